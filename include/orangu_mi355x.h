@@ -412,6 +412,9 @@ int ogm_llama_load_gguf(ogm_ctx *ctx, ogm_gguf *g, uint32_t max_ctx, ogm_llama *
  * "gemm_one_pass", "attn_prefill_variant" and "attn_decode_chunks" can change a result bit; every other
  * setting selects among kernels that produce the same bits.
  *   "gemv_wg_waves"            waves per workgroup of the GEMV kernel, 1..16; 0 = by the row's tile count
+ *   "gemv_prologue"            one-token GEMVs that prepare their own activations (quantizer, or residual add, RMSNorm
+ *                              and quantizer) instead of after a launch that does: 0 by the size of the launch,
+ *                              1 never, 2 whenever the shape allows
  *   "gemm_min_tokens"          ogm_matmul takes a matrix-core GEMM from this many tokens on; 0 = default (6 for
  *                              Q4_K, Q5_K and Q6_K; 9 for Q8_0, Q5_0, Q4_0 and IQ4_NL where their small-batch
  *                              kernel would run, or as soon as the GEMV kernel would need two passes over

@@ -54,6 +54,7 @@ struct ogm_ctx {
   DevBuf hflag;   // pinned word a trailing kernel sets for host_wait
   uint32_t flag_epoch = 0, flag_unsynced = 0;
   int tune_wg_waves = 0;
+  int tune_gemv_prologue = 0;
   // matmul at n_tokens >= this takes the MFMA GEMM; 0 = by type: 9 for Q4_K, Q5_K and Q6_K, whose
   // small-batch kernel beats the GEMV kernel's chunks of 8 tokens from there on (Q4_K 4096 -> 4096 at 9
   // tokens: 12 against 16 us), 17 for the others, whose tiled kernels cost about the same from 9 to 128
@@ -277,6 +278,11 @@ extern "C" int ogm_set_tuning(ogm_ctx *ctx, const char *key, int value) {
   if (strcmp(key, "gemv_wg_waves") == 0) {
     if (value < 0 || value > 16) return fail(ctx, OGM_ERR_INVALID, "gemv_wg_waves must be 0..16");
     ctx->tune_wg_waves = value;
+    return OGM_OK;
+  }
+  if (strcmp(key, "gemv_prologue") == 0) {
+    if (value < 0 || value > 2) return fail(ctx, OGM_ERR_INVALID, "gemv_prologue must be 0, 1 or 2");
+    ctx->tune_gemv_prologue = value;
     return OGM_OK;
   }
   if (strcmp(key, "gemm_min_tokens") == 0) {
@@ -530,13 +536,79 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
                         hipStream_t stream, int32_t *dump_isum, int32_t *dump_imin,
                         const OgmActDev *act_base = nullptr);
 
+// Whether a one-token launch over these matrices (one type and in_dim) prepares its own activations: where the work
+// that every workgroup repeats -- row blocks times runs of 1024 inputs, eight a compute unit at the line -- costs less
+// than the launch it saves.  Measured, whole calls, us, separate / prepared: at 2048 Q4_K 4096 -> 8192 6.9 / 6.3, 2048 ->
+// 2 x 8192 7.1 / 6.4, Q6_K 8.4 / 8.1 and 9.0 / 8.2; above, 11008 -> 4096 (2816) 9.1 / 9.0, 14336 -> 4096 (3584) 9.5 / 9.5,
+// 4096 -> 14336 (3584) 9.0 / 9.4, 8192 -> 8192 (4096) 10.3 / 11.1.  The per-32 types' workgroups have sixteen waves of
+// small tiles and gain less: Q8_0 4096 -> 2048 (512) 6.6 / 6.3, 4096 -> 4096 (1024) 7.1 / 7.6, 8192 -> 2048 (1024) 10.9 / 10.9.
+static const uint32_t OGM_PREPARE_MAX_WORK = 2048, OGM_PREPARE_MAX_WORK_32 = 512;
+static bool gemv_prepares(const ogm_ctx *ctx, const Target *tg, size_t n_tg, bool norm, bool swiglu) {
+  if (ctx->tune_gemv_prologue == 1 || n_tg == 0 || n_tg > OGM_GEMV_MAX_MATS) return false;
+  const uint32_t type = tg[0].w->ggml_type, in_dim = tg[0].w->in_dim;
+  uint32_t rb = 0;
+  for (size_t i = 0; i < n_tg; i++) rb += ogm_gemv_row_blocks(type, in_dim, tg[i].w->out_dim);
+  if (rb == 0 || !ogm_gemv_fused_can(type, in_dim, rb, norm, swiglu, (uint32_t)ctx->tune_wg_waves)) return false;
+  if (ctx->tune_gemv_prologue == 2) return true;
+  return (uint64_t)rb * ((in_dim + 1023u) / 1024u) <= (block_elems_of(type) == 256 ? OGM_PREPARE_MAX_WORK : OGM_PREPARE_MAX_WORK_32);
+}
+
+// Enqueues that launch; the quantized row also ends in the context's scratch.  The scratch is large enough.
+static int enqueue_prepared(ogm_ctx *ctx, const Target *tg, size_t n_tg, const OgmGemvSrc &src, hipStream_t stream) {
+  OgmGemvArgs a;
+  const ogm_weight *w0 = tg[0].w;
+  a.ggml_type = w0->ggml_type;
+  a.wt = w0->dev;
+  a.in_dim = w0->in_dim;
+  a.out_dim = w0->out_dim;
+  a.act = act_view(ctx, w0->in_dim, act_mode_for(w0->ggml_type), 0);
+  a.n_tokens = 1;
+  a.y = tg[0].y;
+  a.gemm_order = 0;
+  a.wg_waves = (uint32_t)ctx->tune_wg_waves;
+  a.dump_isum = a.dump_imin = nullptr;
+  a.n_extra = (uint32_t)n_tg - 1;
+  for (size_t i = 1; i < n_tg; i++) {
+    a.extra_wt[i - 1] = tg[i].w->dev;
+    a.extra_out_dim[i - 1] = tg[i].w->out_dim;
+    a.extra_y[i - 1] = tg[i].y;
+  }
+  HIPCHK(ctx, ogm_launch_gemv_fused(a, src, stream, &ctx->last_kernel));
+  return OGM_OK;
+}
+
+// Whether any output shares memory with the input row.  A launch that prepares its own activations reads x while it
+// writes y; with a quantizer launch before it an output may lie over x.
+static bool outputs_overlap(const Target *tg, size_t n_tg, const float *x, uint32_t in_dim) {
+  const uintptr_t x0 = (uintptr_t)x, x1 = x0 + (size_t)in_dim * 4;
+  for (size_t i = 0; i < n_tg; i++) {
+    const uintptr_t y0 = (uintptr_t)tg[i].y, y1 = y0 + (size_t)tg[i].w->out_dim * 4;
+    if (y0 < x1 && x0 < y1) return true;
+  }
+  return false;
+}
+
 // Enqueues quantize + kernels for tokens of x_dev into the targets' outputs.  Caller holds the
 // lock and has checked that the targets share type and in_dim.
+// x_in_host_memory: x lies behind the bus, where it is read once and not by every workgroup.
 static int enqueue_matmul(ogm_ctx *ctx, const Target *tg, size_t n_tg, const float *x_dev,
                           uint32_t n_tokens, int decode, hipStream_t stream, int32_t *dump_isum,
-                          int32_t *dump_imin) {
+                          int32_t *dump_imin, bool x_in_host_memory = false) {
   if (n_tokens == 0 || n_tg == 0) return OGM_OK;
   const ogm_weight *w = tg[0].w;
+  if (n_tokens == 1 && !dump_isum && !dump_imin && !x_in_host_memory && gemv_prepares(ctx, tg, n_tg, false, false) &&
+      !outputs_overlap(tg, n_tg, x_dev, w->in_dim)) {
+    int rc = ensure_act(ctx, w->in_dim, 1);
+    if (rc != OGM_OK) return rc;
+    OgmGemvSrc src;
+    src.x = x_dev;
+    if ((rc = enqueue_prepared(ctx, tg, n_tg, src, stream)) != OGM_OK) return rc;
+    ctx->act_mode = act_mode_for(w->ggml_type, 1, decode);   // as after a quantizer launch
+    ctx->act_in_dim = w->in_dim;
+    ctx->act_tokens = 1;
+    ctx->act_xt = false;
+    return OGM_OK;
+  }
   // A batch that may go to a matrix-core GEMM of the K-quants has its activations laid out in that kernel's
   // operand chunks by the quantizer itself (from 25 tokens: below, the small-batch kernel's loads gather few enough
   // distinct rows that the plain quantizer's shorter launch decides: 4096 -> 4096 at 24 tokens 11.5 us from rows,
@@ -549,9 +621,9 @@ static int enqueue_matmul(ogm_ctx *ctx, const Target *tg, size_t n_tg, const flo
 
 static int enqueue_matmul(ogm_ctx *ctx, const ogm_weight *w, const float *x_dev, uint32_t n_tokens,
                           float *y_dev, int decode, hipStream_t stream, int32_t *dump_isum,
-                          int32_t *dump_imin) {
+                          int32_t *dump_imin, bool x_in_host_memory = false) {
   const Target t{w, y_dev};
-  return enqueue_matmul(ctx, &t, 1, x_dev, n_tokens, decode, stream, dump_isum, dump_imin);
+  return enqueue_matmul(ctx, &t, 1, x_dev, n_tokens, decode, stream, dump_isum, dump_imin, x_in_host_memory);
 }
 
 // Builds the prefill planes of a K-quant matrix on first use, within the context's budget.  Returns
@@ -855,7 +927,7 @@ static int host_matmul(ogm_ctx *ctx, const ogm_weight *w, const float *x, uint32
     // a decode-sized call: the kernels read x from, and write y to, the pinned staging buffers over
     // the bus themselves; two copy-engine transfers and their latencies fall away
     rc = enqueue_matmul(ctx, w, (const float *)ctx->hx.p, n_tokens, (float *)ctx->hy.p, decode, ctx->stream,
-                        nullptr, nullptr);
+                        nullptr, nullptr, true);
     if (rc != OGM_OK) return rc;
   } else {
     if ((rc = ensure_dev(ctx, ctx->x, xb)) != OGM_OK) return rc;
@@ -1175,7 +1247,7 @@ extern "C" int ogm_matmul_batch(ogm_ctx *ctx, const ogm_op *ops, size_t n_ops, i
       for (size_t k = i; k < e; k++)
         tg.push_back(Target{ops[k].w, (float *)(y_base + yoff[k]) + (size_t)t0 * ops[k].w->out_dim});
       rc = enqueue_matmul(ctx, tg.data(), tg.size(), xd + (size_t)t0 * op.w->in_dim, nt, decode,
-                          ctx->stream, nullptr, nullptr);
+                          ctx->stream, nullptr, nullptr, zc);
       if (rc != OGM_OK) return rc;
     }
     i = e;
@@ -1310,6 +1382,7 @@ struct ogm_llama {
   void *k_cache = nullptr;    // f16 [n_layer][max_ctx][kv_dim]
   void *v_cache = nullptr;
   float *x = nullptr;         // hidden state [n_embd]
+  float *x2 = nullptr;        // the residual stream's second place: a launch that reads it in every workgroup stores its sum here
   float *q = nullptr, *k = nullptr, *v = nullptr;  // projections
   float *proj = nullptr;      // wo / down output [n_embd]
   float *gate = nullptr, *up = nullptr;            // [n_ff]
@@ -1412,6 +1485,7 @@ extern "C" int ogm_llama_create(ogm_ctx *ctx, const ogm_llama_config *cfg, const
   A(&m->k_cache, cache_bytes);
   A(&m->v_cache, cache_bytes);
   A((void **)&m->x, (size_t)c.n_embd * 4);
+  A((void **)&m->x2, (size_t)c.n_embd * 4);
   A((void **)&m->q, (size_t)qd * 4);
   A((void **)&m->k, (size_t)kvd * 4);
   A((void **)&m->v, (size_t)kvd * 4);
@@ -1575,8 +1649,59 @@ static int llama_matmul(ogm_ctx *ctx, const ogm_weight *const *ws, float *const 
   return OGM_OK;
 }
 
-// LlamaModel::run_layers + forward at one token (arch/llama.rs:594-932, 1007-1032), eight launches a layer:
-// norm (+ quantize), q/k/v, attention (+ quantize), wo, norm (+ quantize), gate/up, SwiGLU (+ quantize), down.
+// The residual stream of a decode step: where it is, and what the next norm adds to it first.
+struct DecodeRow {
+  float *x, *spare;           // the stream, and the model's other buffer for it
+  const float *first;         // the caller's row while no norm has stored it to x (null afterwards)
+  const float *delta;         // the last block's output, null before the first
+};
+
+// Norm + quantize + matmuls of one group of a decode step.  The group's first launch prepares the normed row itself
+// where that pays (then its workgroup 0 leaves the quantized row for the others and the new residual stream in the
+// other buffer); else the norm has a launch of its own.  swiglu: the group is gate and up; *did_swiglu says whether
+// ys[0] now holds silu(gate) * up.
+static int llama_norm_matmul(ogm_ctx *ctx, ogm_llama *m, DecodeRow &row, const float *norm_w, const ogm_weight *const *ws,
+                             float *const *ys, size_t n, uint32_t site, hipStream_t s, bool *did_swiglu = nullptr) {
+  const ogm_llama_config &c = m->cfg;
+  const int mode = act_mode_for(ws[0]->ggml_type);
+  Target tg[OGM_GEMV_MAX_MATS];
+  size_t e = 0;
+  while (e < n && e < OGM_GEMV_MAX_MATS && ws[e]->ggml_type == ws[0]->ggml_type) {
+    tg[e] = Target{ws[e], ys[e]};
+    e++;
+  }
+  int rc;
+  const bool swiglu = did_swiglu && e == 2 && n == 2 && ws[0]->out_dim == ws[1]->out_dim && gemv_prepares(ctx, tg, e, true, true);
+  if (did_swiglu) *did_swiglu = swiglu;
+  if (swiglu || gemv_prepares(ctx, tg, e, true, false)) {
+    OgmGemvSrc src;
+    src.x = row.first ? row.first : row.x;
+    src.delta = row.delta;
+    src.weight = norm_w;
+    src.eps = c.rms_eps;
+    src.swiglu = swiglu;
+    if (row.delta) {
+      src.x_out = row.spare;
+      row.spare = row.x;
+      row.x = src.x_out;
+    } else if (row.first) {
+      src.x_out = row.x;
+    }
+    if ((rc = enqueue_prepared(ctx, tg, e, src, s)) != OGM_OK) return rc;
+    if (e < n && (rc = llama_matmul(ctx, ws + e, ys + e, n - e, s)) != OGM_OK) return rc;
+  } else {
+    HIPCHK(ctx, ogm_launch_norm_quant(mode, row.x, row.delta, norm_w, c.n_embd, c.rms_eps, nullptr,
+                                      act_view(ctx, c.n_embd, mode, 0), s, 1, row.first));
+    if ((rc = llama_matmul(ctx, ws, ys, n, s)) != OGM_OK) return rc;
+  }
+  row.first = nullptr;
+  row.delta = nullptr;
+  return llama_capture(ctx, m, site, c.n_embd, mode, s);
+}
+
+// LlamaModel::run_layers + forward at one token (arch/llama.rs:594-932, 1007-1032), five to eight launches a layer:
+// [norm (+ quantize)] q/k/v, attention (+ quantize), wo, [norm (+ quantize)] gate/up [SwiGLU], [SwiGLU (+ quantize)]
+// down; the bracketed parts are inside the matmul launches beside them where gemv_prepares says so.
 static int llama_decode_enqueue(ogm_ctx *ctx, ogm_llama *m, const float *x_dev, uint32_t pos, float *logits_dev,
                                 uint32_t *argmax_dev, hipStream_t s) {
   const ogm_llama_config &c = m->cfg;
@@ -1586,9 +1711,8 @@ static int llama_decode_enqueue(ogm_ctx *ctx, ogm_llama *m, const float *x_dev, 
   // (the table of this position: from the one made at creation, or computed now)
   const float *rope_cs = m->rope_all ? m->rope_all + (size_t)pos * (c.rope_dim / 2) * 2 : m->rope_cs;
   if (!m->rope_all) HIPCHK(ctx, ogm_launch_rope_table(m->freq, pos, 1, c.rope_dim, m->rope_cs, s));
-  const float *delta = nullptr;  // what the next norm adds to x first: the last block's output
   // The caller's row becomes the residual stream: the first norm reads it where it lies and stores it to m->x.
-  const float *x_first = x_dev != m->x ? x_dev : nullptr;
+  DecodeRow row{m->x, m->x2, x_dev != m->x ? x_dev : nullptr, nullptr};
   const int mode_out = act_mode_for(m->output->ggml_type);
   const float *out_norm = m->norms + (size_t)c.n_layer * 2 * c.n_embd;
   int rc;
@@ -1602,40 +1726,46 @@ static int llama_decode_enqueue(ogm_ctx *ctx, ogm_llama *m, const float *x_dev, 
     const int mode_qkv = act_mode_for(L.wq->ggml_type);
     if (act_mode_for(L.wk->ggml_type) != mode_qkv || act_mode_for(L.wv->ggml_type) != mode_qkv)
       return fail(ctx, OGM_ERR_UNSUPPORTED, "wq, wk and wv must share an activation mode");
+    const int mode_ff = act_mode_for(L.w_gate->ggml_type);
+    if (act_mode_for(L.w_up->ggml_type) != mode_ff)
+      return fail(ctx, OGM_ERR_UNSUPPORTED, "w_gate and w_up must share an activation mode");
     const ogm_weight *w3[3] = {L.wq, L.wk, L.wv};
     float *y3[3] = {m->q, m->k, m->v};
-    HIPCHK(ctx, ogm_launch_norm_quant(mode_qkv, m->x, delta, attn_norm, c.n_embd, c.rms_eps, nullptr,
-                                      act_view(ctx, c.n_embd, mode_qkv, 0), s, 1, l == 0 ? x_first : nullptr));
-    if ((rc = llama_capture(ctx, m, 4 * l, c.n_embd, mode_qkv, s)) != OGM_OK) return rc;
-    if ((rc = llama_matmul(ctx, w3, y3, 3, s)) != OGM_OK) return rc;
+    if ((rc = llama_norm_matmul(ctx, m, row, attn_norm, w3, y3, 3, 4 * l, s)) != OGM_OK) return rc;
     const int mode_o = act_mode_for(L.wo->ggml_type);
     const OgmAttnPre pre{L.q_bias, L.k_bias, L.v_bias, L.q_norm, L.k_norm, c.rms_eps, c.rope_neox};
     HIPCHK(ctx, ogm_launch_attn_decode(m->q, m->k, m->v, rope_cs, c.rope_dim, pre, kc, vc, pos, m->max_splits,
                                        c.n_head, c.n_head_kv, c.head_dim, scale, m->part_o, m->part_ml,
                                        m->attn_counters, mode_o, nullptr, act_view(ctx, qd, mode_o, 0), s, 0u,
                                        (uint32_t)ctx->tune_attn_decode_chunks));
-    const int mode_ff = act_mode_for(L.w_gate->ggml_type);
-    if (act_mode_for(L.w_up->ggml_type) != mode_ff)
-      return fail(ctx, OGM_ERR_UNSUPPORTED, "w_gate and w_up must share an activation mode");
     const ogm_weight *w1[1] = {L.wo};
     float *y1[1] = {m->proj};
     if ((rc = llama_capture(ctx, m, 4 * l + 1, qd, mode_o, s)) != OGM_OK) return rc;
     if ((rc = llama_matmul(ctx, w1, y1, 1, s)) != OGM_OK) return rc;
-    HIPCHK(ctx, ogm_launch_norm_quant(mode_ff, m->x, m->proj, ffn_norm, c.n_embd, c.rms_eps, nullptr,
-                                      act_view(ctx, c.n_embd, mode_ff, 0), s));
+    row.delta = m->proj;
     const ogm_weight *w2[2] = {L.w_gate, L.w_up};
     float *y2[2] = {m->gate, m->up};
+    bool h_ready = false;   // m->gate holds silu(gate) * up
+    if ((rc = llama_norm_matmul(ctx, m, row, ffn_norm, w2, y2, 2, 4 * l + 2, s, &h_ready)) != OGM_OK) return rc;
     const int mode_d = act_mode_for(L.w_down->ggml_type);
-    if ((rc = llama_capture(ctx, m, 4 * l + 2, c.n_embd, mode_ff, s)) != OGM_OK) return rc;
-    if ((rc = llama_matmul(ctx, w2, y2, 2, s)) != OGM_OK) return rc;
-    HIPCHK(ctx, ogm_launch_swiglu_quant(mode_d, m->gate, m->up, c.n_ff, nullptr, act_view(ctx, c.n_ff, mode_d, 0), s));
     const ogm_weight *wd[1] = {L.w_down};
+    const Target td{L.w_down, m->proj};
+    if (h_ready && gemv_prepares(ctx, &td, 1, false, false)) {
+      OgmGemvSrc src;
+      src.x = m->gate;
+      if ((rc = enqueue_prepared(ctx, &td, 1, src, s)) != OGM_OK) return rc;
+    } else {
+      const OgmActDev act = act_view(ctx, c.n_ff, mode_d, 0);
+      if (h_ready) HIPCHK(ctx, ogm_launch_quantize(mode_d, m->gate, c.n_ff, 1, act, s));
+      else HIPCHK(ctx, ogm_launch_swiglu_quant(mode_d, m->gate, m->up, c.n_ff, nullptr, act, s));
+      if ((rc = llama_matmul(ctx, wd, y1, 1, s)) != OGM_OK) return rc;
+    }
     if ((rc = llama_capture(ctx, m, 4 * l + 3, c.n_ff, mode_d, s)) != OGM_OK) return rc;
-    if ((rc = llama_matmul(ctx, wd, y1, 1, s)) != OGM_OK) return rc;
-    delta = m->proj;
+    row.delta = m->proj;
   }
-  HIPCHK(ctx, ogm_launch_norm_quant(mode_out, m->x, delta, out_norm, c.n_embd, c.rms_eps, nullptr,
-                                    act_view(ctx, c.n_embd, mode_out, 0), s));
+  // (the sum ends in m->x, whichever buffer the stream is in)
+  HIPCHK(ctx, ogm_launch_norm_quant(mode_out, m->x, row.delta, out_norm, c.n_embd, c.rms_eps, nullptr,
+                                    act_view(ctx, c.n_embd, mode_out, 0), s, 1, row.first ? row.first : row.x != m->x ? row.x : nullptr));
   float *lg = logits_dev ? logits_dev : m->logits;
   const ogm_weight *wo_[1] = {m->output};
   float *yo[1] = {lg};

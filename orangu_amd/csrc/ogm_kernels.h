@@ -52,6 +52,22 @@ struct OgmGemvArgs {
 // Largest token count one launch can take for this shape (LDS budget), at least 1.
 uint32_t ogm_gemv_max_tokens(uint32_t ggml_type, uint32_t in_dim, int gemm_order);
 hipError_t ogm_launch_gemv(const OgmGemvArgs &a, hipStream_t stream, const char **kernel_name);
+
+// One token whose activations the GEMV prepares itself (ogm_gemv_fused_kernel): what it reads in place of a quantized row.
+struct OgmGemvSrc {
+  const float *x = nullptr;        // the row to quantize; with `weight`, the residual stream
+  const float *delta = nullptr;    // with `weight`: added to x first
+  const float *weight = nullptr;   // RMSNorm weights (null: x is quantized as it is)
+  float *x_out = nullptr;          // with `weight`: where x + delta goes; not x itself
+  float eps = 0.0f;
+  bool swiglu = false;             // the two matrices are gate and up: y gets silu(gate) * up, extra_y is not written
+};
+// Row blocks (workgroups of the plain GEMV) of a matrix.
+uint32_t ogm_gemv_row_blocks(uint32_t ggml_type, uint32_t in_dim, uint32_t out_dim);
+// Whether the launch can prepare its own activations at this shape.
+bool ogm_gemv_fused_can(uint32_t ggml_type, uint32_t in_dim, uint32_t n_row_blocks, bool norm, bool swiglu, uint32_t wg_waves);
+// a.act: where workgroup 0 leaves the quantized row, as ogm_launch_quantize would.
+hipError_t ogm_launch_gemv_fused(const OgmGemvArgs &a, const OgmGemvSrc &src, hipStream_t stream, const char **kernel_name);
 // Prefill GEMM on MFMA (ogm_gemm.hip).  Same operands as the GEMV plus a scratch buffer `xh` of
 // ogm_gemm_xh_bytes() for the int8 activations in operand chunks.  Follows the CPU path's GEMM float order.
 #define OGM_GEMM_MAX_MATS 3   // matrices one GEMM launch can take (q, k, v)

@@ -1166,6 +1166,228 @@ __global__ __launch_bounds__((SINGLE && !DUMP) ? F::MAX_THREADS_SINGLE : F::MAX_
 }
 
 // ------------------------------------------------------------------------------------------
+// one token, the activations prepared inside the GEMV
+//
+// A decode step's small launches are latency: a quantizer or norm launch of its own takes 2.5 to 4.5 us, and the
+// arithmetic in it a tenth of that.  Here every
+// workgroup prepares the whole row itself -- from x (PRE 1), or from the residual stream through the residual add and
+// RMSNorm (PRE 2) -- while its first tile of weights is in flight, and keeps it in LDS; workgroup 0 also stores what the
+// separate launch would have (the quantized row, the new residual stream), so the scratch holds the same bytes
+// afterwards.  What it costs is the row's preparation once per workgroup: a lane takes sixteen elements in a row (the
+// per-16 sums stay in the lane, a wave's reductions serve four runs of 256 at once, one 16-byte LDS store holds the
+// result), and `teams` row blocks share one workgroup on launches of many row blocks (each team of waves takes a row
+// block, as a workgroup of ogm_gemv_kernel does).
+// SWIGLU: the launch is gate and up (two teams, the same row block of each); the epilogue leaves silu(gate) * up.
+struct GemvFusedParams {
+  GemvParams g;
+  const float *x;        // the row (PRE 1), the residual stream (PRE 2)
+  const float *delta;    // PRE 2: added to x first; may be null
+  const float *weight;   // PRE 2: the norm's weights
+  float *x_out;          // PRE 2: where x + delta goes, never x itself (other workgroups still read that); may be null
+  float eps;
+  uint32_t teams, team_waves;
+};
+
+// NQ: runs of 1024 elements a wave prepares.
+template <class F, int UPR, int PRE, int NQ, bool SWIGLU>
+__global__ __launch_bounds__(F::ELEMS == 32 ? 1024 : 512) void ogm_gemv_fused_kernel(GemvFusedParams fp) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  const GemvParams &p = fp.g;
+  constexpr int GROUP = F::ACT_GROUP;
+  const uint32_t tid = threadIdx.x, nthr = blockDim.x;
+  const uint32_t lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n_wave = nthr >> 6;
+  const uint32_t tw = fp.team_waves, teams = SWIGLU ? 2u : fp.teams;
+  const uint32_t upr = UPR ? (uint32_t)UPR : p.upr;
+  const uint32_t C = UPR ? ((UPR % 4 == 0) ? 4u : ((UPR % 2 == 0) ? 2u : 1u)) : p.C;
+  const uint32_t R = 64u / C, nct = UPR ? upr / C : p.nct;
+  const uint32_t xch = upr * F::XPIECES;
+  const uint32_t n = upr * F::ELEMS;
+  const uint32_t n_scale = upr * (F::ELEMS / F::ACT_GROUP);
+  const uint32_t term_stride = upr * R;
+
+  uint4 *l_xq = (uint4 *)lds;                          // as ogm_gemv_kernel at one token
+  uint4 *l_aux = l_xq + xch;
+  float *l_d = (float *)(l_aux + upr * F::AUX16);
+  const uint32_t head = (xch * 16 + upr * F::AUX16 * 16 + n_scale * 4 + 15) & ~15u;
+  float *l_term = (float *)(lds + head);               // [teams][upr][R]
+  float *l_red = l_term + (size_t)teams * term_stride; // PRE 2: a run of 256's sum of squares each
+
+  // ---- this wave's team and its row block (a team past the last one multiplies the last again and stores nothing)
+  const uint32_t team = teams == 1u ? 0u : wave / tw, wv = wave - team * tw;
+  auto locate = [&](uint32_t team_, uint32_t &m, uint32_t &rb) -> bool {
+    if (SWIGLU) {
+      m = team_;
+      rb = blockIdx.x;
+      return true;
+    }
+    const uint32_t last = p.wg_end[OGM_GEMV_MAX_MATS - 1] - 1u, want = blockIdx.x * teams + team_;
+    const uint32_t b = min(want, last);
+    m = (b >= p.wg_end[0] ? 1u : 0u) + (b >= p.wg_end[1] ? 1u : 0u) + (b >= p.wg_end[2] ? 1u : 0u);
+    rb = b - (m == 0 ? 0u : m == 1 ? p.wg_end[0] : m == 2 ? p.wg_end[1] : p.wg_end[2]);
+    return want <= last;
+  };
+  uint32_t m, rb0;
+  locate(team, m, rb0);
+  const uint8_t *wt = m == 0 ? p.wt[0] : m == 1 ? p.wt[1] : m == 2 ? p.wt[2] : p.wt[3];
+  const size_t tile0 = (size_t)rb0 * nct;
+
+  // ---- the row's loads, ahead of every weight load of the workgroup (as in ogm_gemv_kernel)
+  float4 v[NQ][4], dl[PRE == 2 ? 4 : 1], wv4[PRE == 2 ? 4 : 1];
+  static_assert(PRE == 1 || NQ == 1, "a norm's wave prepares one run of 1024");
+#pragma unroll
+  for (int k = 0; k < NQ; k++) {
+    const uint32_t e0 = min((wave + (uint32_t)k * n_wave) * 1024u + lane * 16u, n - 16u);
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[k][i] = *(const float4 *)(fp.x + e0 + 4 * i);
+    if (PRE == 2) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) wv4[i] = *(const float4 *)(fp.weight + e0 + 4 * i);
+      const float *dsrc = fp.delta ? fp.delta : fp.x;   // (no branch around the loads: the compiler counts them)
+#pragma unroll
+      for (int i = 0; i < 4; i++) dl[i] = *(const float4 *)(dsrc + e0 + 4 * i);
+    }
+  }
+  __syncthreads();
+  const uint32_t r_local = lane & (R - 1), c_local = lane / R;
+  uint32_t it = wv;   // tw <= nct
+  typename F::Regs cur;
+  F::load(cur, wt, tile0 + it, lane);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- prepare the row while they are in flight
+  if constexpr (PRE == 2) {
+    // ogm_norm_quant_row's arithmetic: the squares of four elements, a butterfly over the run (its first two levels
+    // are in this lane), the runs in ascending order -- the same bits
+    const uint32_t e0 = wave * 1024u + lane * 16u;
+    const bool active = e0 < n;
+    float ss4[4];
+    if (fp.delta) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        float4 &a = v[0][i];
+        a.x += dl[i].x; a.y += dl[i].y; a.z += dl[i].z; a.w += dl[i].w;
+      }
+    }
+    if (blockIdx.x == 0 && fp.x_out && active) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) *(float4 *)(fp.x_out + e0 + 4 * i) = v[0][i];
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float4 &a = v[0][i];
+      ss4[i] = a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w;
+    }
+    float ss = active ? (ss4[0] + ss4[1]) + (ss4[2] + ss4[3]) : 0.0f;
+    ss = ogm_butterfly_step<1>(ss, OgmOpAdd());
+    ss = ogm_butterfly_step<2>(ss, OgmOpAdd());
+    ss = ogm_butterfly_step<4>(ss, OgmOpAdd());
+    ss = ogm_butterfly_step<8>(ss, OgmOpAdd());
+    if ((lane & 15u) == 0 && active) l_red[e0 >> 8] = ss;
+    __syncthreads();
+    float total = 0.0f;
+    for (uint32_t r = 0; r * 256u < n; r++) total += l_red[r];
+    const float mean_sq = total / (float)n;
+    const float scale = 1.0f / sqrtf(mean_sq + fp.eps);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      float4 &a = v[0][i];
+      a.x = a.x * scale * wv4[i].x; a.y = a.y * scale * wv4[i].y;
+      a.z = a.z * scale * wv4[i].z; a.w = a.w * scale * wv4[i].w;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NQ; k++) {
+    if ((wave + (uint32_t)k * n_wave) * 1024u >= n) continue;   // wave-uniform
+    const uint32_t e0 = (wave + (uint32_t)k * n_wave) * 1024u + lane * 16u;
+    const bool active = e0 < n;   // (a group of 32 or 256 is wholly active or wholly not)
+    float am[4];   // (four short chains: a lone wave pays every dependent instruction's latency)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      am[i] = ogm_nan_blind_max(0.0f, fabsf(v[k][i].x));
+      am[i] = ogm_nan_blind_max(am[i], fabsf(v[k][i].y));
+      am[i] = ogm_nan_blind_max(am[i], fabsf(v[k][i].z));
+      am[i] = ogm_nan_blind_max(am[i], fabsf(v[k][i].w));
+    }
+    float amax = ogm_nan_blind_max(ogm_nan_blind_max(am[0], am[1]), ogm_nan_blind_max(am[2], am[3]));
+    amax = ogm_butterfly_step<1>(amax, OgmOpNanBlindMax());
+    if constexpr (GROUP == 256) {
+      amax = ogm_butterfly_step<2>(amax, OgmOpNanBlindMax());
+      amax = ogm_butterfly_step<4>(amax, OgmOpNanBlindMax());
+      amax = ogm_butterfly_step<8>(amax, OgmOpNanBlindMax());
+    }
+    const float scale = amax / 127.0f;
+    const float inv = scale > 0.0f ? 1.0f / scale : 0.0f;
+    uint32_t pk[4];
+    int s16 = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float4 &a = v[k][i];
+      pk[i] = ogm_pack4(ogm_quantize_one(a.x, inv), ogm_quantize_one(a.y, inv), ogm_quantize_one(a.z, inv),
+                        ogm_quantize_one(a.w, inv));
+      s16 = dot4(pk[i], 0x01010101u, s16);
+    }
+    const int s32 = ogm_butterfly_add_i32<1>(s16);
+    const uint4 q16 = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+    if (active) {
+      const uint32_t ch = e0 / 16u, col = ch / F::XPIECES, c = ch - col * F::XPIECES;
+      l_xq[c * upr + col] = q16;
+      if (F::AUX16 == 1 && (lane & 1u) == 0) ((int16_t *)(l_aux + col))[c >> 1] = (int16_t)s32;
+      if (F::AUX16 == 2) ((int16_t *)(l_aux + (c >> 3) * upr + col))[c & 7u] = (int16_t)s16;
+      if ((lane & (GROUP / 16 - 1)) == 0) l_d[e0 / GROUP] = scale;
+      if (blockIdx.x == 0) {   // the scratch, as the quantizer's own launch leaves it
+        *(uint4 *)(p.act.q + e0) = q16;
+        p.act.sums[e0 / 16u] = s16;
+        if ((lane & 1u) == 0) {
+          p.act.bsum[e0 / 32u] = (int16_t)s32;
+          if (GROUP == 256 && p.act.bs16 != nullptr) {
+            uint16_t *b = p.act.bs16 + (e0 / 256u) * 16u + ((e0 / 32u) & 7u);
+            b[0] = __half_as_ushort(__float2half_rn((float)(s32 >> 6)));
+            b[8] = __half_as_ushort(__float2half_rn((float)(s32 & 63)));
+          }
+        }
+        if ((lane & (GROUP / 16 - 1)) == 0) p.act.d[e0 / GROUP] = scale;
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- tiles of this wave, as ogm_gemv_kernel at one token in GEMV order
+  ActLds a;
+  a.xq = l_xq;
+  a.aux = l_aux;
+  a.d = l_d;
+  a.upr = upr;
+  float *my_term = l_term + (size_t)team * term_stride;
+  for (; it < nct; it += tw) {
+    const uint32_t col_own = it * C + c_local;
+    const bool live = col_own < upr;
+    const uint32_t col = live ? col_own : upr - 1u;
+    int isum, imin;
+    F::template sums<UPR>(cur, a, col, isum, imin);
+    if (live) my_term[col * R + r_local] = F::term_gemv(cur, a.d[col], isum, imin);
+    if (it + tw < nct) F::load(cur, wt, tile0 + it + tw, lane);
+  }
+  __syncthreads();
+
+  for (uint32_t i = tid; i < teams * R; i += nthr) {
+    const uint32_t t = i / R, r = i - t * R;
+    uint32_t om, orb;
+    const bool mine = locate(t, om, orb);
+    const uint32_t out_dim = om == 0 ? p.out_dim[0] : om == 1 ? p.out_dim[1] : om == 2 ? p.out_dim[2] : p.out_dim[3];
+    const uint32_t orow = orb * R + r;
+    const bool store = mine && orow < out_dim;
+    const float acc = store ? ordered_sum<false>(0.0f, l_term + (size_t)t * term_stride + r, upr, R) : 0.0f;
+    if constexpr (SWIGLU) {   // R <= 32: gate and up of a row are in one wave, and so are all 2 R lanes of this pass
+      const float up = __shfl(acc, (int)((lane + R) & 63u));
+      if (store && t == 0) p.y[0][orow] = acc / (1.0f + expf(-acc)) * up;
+    } else {
+      float *y = om == 0 ? p.y[0] : om == 1 ? p.y[1] : om == 2 ? p.y[2] : p.y[3];
+      if (store) y[orow] = acc;
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------
 // host side of the launch
 
 
@@ -1360,6 +1582,137 @@ hipError_t ogm_launch_gemv(const OgmGemvArgs &a, hipStream_t stream, const char 
     default:
       return hipErrorInvalidValue;
   }
+}
+
+// The one-token GEMV's name for each type (ogm_last_kernel), whichever of its two kernels runs.
+static const char *gemv_name(uint32_t ggml_type) {
+  switch (ggml_type) {
+    case OGM_Q4_K: return "ogm_gemv_kernel<FmtQ4K,gemv>";
+    case OGM_Q5_K: return "ogm_gemv_kernel<FmtQ5K,gemv>";
+    case OGM_Q3_K: return "ogm_gemv_kernel<FmtQ3K,gemv>";
+    case OGM_Q6_K: return "ogm_gemv_kernel<FmtQ6K,gemv>";
+    case OGM_Q8_0: return "ogm_gemv_kernel<FmtQ80,gemv>";
+    case OGM_Q4_0: return "ogm_gemv_kernel<FmtQ40,gemv>";
+    case OGM_Q5_0: return "ogm_gemv_kernel<FmtQ50,gemv>";
+    case OGM_IQ4_NL: return "ogm_gemv_kernel<FmtIQ4NL,gemv>";
+    case OGM_Q5_1: return "ogm_gemv_kernel<FmtQ51,gemv>";
+    case OGM_IQ4_XS: return "ogm_gemv_kernel<FmtIQ4XS,gemv>";
+    default: return "ogm_gemv_kernel<FmtQ2K,gemv>";
+  }
+}
+
+// How a fused launch of this shape is cut: waves a team, teams a workgroup, runs of 1024 a wave prepares (0: it can't).
+struct FusedShape {
+  uint32_t team_waves, teams, nq;
+  size_t lds;
+};
+template <class F>
+static FusedShape fused_shape(uint32_t in_dim, uint32_t n_row_blocks, bool norm, bool swiglu, uint32_t wg_waves) {
+  FusedShape f = {0, 0, 0, 0};
+  const uint32_t upr = in_dim / F::ELEMS;
+  const OgmTiling tl = ogm_tiling_for(upr, 1);
+  const uint32_t max_waves = F::ELEMS == 32 ? 16u : 8u;
+  f.team_waves = pick_waves(tl.nct, wg_waves, (int)max_waves * 64, max_waves);
+  // two row blocks a workgroup where the launch has several workgroups a compute unit and the waves fit
+  f.teams = swiglu ? 2u : (n_row_blocks > 512u && 2u * f.team_waves <= max_waves) ? 2u : 1u;
+  if (swiglu && (2u * f.team_waves > max_waves || tl.R > 32u)) return f;
+  const uint32_t runs = (in_dim + 1023u) / 1024u, waves = f.team_waves * f.teams;
+  f.lds = gemv_lds_bytes<F, false>(in_dim, 1) + (size_t)(f.teams - 1u) * upr * tl.R * 4u + (norm ? (in_dim + 255u) / 256u * 4u : 0u);
+  if (f.lds > OGM_LDS_UNASKED) return f;
+  const uint32_t nq = (runs + waves - 1u) / waves;
+  f.nq = nq <= (norm ? 1u : 2u) ? nq : 0u;
+  return f;
+}
+
+template <class F>
+static hipError_t launch_fused_t(const OgmGemvArgs &a, const OgmGemvSrc &src, hipStream_t stream) {
+  GemvFusedParams fp;
+  GemvParams &p = fp.g;
+  p.act = a.act;
+  p.dump_isum = p.dump_imin = nullptr;
+  p.in_dim = a.in_dim;
+  p.upr = a.in_dim / F::ELEMS;
+  p.n_tokens = 1;
+  p.lane_acc = 0;
+  const OgmTiling tl = ogm_tiling_for(p.upr, a.out_dim);
+  p.C = tl.C;
+  p.nct = tl.nct;
+  uint32_t n_rb = 0;
+  for (uint32_t m = 0; m < OGM_GEMV_MAX_MATS; m++) {
+    const bool has = m <= a.n_extra;
+    p.wt[m] = !has ? nullptr : m ? a.extra_wt[m - 1] : a.wt;
+    p.y[m] = !has ? nullptr : m ? a.extra_y[m - 1] : a.y;
+    p.out_dim[m] = !has ? 0u : m ? a.extra_out_dim[m - 1] : a.out_dim;
+    n_rb += (p.out_dim[m] + tl.R - 1) / tl.R;
+    p.wg_end[m] = n_rb;
+  }
+  if (n_rb == 0) return hipSuccess;
+  const bool norm = src.weight != nullptr;
+  const FusedShape f = fused_shape<F>(a.in_dim, n_rb, norm, src.swiglu, a.wg_waves);
+  if (f.nq == 0) return hipErrorInvalidValue;
+  if (src.swiglu && (a.n_extra != 1 || a.extra_out_dim[0] != a.out_dim || !norm)) return hipErrorInvalidValue;
+  fp.x = src.x;
+  fp.delta = src.delta;
+  fp.weight = src.weight;
+  fp.x_out = src.x_out;
+  fp.eps = src.eps;
+  fp.teams = f.teams;
+  fp.team_waves = f.team_waves;
+  const dim3 g(src.swiglu ? p.wg_end[0] : (n_rb + f.teams - 1u) / f.teams), b(f.team_waves * f.teams * 64u);
+  constexpr bool K = F::ELEMS == 256;
+  constexpr int HOT = K ? 16 : 128;   // rows of 4096
+#define OGM_FUSED(UPR, PRE, NQ, SW) hipLaunchKernelGGL((ogm_gemv_fused_kernel<F, UPR, PRE, NQ, SW>), g, b, f.lds, stream, fp)
+  if (norm && src.swiglu) {
+    if (p.upr == HOT) OGM_FUSED(HOT, 2, 1, true);
+    else OGM_FUSED(0, 2, 1, true);
+  } else if (norm) {
+    if (p.upr == HOT) OGM_FUSED(HOT, 2, 1, false);
+    else OGM_FUSED(0, 2, 1, false);
+  } else if (f.nq == 1) {
+    if (p.upr == HOT) OGM_FUSED(HOT, 1, 1, false);
+    else OGM_FUSED(0, 1, 1, false);
+  } else {
+    if (K && p.upr == 56) OGM_FUSED((K ? 56 : 0), 1, 2, false);
+    else OGM_FUSED(0, 1, 2, false);
+  }
+#undef OGM_FUSED
+  return hipGetLastError();
+}
+
+#define OGM_FOR_TYPE(type, CALL, NONE)       \
+  switch (type) {                            \
+    case OGM_Q4_K: return CALL(FmtQ4K);      \
+    case OGM_Q5_K: return CALL(FmtQ5K);      \
+    case OGM_Q3_K: return CALL(FmtQ3K);      \
+    case OGM_Q6_K: return CALL(FmtQ6K);      \
+    case OGM_Q8_0: return CALL(FmtQ80);      \
+    case OGM_Q4_0: return CALL(FmtQ40);      \
+    case OGM_Q5_0: return CALL(FmtQ50);      \
+    case OGM_IQ4_NL: return CALL(FmtIQ4NL);  \
+    case OGM_Q5_1: return CALL(FmtQ51);      \
+    case OGM_IQ4_XS: return CALL(FmtIQ4XS);  \
+    case OGM_Q2_K: return CALL(FmtQ2K);      \
+    default: return NONE;                    \
+  }
+
+bool ogm_gemv_fused_can(uint32_t ggml_type, uint32_t in_dim, uint32_t n_row_blocks, bool norm, bool swiglu, uint32_t wg_waves) {
+#define OGM_CAN(F) (fused_shape<F>(in_dim, n_row_blocks, norm, swiglu, wg_waves).nq != 0)
+  OGM_FOR_TYPE(ggml_type, OGM_CAN, false)
+#undef OGM_CAN
+}
+
+uint32_t ogm_gemv_row_blocks(uint32_t ggml_type, uint32_t in_dim, uint32_t out_dim) {
+#define OGM_RB(F) ((out_dim + ogm_tiling_for(in_dim / F::ELEMS, out_dim).R - 1u) / ogm_tiling_for(in_dim / F::ELEMS, out_dim).R)
+  OGM_FOR_TYPE(ggml_type, OGM_RB, 0u)
+#undef OGM_RB
+}
+
+hipError_t ogm_launch_gemv_fused(const OgmGemvArgs &a, const OgmGemvSrc &src, hipStream_t stream, const char **kernel_name) {
+  if (a.n_tokens != 1 || a.gemm_order || a.dump_isum || a.dump_imin || a.n_extra > OGM_GEMV_MAX_MATS - 1) return hipErrorInvalidValue;
+  if (kernel_name) *kernel_name = gemv_name(a.ggml_type);
+#define OGM_GO(F) launch_fused_t<F>(a, src, stream)
+  OGM_FOR_TYPE(a.ggml_type, OGM_GO, hipErrorInvalidValue)
+#undef OGM_GO
 }
 
 // ------------------------------------------------------------------------------------------

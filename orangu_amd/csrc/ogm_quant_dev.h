@@ -12,7 +12,9 @@
 
 #include "ogm_kernels.h"
 
-__device__ __forceinline__ float ogm_nan_blind_max(float m, float a) { return a > m ? a : m; }
+// max(m, a) ignoring a NaN `a`; m is never one (the folds start at 0).  (fmaxf returns the other operand for a NaN, and
+// is one instruction where the compiler knows that `a` is no signalling NaN, two otherwise.)
+__device__ __forceinline__ float ogm_nan_blind_max(float m, float a) { return fmaxf(m, a); }
 
 // One step of a butterfly all-reduce over the wave: joins groups of M lanes pairwise with a commutative
 // `op`.  For a value that is already equal within each group of M lanes (the state of a butterfly after its
@@ -82,11 +84,22 @@ __device__ __forceinline__ float ogm_wave_sum(float v) {
   return ogm_butterfly_step<32>(v, OgmOpAdd());
 }
 
+// Round half away from zero, clamp, NaN -> 0, in five instructions.  t + copysign(largest float below 0.5, t), cut off,
+// is roundf(t) for every |t| < 2^22: at a tie the sum lies halfway between two floats and rounds to the even one, the
+// next integer; just below a tie it stays below.  v_cvt_i32_f32 cuts off, saturates and turns NaN into 0 (the
+// instruction by name: a C conversion is undefined for NaN and out of range, where 1 / scale has overflowed).
 __device__ __forceinline__ int ogm_quantize_one(float v, float inv) {
-  float r = roundf(v * inv);
-  if (r != r) r = 0.0f;
-  r = fminf(fmaxf(r, -127.0f), 127.0f);
-  return (int)r;
+  const float t = v * inv;
+  const float s = t + copysignf(0x1.fffffep-2f, t);
+  int r;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(s));
+  return r < -127 ? -127 : r > 127 ? 127 : r;
+}
+// the low bytes of four words, little-endian, by three byte permutes
+__device__ __forceinline__ uint32_t ogm_pack4(int q0, int q1, int q2, int q3) {
+  const uint32_t lo = __builtin_amdgcn_perm((uint32_t)q1, (uint32_t)q0, 0x0C0C0400u);
+  const uint32_t hi = __builtin_amdgcn_perm((uint32_t)q3, (uint32_t)q2, 0x0C0C0400u);
+  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
 }
 
 // Quantizes the four values a lane holds (elements 4*lane .. 4*lane+3 of a run of 256 spread
@@ -120,8 +133,7 @@ __device__ __forceinline__ uint32_t ogm_quantize4(const float4 &v, float &scale,
   s = ogm_butterfly_add_i32<2>(s);
   s16 = s;
   s32 = ogm_butterfly_add_i32<4>(s);
-  return (uint32_t)(q0 & 0xFF) | ((uint32_t)(q1 & 0xFF) << 8) | ((uint32_t)(q2 & 0xFF) << 16) |
-         ((uint32_t)(q3 & 0xFF) << 24);
+  return ogm_pack4(q0, q1, q2, q3);
 }
 
 // A store that workgroups of the same kernel on other compute dies may read (with a device-coherent

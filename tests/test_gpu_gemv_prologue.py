@@ -1,0 +1,123 @@
+"""One-token launches that prepare their own activations (quantizer, or residual add + RMSNorm + quantizer, inside the
+GEMV) against the same call after a launch that does: the arithmetic is the same sequence of roundings, so outputs, the
+quantized row left in the scratch and a decode step's logits are equal to the bit."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helpers import IQ4_NL, IQ4_XS, Q2_K, Q3_K, Q4_0, Q4_K, Q5_0, Q5_1, Q5_K, Q6_K, Q8_0, synth_weights
+from test_gpu_llama import build
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+@pytest.fixture(scope="module")
+def be():
+    from orangu_amd import Mi355xBackend
+    b = Mi355xBackend()
+    yield b
+    b.close()
+
+
+def special_row(n, seed):
+    """Ties and near-ties of the int8 rounding, a run of zeros, one of subnormals, NaN and infinities."""
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal(n).astype(f32)
+    x[:32] = (np.arange(32) - 16).astype(f32) + f32(0.5)      # with 127 as the group's maximum: exact ties
+    x[31] = 127.0
+    x[5] = np.nextafter(f32(2.5), f32(0))
+    if n >= 1024:
+        x[256:512] = 0.0
+        x[512:544] = f32(1e-42)
+        x[768], x[780] = np.nan, 3.0
+        x[800] = np.inf
+    return x
+
+
+# (edges: one block; a last run of 1024 partly empty; a row of 43 blocks; one run a wave, two runs a wave; rows that end
+# inside a row block; several row blocks a workgroup with an odd number of them)
+SHAPES_K = [(256, 5), (1024, 48), (1280, 33), (4096, 8192 + 272), (11008, 40), (14336, 17)]
+SHAPES_32 = [(32, 3), (1056, 40), (4096, 300), (14336, 65)]
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q3_K, Q6_K, Q2_K, IQ4_XS, Q8_0, Q4_0, Q5_0, IQ4_NL, Q5_1])
+def test_prepared_rows_give_the_same_bits(be, t):
+    per_256 = t in (Q4_K, Q5_K, Q3_K, Q6_K, Q2_K, IQ4_XS)
+    for in_dim, out_dim in SHAPES_K if per_256 else SHAPES_32:
+        print(t, in_dim, out_dim, flush=True)
+        raw = synth_weights(t, in_dim, out_dim, seed=in_dim)
+        raw2 = synth_weights(t, in_dim, 19, seed=in_dim + 1)
+        ws = [be.upload_raw(raw, t, in_dim, out_dim), be.upload_raw(raw2, t, in_dim, 19)]
+        for x in (np.random.default_rng(1).standard_normal(in_dim).astype(f32), special_row(in_dim, 2)):
+            xd = torch.from_numpy(x).cuda()
+            got = {}
+            for mode in (1, 2):
+                be.set_tuning("gemv_prologue", mode)
+                y = [torch.full((o,), 7.0, device="cuda") for o in (out_dim, 19, out_dim, 19)]
+                torch.cuda.synchronize()
+                be.matmul_dev(ws[0], xd.data_ptr(), 1, y[0].data_ptr(), False, 0)
+                be.matmul_multi_dev(ws, xd.data_ptr(), 1, [y[2].data_ptr(), y[1].data_ptr()], True, 0)
+                be.matmul_act_dev(ws[1], 1, y[3].data_ptr(), True, 0)   # over the scratch that call left
+                torch.cuda.synchronize()
+                got[mode] = [v.cpu().numpy() for v in y]
+            for a, b in zip(got[1], got[2]):
+                assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (t, in_dim, out_dim)
+            if np.isfinite(x).all() and out_dim < 1000:
+                want = oracle.matmul(t, raw, in_dim, out_dim, x, 1).reshape(-1)
+                assert np.array_equal(got[2][0].view(np.uint32), want.view(np.uint32)), (t, in_dim, out_dim)
+        for w in ws:
+            be.free_weight(w)
+    be.set_tuning("gemv_prologue", 0)
+
+
+def test_output_over_its_input(be):
+    """y may lie over x: such a call quantizes first."""
+    n = 1024
+    raw = synth_weights(Q4_K, n, n, seed=3)
+    w = be.upload_raw(raw, Q4_K, n, n)
+    x = np.random.default_rng(4).standard_normal(n).astype(f32)
+    want = oracle.matmul(Q4_K, raw, n, n, x, 1).reshape(-1)
+    be.set_tuning("gemv_prologue", 2)
+    for shift in (0, 64):
+        buf = torch.zeros(2 * n, device="cuda")
+        buf[shift:shift + n] = torch.from_numpy(x).cuda()
+        torch.cuda.synchronize()
+        be.matmul_dev(w, buf.data_ptr() + 4 * shift, 1, buf.data_ptr(), False, 0)
+        torch.cuda.synchronize()
+        assert np.array_equal(buf[:n].cpu().numpy().view(np.uint32), want.view(np.uint32))
+    be.set_tuning("gemv_prologue", 0)
+    be.free_weight(w)
+
+
+# (types: q/k/gate/up, v, down, output; a group of two types leaves its second launch the first one's scratch; Q5_0's
+# 1056 inputs end inside a run of 256; 2304 / 6400: an odd number of blocks a row)
+@pytest.mark.parametrize("types,n_embd,n_ff", [((Q4_K, Q4_K, Q6_K, Q6_K), 2048, 8192), ((Q4_K, Q6_K, Q4_K, Q6_K), 1024, 2816),
+                                               ((Q8_0, Q8_0, Q8_0, Q8_0), 1024, 3072), ((Q5_0, Q8_0, Q5_1, Q8_0), 1056, 2080),
+                                               ((Q5_K, Q5_K, Q3_K, Q4_K), 4096, 4352), ((Q6_K, Q6_K, IQ4_XS, Q4_K), 2304, 6400)])
+def test_decode_steps_give_the_same_bits(be, types, n_embd, n_ff):
+    _, dev, rng = build(be, n_embd=n_embd, n_head=4, n_kv=2, hd=64, n_ff=n_ff, n_vocab=500, n_layer=3, types=types,
+                        max_ctx=16, seed=n_embd)
+    xs = rng.standard_normal((4, n_embd)).astype(f32)
+    got = {}
+    for mode in (1, 2):
+        be.set_tuning("gemv_prologue", mode)
+        out = []
+        for pos in range(4):
+            if pos % 2 == 0:
+                out.append(dev.decode(xs[pos], pos)[0])
+            else:
+                xd, lg, tok = torch.from_numpy(xs[pos]).cuda(), torch.empty(500, device="cuda"), torch.empty(1, dtype=torch.int32, device="cuda")
+                torch.cuda.synchronize()
+                dev.decode_dev(xd.data_ptr(), pos, lg.data_ptr(), tok.data_ptr(), 0)
+                torch.cuda.synchronize()
+                out.append(lg.cpu().numpy())
+                assert np.array_equal(xd.cpu().numpy(), xs[pos])   # the caller's row stays as it was
+            out.append(dev.hidden())
+        got[mode] = out
+    be.set_tuning("gemv_prologue", 0)
+    dev.close()
+    for a, b in zip(got[1], got[2]):
+        assert np.isfinite(a).all()
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
