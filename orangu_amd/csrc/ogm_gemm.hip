@@ -23,6 +23,7 @@
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float16v __attribute__((ext_vector_type(16)));
+typedef float float32v __attribute__((ext_vector_type(32)));
 
 #define GM_BN 128   // rows per workgroup of the tiled kernels
 #define GM_BT 128   // tokens per workgroup
@@ -2544,11 +2545,17 @@ __device__ __forceinline__ half8 gw_i8_to_f16(uint32_t w0, uint32_t w1) {
 // A block's integer dot is exact on the matrix cores: weights and activations are int8 values as
 // f16, a 32-long sum is at most 32 * 127 * 127 < 2^24.  Each block (two K = 16 MFMA steps) starts a
 // fresh accumulator and ends with the reference's f32 step, so the f32 work per MFMA is eight times
-// Q4_K's: this kernel is bound by the vector pipe, not by the matrix cores.
+// Q4_K's.  Bound: a SIMD's vector and matrix instructions take their turns -- counters at 4096 -> 14336, 512 tokens:
+// 174 k cycles of vector instructions and 86 k of matrix instructions in the 266 k a SIMD has work for -- so what
+// counts is the sum.  Hence the scales' products ad * dw come from an outer product (one v_mfma_f32_32x32x1_2b for 64
+// rows x 32 tokens, 32 cycles a 32 x 32 block where sixteen multiplies take 64) and the activations become f16 once,
+// in the feeding waves, instead of in each of the multiplying ones: 149 -> 130 us (Q4_0) and 157 -> 133 (Q8_0).
+// Interleaving the f32 step with the next block's matrix instructions, operands fetched a block ahead, 64 x 64 outputs
+// a wave: no faster (132 to 155).
 //
 // Workgroup = 128 rows x 128 tokens, twelve waves: eight multiplying (64 rows x 32 tokens each),
 // four feeding.  A stage is 64 k = two blocks.  LDS rows are padded by one chunk (see the wide
-// Q4_K kernel); activations stay int8 in LDS.  Loads run three stages ahead of the MFMAs.
+// Q4_K kernel).  Loads run three stages ahead of the MFMAs.
 
 struct GemmFlatParams {
   const uint8_t *wt;      // tile-planar weights
@@ -2560,9 +2567,8 @@ struct GemmFlatParams {
 };
 
 #define GF_A_ROW 72u                       // f16 per staged weight row (64 + one chunk of padding)
-#define GF_B_ROW 80u                       // bytes per staged activation row
-#define GF_A_STAGE (128u * GF_A_ROW)       // f16
-#define GF_B_STAGE (128u * GF_B_ROW)       // bytes
+#define GF_STAGE (128u * GF_A_ROW)         // f16 of one operand's stage
+#define GF_LDS (4u * GF_STAGE * 2u + 2u * 2u * 128u * 4u)   // bytes: two stages of both operands and of the weight scales
 
 // KIND 0: Q4_0, 1: Q5_0, 2: IQ4_NL, 3: Q8_0
 template <int KIND>
@@ -2570,9 +2576,10 @@ __global__ __launch_bounds__(768) void ogm_gemm_flat_kernel(GemmFlatParams p) {
   constexpr uint32_t PIECES = KIND == 3 ? 2u : 1u;
   constexpr uint32_t TAIL = KIND == 1 ? 6u : 2u;
   constexpr uint32_t TILE = 64u * (16u * PIECES + TAIL);
-  __shared__ __align__(16) _Float16 A_l[2 * GF_A_STAGE];   // [2][128][72]
-  __shared__ __align__(16) uint8_t B_l[2 * GF_B_STAGE];    // [2][128][80]
-  __shared__ __align__(16) float dw_l[2 * 2 * 128];        // [2][block of the stage][128 rows]
+  extern __shared__ __align__(16) uint8_t gf_lds[];
+  _Float16 *A_l = (_Float16 *)gf_lds;        // [2][128][72] weights
+  _Float16 *B_l = A_l + 2 * GF_STAGE;        // [2][128][72] activations
+  float *dw_l = (float *)(B_l + 2 * GF_STAGE);   // [2][block of the stage][128 rows]
 
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const bool producer = wave >= 8u;
@@ -2598,7 +2605,7 @@ __global__ __launch_bounds__(768) void ogm_gemm_flat_kernel(GemmFlatParams p) {
     const uint32_t btok0 = rt >> 2, bch = rt & 3u;   // chunk i: token btok0 + 64 i, 16-byte chunk bch
     const uint32_t bo0 = min(t0 + btok0, p.n_tokens - 1u) * p.in_dim + 16u * bch;
     const uint32_t bo1 = min(t0 + btok0 + 64u, p.n_tokens - 1u) * p.in_dim + 16u * bch;
-    const uint32_t bso = btok0 * GF_B_ROW + 16u * bch;
+    const uint32_t bso = btok0 * GF_A_ROW + 16u * bch;   // f16
     const uint32_t aso = arow * GF_A_ROW + 32u * abl;   // f16 offset of the block's first chunk
 
     uint4 qa_0, qa_1, qa_2, qb_0, qb_1, qb_2;          // weight pieces (qb only for Q8_0)
@@ -2633,13 +2640,15 @@ __global__ __launch_bounds__(768) void ogm_gemm_flat_kernel(GemmFlatParams p) {
                                              (th_##K >> (16 + 4 * k_)) & 0xFu);                    \
       }                                                                                            \
     }                                                                                              \
-    _Float16 *ab_ = A_l + (BUF) * GF_A_STAGE + aso;                                                \
+    _Float16 *ab_ = A_l + (BUF) * GF_STAGE + aso;                                                  \
     _Pragma("unroll") for (int c_ = 0; c_ < 4; c_++)                                               \
       *(half8 *)(ab_ + 8 * c_) = gw_i8_to_f16(w_[2 * c_], w_[2 * c_ + 1]);                         \
     dw_l[(BUF) * 256u + abl * 128u + arow] = gm_f16_bits_to_f32(tl_##K);                           \
-    uint8_t *bb_ = B_l + (BUF) * GF_B_STAGE + bso;                                                 \
-    *(uint4 *)(bb_) = bx_##K;                                                                      \
-    *(uint4 *)(bb_ + 64u * GF_B_ROW) = by_##K;                                                     \
+    _Float16 *bb_ = B_l + (BUF) * GF_STAGE + bso;                                                  \
+    *(half8 *)(bb_) = gw_i8_to_f16(bx_##K.x, bx_##K.y);                                            \
+    *(half8 *)(bb_ + 8) = gw_i8_to_f16(bx_##K.z, bx_##K.w);                                        \
+    *(half8 *)(bb_ + 64u * GF_A_ROW) = gw_i8_to_f16(by_##K.x, by_##K.y);                           \
+    *(half8 *)(bb_ + 64u * GF_A_ROW + 8) = gw_i8_to_f16(by_##K.z, by_##K.w);                       \
   } while (0)
 
     // stage m uses register set m mod 3; at the barrier of stage st the loads of st + 3 are
@@ -2675,48 +2684,40 @@ __global__ __launch_bounds__(768) void ogm_gemm_flat_kernel(GemmFlatParams p) {
   const uint32_t ra = 64u * wr + l32, tl = 32u * wt_ + l32;
   const uint32_t tk = min(t0 + tl, p.n_tokens - 1u);
   const uint32_t aro = ra * GF_A_ROW + 16u * lh;    // f16 offset of chunk 2 lh of row ra
-  const uint32_t bro = tl * GF_B_ROW + 16u * lh;    // byte offset of the lane half's 16 bytes
+  const uint32_t bro = tl * GF_A_ROW + 16u * lh;    // likewise of the token's activations
   const float *adp = p.ad + (size_t)tk * p.nblk;
   float16v y0, y1;
 #pragma unroll
   for (int r = 0; r < 16; r++) y0[r] = y1[r] = 0.0f;
   const float16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  const float32v zero2 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f,
+                          0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   float2 adv = *(const float2 *)adp;   // the two blocks of stage 0
   __syncthreads();
 #pragma unroll 1
   for (uint32_t st = 0; st < n_st; st++) {
     const uint32_t buf = st & 1u;
     const float2 adn = *(const float2 *)(adp + 2u * min(st + 1u, n_st - 1u));
-    const _Float16 *ab = A_l + buf * GF_A_STAGE + aro;
-    const uint8_t *bb = B_l + buf * GF_B_STAGE + bro;
-    const float *dwp = dw_l + buf * 256u + 64u * wr + 4u * lh;
+    const _Float16 *ab = A_l + buf * GF_STAGE + aro;
+    const _Float16 *bb = B_l + buf * GF_STAGE + bro;
+    const float *dwp = dw_l + buf * 256u + 64u * wr + lane;
 #pragma unroll
     for (int bl = 0; bl < 2; bl++) {
-      // the lane's 16 activations of this block: MFMA step kk takes bytes 8 kk .. 8 kk + 7
-      const uint4 bq = *(const uint4 *)(bb + 32u * bl);
       float16v c0, c1;
 #pragma unroll
       for (int kk = 0; kk < 2; kk++) {
         const half8 a0 = *(const half8 *)(ab + 32u * bl + 8u * kk);
         const half8 a1 = *(const half8 *)(ab + 32u * GF_A_ROW + 32u * bl + 8u * kk);
-        const half8 b = kk ? gw_i8_to_f16(bq.z, bq.w) : gw_i8_to_f16(bq.x, bq.y);
+        const half8 b = *(const half8 *)(bb + 32u * bl + 8u * kk);
         c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b, kk ? c0 : zero, 0, 0, 0);
         c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b, kk ? c1 : zero, 0, 0, 0);
       }
-      // acc += d * s * dot32 (vecdot.rs:2622): (ad * dw) * (f32)isum
-      const float ad = bl ? adv.y : adv.x;
+      // acc += d * s * dot32 (vecdot.rs:2622): (ad * dw) * (f32)isum, the products of the scales from an outer product
+      const float32v s = __builtin_amdgcn_mfma_f32_32x32x1f32(dwp[128 * bl], bl ? adv.y : adv.x, zero2, 0, 0, 0);
 #pragma unroll
-      for (int q4 = 0; q4 < 4; q4++) {
-        const float4 d0 = *(const float4 *)(dwp + 128 * bl + 8 * q4);
-        const float4 d1 = *(const float4 *)(dwp + 128 * bl + 32 + 8 * q4);
-        y0[4 * q4 + 0] += ad * d0.x * c0[4 * q4 + 0];
-        y0[4 * q4 + 1] += ad * d0.y * c0[4 * q4 + 1];
-        y0[4 * q4 + 2] += ad * d0.z * c0[4 * q4 + 2];
-        y0[4 * q4 + 3] += ad * d0.w * c0[4 * q4 + 3];
-        y1[4 * q4 + 0] += ad * d1.x * c1[4 * q4 + 0];
-        y1[4 * q4 + 1] += ad * d1.y * c1[4 * q4 + 1];
-        y1[4 * q4 + 2] += ad * d1.z * c1[4 * q4 + 2];
-        y1[4 * q4 + 3] += ad * d1.w * c1[4 * q4 + 3];
+      for (int r = 0; r < 16; r++) {
+        y0[r] += s[r] * c0[r];
+        y1[r] += s[16 + r] * c1[r];
       }
     }
     adv = adn;
@@ -3182,12 +3183,13 @@ hipError_t ogm_launch_gemm(const OgmGemmArgs &a, hipStream_t stream, const char 
     }
     if (q51) return hipErrorInvalidValue;
     const dim3 grid((a.n_tokens + 127u) / 128u, (a.out_dim + 127u) / 128u);
-    switch (a.ggml_type) {
-      case OGM_Q4_0: hipLaunchKernelGGL(ogm_gemm_flat_kernel<0>, grid, dim3(768), 0, stream, p); break;
-      case OGM_Q5_0: hipLaunchKernelGGL(ogm_gemm_flat_kernel<1>, grid, dim3(768), 0, stream, p); break;
-      case OGM_IQ4_NL: hipLaunchKernelGGL(ogm_gemm_flat_kernel<2>, grid, dim3(768), 0, stream, p); break;
-      default: hipLaunchKernelGGL(ogm_gemm_flat_kernel<3>, grid, dim3(768), 0, stream, p); break;
-    }
+    void (*const flat)(GemmFlatParams) = a.ggml_type == OGM_Q4_0     ? ogm_gemm_flat_kernel<0>
+                                         : a.ggml_type == OGM_Q5_0   ? ogm_gemm_flat_kernel<1>
+                                         : a.ggml_type == OGM_IQ4_NL ? ogm_gemm_flat_kernel<2>
+                                                                     : ogm_gemm_flat_kernel<3>;
+    const hipError_t e = hipFuncSetAttribute((const void *)flat, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GF_LDS);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(flat, grid, dim3(768), GF_LDS, stream, p);
     if (kernel_name) *kernel_name = "ogm_gemm_flat_kernel";
     return hipGetLastError();
   }
