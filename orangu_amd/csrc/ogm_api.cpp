@@ -1368,6 +1368,8 @@ extern "C" int ogm_f16_to_f32(ogm_ctx *ctx, const uint16_t *bits, size_t n, floa
 
 #include "ogm_llama.h"
 
+static const uint32_t OGM_ALL_LOGITS_MAX_TOKENS = 64;
+
 struct ogm_llama {
   ogm_llama_config cfg;
   std::vector<ogm_llama_layer> layers;  // weight handles; the optional vectors as device pointers
@@ -1495,7 +1497,7 @@ extern "C" int ogm_llama_create(ogm_ctx *ctx, const ogm_llama_config *cfg, const
   A((void **)&m->part_o, (size_t)c.n_head * m->max_splits * c.head_dim * 4);
   A((void **)&m->part_ml, (size_t)c.n_head * m->max_splits * 2 * 4);
   A((void **)&m->logits, (size_t)c.n_vocab * 4);
-  A((void **)&m->amax_scratch, 512 * 4);
+  A((void **)&m->amax_scratch, (size_t)OGM_ALL_LOGITS_MAX_TOKENS * OGM_ARGMAX_SCRATCH * 4);
   A((void **)&m->amax_out, 4);
   if (rc != OGM_OK) { llama_free(m); return rc; }
   // activation scratch for the widest matmul input
@@ -2144,8 +2146,7 @@ static int llama_prefill_chunk(ogm_ctx *ctx, ogm_llama *m, uint32_t pos0, uint32
     const ogm_weight *wo_[1] = {m->output};
     float *yo[1] = {m->logits_all};
     if ((rc = llama_matmul_quantized_rows(ctx, wo_, yo, 1, mode_out, c.n_embd, T, s)) != OGM_OK) return rc;
-    for (uint32_t t = 0; t < T; t++)
-      HIPCHK(ctx, ogm_launch_argmax(m->logits_all + (size_t)t * c.n_vocab, c.n_vocab, m->amax_scratch, m->amax_all + t, s));
+    HIPCHK(ctx, ogm_launch_argmax(m->logits_all, c.n_vocab, m->amax_scratch, m->amax_all, s, T));
     ctx->act_mode = -1;
     return OGM_OK;
   }
@@ -2225,7 +2226,6 @@ extern "C" int ogm_llama_prefill(ogm_ctx *ctx, ogm_llama *m, const float *x, uin
   return llama_prefill(ctx, m, x, nullptr, nullptr, pos0, n_tokens, last_logits, argmax);
 }
 
-static const uint32_t OGM_ALL_LOGITS_MAX_TOKENS = 64;
 
 extern "C" int ogm_llama_forward_all_logits(ogm_ctx *ctx, ogm_llama *m, const float *x, const ogm_weight *tok_embd,
                                             const uint32_t *tokens, uint32_t pos0, uint32_t n_tokens, float *logits,

@@ -79,9 +79,10 @@ hipError_t ogm_launch_swiglu_quant(int mode, const float *gate, const float *up,
                                    OgmActDev act, hipStream_t stream, uint32_t n_rows = 1);
 
 // Index of the largest logit; of several equal ones the last (sampling.rs:336-343).  `scratch`
-// holds 2 * 256 words.
+// holds 2 * 256 words a row of n logits.
+#define OGM_ARGMAX_SCRATCH 512u   // words of scratch a row
 hipError_t ogm_launch_argmax(const float *logits, uint32_t n, uint32_t *scratch, uint32_t *out,
-                             hipStream_t stream);
+                             hipStream_t stream, uint32_t n_rows = 1);
 
 // f32 -> f16 (round to nearest even) for cache rows handed over by the host.
 hipError_t ogm_launch_f32_to_f16(const float *src, void *dst, size_t n, hipStream_t stream);

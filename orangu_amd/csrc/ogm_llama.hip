@@ -936,9 +936,12 @@ __global__ __launch_bounds__(256) void ogm_argmax_kernel(const float *__restrict
   __shared__ int32_t sv[256];
   __shared__ uint32_t si[256];
   const uint32_t tid = threadIdx.x;
+  // one row of logits per grid row (a verify batch's rows in one launch each stage: launches of their own cost 9 us a row)
+  scratch += (size_t)blockIdx.y * OGM_ARGMAX_SCRATCH;
   int32_t bk = INT32_MIN;   // the key of the smallest value there is
   uint32_t bi = 0;
   if (!final_stage) {
+    x += (size_t)blockIdx.y * n;
     for (uint32_t i = blockIdx.x * 256u + tid; i < n; i += gridDim.x * 256u) {
       const int32_t k = argmax_key(x[i]);
       if (argmax_better(k, i, bk, bi)) { bk = k; bi = i; }
@@ -962,18 +965,18 @@ __global__ __launch_bounds__(256) void ogm_argmax_kernel(const float *__restrict
       scratch[blockIdx.x] = (uint32_t)sv[0];
       scratch[256 + blockIdx.x] = si[0];
     } else {
-      *out = si[0];
+      out[blockIdx.y] = si[0];
     }
   }
 }
 
 hipError_t ogm_launch_argmax(const float *logits, uint32_t n, uint32_t *scratch, uint32_t *out,
-                             hipStream_t stream) {
-  if (n == 0) return hipErrorInvalidValue;
+                             hipStream_t stream, uint32_t n_rows) {
+  if (n == 0 || n_rows == 0 || n_rows > 65535u) return hipErrorInvalidValue;
   uint32_t wgs = (n + 255u) / 256u;
   if (wgs > 256u) wgs = 256u;
-  hipLaunchKernelGGL(ogm_argmax_kernel, dim3(wgs), dim3(256), 0, stream, logits, n, scratch, out, 0);
-  hipLaunchKernelGGL(ogm_argmax_kernel, dim3(1), dim3(256), 0, stream, logits, wgs, scratch, out, 1);
+  hipLaunchKernelGGL(ogm_argmax_kernel, dim3(wgs, n_rows), dim3(256), 0, stream, logits, n, scratch, out, 0);
+  hipLaunchKernelGGL(ogm_argmax_kernel, dim3(1, n_rows), dim3(256), 0, stream, logits, wgs, scratch, out, 1);
   return hipGetLastError();
 }
 
