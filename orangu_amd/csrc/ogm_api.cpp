@@ -553,8 +553,7 @@ static bool gemv_prepares(const ogm_ctx *ctx, const Target *tg, size_t n_tg, boo
   return (uint64_t)rb * ((in_dim + 1023u) / 1024u) <= (block_elems_of(type) == 256 ? OGM_PREPARE_MAX_WORK : OGM_PREPARE_MAX_WORK_32);
 }
 
-// Enqueues that launch; the quantized row also ends in the context's scratch.  The scratch is large enough.
-static int enqueue_prepared(ogm_ctx *ctx, const Target *tg, size_t n_tg, const OgmGemvSrc &src, hipStream_t stream) {
+static OgmGemvArgs prepared_args(ogm_ctx *ctx, const Target *tg, size_t n_tg) {
   OgmGemvArgs a;
   const ogm_weight *w0 = tg[0].w;
   a.ggml_type = w0->ggml_type;
@@ -573,7 +572,12 @@ static int enqueue_prepared(ogm_ctx *ctx, const Target *tg, size_t n_tg, const O
     a.extra_out_dim[i - 1] = tg[i].w->out_dim;
     a.extra_y[i - 1] = tg[i].y;
   }
-  HIPCHK(ctx, ogm_launch_gemv_fused(a, src, stream, &ctx->last_kernel));
+  return a;
+}
+
+// Enqueues that launch; the quantized row also ends in the context's scratch.  The scratch is large enough.
+static int enqueue_prepared(ogm_ctx *ctx, const Target *tg, size_t n_tg, const OgmGemvSrc &src, hipStream_t stream) {
+  HIPCHK(ctx, ogm_launch_gemv_fused(prepared_args(ctx, tg, n_tg), src, stream, &ctx->last_kernel));
   return OGM_OK;
 }
 
@@ -1675,6 +1679,14 @@ static int llama_norm_matmul(ogm_ctx *ctx, ogm_llama *m, DecodeRow &row, const f
   int rc;
   const bool swiglu = did_swiglu && e == 2 && n == 2 && ws[0]->out_dim == ws[1]->out_dim && gemv_prepares(ctx, tg, e, true, true);
   if (did_swiglu) *did_swiglu = swiglu;
+  // what is left of the group, of one other type: in the same launch where both would fit the line
+  Target tg2[OGM_GEMV_MAX_MATS];
+  bool both = e < n && n - e <= OGM_GEMV_MAX_MATS && ogm_gemv_fused_pair_can(ws[0]->ggml_type, ws[e]->ggml_type, ws[0]->in_dim, (uint32_t)ctx->tune_wg_waves);
+  for (size_t i = e; both && i < n; i++) {
+    both = ws[i]->ggml_type == ws[e]->ggml_type;
+    tg2[i - e] = Target{ws[i], ys[i]};
+  }
+  both = both && gemv_prepares(ctx, tg2, n - e, true, false);
   if (swiglu || gemv_prepares(ctx, tg, e, true, false)) {
     OgmGemvSrc src;
     src.x = row.first ? row.first : row.x;
@@ -1689,8 +1701,12 @@ static int llama_norm_matmul(ogm_ctx *ctx, ogm_llama *m, DecodeRow &row, const f
     } else if (row.first) {
       src.x_out = row.x;
     }
-    if ((rc = enqueue_prepared(ctx, tg, e, src, s)) != OGM_OK) return rc;
-    if (e < n && (rc = llama_matmul(ctx, ws + e, ys + e, n - e, s)) != OGM_OK) return rc;
+    if (both) {
+      HIPCHK(ctx, ogm_launch_gemv_fused_pair(prepared_args(ctx, tg, e), prepared_args(ctx, tg2, n - e), src, s, &ctx->last_kernel));
+    } else {
+      if ((rc = enqueue_prepared(ctx, tg, e, src, s)) != OGM_OK) return rc;
+      if (e < n && (rc = llama_matmul(ctx, ws + e, ys + e, n - e, s)) != OGM_OK) return rc;
+    }
   } else {
     HIPCHK(ctx, ogm_launch_norm_quant(mode, row.x, row.delta, norm_w, c.n_embd, c.rms_eps, nullptr,
                                       act_view(ctx, c.n_embd, mode, 0), s, 1, row.first));

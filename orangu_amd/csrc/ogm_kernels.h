@@ -68,6 +68,10 @@ uint32_t ogm_gemv_row_blocks(uint32_t ggml_type, uint32_t in_dim, uint32_t out_d
 bool ogm_gemv_fused_can(uint32_t ggml_type, uint32_t in_dim, uint32_t n_row_blocks, bool norm, bool swiglu, uint32_t wg_waves);
 // a.act: where workgroup 0 leaves the quantized row, as ogm_launch_quantize would.
 hipError_t ogm_launch_gemv_fused(const OgmGemvArgs &a, const OgmGemvSrc &src, hipStream_t stream, const char **kernel_name);
+// The same for matrices of two types (Q4_K or Q5_K, and Q6_K) over one normed row, in one launch.
+bool ogm_gemv_fused_pair_can(uint32_t type1, uint32_t type2, uint32_t in_dim, uint32_t wg_waves);
+hipError_t ogm_launch_gemv_fused_pair(const OgmGemvArgs &a, const OgmGemvArgs &b, const OgmGemvSrc &src, hipStream_t stream,
+                                      const char **kernel_name);
 // Prefill GEMM on MFMA (ogm_gemm.hip).  Same operands as the GEMV plus a scratch buffer `xh` of
 // ogm_gemm_xh_bytes() for the int8 activations in operand chunks.  Follows the CPU path's GEMM float order.
 #define OGM_GEMM_MAX_MATS 3   // matrices one GEMM launch can take (q, k, v)

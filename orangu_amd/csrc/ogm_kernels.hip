@@ -1188,9 +1188,10 @@ struct GemvFusedParams {
   uint32_t teams, team_waves;
 };
 
-// NQ: runs of 1024 elements a wave prepares.
+// NQ: runs of 1024 elements a wave prepares.  bid: the workgroup's number among those of its type; leads: it stores the
+// quantized row and the residual stream.
 template <class F, int UPR, int PRE, int NQ, bool SWIGLU>
-__global__ __launch_bounds__(F::ELEMS == 32 ? 1024 : 512) void ogm_gemv_fused_kernel(GemvFusedParams fp) {
+__device__ __forceinline__ void gemv_fused_body(const GemvFusedParams &fp, const uint32_t bid, const bool leads) {
   extern __shared__ __align__(16) uint8_t lds[];
   const GemvParams &p = fp.g;
   constexpr int GROUP = F::ACT_GROUP;
@@ -1217,10 +1218,10 @@ __global__ __launch_bounds__(F::ELEMS == 32 ? 1024 : 512) void ogm_gemv_fused_ke
   auto locate = [&](uint32_t team_, uint32_t &m, uint32_t &rb) -> bool {
     if (SWIGLU) {
       m = team_;
-      rb = blockIdx.x;
+      rb = bid;
       return true;
     }
-    const uint32_t last = p.wg_end[OGM_GEMV_MAX_MATS - 1] - 1u, want = blockIdx.x * teams + team_;
+    const uint32_t last = p.wg_end[OGM_GEMV_MAX_MATS - 1] - 1u, want = bid * teams + team_;
     const uint32_t b = min(want, last);
     m = (b >= p.wg_end[0] ? 1u : 0u) + (b >= p.wg_end[1] ? 1u : 0u) + (b >= p.wg_end[2] ? 1u : 0u);
     rb = b - (m == 0 ? 0u : m == 1 ? p.wg_end[0] : m == 2 ? p.wg_end[1] : p.wg_end[2]);
@@ -1268,7 +1269,7 @@ __global__ __launch_bounds__(F::ELEMS == 32 ? 1024 : 512) void ogm_gemv_fused_ke
         a.x += dl[i].x; a.y += dl[i].y; a.z += dl[i].z; a.w += dl[i].w;
       }
     }
-    if (blockIdx.x == 0 && fp.x_out && active) {
+    if (leads && fp.x_out && active) {
 #pragma unroll
       for (int i = 0; i < 4; i++) *(float4 *)(fp.x_out + e0 + 4 * i) = v[0][i];
     }
@@ -1334,7 +1335,7 @@ __global__ __launch_bounds__(F::ELEMS == 32 ? 1024 : 512) void ogm_gemv_fused_ke
       if (F::AUX16 == 1 && (lane & 1u) == 0) ((int16_t *)(l_aux + col))[c >> 1] = (int16_t)s32;
       if (F::AUX16 == 2) ((int16_t *)(l_aux + (c >> 3) * upr + col))[c & 7u] = (int16_t)s16;
       if ((lane & (GROUP / 16 - 1)) == 0) l_d[e0 / GROUP] = scale;
-      if (blockIdx.x == 0) {   // the scratch, as the quantizer's own launch leaves it
+      if (leads) {   // the scratch, as the quantizer's own launch leaves it
         *(uint4 *)(p.act.q + e0) = q16;
         p.act.sums[e0 / 16u] = s16;
         if ((lane & 1u) == 0) {
@@ -1385,6 +1386,19 @@ __global__ __launch_bounds__(F::ELEMS == 32 ? 1024 : 512) void ogm_gemv_fused_ke
       if (store) y[orow] = acc;
     }
   }
+}
+
+template <class F, int UPR, int PRE, int NQ, bool SWIGLU>
+__global__ __launch_bounds__(F::ELEMS == 32 ? 1024 : 512) void ogm_gemv_fused_kernel(GemvFusedParams fp) {
+  gemv_fused_body<F, UPR, PRE, NQ, SWIGLU>(fp, blockIdx.x, blockIdx.x == 0);
+}
+
+// Matrices of two K-quants over one normed row (q and k in Q4_K beside v in Q6_K, as mixed files have them in half of
+// their layers): the workgroups of both in one launch.
+template <class F1, class F2, int UPR>
+__global__ __launch_bounds__(512) void ogm_gemv_fused_pair_kernel(GemvFusedParams fp1, GemvFusedParams fp2, uint32_t wgs1) {
+  if (blockIdx.x < wgs1) gemv_fused_body<F1, UPR, 2, 1, false>(fp1, blockIdx.x, blockIdx.x == 0);
+  else gemv_fused_body<F2, UPR, 2, 1, false>(fp2, blockIdx.x - wgs1, false);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1624,9 +1638,9 @@ static FusedShape fused_shape(uint32_t in_dim, uint32_t n_row_blocks, bool norm,
   return f;
 }
 
+// Fills the kernel's parameters; `f` has nq 0 if the shape can't be launched.  Returns the row blocks.
 template <class F>
-static hipError_t launch_fused_t(const OgmGemvArgs &a, const OgmGemvSrc &src, hipStream_t stream) {
-  GemvFusedParams fp;
+static uint32_t fused_params(const OgmGemvArgs &a, const OgmGemvSrc &src, GemvFusedParams &fp, FusedShape &f) {
   GemvParams &p = fp.g;
   p.act = a.act;
   p.dump_isum = p.dump_imin = nullptr;
@@ -1646,11 +1660,7 @@ static hipError_t launch_fused_t(const OgmGemvArgs &a, const OgmGemvSrc &src, hi
     n_rb += (p.out_dim[m] + tl.R - 1) / tl.R;
     p.wg_end[m] = n_rb;
   }
-  if (n_rb == 0) return hipSuccess;
-  const bool norm = src.weight != nullptr;
-  const FusedShape f = fused_shape<F>(a.in_dim, n_rb, norm, src.swiglu, a.wg_waves);
-  if (f.nq == 0) return hipErrorInvalidValue;
-  if (src.swiglu && (a.n_extra != 1 || a.extra_out_dim[0] != a.out_dim || !norm)) return hipErrorInvalidValue;
+  f = fused_shape<F>(a.in_dim, n_rb, src.weight != nullptr, src.swiglu, a.wg_waves);
   fp.x = src.x;
   fp.delta = src.delta;
   fp.weight = src.weight;
@@ -1658,6 +1668,19 @@ static hipError_t launch_fused_t(const OgmGemvArgs &a, const OgmGemvSrc &src, hi
   fp.eps = src.eps;
   fp.teams = f.teams;
   fp.team_waves = f.team_waves;
+  return n_rb;
+}
+
+template <class F>
+static hipError_t launch_fused_t(const OgmGemvArgs &a, const OgmGemvSrc &src, hipStream_t stream) {
+  GemvFusedParams fp;
+  FusedShape f;
+  const GemvParams &p = fp.g;
+  const uint32_t n_rb = fused_params<F>(a, src, fp, f);
+  const bool norm = src.weight != nullptr;
+  if (n_rb == 0) return hipSuccess;
+  if (f.nq == 0) return hipErrorInvalidValue;
+  if (src.swiglu && (a.n_extra != 1 || a.extra_out_dim[0] != a.out_dim || !norm)) return hipErrorInvalidValue;
   const dim3 g(src.swiglu ? p.wg_end[0] : (n_rb + f.teams - 1u) / f.teams), b(f.team_waves * f.teams * 64u);
   constexpr bool K = F::ELEMS == 256;
   constexpr int HOT = K ? 16 : 128;   // rows of 4096
@@ -1677,6 +1700,38 @@ static hipError_t launch_fused_t(const OgmGemvArgs &a, const OgmGemvSrc &src, hi
   }
 #undef OGM_FUSED
   return hipGetLastError();
+}
+
+template <class F1, class F2>
+static hipError_t launch_fused_pair_t(const OgmGemvArgs &a, const OgmGemvArgs &b, const OgmGemvSrc &src, hipStream_t stream) {
+  GemvFusedParams fp1, fp2;
+  FusedShape f1, f2;
+  const uint32_t rb1 = fused_params<F1>(a, src, fp1, f1), rb2 = fused_params<F2>(b, src, fp2, f2);
+  if (rb1 == 0 || rb2 == 0 || f1.nq != 1 || f2.nq != 1 || f1.team_waves != f2.team_waves) return hipErrorInvalidValue;
+  fp1.teams = fp2.teams = 1;   // (f.lds holds for more)
+  const dim3 g(rb1 + rb2), t(f1.team_waves * 64u);
+  const size_t lds = f1.lds > f2.lds ? f1.lds : f2.lds;
+  if (fp1.g.upr == 16) hipLaunchKernelGGL((ogm_gemv_fused_pair_kernel<F1, F2, 16>), g, t, lds, stream, fp1, fp2, rb1);
+  else hipLaunchKernelGGL((ogm_gemv_fused_pair_kernel<F1, F2, 0>), g, t, lds, stream, fp1, fp2, rb1);
+  return hipGetLastError();
+}
+
+bool ogm_gemv_fused_pair_can(uint32_t type1, uint32_t type2, uint32_t in_dim, uint32_t wg_waves) {
+  if (type2 != OGM_Q6_K || (type1 != OGM_Q4_K && type1 != OGM_Q5_K)) return false;
+  // (one row block a workgroup: a wave must be able to prepare its run without a second team)
+  const FusedShape f = type1 == OGM_Q4_K ? fused_shape<FmtQ4K>(in_dim, 1u, true, false, wg_waves) : fused_shape<FmtQ5K>(in_dim, 1u, true, false, wg_waves);
+  const FusedShape f6 = fused_shape<FmtQ6K>(in_dim, 1u, true, false, wg_waves);
+  return f.nq == 1 && f6.nq == 1 && f.team_waves == f6.team_waves;
+}
+
+hipError_t ogm_launch_gemv_fused_pair(const OgmGemvArgs &a, const OgmGemvArgs &b, const OgmGemvSrc &src, hipStream_t stream,
+                                      const char **kernel_name) {
+  if (!ogm_gemv_fused_pair_can(a.ggml_type, b.ggml_type, a.in_dim, a.wg_waves) || a.in_dim != b.in_dim || !src.weight ||
+      src.swiglu || a.n_extra > OGM_GEMV_MAX_MATS - 1 || b.n_extra > OGM_GEMV_MAX_MATS - 1)
+    return hipErrorInvalidValue;
+  if (kernel_name) *kernel_name = gemv_name(a.ggml_type);
+  return a.ggml_type == OGM_Q4_K ? launch_fused_pair_t<FmtQ4K, FmtQ6K>(a, b, src, stream)
+                                 : launch_fused_pair_t<FmtQ5K, FmtQ6K>(a, b, src, stream);
 }
 
 #define OGM_FOR_TYPE(type, CALL, NONE)       \

@@ -95,7 +95,7 @@ def test_output_over_its_input(be):
 # 1056 inputs end inside a run of 256; 2304 / 6400: an odd number of blocks a row)
 @pytest.mark.parametrize("types,n_embd,n_ff", [((Q4_K, Q4_K, Q6_K, Q6_K), 2048, 8192), ((Q4_K, Q6_K, Q4_K, Q6_K), 1024, 2816),
                                                ((Q8_0, Q8_0, Q8_0, Q8_0), 1024, 3072), ((Q5_0, Q8_0, Q5_1, Q8_0), 1056, 2080),
-                                               ((Q5_K, Q5_K, Q3_K, Q4_K), 4096, 4352), ((Q6_K, Q6_K, IQ4_XS, Q4_K), 2304, 6400)])
+                                               ((Q5_K, Q6_K, Q3_K, Q4_K), 4096, 4352), ((Q6_K, Q6_K, IQ4_XS, Q4_K), 2304, 6400)])
 def test_decode_steps_give_the_same_bits(be, types, n_embd, n_ff):
     _, dev, rng = build(be, n_embd=n_embd, n_head=4, n_kv=2, hd=64, n_ff=n_ff, n_vocab=500, n_layer=3, types=types,
                         max_ctx=16, seed=n_embd)
