@@ -121,3 +121,24 @@ def test_decode_steps_give_the_same_bits(be, types, n_embd, n_ff):
     for a, b in zip(got[1], got[2]):
         assert np.isfinite(a).all()
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+# (the kernel between the projections and the attention takes several tokens a wave from 256 on, two at a time where a
+# head has 64 elements; the norm four runs of 256 a wave from 1024 rows, and on rows of more than 4096)
+@pytest.mark.parametrize("n_embd,n_head,n_kv,hd,neox,pre,n_tokens", [
+    (256, 4, 2, 64, False, (), 257), (256, 4, 1, 64, True, ("q_bias", "k_bias", "v_bias"), 263),
+    (256, 2, 2, 128, False, ("q_norm", "k_norm"), 259), (512, 4, 4, 64, False, ("q_norm", "k_norm"), 1027),
+    (1280, 2, 1, 128, True, (), 1025)])
+def test_batches_leave_the_rows_of_smaller_ones(be, n_embd, n_head, n_kv, hd, neox, pre, n_tokens):
+    """Cache rows of a batch against those of the same tokens in parts of at most 100 (a wave a token)."""
+    _, dev, rng = build(be, n_embd=n_embd, n_head=n_head, n_kv=n_kv, hd=hd, n_ff=512, n_vocab=300, n_layer=1,
+                        types=(Q8_0, Q8_0, Q8_0, Q8_0), max_ctx=n_tokens + 8, seed=n_tokens, neox=neox, pre=pre)
+    X = rng.standard_normal((n_tokens, n_embd)).astype(f32)
+    dev.prefill(X, 3)
+    whole = [a.copy() for a in dev.kv_read(0, 3, n_tokens)]
+    for at in range(0, n_tokens, 100):
+        dev.prefill(X[at:at + 100], 3 + at)
+    parts = dev.kv_read(0, 3, n_tokens)
+    dev.close()
+    for a, b in zip(whole, parts):
+        assert np.array_equal(np.asarray(a), np.asarray(b))
