@@ -18,7 +18,7 @@
 // residual add + RMSNorm + quantize
 
 // One workgroup per row (ogm_norm_quant_row).
-template <int GROUP>
+template <int GROUP, int RUNS>
 __global__ __launch_bounds__(1024) void ogm_norm_quant_kernel(float *__restrict__ x,
                                                               const float *__restrict__ delta,
                                                               const float *__restrict__ weight, uint32_t n,
@@ -40,7 +40,7 @@ __global__ __launch_bounds__(1024) void ogm_norm_quant_kernel(float *__restrict_
     if (act.bs16) act.bs16 += (size_t)r * (n / 16u);
     act.xt = ogm_xt_row(act.xt, r, n);
   }
-  ogm_norm_quant_row<GROUP, false>(x, delta, weight, n, eps, normed, act, red, tid, n_wave, x_src);
+  ogm_norm_quant_row<GROUP, RUNS>(x, delta, weight, n, eps, normed, act, red, tid, n_wave, x_src);
 }
 
 hipError_t ogm_launch_norm_quant(int mode, float *x, const float *delta, const float *weight, uint32_t n,
@@ -48,15 +48,21 @@ hipError_t ogm_launch_norm_quant(int mode, float *x, const float *delta, const f
                                  const float *x_src) {
   if (n == 0 || n % 32u != 0 || n > 16384u || n_rows == 0) return hipErrorInvalidValue;
   const uint32_t runs = (n + 255u) / 256u;
-  // few rows: a wave per run, the shortest chain; from 1024 rows (2048 rows: 2 % of a prefill): four runs per wave
-  // (the row's bits do not depend on it)
-  const uint32_t waves = n_rows >= 1024u ? (runs + 3u) / 4u : (runs < 16u ? runs : 16u);
-  if (mode == 0)
-    hipLaunchKernelGGL(ogm_norm_quant_kernel<32>, dim3(n_rows), dim3(waves * 64), 0, stream, x, delta, weight,
-                       n, eps, normed, act, x_src);
-  else
-    hipLaunchKernelGGL(ogm_norm_quant_kernel<256>, dim3(n_rows), dim3(waves * 64), 0, stream, x, delta, weight,
-                       n, eps, normed, act, x_src);
+  // few rows: a wave per run, the shortest chain (rows of more than sixteen: four runs a wave); from 1024 rows four runs
+  // per wave (the row's bits do not depend on it)
+  const bool one = n_rows < 1024u && runs <= 16u;
+  const dim3 threads((one ? runs : (runs + 3u) / 4u) * 64u);
+#define OGM_NORM(GROUP, RUNS)                                                                                      \
+  hipLaunchKernelGGL((ogm_norm_quant_kernel<GROUP, RUNS>), dim3(n_rows), threads, 0, stream, x, delta, weight, n, \
+                     eps, normed, act, x_src)
+  if (mode == 0) {
+    if (one) OGM_NORM(32, 1);
+    else OGM_NORM(32, 4);
+  } else {
+    if (one) OGM_NORM(256, 1);
+    else OGM_NORM(256, 4);
+  }
+#undef OGM_NORM
   return hipGetLastError();
 }
 

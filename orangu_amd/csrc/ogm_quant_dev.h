@@ -204,41 +204,40 @@ __device__ __forceinline__ float4 ogm_ld4(const float *p) {
   }
 }
 
-// Residual add, RMSNorm and quantization of one row by one workgroup of n_wave waves (n <= 1024 *
-// n_wave): wave w owns the 256-runs w, w + n_wave, ... (at most four), lane l their elements
-// 4l..4l+3, kept in registers between the two passes.  red: 64 floats of LDS.  COHERENT_DELTA:
-// delta was written by other workgroups of the calling kernel.  COHERENT_OUT: the quantized row is
-// for other workgroups of the calling kernel.  x_src (optional): the row is read from there instead of
-// from x, and stored to x.
-template <int GROUP, bool COHERENT_DELTA, bool COHERENT_OUT = false>
+// Residual add, RMSNorm and quantization of one row by one workgroup of n_wave waves (n <= 256 * RUNS * n_wave): wave w
+// owns the 256-runs w, w + n_wave, ... (RUNS at most), lane l their elements 4l..4l+3, kept in registers between the two
+// passes.  red: 64 floats of LDS.  x_src (optional): the row is read from there instead of from x, and stored to x.
+template <int GROUP, int RUNS>
 __device__ __forceinline__ void ogm_norm_quant_row(float *__restrict__ x, const float *__restrict__ delta,
                                                    const float *__restrict__ weight, uint32_t n, float eps,
                                                    float *__restrict__ normed, const OgmActDev &act,
                                                    float *red, uint32_t tid, uint32_t n_wave,
                                                    const float *__restrict__ x_src = nullptr) {
   const uint32_t lane = tid & 63u, wave = tid >> 6;
-  float4 v[4], wv[4];
-  float ss[4];
-  // every load first (x, the residual delta and the norm weights share one trip to memory)
+  float4 v[RUNS], wv[RUNS], d[RUNS];
+  float ss[RUNS];
+  // every load first, at clamped places instead of behind branches: x, the residual delta and the norm weights of all
+  // runs share one trip to memory
+  const float *xs = x_src ? x_src : x, *ds = delta ? delta : xs;
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
+  for (int k = 0; k < RUNS; k++) {
+    const uint32_t e0 = min((wave + k * n_wave) * 256u + 4u * lane, n - 4u);
+    v[k] = *(const float4 *)(xs + e0);
+    d[k] = *(const float4 *)(ds + e0);
+    wv[k] = *(const float4 *)(weight + e0);
+  }
+#pragma unroll
+  for (int k = 0; k < RUNS; k++) {
     const uint32_t e0 = (wave + k * n_wave) * 256u + 4u * lane;
-    v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-    wv[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 d = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (e0 < n) {
-      v[k] = *(const float4 *)((x_src ? x_src : x) + e0);
-      wv[k] = *(const float4 *)(weight + e0);
-      if (delta) d = ogm_ld4<COHERENT_DELTA>(delta + e0);
-    }
-    if (e0 < n && delta) { v[k].x += d.x; v[k].y += d.y; v[k].z += d.z; v[k].w += d.w; }
+    if (e0 >= n) v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (e0 < n && delta) { v[k].x += d[k].x; v[k].y += d[k].y; v[k].z += d[k].z; v[k].w += d[k].w; }
     if (e0 < n && (delta || x_src)) *(float4 *)(x + e0) = v[k];
     ss[k] = v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
   }
   // one sum per 256-run, then the runs in ascending order: the same value whatever the
   // number of waves
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
+  for (int k = 0; k < RUNS; k++) {
     if ((wave + k * n_wave) * 256u < n) {   // wave-uniform: the run exists
       ss[k] = ogm_wave_sum(ss[k]);
       if (lane == 0) red[wave + k * n_wave] = ss[k];
@@ -250,7 +249,7 @@ __device__ __forceinline__ void ogm_norm_quant_row(float *__restrict__ x, const 
   const float mean_sq = total / (float)n;
   const float scale = 1.0f / sqrtf(mean_sq + eps);
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
+  for (int k = 0; k < RUNS; k++) {
     const uint32_t e0 = (wave + k * n_wave) * 256u + 4u * lane;
     const bool active = e0 < n;
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -260,7 +259,7 @@ __device__ __forceinline__ void ogm_norm_quant_row(float *__restrict__ x, const 
       if (normed) *(float4 *)(normed + e0) = o;
     }
     if ((wave + k * n_wave) * 256u < n)  // wave-uniform: the run exists
-      ogm_quantize_store<GROUP, COHERENT_OUT>(o, e0, active, lane, act.q, act.d, act.sums, act.bsum, act.bs16, act.xt);
+      ogm_quantize_store<GROUP>(o, e0, active, lane, act.q, act.d, act.sums, act.bsum, act.bs16, act.xt);
   }
 }
 
