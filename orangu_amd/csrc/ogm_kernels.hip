@@ -1310,11 +1310,11 @@ __device__ __forceinline__ void gemv_fused_body(const GemvFusedParams &fp, const
       am[i] = ogm_nan_blind_max(am[i], fabsf(v[k][i].w));
     }
     float amax = ogm_nan_blind_max(ogm_nan_blind_max(am[0], am[1]), ogm_nan_blind_max(am[2], am[3]));
-    amax = ogm_butterfly_step<1>(amax, OgmOpNanBlindMax());
+    amax = ogm_butterfly_step<1>(amax, OgmOpMax());
     if constexpr (GROUP == 256) {
-      amax = ogm_butterfly_step<2>(amax, OgmOpNanBlindMax());
-      amax = ogm_butterfly_step<4>(amax, OgmOpNanBlindMax());
-      amax = ogm_butterfly_step<8>(amax, OgmOpNanBlindMax());
+      amax = ogm_butterfly_step<2>(amax, OgmOpMax());
+      amax = ogm_butterfly_step<4>(amax, OgmOpMax());
+      amax = ogm_butterfly_step<8>(amax, OgmOpMax());
     }
     const float scale = amax / 127.0f;
     const float inv = scale > 0.0f ? 1.0f / scale : 0.0f;

@@ -12,9 +12,10 @@
 
 #include "ogm_kernels.h"
 
-// max(m, a) ignoring a NaN `a`; m is never one (the folds start at 0).  (fmaxf returns the other operand for a NaN, and
-// is one instruction where the compiler knows that `a` is no signalling NaN, two otherwise.)
-__device__ __forceinline__ float ogm_nan_blind_max(float m, float a) { return fmaxf(m, a); }
+// max(m, a) ignoring a NaN `a` of any payload; m is never one (the folds start at 0).  (A comparison and a select:
+// fmaxf may become v_max_f32 or v_max3_f32 over the bare operands, which answer a signalling NaN with a NaN, and then
+// what came before it in the fold is lost.)
+__device__ __forceinline__ float ogm_nan_blind_max(float m, float a) { return a > m ? a : m; }
 
 // One step of a butterfly all-reduce over the wave: joins groups of M lanes pairwise with a commutative
 // `op`.  For a value that is already equal within each group of M lanes (the state of a butterfly after its
@@ -73,7 +74,6 @@ __device__ __forceinline__ float ogm_row_quads_allreduce(float v, Op op) {
 }
 struct OgmOpMax { __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); } };
 struct OgmOpAdd { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
-struct OgmOpNanBlindMax { __device__ __forceinline__ float operator()(float a, float b) const { return ogm_nan_blind_max(a, b); } };
 // v summed over the wave, in the butterfly's order: ((lane + lane^1) + ...) level by level
 __device__ __forceinline__ float ogm_wave_sum(float v) {
   v = ogm_butterfly_step<1>(v, OgmOpAdd());
@@ -113,14 +113,14 @@ __device__ __forceinline__ uint32_t ogm_quantize4(const float4 &v, float &scale,
   amax = ogm_nan_blind_max(amax, fabsf(v.y));
   amax = ogm_nan_blind_max(amax, fabsf(v.z));
   amax = ogm_nan_blind_max(amax, fabsf(v.w));
-  // (no lane's amax is NaN -- the fold starts at 0 and skips them -- so the max commutes)
-  amax = ogm_butterfly_step<1>(amax, OgmOpNanBlindMax());
-  amax = ogm_butterfly_step<2>(amax, OgmOpNanBlindMax());
-  amax = ogm_butterfly_step<4>(amax, OgmOpNanBlindMax());
+  // (no lane's amax is NaN -- the fold starts at 0 and skips them -- so any max joins the lanes)
+  amax = ogm_butterfly_step<1>(amax, OgmOpMax());
+  amax = ogm_butterfly_step<2>(amax, OgmOpMax());
+  amax = ogm_butterfly_step<4>(amax, OgmOpMax());
   if constexpr (GROUP == 256) {
-    amax = ogm_butterfly_step<8>(amax, OgmOpNanBlindMax());
-    amax = ogm_butterfly_step<16>(amax, OgmOpNanBlindMax());
-    amax = ogm_butterfly_step<32>(amax, OgmOpNanBlindMax());
+    amax = ogm_butterfly_step<8>(amax, OgmOpMax());
+    amax = ogm_butterfly_step<16>(amax, OgmOpMax());
+    amax = ogm_butterfly_step<32>(amax, OgmOpMax());
   } else {
     static_assert(GROUP == 32, "groups of 32 or 256");
   }
