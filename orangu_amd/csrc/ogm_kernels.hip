@@ -1598,21 +1598,23 @@ hipError_t ogm_launch_gemv(const OgmGemvArgs &a, hipStream_t stream, const char 
   }
 }
 
-// The one-token GEMV's name for each type (ogm_last_kernel), whichever of its two kernels runs.
-static const char *gemv_name(uint32_t ggml_type) {
+// What ogm_last_kernel says of a launch that prepares its own activations.
+static const char *fused_name(uint32_t ggml_type, bool swiglu) {
+#define OGM_FUSED_NAME(F) (swiglu ? "ogm_gemv_fused_kernel<" #F ",swiglu>" : "ogm_gemv_fused_kernel<" #F ">")
   switch (ggml_type) {
-    case OGM_Q4_K: return "ogm_gemv_kernel<FmtQ4K,gemv>";
-    case OGM_Q5_K: return "ogm_gemv_kernel<FmtQ5K,gemv>";
-    case OGM_Q3_K: return "ogm_gemv_kernel<FmtQ3K,gemv>";
-    case OGM_Q6_K: return "ogm_gemv_kernel<FmtQ6K,gemv>";
-    case OGM_Q8_0: return "ogm_gemv_kernel<FmtQ80,gemv>";
-    case OGM_Q4_0: return "ogm_gemv_kernel<FmtQ40,gemv>";
-    case OGM_Q5_0: return "ogm_gemv_kernel<FmtQ50,gemv>";
-    case OGM_IQ4_NL: return "ogm_gemv_kernel<FmtIQ4NL,gemv>";
-    case OGM_Q5_1: return "ogm_gemv_kernel<FmtQ51,gemv>";
-    case OGM_IQ4_XS: return "ogm_gemv_kernel<FmtIQ4XS,gemv>";
-    default: return "ogm_gemv_kernel<FmtQ2K,gemv>";
+    case OGM_Q4_K: return OGM_FUSED_NAME(FmtQ4K);
+    case OGM_Q5_K: return OGM_FUSED_NAME(FmtQ5K);
+    case OGM_Q3_K: return OGM_FUSED_NAME(FmtQ3K);
+    case OGM_Q6_K: return OGM_FUSED_NAME(FmtQ6K);
+    case OGM_Q8_0: return OGM_FUSED_NAME(FmtQ80);
+    case OGM_Q4_0: return OGM_FUSED_NAME(FmtQ40);
+    case OGM_Q5_0: return OGM_FUSED_NAME(FmtQ50);
+    case OGM_IQ4_NL: return OGM_FUSED_NAME(FmtIQ4NL);
+    case OGM_Q5_1: return OGM_FUSED_NAME(FmtQ51);
+    case OGM_IQ4_XS: return OGM_FUSED_NAME(FmtIQ4XS);
+    default: return OGM_FUSED_NAME(FmtQ2K);
   }
+#undef OGM_FUSED_NAME
 }
 
 // How a fused launch of this shape is cut: waves a team, teams a workgroup, runs of 1024 a wave prepares (0: it can't).
@@ -1729,7 +1731,7 @@ hipError_t ogm_launch_gemv_fused_pair(const OgmGemvArgs &a, const OgmGemvArgs &b
   if (!ogm_gemv_fused_pair_can(a.ggml_type, b.ggml_type, a.in_dim, a.wg_waves) || a.in_dim != b.in_dim || !src.weight ||
       src.swiglu || a.n_extra > OGM_GEMV_MAX_MATS - 1 || b.n_extra > OGM_GEMV_MAX_MATS - 1)
     return hipErrorInvalidValue;
-  if (kernel_name) *kernel_name = gemv_name(a.ggml_type);
+  if (kernel_name) *kernel_name = a.ggml_type == OGM_Q4_K ? "ogm_gemv_fused_pair_kernel<FmtQ4K,FmtQ6K>" : "ogm_gemv_fused_pair_kernel<FmtQ5K,FmtQ6K>";
   return a.ggml_type == OGM_Q4_K ? launch_fused_pair_t<FmtQ4K, FmtQ6K>(a, b, src, stream)
                                  : launch_fused_pair_t<FmtQ5K, FmtQ6K>(a, b, src, stream);
 }
@@ -1764,7 +1766,7 @@ uint32_t ogm_gemv_row_blocks(uint32_t ggml_type, uint32_t in_dim, uint32_t out_d
 
 hipError_t ogm_launch_gemv_fused(const OgmGemvArgs &a, const OgmGemvSrc &src, hipStream_t stream, const char **kernel_name) {
   if (a.n_tokens != 1 || a.gemm_order || a.dump_isum || a.dump_imin || a.n_extra > OGM_GEMV_MAX_MATS - 1) return hipErrorInvalidValue;
-  if (kernel_name) *kernel_name = gemv_name(a.ggml_type);
+  if (kernel_name) *kernel_name = fused_name(a.ggml_type, src.swiglu);
 #define OGM_GO(F) launch_fused_t<F>(a, src, stream)
   OGM_FOR_TYPE(a.ggml_type, OGM_GO, hipErrorInvalidValue)
 #undef OGM_GO

@@ -180,3 +180,47 @@ def synth_weights(ggml_type: int, in_dim: int, out_dim: int, seed: int) -> np.nd
 def synth_x(n_tokens: int, in_dim: int, seed: int) -> np.ndarray:
     rng = np.random.default_rng(seed ^ 0x5EED)
     return rng.standard_normal((n_tokens, in_dim)).astype(np.float32)
+
+
+def captured_launches(stream, enqueue):
+    """The kernels that `enqueue` puts on `stream` (a hipStream_t), in order, as (name, template arguments as mangled,
+    workgroups, threads): taken from a stream capture whose graph is never launched.  What `enqueue` allocates on first
+    use must be there already."""
+    import ctypes as C
+    import re
+    from orangu_amd import hiprt
+
+    class Dim3(C.Structure):
+        _fields_ = [(d, C.c_uint32) for d in "xyz"]
+
+    class KernelNode(C.Structure):
+        _fields_ = [("block", Dim3), ("extra", C.c_void_p), ("func", C.c_void_p), ("grid", Dim3), ("params", C.c_void_p),
+                    ("lds", C.c_uint)]
+
+    L = hiprt.hip()
+    L.hipKernelNameRefByPtr.restype = C.c_char_p
+    s, graph, n = C.c_void_p(stream), C.c_void_p(), C.c_size_t()
+    hiprt.check(L.hipStreamBeginCapture(s, C.c_int(0)), "hipStreamBeginCapture")
+    try:
+        enqueue()
+    finally:
+        hiprt.check(L.hipStreamEndCapture(s, C.byref(graph)), "hipStreamEndCapture")
+    out = []
+    try:
+        hiprt.check(L.hipGraphGetNodes(graph, None, C.byref(n)), "hipGraphGetNodes")
+        nodes = (C.c_void_p * n.value)()
+        hiprt.check(L.hipGraphGetNodes(graph, nodes, C.byref(n)), "hipGraphGetNodes")
+        for node in nodes:
+            kind, k = C.c_int(), KernelNode()
+            hiprt.check(L.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)), "hipGraphNodeGetType")
+            if kind.value != 0:   # hipGraphNodeTypeKernel
+                continue
+            hiprt.check(L.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(k)), "hipGraphKernelNodeGetParams")
+            mangled = L.hipKernelNameRefByPtr(C.c_void_p(k.func), s).decode()
+            digits = re.match(r"_Z(\d+)", mangled)
+            at = digits.end()
+            end = at + int(digits.group(1))
+            out.append((mangled[at:end], mangled[end:], (k.grid.x, k.grid.y, k.grid.z), k.block.x))
+    finally:
+        hiprt.check(L.hipGraphDestroy(graph), "hipGraphDestroy")
+    return out

@@ -1,0 +1,57 @@
+"""Which kernels one-token calls run: read from a capture of the call (helpers.captured_launches), so that a comparison of
+two routes elsewhere is known to compare two routes."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import IQ4_NL, IQ4_XS, Q2_K, Q3_K, Q4_0, Q4_K, Q5_0, Q5_1, Q5_K, Q6_K, Q8_0, captured_launches, synth_weights
+
+pytestmark = pytest.mark.gpu
+FMT = {Q4_K: "FmtQ4K", Q5_K: "FmtQ5K", Q3_K: "FmtQ3K", Q6_K: "FmtQ6K", Q2_K: "FmtQ2K", IQ4_XS: "FmtIQ4XS", Q8_0: "FmtQ80",
+       Q4_0: "FmtQ40", Q5_0: "FmtQ50", IQ4_NL: "FmtIQ4NL", Q5_1: "FmtQ51"}
+# the template argument of the types whose Fmt name is an alias
+MANGLED = {Q4_0: "8FmtNib32ILi0E", Q5_0: "8FmtNib32ILi1E", IQ4_NL: "8FmtNib32ILi2E", Q5_1: "8FmtNib32ILi3E", Q2_K: "7FmtQ2KTILb0E"}
+
+
+@pytest.fixture(scope="module")
+def be():
+    from orangu_amd import Mi355xBackend
+    b = Mi355xBackend()
+    yield b
+    b.close()
+
+
+@pytest.fixture(scope="module")
+def stream():
+    from orangu_amd import hiprt
+    s = hiprt.Stream()
+    yield s
+    s.destroy()
+
+
+def launches(stream, call):
+    """The call's launches; it runs once before, so that its scratch is there."""
+    call()
+    stream.synchronize()
+    return captured_launches(stream.ptr, call)
+
+
+@pytest.mark.parametrize("t", sorted(FMT))
+@pytest.mark.parametrize("prologue", [1, 2])
+def test_last_kernel_names_the_kernel_that_ran(be, stream, t, prologue):
+    in_dim, out_dim = 1024, 40
+    w = be.upload_raw(synth_weights(t, in_dim, out_dim, seed=t), t, in_dim, out_dim)
+    x, y = torch.ones(in_dim, device="cuda"), torch.empty(out_dim, device="cuda")
+    torch.cuda.synchronize()
+    be.set_tuning("gemv_prologue", prologue)
+    try:
+        ran = launches(stream, lambda: be.matmul_dev(w, x.data_ptr(), 1, y.data_ptr(), False, stream.ptr))
+    finally:
+        be.set_tuning("gemv_prologue", 0)
+    name = be.last_kernel()
+    be.free_weight(w)
+    print(t, prologue, name, ran, flush=True)
+    assert [k[0] for k in ran] == (["ogm_quantize_kernel", "ogm_gemv_kernel"] if prologue == 1 else ["ogm_gemv_fused_kernel"])
+    assert name.split("<")[0] == ran[-1][0]
+    assert name.split("<")[1].rstrip(">").split(",")[0] == FMT[t]
+    assert ran[-1][1].startswith("I" + MANGLED.get(t, str(len(FMT[t])) + FMT[t]))
