@@ -17,9 +17,10 @@
 // ------------------------------------------------------------------------------------------
 // residual add + RMSNorm + quantize
 
-// One workgroup per row (ogm_norm_quant_row).
-template <int GROUP, int RUNS>
-__global__ __launch_bounds__(1024) void ogm_norm_quant_kernel(float *__restrict__ x,
+// One workgroup per row (ogm_norm_quant_row).  DENSE: in 64 registers, where RUNS 4 takes one more and a compute unit then
+// holds one workgroup of sixteen waves instead of two.
+template <int GROUP, int RUNS, bool DENSE>
+__global__ __launch_bounds__(1024, DENSE ? 8 : 1) void ogm_norm_quant_kernel(float *__restrict__ x,
                                                               const float *__restrict__ delta,
                                                               const float *__restrict__ weight, uint32_t n,
                                                               float eps, float *__restrict__ normed,
@@ -48,20 +49,32 @@ hipError_t ogm_launch_norm_quant(int mode, float *x, const float *delta, const f
                                  const float *x_src) {
   if (n == 0 || n % 32u != 0 || n > 16384u || n_rows == 0) return hipErrorInvalidValue;
   const uint32_t runs = (n + 255u) / 256u;
-  // few rows: a wave per run, the shortest chain (rows of more than sixteen: four runs a wave); from 1024 rows four runs
-  // per wave (the row's bits do not depend on it)
-  const bool one = n_rows < 1024u && runs <= 16u;
-  const dim3 threads((one ? runs : (runs + 3u) / 4u) * 64u);
-#define OGM_NORM(GROUP, RUNS)                                                                                      \
-  hipLaunchKernelGGL((ogm_norm_quant_kernel<GROUP, RUNS>), dim3(n_rows), threads, 0, stream, x, delta, weight, n, \
-                     eps, normed, act, x_src)
-  if (mode == 0) {
-    if (one) OGM_NORM(32, 1);
-    else OGM_NORM(32, 4);
-  } else {
-    if (one) OGM_NORM(256, 1);
-    else OGM_NORM(256, 4);
-  }
+  // A wave's loads leave together, so few runs a wave make the shortest chain: one on rows of up to sixteen runs, two on
+  // up to 32, three and four beyond, where a workgroup has its sixteen waves.  From 1024 narrow rows on the device is
+  // full and two runs a wave halve the waves; more rows than compute units at four runs a wave run two to a unit.
+  // us, sixteen waves with loads behind branches (a quarter as many waves as runs from 1024 rows) / four runs a wave /
+  // this rule:
+  //   1 row      5120 inputs 4.18 / 4.86 / 3.83, 8192 5.26 / 5.11 / 4.56, 10240 5.87 / 6.02 / 5.36, 16384 8.27 / 7.65 / 7.65
+  //   128 rows   5120 inputs 4.85 / 5.49 / 4.57, 8192 6.10 / 5.92 / 5.46, 16384 10.5 / 9.2 / 9.2 (DENSE 9.8)
+  //   1000 rows  5120 inputs 14.8 / 12.6 / 13.4, 10240 24.8 / 27.2 / 20.7, 14336 32.7 / 36.7 / 29.1, 16384 36.9 / 39.9 / 34.6
+  //   2048 rows  2048 inputs 10.8 / 9.6 / 8.7, 4096 20.9 / 18.4 / 17.0, 5120 26.1 / 22.5 / 22.9, 16384 76 / 85 / 77
+  // (the row's bits do not depend on it)
+  const uint32_t per_wave = runs > 48u ? 4u : runs > 32u ? 3u : (runs > 16u || n_rows >= 1024u) ? 2u : 1u;
+  const dim3 threads((per_wave > 2u ? 16u : (runs + per_wave - 1u) / per_wave) * 64u);
+#define OGM_NORM(GROUP, RUNS, DENSE)                                                                            \
+  hipLaunchKernelGGL((ogm_norm_quant_kernel<GROUP, RUNS, DENSE>), dim3(n_rows), threads, 0, stream, x, delta,   \
+                     weight, n, eps, normed, act, x_src)
+#define OGM_NORM_GROUP(GROUP)                                     \
+  do {                                                            \
+    if (per_wave == 1u) OGM_NORM(GROUP, 1, false);                \
+    else if (per_wave == 2u) OGM_NORM(GROUP, 2, false);           \
+    else if (per_wave == 3u) OGM_NORM(GROUP, 3, false);           \
+    else if (n_rows <= 256u) OGM_NORM(GROUP, 4, false);           \
+    else OGM_NORM(GROUP, 4, true);                                \
+  } while (0)
+  if (mode == 0) OGM_NORM_GROUP(32);
+  else OGM_NORM_GROUP(256);
+#undef OGM_NORM_GROUP
 #undef OGM_NORM
   return hipGetLastError();
 }
