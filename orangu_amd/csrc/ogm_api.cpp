@@ -592,16 +592,28 @@ static bool outputs_overlap(const Target *tg, size_t n_tg, const float *x, uint3
   return false;
 }
 
+// Whether p lies in the context's own GPU's memory.  Elsewhere -- the library's or a caller's pinned row, another GPU's
+// memory -- a row is read once, by a quantizer launch, and not over the bus by every workgroup of a launch that prepares
+// its own (pinned x, separate / prepared, us: Q4_K 4096 -> 8192 6.9 / 8.6, 14336 -> 2048 9.3 / 15.8).  The question
+// takes 0.06 us and is put again on every call.
+static bool in_device_memory(const ogm_ctx *ctx, const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && a.device == ctx->device;
+}
+
 // Enqueues quantize + kernels for tokens of x_dev into the targets' outputs.  Caller holds the
 // lock and has checked that the targets share type and in_dim.
-// x_in_host_memory: x lies behind the bus, where it is read once and not by every workgroup.
 static int enqueue_matmul(ogm_ctx *ctx, const Target *tg, size_t n_tg, const float *x_dev,
                           uint32_t n_tokens, int decode, hipStream_t stream, int32_t *dump_isum,
-                          int32_t *dump_imin, bool x_in_host_memory = false) {
+                          int32_t *dump_imin) {
   if (n_tokens == 0 || n_tg == 0) return OGM_OK;
   const ogm_weight *w = tg[0].w;
-  if (n_tokens == 1 && !dump_isum && !dump_imin && !x_in_host_memory && gemv_prepares(ctx, tg, n_tg, false, false) &&
-      !outputs_overlap(tg, n_tg, x_dev, w->in_dim)) {
+  if (n_tokens == 1 && !dump_isum && !dump_imin && gemv_prepares(ctx, tg, n_tg, false, false) &&
+      !outputs_overlap(tg, n_tg, x_dev, w->in_dim) && in_device_memory(ctx, x_dev)) {
     int rc = ensure_act(ctx, w->in_dim, 1);
     if (rc != OGM_OK) return rc;
     OgmGemvSrc src;
@@ -625,9 +637,9 @@ static int enqueue_matmul(ogm_ctx *ctx, const Target *tg, size_t n_tg, const flo
 
 static int enqueue_matmul(ogm_ctx *ctx, const ogm_weight *w, const float *x_dev, uint32_t n_tokens,
                           float *y_dev, int decode, hipStream_t stream, int32_t *dump_isum,
-                          int32_t *dump_imin, bool x_in_host_memory = false) {
+                          int32_t *dump_imin) {
   const Target t{w, y_dev};
-  return enqueue_matmul(ctx, &t, 1, x_dev, n_tokens, decode, stream, dump_isum, dump_imin, x_in_host_memory);
+  return enqueue_matmul(ctx, &t, 1, x_dev, n_tokens, decode, stream, dump_isum, dump_imin);
 }
 
 // Builds the prefill planes of a K-quant matrix on first use, within the context's budget.  Returns
@@ -931,7 +943,7 @@ static int host_matmul(ogm_ctx *ctx, const ogm_weight *w, const float *x, uint32
     // a decode-sized call: the kernels read x from, and write y to, the pinned staging buffers over
     // the bus themselves; two copy-engine transfers and their latencies fall away
     rc = enqueue_matmul(ctx, w, (const float *)ctx->hx.p, n_tokens, (float *)ctx->hy.p, decode, ctx->stream,
-                        nullptr, nullptr, true);
+                        nullptr, nullptr);
     if (rc != OGM_OK) return rc;
   } else {
     if ((rc = ensure_dev(ctx, ctx->x, xb)) != OGM_OK) return rc;
@@ -1251,7 +1263,7 @@ extern "C" int ogm_matmul_batch(ogm_ctx *ctx, const ogm_op *ops, size_t n_ops, i
       for (size_t k = i; k < e; k++)
         tg.push_back(Target{ops[k].w, (float *)(y_base + yoff[k]) + (size_t)t0 * ops[k].w->out_dim});
       rc = enqueue_matmul(ctx, tg.data(), tg.size(), xd + (size_t)t0 * op.w->in_dim, nt, decode,
-                          ctx->stream, nullptr, nullptr, zc);
+                          ctx->stream, nullptr, nullptr);
       if (rc != OGM_OK) return rc;
     }
     i = e;

@@ -55,3 +55,27 @@ def test_last_kernel_names_the_kernel_that_ran(be, stream, t, prologue):
     assert name.split("<")[0] == ran[-1][0]
     assert name.split("<")[1].rstrip(">").split(",")[0] == FMT[t]
     assert ran[-1][1].startswith("I" + MANGLED.get(t, str(len(FMT[t])) + FMT[t]))
+
+
+def test_a_row_behind_the_bus_is_read_once(be, stream):
+    """A caller's pinned row goes through a quantizer launch, alone and for several matrices; one in device memory (also
+    from the middle of an allocation) is prepared by the launch.  Same bits."""
+    in_dim, out_dim = 4096, 600
+    ws = [be.upload_raw(synth_weights(Q4_K, in_dim, o, seed=o), Q4_K, in_dim, o) for o in (out_dim, 40)]
+    x = torch.randn(8 + in_dim)
+    on_device, pinned = x.cuda(), x.pin_memory()
+    got = []
+    for rows in (on_device, pinned):
+        y = [torch.zeros(o, device="cuda") for o in (out_dim, out_dim, 40)]
+        torch.cuda.synchronize()
+        ran = launches(stream, lambda: (be.matmul_dev(ws[0], rows.data_ptr() + 32, 1, y[0].data_ptr(), False, stream.ptr),
+                                        be.matmul_multi_dev(ws, rows.data_ptr() + 32, 1, [y[1].data_ptr(), y[2].data_ptr()],
+                                                            True, stream.ptr)))
+        stream.synchronize()
+        assert [k[0] for k in ran] == 2 * (["ogm_gemv_fused_kernel"] if rows is on_device else
+                                           ["ogm_quantize_kernel", "ogm_gemv_kernel"])
+        got.append([v.cpu().numpy().view(np.uint32) for v in y])
+    for w in ws:
+        be.free_weight(w)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
