@@ -1691,7 +1691,11 @@ static int llama_norm_matmul(ogm_ctx *ctx, ogm_llama *m, DecodeRow &row, const f
   int rc;
   const bool swiglu = did_swiglu && e == 2 && n == 2 && ws[0]->out_dim == ws[1]->out_dim && gemv_prepares(ctx, tg, e, true, true);
   if (did_swiglu) *did_swiglu = swiglu;
-  // what is left of the group, of one other type: in the same launch where both would fit the line
+  // What is left of the group, of one other type, joins the launch where its own share is within the line too; together
+  // they may reach one and a half lines (v has k's rows, at most q's) or two (gate and up).  Measured with 12 layers, us a
+  // layer, one launch / prepared q and k, then a launch for v / norm and two launches: 4096 wide, q/k 2048 + v 1024
+  // 33.5 / 34.9 / 40.3; 3072 wide, 1536 + 768 31.7 / 33.7 / 39.9; 5120 wide, 1920 + 320 43.9 / 47.9 / 50.5; gate 2048 + up
+  // 2048 at 4096 wide 39.9 / 39.9 / 41.7, at 2048 wide 40.7 / 40.2 / 42.1.
   Target tg2[OGM_GEMV_MAX_MATS];
   bool both = e < n && n - e <= OGM_GEMV_MAX_MATS && ogm_gemv_fused_pair_can(ws[0]->ggml_type, ws[e]->ggml_type, ws[0]->in_dim, (uint32_t)ctx->tune_wg_waves);
   for (size_t i = e; both && i < n; i++) {
