@@ -922,7 +922,7 @@ __global__ __launch_bounds__(64) void ogm_swiglu_quant_kernel(const float *__res
     if (act.bs16) act.bs16 += (size_t)r * (n / 16u);
     act.xt = ogm_xt_row(act.xt, r, n);
   }
-  ogm_swiglu_quant_run<GROUP, false>(gate, up, n, h, act, run, lane);
+  ogm_swiglu_quant_run<GROUP>(gate, up, n, h, act, run, lane);
 }
 
 hipError_t ogm_launch_swiglu_quant(int mode, const float *gate, const float *up, uint32_t n, float *h,

@@ -136,19 +136,10 @@ __device__ __forceinline__ uint32_t ogm_quantize4(const float4 &v, float &scale,
   return ogm_pack4(q0, q1, q2, q3);
 }
 
-// A store that workgroups of the same kernel on other compute dies may read (with a device-coherent
-// load) once this wave's stores are acknowledged: it goes through to the level all dies share.
-template <bool COHERENT, class T>
-__device__ __forceinline__ void ogm_st(T *p, T v) {
-  if constexpr (COHERENT) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  else *p = v;
-}
-
 // Quantizes and stores one lane's share of a 256-run whose first element is e0 (= 256*run +
 // 4*lane) of token-major activations with row length in_dim; t_off* are the token's offsets.  Returns the
 // lane's four quantized values, packed.
-// COHERENT_OUT: the stores are for other workgroups of the same kernel (ogm_st).
-template <int GROUP, bool COHERENT_OUT = false>
+template <int GROUP>
 __device__ __forceinline__ uint32_t ogm_quantize_store(const float4 &v, uint32_t e0, bool active, uint32_t lane,
                                                        int8_t *q, float *d, int32_t *sums, int16_t *bsum,
                                                        uint16_t *bs16, int8_t *xt_row = nullptr) {
@@ -156,18 +147,18 @@ __device__ __forceinline__ uint32_t ogm_quantize_store(const float4 &v, uint32_t
   int s16, s32;
   const uint32_t packed = ogm_quantize4<GROUP>(v, scale, s16, s32);
   if (active) {
-    ogm_st<COHERENT_OUT>((uint32_t *)(q + e0), packed);
-    if ((lane & 3u) == 0) ogm_st<COHERENT_OUT>(sums + e0 / 16, (int32_t)s16);
+    *(uint32_t *)(q + e0) = packed;
+    if ((lane & 3u) == 0) sums[e0 / 16] = s16;
     if ((lane & 7u) == 0) {
-      ogm_st<COHERENT_OUT>(bsum + e0 / 32, (int16_t)s32);
+      bsum[e0 / 32] = (int16_t)s32;
       if (GROUP == 256 && bs16 != nullptr) {
         // |s32| <= 32 * 127: floor(s32 / 64) and s32 mod 64 are exact in f16
         uint16_t *b = bs16 + (e0 / 256u) * 16u + ((e0 / 32u) & 7u);
-        ogm_st<COHERENT_OUT>(b, __half_as_ushort(__float2half_rn((float)(s32 >> 6))));
-        ogm_st<COHERENT_OUT>(b + 8, __half_as_ushort(__float2half_rn((float)(s32 & 63))));
+        b[0] = __half_as_ushort(__float2half_rn((float)(s32 >> 6)));
+        b[8] = __half_as_ushort(__float2half_rn((float)(s32 & 63)));
       }
     }
-    if ((lane & (GROUP / 4 - 1)) == 0) ogm_st<COHERENT_OUT>(d + e0 / GROUP, scale);
+    if ((lane & (GROUP / 4 - 1)) == 0) d[e0 / GROUP] = scale;
     // the token's place in the operand chunks (ogm_xt_row): chunk e0 / 32, half (e0 / 16) & 1 of its k, byte e0 & 15
     if (xt_row != nullptr) *(uint32_t *)(xt_row + (e0 >> 5) * 1024u + ((e0 >> 4) & 1u) * 512u + (e0 & 15u)) = packed;
   }
@@ -189,19 +180,6 @@ __device__ __forceinline__ int8_t *ogm_xt_row(int8_t *xt, uint32_t t, uint32_t n
 __device__ __forceinline__ uint32_t ogm_xt_row_of_workgroup(uint32_t b, uint32_t n) {
   if ((b | 63u) >= n) return b;
   return (b & ~63u) | ((b & 7u) << 3) | ((b >> 3) & 7u);
-}
-
-// Four floats that another workgroup of the same kernel may have stored device-coherently.
-template <bool COHERENT>
-__device__ __forceinline__ float4 ogm_ld4(const float *p) {
-  if constexpr (COHERENT) {
-    const uint64_t a = __hip_atomic_load((const uint64_t *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint64_t b = __hip_atomic_load((const uint64_t *)p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return make_float4(__uint_as_float((uint32_t)a), __uint_as_float((uint32_t)(a >> 32)),
-                       __uint_as_float((uint32_t)b), __uint_as_float((uint32_t)(b >> 32)));
-  } else {
-    return *(const float4 *)p;
-  }
 }
 
 // Residual add, RMSNorm and quantization of one row by one workgroup of n_wave waves (n <= 256 * RUNS * n_wave): wave w
@@ -263,9 +241,8 @@ __device__ __forceinline__ void ogm_norm_quant_row(float *__restrict__ x, const 
   }
 }
 
-// SwiGLU and quantization of one 256-run by one wave: h = silu(gate) * up.  COHERENT: gate and up were
-// written by other workgroups of the calling kernel; COHERENT_OUT: the quantized run is for them.
-template <int GROUP, bool COHERENT, bool COHERENT_OUT = false>
+// SwiGLU and quantization of one 256-run by one wave: h = silu(gate) * up.
+template <int GROUP>
 __device__ __forceinline__ void ogm_swiglu_quant_run(const float *__restrict__ gate, const float *__restrict__ up,
                                                      uint32_t n, float *__restrict__ h, const OgmActDev &act,
                                                      uint32_t run, uint32_t lane) {
@@ -273,12 +250,12 @@ __device__ __forceinline__ void ogm_swiglu_quant_run(const float *__restrict__ g
   const bool active = e0 < n;
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
   if (active) {
-    const float4 g = ogm_ld4<COHERENT>(gate + e0), u = ogm_ld4<COHERENT>(up + e0);
+    const float4 g = *(const float4 *)(gate + e0), u = *(const float4 *)(up + e0);
     o.x = g.x / (1.0f + expf(-g.x)) * u.x;
     o.y = g.y / (1.0f + expf(-g.y)) * u.y;
     o.z = g.z / (1.0f + expf(-g.z)) * u.z;
     o.w = g.w / (1.0f + expf(-g.w)) * u.w;
     if (h) *(float4 *)(h + e0) = o;
   }
-  ogm_quantize_store<GROUP, COHERENT_OUT>(o, e0, active, lane, act.q, act.d, act.sums, act.bsum, act.bs16, act.xt);
+  ogm_quantize_store<GROUP>(o, e0, active, lane, act.q, act.d, act.sums, act.bsum, act.bs16, act.xt);
 }
