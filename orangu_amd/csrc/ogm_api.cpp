@@ -538,10 +538,12 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
 
 // Whether a one-token launch over these matrices (one type and in_dim) prepares its own activations: where the work
 // that every workgroup repeats -- row blocks times runs of 1024 inputs, eight a compute unit at the line -- costs less
-// than the launch it saves.  Measured, whole calls, us, separate / prepared: at 2048 Q4_K 4096 -> 8192 6.9 / 6.3, 2048 ->
-// 2 x 8192 7.1 / 6.4, Q6_K 8.4 / 8.1 and 9.0 / 8.2; above, 11008 -> 4096 (2816) 9.1 / 9.0, 14336 -> 4096 (3584) 9.5 / 9.5,
-// 4096 -> 14336 (3584) 9.0 / 9.4, 8192 -> 8192 (4096) 10.3 / 11.1.  The per-32 types' workgroups have sixteen waves of
-// small tiles and gain less: Q8_0 4096 -> 2048 (512) 6.6 / 6.3, 4096 -> 4096 (1024) 7.1 / 7.6, 8192 -> 2048 (1024) 10.9 / 10.9.
+// than the launch it saves.  Measured, whole calls, us, separate / prepared, at 2048: Q4_K 4096 -> 8192 6.2 / 4.7, 2048 ->
+// 16384 6.8 / 5.4, 7680 -> 4096 7.0 / 5.8, 3328 -> 32768 12.8 / 11.7, 16384 -> 2048 8.9 / 8.8; Q6_K 4096 -> 8192 7.6 / 6.1,
+// 2048 -> 16384 8.7 / 6.7; the per-32 types at 512: Q8_0 4096 -> 2048 6.4 / 4.9, 16384 -> 512 1.2 less.  The line lies where
+// the launches' pointers in private memory had put it; above it prepared launches are ahead too by now, by less of the call: Q4_K
+// 4096 -> 14336 (3584) 8.8 / 7.0, 11008 -> 4096 (2816) 8.5 / 8.3, 8192 -> 8192 (4096) 9.4 / 8.6, 4096 -> 28672 (7168) 13.1 /
+// 11.8, Q8_0 4096 -> 4096 (1024) 6.8 / 5.2; until rows of several tiles a wave: Q6_K 2816 -> 27264 (5112) 14.5 / 17.4.
 static const uint32_t OGM_PREPARE_MAX_WORK = 2048, OGM_PREPARE_MAX_WORK_32 = 512;
 static bool gemv_prepares(const ogm_ctx *ctx, const Target *tg, size_t n_tg, bool norm, bool swiglu) {
   if (ctx->tune_gemv_prologue == 1 || n_tg == 0 || n_tg > OGM_GEMV_MAX_MATS) return false;

@@ -1188,6 +1188,20 @@ struct GemvFusedParams {
   uint32_t teams, team_waves;
 };
 
+// v[m] for the wave's own matrix m, by selects over scalar registers.  (Left to itself the compiler indexes the kernel's
+// arguments by m in private memory: 40 bytes a lane, stored by every wave at its start and loaded again between the
+// ordered sum and the output's store.)
+template <class T>
+__device__ __forceinline__ T of_matrix(T a, T b, T c, T d, uint32_t m) {
+  asm("" : "+s"(a), "+s"(b), "+s"(c), "+s"(d));
+  return m == 0 ? a : m == 1 ? b : m == 2 ? c : d;
+}
+// Likewise of pointers, which are to global memory (through the asm alone they would be to any, and every load a flat one).
+template <class T>
+__device__ __forceinline__ T *of_matrix(T *const (&v)[OGM_GEMV_MAX_MATS], uint32_t m) {
+  return (T *)(__attribute__((address_space(1))) T *)of_matrix((uint64_t)v[0], (uint64_t)v[1], (uint64_t)v[2], (uint64_t)v[3], m);
+}
+
 // NQ: runs of 1024 elements a wave prepares.  bid: the workgroup's number among those of its type; leads: it stores the
 // quantized row and the residual stream.
 template <class F, int UPR, int PRE, int NQ, bool SWIGLU>
@@ -1215,21 +1229,20 @@ __device__ __forceinline__ void gemv_fused_body(const GemvFusedParams &fp, const
 
   // ---- this wave's team and its row block (a team past the last one multiplies the last again and stores nothing)
   const uint32_t team = teams == 1u ? 0u : wave / tw, wv = wave - team * tw;
-  auto locate = [&](uint32_t team_, uint32_t &m, uint32_t &rb) -> bool {
-    if (SWIGLU) {
-      m = team_;
-      rb = bid;
-      return true;
-    }
-    const uint32_t last = p.wg_end[OGM_GEMV_MAX_MATS - 1] - 1u, want = bid * teams + team_;
+  uint32_t m = 0, rb0 = bid;
+  bool mine = true;
+  if (SWIGLU) {
+    m = team;
+  } else {
+    const uint32_t last = p.wg_end[OGM_GEMV_MAX_MATS - 1] - 1u, want = bid * teams + team;
     const uint32_t b = min(want, last);
     m = (b >= p.wg_end[0] ? 1u : 0u) + (b >= p.wg_end[1] ? 1u : 0u) + (b >= p.wg_end[2] ? 1u : 0u);
-    rb = b - (m == 0 ? 0u : m == 1 ? p.wg_end[0] : m == 2 ? p.wg_end[1] : p.wg_end[2]);
-    return want <= last;
-  };
-  uint32_t m, rb0;
-  locate(team, m, rb0);
-  const uint8_t *wt = m == 0 ? p.wt[0] : m == 1 ? p.wt[1] : m == 2 ? p.wt[2] : p.wt[3];
+    rb0 = b - of_matrix(0u, p.wg_end[0], p.wg_end[1], p.wg_end[2], m);
+    mine = want <= last;
+  }
+  const uint8_t *wt = of_matrix(p.wt, m);
+  float *y = SWIGLU ? p.y[0] : of_matrix(p.y, m);
+  const uint32_t out_dim = SWIGLU ? p.out_dim[0] : of_matrix(p.out_dim[0], p.out_dim[1], p.out_dim[2], p.out_dim[3], m);
   const size_t tile0 = (size_t)rb0 * nct;
 
   // ---- the row's loads, ahead of every weight load of the workgroup (as in ogm_gemv_kernel)
@@ -1370,21 +1383,17 @@ __device__ __forceinline__ void gemv_fused_body(const GemvFusedParams &fp, const
   }
   __syncthreads();
 
-  for (uint32_t i = tid; i < teams * R; i += nthr) {
-    const uint32_t t = i / R, r = i - t * R;
-    uint32_t om, orb;
-    const bool mine = locate(t, om, orb);
-    const uint32_t out_dim = om == 0 ? p.out_dim[0] : om == 1 ? p.out_dim[1] : om == 2 ? p.out_dim[2] : p.out_dim[3];
-    const uint32_t orow = orb * R + r;
-    const bool store = mine && orow < out_dim;
-    const float acc = store ? ordered_sum<false>(0.0f, l_term + (size_t)t * term_stride + r, upr, R) : 0.0f;
-    if constexpr (SWIGLU) {   // R <= 32: gate and up of a row are in one wave, and so are all 2 R lanes of this pass
-      const float up = __shfl(acc, (int)((lane + R) & 63u));
-      if (store && t == 0) p.y[0][orow] = acc / (1.0f + expf(-acc)) * up;
-    } else {
-      float *y = om == 0 ? p.y[0] : om == 1 ? p.y[1] : om == 2 ? p.y[2] : p.y[3];
-      if (store) y[orow] = acc;
-    }
+  if constexpr (SWIGLU) {   // R <= 32: the first wave adds gate and up of a row up, one in each half
+    if (wave != 0u) return;
+    const uint32_t t = lane / R, r = lane - t * R, orow = rb0 * R + r;
+    const bool have = t < 2u && orow < out_dim;
+    const float acc = have ? ordered_sum<false>(0.0f, l_term + (size_t)t * term_stride + r, upr, R) : 0.0f;
+    const float up = __shfl(acc, (int)((lane + R) & 63u));
+    if (have && t == 0u) y[orow] = acc / (1.0f + expf(-acc)) * up;
+  } else {   // a team's first wave adds its row block up
+    if (wv != 0u || !mine) return;
+    const uint32_t orow = rb0 * R + lane;
+    if (lane < R && orow < out_dim) y[orow] = ordered_sum<false>(0.0f, my_term + lane, upr, R);
   }
 }
 

@@ -184,7 +184,7 @@ def synth_x(n_tokens: int, in_dim: int, seed: int) -> np.ndarray:
 
 def captured_launches(stream, enqueue):
     """The kernels that `enqueue` puts on `stream` (a hipStream_t), in order, as (name, template arguments as mangled,
-    workgroups, threads): taken from a stream capture whose graph is never launched.  What `enqueue` allocates on first
+    workgroups, threads, bytes of private memory a lane): taken from a stream capture whose graph is never launched.  What `enqueue` allocates on first
     use must be there already."""
     import ctypes as C
     import re
@@ -196,6 +196,10 @@ def captured_launches(stream, enqueue):
     class KernelNode(C.Structure):
         _fields_ = [("block", Dim3), ("extra", C.c_void_p), ("func", C.c_void_p), ("grid", Dim3), ("params", C.c_void_p),
                     ("lds", C.c_uint)]
+
+    class FuncAttributes(C.Structure):
+        _fields_ = [("binary", C.c_int), ("cache", C.c_int), ("const_bytes", C.c_size_t), ("local_bytes", C.c_size_t),
+                    ("rest", C.c_int * 16)]
 
     L = hiprt.hip()
     L.hipKernelNameRefByPtr.restype = C.c_char_p
@@ -220,7 +224,9 @@ def captured_launches(stream, enqueue):
             digits = re.match(r"_Z(\d+)", mangled)
             at = digits.end()
             end = at + int(digits.group(1))
-            out.append((mangled[at:end], mangled[end:], (k.grid.x, k.grid.y, k.grid.z), k.block.x))
+            attrs = FuncAttributes()
+            hiprt.check(L.hipFuncGetAttributes(C.byref(attrs), C.c_void_p(k.func)), "hipFuncGetAttributes")
+            out.append((mangled[at:end], mangled[end:], (k.grid.x, k.grid.y, k.grid.z), k.block.x, attrs.local_bytes))
     finally:
         hiprt.check(L.hipGraphDestroy(graph), "hipGraphDestroy")
     return out

@@ -137,7 +137,9 @@ def test_decode_steps_give_the_same_bits(be, types, n_embd, n_ff, layer):
                 assert np.array_equal(xd.cpu().numpy(), xs[pos])   # the caller's row stays as it was
             out.append(dev.hidden())
         got[mode] = out
-        ran = route(captured_launches(stream.ptr, lambda: dev.decode_dev(xd.data_ptr(), 3, lg.data_ptr(), tok.data_ptr(), stream.ptr)))
+        launched = captured_launches(stream.ptr, lambda: dev.decode_dev(xd.data_ptr(), 3, lg.data_ptr(), tok.data_ptr(), stream.ptr))
+        ran = route(launched)
+        assert all(k[4] == 0 for k in launched if "fused" in k[0])
         v_apart = "G" if types[0] != types[1] else ""
         assert ran == 3 * (layer if mode == 2 else "NG" + v_apart + "AGNGsG") + "NG"
     be.set_tuning("gemv_prologue", 0)

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import IQ4_NL, IQ4_XS, Q2_K, Q3_K, Q4_0, Q4_K, Q5_0, Q5_1, Q5_K, Q6_K, Q8_0, captured_launches, synth_weights
+from helpers import BLOCK, IQ4_NL, IQ4_XS, Q2_K, Q3_K, Q4_0, Q4_K, Q5_0, Q5_1, Q5_K, Q6_K, Q8_0, captured_launches, synth_weights
 
 pytestmark = pytest.mark.gpu
 FMT = {Q4_K: "FmtQ4K", Q5_K: "FmtQ5K", Q3_K: "FmtQ3K", Q6_K: "FmtQ6K", Q2_K: "FmtQ2K", IQ4_XS: "FmtIQ4XS", Q8_0: "FmtQ80",
@@ -79,3 +79,38 @@ def test_a_row_behind_the_bus_is_read_once(be, stream):
         be.free_weight(w)
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("t", sorted(FMT))
+def test_prepared_rows_use_no_private_memory(be, stream, t):
+    """Alone and several matrices at a time, at row lengths that are constants of the kernel and at others, a wave
+    preparing one run of 1024 or two.  (An array indexed by a lane's own number ends there: every wave stored it at its
+    start, and at the line calls took up to an eighth longer than after a quantizer launch.)"""
+    be.set_tuning("gemv_prologue", 2)
+    try:
+        for in_dim in (1024, 4096, 8960, 14336):
+            ws = [be.upload_raw(synth_weights(t, in_dim, o, seed=o), t, in_dim, o) for o in (33, 20)]
+            x, y = torch.ones(in_dim, device="cuda"), [torch.empty(33, device="cuda") for _ in ws]
+            torch.cuda.synchronize()
+            ran = launches(stream, lambda: (be.matmul_dev(ws[0], x.data_ptr(), 1, y[0].data_ptr(), False, stream.ptr),
+                                            be.matmul_multi_dev(ws, x.data_ptr(), 1, [v.data_ptr() for v in y], True, stream.ptr)))
+            for w in ws:
+                be.free_weight(w)
+            assert [(k[0], k[4]) for k in ran] == 2 * [("ogm_gemv_fused_kernel", 0)], (in_dim, ran)
+    finally:
+        be.set_tuning("gemv_prologue", 0)
+
+
+# (row blocks x runs of 1024 up to 2048, 512 for the per-32 types; row blocks of 16 rows, of 64 at 7 blocks a row)
+@pytest.mark.parametrize("t,in_dim,out_dim,prepared", [
+    (Q4_K, 4096, 512 * 16, True), (Q4_K, 4096, 512 * 16 + 1, False), (Q6_K, 2816, 682 * 16, True), (Q6_K, 2816, 682 * 16 + 1, False),
+    (Q4_K, 1792, 1024 * 64, True), (Q8_0, 2048, 256 * 16, True), (Q8_0, 2048, 256 * 16 + 1, False)])
+def test_the_line(be, stream, t, in_dim, out_dim, prepared):
+    bytes_, elems = BLOCK[t]
+    raw = np.zeros(out_dim * (in_dim // elems) * bytes_, np.uint8)
+    w = be.upload_raw(raw, t, in_dim, out_dim)
+    x, y = torch.ones(in_dim, device="cuda"), torch.empty(out_dim, device="cuda")
+    torch.cuda.synchronize()
+    ran = launches(stream, lambda: be.matmul_dev(w, x.data_ptr(), 1, y.data_ptr(), False, stream.ptr))
+    be.free_weight(w)
+    assert [k[0] for k in ran] == (["ogm_gemv_fused_kernel"] if prepared else ["ogm_quantize_kernel", "ogm_gemv_kernel"])
