@@ -1171,18 +1171,67 @@ hipError_t ogm_launch_dequant_row(const uint8_t *wt, uint32_t ggml_type, uint32_
 // prefill: the same layer over a batch of tokens.  The matmuls are GEMMs that quantize their
 // own input, so these kernels leave plain f32 rows.
 
-// A wave takes one head of q | k | v over IT tokens (twice as many at HD 64, whose pairs fill half a wave): bias,
-// per-head norm and RoPE as the decode kernel's first phase; q is rewritten in place, k and v go to their cache rows as
-// f16.  Bound: the trip to memory, of which a wave of one token makes one after the other with the launch's other
-// waves (a 2048-wide layer's 48 heads at 1901 tokens: eleven rounds of waves, 18 us for 47 MB); so from 256 tokens on a
-// wave requests four (eight) tokens' values before it works on the first.
-template <int HD, int IT>
+// One wave per (token, head of q | k | v): bias, per-head norm and RoPE as the decode kernel's
+// first phase; q is rewritten in place, k and v go to their cache rows as f16.
+template <int HD>
 __global__ __launch_bounds__(256) void ogm_qkv_pre_kernel(float *__restrict__ q, const float *__restrict__ k,
                                                           const float *__restrict__ v,
                                                           const float2 *__restrict__ cs, uint32_t rope_half,
                                                           OgmAttnPre pre, uint32_t n_head, uint32_t n_head_kv,
                                                           __half *__restrict__ kc, __half *__restrict__ vc,
-                                                          uint32_t pos0, uint32_t n_tokens) {
+                                                          uint32_t pos0) {
+  static_assert(HD == 64 || HD == 128, "a lane holds one pair");
+  const uint32_t p = threadIdx.x & 63u;
+  const uint32_t u = blockIdx.x * 4u + (threadIdx.x >> 6), tok = blockIdx.y;
+  if (u >= n_head + 2u * n_head_kv) return;
+  const bool is_q = u < n_head, is_v = u >= n_head + n_head_kv;
+  const uint32_t head = is_q ? u : (is_v ? u - n_head - n_head_kv : u - n_head);
+  const size_t kv_dim = (size_t)n_head_kv * HD;
+  const size_t row = (size_t)head * HD;   // within a token's vector and within the bias
+  float *qrow = q + (size_t)tok * n_head * HD + row;
+  const float *src = is_q ? qrow : (is_v ? v : k) + (size_t)tok * kv_dim + row;
+  const float *bias = is_q ? pre.q_bias : is_v ? pre.v_bias : pre.k_bias;
+  const float *nw = is_q ? pre.q_norm : is_v ? nullptr : pre.k_norm;
+  cs += (size_t)tok * rope_half;
+  const bool have = p < (uint32_t)(HD / 2);
+  const bool split_pair = pre.neox != 0u && !is_v && p < rope_half;
+  const uint32_t ia = split_pair ? p : 2u * p, ib = split_pair ? p + rope_half : 2u * p + 1u;
+  float2 ab = make_float2(have ? src[ia] : 0.0f, have ? src[ib] : 0.0f);
+  if (bias != nullptr && have) {
+    ab.x += bias[row + ia];
+    ab.y += bias[row + ib];
+  }
+  if (nw != nullptr) {
+    const float ss = ogm_wave_sum(ab.x * ab.x + ab.y * ab.y);
+    const float sc_n = 1.0f / sqrtf(ss / (float)HD + pre.eps);
+    if (have) {
+      ab.x = ab.x * sc_n * nw[ia];
+      ab.y = ab.y * sc_n * nw[ib];
+    }
+  }
+  if (!have) return;
+  if (!is_v && p < rope_half) ab = rope_pair(ab, cs[p]);
+  if (is_q) {
+    qrow[ia] = ab.x;
+    qrow[ib] = ab.y;
+  } else {
+    __half *cache = (is_v ? vc : kc) + (size_t)(pos0 + tok) * kv_dim + row;
+    cache[ia] = ogm_f16_sat(ab.x);
+    cache[ib] = ogm_f16_sat(ab.y);
+  }
+}
+
+// The same where the launch would have several rounds of such waves, each a trip to memory after the other (a 2048-wide
+// layer's 48 heads at 1901 tokens: eleven rounds, 18 us for 47 MB): a wave takes one head over four tokens (eight at HD
+// 64, whose pairs fill half a wave) and requests all their values before it works on the first.
+template <int HD>
+__global__ __launch_bounds__(256) void ogm_qkv_pre_tokens_kernel(float *__restrict__ q, const float *__restrict__ k,
+                                                                 const float *__restrict__ v,
+                                                                 const float2 *__restrict__ cs, uint32_t rope_half,
+                                                                 OgmAttnPre pre, uint32_t n_head, uint32_t n_head_kv,
+                                                                 __half *__restrict__ kc, __half *__restrict__ vc,
+                                                                 uint32_t pos0, uint32_t n_tokens) {
+  constexpr int IT = 4;
   static_assert(HD == 64 || HD == 128, "a lane holds one pair");
   constexpr uint32_t LPT = HD / 2, TPI = 64u / LPT;   // lanes a token, tokens an iteration
   const uint32_t lane = threadIdx.x & 63u, p = lane % LPT;
@@ -1255,19 +1304,27 @@ hipError_t ogm_launch_qkv_pre(float *q, const float *k, const float *v, const vo
                               hipStream_t stream) {
   if (rope_dim > head_dim || rope_dim % 2u != 0 || n_tokens == 0 || n_tokens > 65535u) return hipErrorInvalidValue;
   if (head_dim != 64 && head_dim != 128) return hipErrorInvalidValue;
-  const bool many = n_tokens >= 256u;
-  const uint32_t per_wave = (many ? 4u : 1u) * (head_dim == 64 ? 2u : 1u);
-  const dim3 grid((n_head + 2u * n_head_kv + 3u) / 4u, (n_tokens + per_wave - 1u) / per_wave);
-#define OGM_PRE(HD, IT)                                                                                            \
-  hipLaunchKernelGGL((ogm_qkv_pre_kernel<HD, IT>), grid, dim3(256), 0, stream, q, k, v, (const float2 *)cs,       \
-                     rope_dim / 2u, pre, n_head, n_head_kv, (__half *)k_cache_layer, (__half *)v_cache_layer, pos0, n_tokens)
-  if (head_dim == 128) {
-    if (many) OGM_PRE(128, 4);
-    else OGM_PRE(128, 1);
-  } else {
-    if (many) OGM_PRE(64, 4);
-    else OGM_PRE(64, 1);
-  }
+  // The line lies where the device's 8192 waves have been dealt out once or twice.  us, a wave a token / four (eight)
+  // tokens a wave: heads of 64, 8 x 1024 (8192 waves) 2.76 / 3.00, 48 x 256 (12288) 3.32 / 3.26, 48 x 512 (24576) 4.88 /
+  // 3.97, 48 x 2048 14.7 / 8.9; heads of 128, 20 x 512 (10240) 3.56 / 3.90, 48 x 300 (14400) 4.26 / 4.40, 80 x 256 (20480)
+  // 5.37 / 5.20, 48 x 512 (24576) 6.07 / 5.69, 80 x 2048 27.3 / 22.2; below, 6 to 8 heads at up to 512 tokens 2.5 / 2.9,
+  // with per-head norms 2.5 / 3.3.
+  const uint32_t heads = n_head + 2u * n_head_kv, gx = (heads + 3u) / 4u;
+  const bool many = (uint64_t)heads * n_tokens >= (head_dim == 64 ? 12288u : 20480u);
+  const uint32_t per_wave = head_dim == 64 ? 8u : 4u;
+#define OGM_PRE(HD)                                                                                                  \
+  do {                                                                                                               \
+    if (many)                                                                                                        \
+      hipLaunchKernelGGL(ogm_qkv_pre_tokens_kernel<HD>, dim3(gx, (n_tokens + per_wave - 1u) / per_wave), dim3(256),  \
+                         0, stream, q, k, v, (const float2 *)cs, rope_dim / 2u, pre, n_head, n_head_kv,              \
+                         (__half *)k_cache_layer, (__half *)v_cache_layer, pos0, n_tokens);                          \
+    else                                                                                                             \
+      hipLaunchKernelGGL(ogm_qkv_pre_kernel<HD>, dim3(gx, n_tokens), dim3(256), 0, stream, q, k, v,                  \
+                         (const float2 *)cs, rope_dim / 2u, pre, n_head, n_head_kv, (__half *)k_cache_layer,         \
+                         (__half *)v_cache_layer, pos0);                                                             \
+  } while (0)
+  if (head_dim == 128) OGM_PRE(128);
+  else OGM_PRE(64);
 #undef OGM_PRE
   return hipGetLastError();
 }

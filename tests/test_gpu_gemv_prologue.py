@@ -179,13 +179,13 @@ def test_two_types_at_the_line(be, n_head, n_kv, layer, wgs):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
-# (the kernel between the projections and the attention takes several tokens a wave from 256 on, two at a time where a
-# head has 64 elements; the norm two runs of 256 a wave from 1024 rows)
+# (the kernel between the projections and the attention takes several tokens a wave from 12288 waves of one on at heads of
+# 64, from 20480 at 128; the norm two runs of 256 a wave from 1024 rows)
 @pytest.mark.parametrize("n_embd,n_head,n_kv,hd,rope_dim,neox,pre,n_tokens", [
-    (256, 4, 2, 64, 64, False, (), 257), (256, 4, 1, 64, 64, True, ("q_bias", "k_bias", "v_bias"), 263),
+    (256, 32, 8, 64, 64, False, (), 257), (256, 4, 1, 64, 64, True, ("q_bias", "k_bias", "v_bias"), 263),
     (256, 2, 2, 128, 128, False, ("q_norm", "k_norm"), 259), (512, 4, 4, 64, 64, False, ("q_norm", "k_norm"), 1027),
-    (1280, 2, 1, 128, 128, True, (), 1025), (256, 4, 2, 64, 24, False, ("q_norm", "k_norm"), 258),
-    (256, 4, 2, 64, 48, True, ("q_bias", "k_bias", "v_bias"), 261), (512, 4, 1, 128, 96, True, (), 260),
+    (1280, 32, 4, 128, 128, True, (), 1025), (256, 32, 8, 64, 24, False, ("q_norm", "k_norm"), 258),
+    (256, 32, 8, 64, 48, True, ("q_bias", "k_bias", "v_bias"), 261), (512, 64, 8, 128, 96, True, (), 260),
     (512, 4, 2, 128, 2, False, (), 262)])
 def test_batches_leave_the_rows_of_smaller_ones(be, n_embd, n_head, n_kv, hd, rope_dim, neox, pre, n_tokens):
     """Cache rows of a batch against those of the same tokens in parts of at most 100 (a wave a token).  The second
