@@ -2545,13 +2545,13 @@ __device__ __forceinline__ half8 gw_i8_to_f16(uint32_t w0, uint32_t w1) {
 // A block's integer dot is exact on the matrix cores: weights and activations are int8 values as
 // f16, a 32-long sum is at most 32 * 127 * 127 < 2^24.  Each block (two K = 16 MFMA steps) starts a
 // fresh accumulator and ends with the reference's f32 step, so the f32 work per MFMA is eight times
-// Q4_K's.  Bound: a SIMD's vector and matrix instructions take their turns -- counters at 4096 -> 14336, 512 tokens:
-// 174 k cycles of vector instructions and 86 k of matrix instructions in the 266 k a SIMD has work for -- so what
-// counts is the sum.  Hence the scales' products ad * dw come from an outer product (one v_mfma_f32_32x32x1_2b for 64
+// Q4_K's.  Bound: a SIMD's vector and matrix instructions together fill its time -- counters at 4096 -> 14336, 512 tokens:
+// 174 k cycles of vector instructions and 86 k of matrix instructions in the 266 k a SIMD has work for -- so the sum
+// is what counted.  Hence the scales' products ad * dw come from an outer product (one v_mfma_f32_32x32x1_2b for 64
 // rows x 32 tokens, 32 cycles a 32 x 32 block where sixteen multiplies take 64) and the activations become f16 once,
 // in the feeding waves, instead of in each of the multiplying ones: 149 -> 130 us (Q4_0) and 157 -> 133 (Q8_0).
 // Interleaving the f32 step with the next block's matrix instructions, operands fetched a block ahead, 64 x 64 outputs
-// a wave: no faster (132 to 155).
+// a wave: no faster (132 to 155), for a reason that is not known.
 //
 // Workgroup = 128 rows x 128 tokens, twelve waves: eight multiplying (64 rows x 32 tokens each),
 // four feeding.  A stage is 64 k = two blocks.  LDS rows are padded by one chunk (see the wide

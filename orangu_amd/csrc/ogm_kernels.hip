@@ -1706,6 +1706,8 @@ static hipError_t launch_fused_t(const OgmGemvArgs &a, const OgmGemvSrc &src, hi
     if (p.upr == HOT) OGM_FUSED(HOT, 1, 1, false);
     else OGM_FUSED(0, 1, 1, false);
   } else {
+    // (two runs a wave over two tiles: with the row length a constant Q4_K 14336 -> 512 takes 7.2 us, without 8.4, after a
+    // quantizer launch 7.6; -> 2048 7.6, 8.8 and 8.2)
     if (K && p.upr == 56) OGM_FUSED((K ? 56 : 0), 1, 2, false);
     else OGM_FUSED(0, 1, 2, false);
   }
