@@ -96,6 +96,15 @@ __host__ __device__ inline size_t gp_plane_offset(uint32_t rb, uint32_t nsb, uin
                                                   uint32_t npl) {
   return ((((size_t)rb * nsb + s) * 4u + g) * 4u + t16) * (npl * 1024u);
 }
+// Behind the planes of `nrb` row blocks of 64: the rows' d as f32 ([32-row block][super-block][32], negated for Q3_K),
+// then for Q4_K / Q5_K the rows' dmin alike and the mins as the K = 16 operand of the first pass ([32-row block]
+// [super-block][64 lanes] of 16 bytes).
+__host__ __device__ inline size_t gp_d_offset(uint32_t nrb, uint32_t nsb, uint32_t npl) { return gp_plane_offset(nrb, nsb, 0, 0, 0, npl); }
+__host__ __device__ inline size_t gp_dmin_offset(uint32_t nrb, uint32_t nsb, uint32_t npl) { return gp_d_offset(nrb, nsb, npl) + (size_t)nrb * nsb * 256u; }
+__host__ __device__ inline size_t gp_mins_offset(uint32_t nrb, uint32_t nsb, uint32_t npl) { return gp_dmin_offset(nrb, nsb, npl) + (size_t)nrb * nsb * 256u; }
+__host__ __device__ inline size_t gp_total_bytes(uint32_t nrb, uint32_t nsb, uint32_t npl, bool mins) {
+  return mins ? gp_mins_offset(nrb, nsb, npl) + (size_t)nrb * nsb * 2048u : gp_dmin_offset(nrb, nsb, npl);
+}
 
 // ROWS = 128: eight multiplying waves (32 rows x 64 tokens each) and eight feeding ones; ROWS = 64:
 // four and four, and half the LDS: twice as many workgroups, which fills the chip when a launch has
@@ -639,31 +648,52 @@ __global__ __launch_bounds__(256) void ogm_gemm_build_planes_kernel(GemmPlaneBui
   if constexpr (!Q3) *(uint4 *)(dst + 1024u) = make_uint4(pl[0], pl[1], pl[2], pl[3]);
 }
 
+// What the plane kernels read of a block's header, in their order (gp_d_offset ..): a wave per 32 rows of a super-block.
+template <int KIND>
+__global__ __launch_bounds__(64) void ogm_gemm_build_side_kernel(GemmPlaneBuildParams p) {
+  constexpr bool Q3 = KIND == GP_Q3K, Q45 = KIND == GP_Q4K || KIND == GP_Q5K, Q6 = KIND == GP_Q6K, XS = KIND == GP_IQ4XS;
+  constexpr uint32_t TILE_BYTES = Q3 ? 7168u : (KIND == GP_Q4K || XS) ? 9216u : Q6 ? 13440u : 11264u;
+  constexpr uint32_t NPL = Q3 ? 1u : 2u;
+  const uint32_t lane = threadIdx.x, l32 = lane & 31u, lh = lane >> 5, b = blockIdx.x, s = blockIdx.y;
+  const uint32_t row = min(32u * b + l32, p.out_dim - 1u);   // rows past the matrix repeat its last one
+  const uint32_t r = row & ((1u << p.r_shift) - 1u), c = s & ((1u << p.c_shift) - 1u);
+  const uint8_t *tile = p.wt + ((size_t)(row >> p.r_shift) * p.nct + (s >> p.c_shift)) * TILE_BYTES;
+  const uint32_t unit = (c << p.r_shift) + r;   // this row's lane of the tile
+  const uint4 hd = *(const uint4 *)(tile + unit * 16u + (Q3 ? 6u * 1024u : 0u));
+  const uint32_t db = Q3 ? hd.w : Q6 ? *(const uint16_t *)(tile + 13u * 1024u + unit * 2u) : hd.x;
+  const float d = gm_f16_bits_to_f32(db & 0xFFFFu);
+  const uint32_t nrb = (p.out_dim + 63u) / 64u;
+  const size_t at = ((size_t)b * p.nsb + s) * 32u;
+  if (lh == 0u) ((float *)(p.planes + gp_d_offset(nrb, p.nsb, NPL)))[at + l32] = Q3 ? -d : d;
+  if constexpr (Q45) {
+    if (lh == 0u) ((float *)(p.planes + gp_dmin_offset(nrb, p.nsb, NPL)))[at + l32] = gm_f16_bits_to_f32(hd.x >> 16);
+    uint32_t mna, mnb;
+    q4k_mins(hd, mna, mnb);
+    *(half8 *)(p.planes + gp_mins_offset(nrb, p.nsb, NPL) + at * 32u + lane * 16u) = side_operand(mna, mnb, lh ? 1.0f : 64.0f);
+  }
+}
+
 // ------------------------------------------------------------------------------------------
-// The K-quant GEMM over prebuilt planes with every wave multiplying (no feeding waves): operands
-// go from global memory straight into LDS (global_load_lds_dwordx4: no registers, no vector
-// work), in the order the matrix instruction wants them, so a wave's operand read is 64 lanes x 16
-// consecutive bytes.  Same arithmetic and f32 order as gemm_q6k_i8_body; bit-identical results.
+// The K-quant GEMMs over prebuilt planes with every wave multiplying (no feeding waves): operands go from global memory
+// straight into LDS (load-to-LDS: no registers, no vector work), in the order the matrix instruction wants them, so a
+// wave's operand read is 64 lanes x 16 consecutive bytes.
 //
+// First the option without a first pass:
 //   workgroup  256 threads = 4 waves; 128 rows x 128 tokens; wave w: rows 32 w .. + 31, all tokens.
-//              Two workgroups share a compute unit (two waves per SIMD, 74 KiB of LDS each): while
-//              one adds a super-block's sums up in f32 the other multiplies.
+//              Two workgroups share a compute unit (two waves per SIMD).
 //   step       32 weights of k: per wave the planes of its 32 rows (1 KiB each, fetched by the wave
 //              itself), per workgroup four token blocks of activations (1 KiB each, one per wave)
-//   ring       six steps in LDS: one multiplied, the next being read into registers behind it,
-//              four in flight.  At the top of step k a wave waits until its loads of step k + 1
-//              have landed (all but the newest three steps' loads), meets the others at a barrier,
-//              and fetches step k + 5 into the slot step k - 1 left.
-//   per super-block: the tokens' activation scales and the rows' d, fetched the same way one
-//              super-block ahead (4 bytes a lane), then acc += ad * (d * isum) as the CPU path adds it
+//   ring       five steps in LDS: one multiplied, the next being read into registers behind it,
+//              three in flight.  At the top of step k a wave waits until its loads of step k + 1
+//              have landed, meets the others at a barrier, and fetches step k + 4 into the slot step k - 1 left.
+//   per super-block: the tokens' activation scales, sums and the rows' headers, fetched the same way one
+//              super-block ahead
 //
 // The compiler cannot tell which LDS reads a load-to-LDS in flight may alias and would wait for all
-// of them before every LDS read; the operand and table reads of the main loop are therefore written
+// of them before every LDS read; the operand and table reads of the main loops are therefore written
 // as ds_read instructions with their own waits (LDS reads return in order: "at most N outstanding"
-// means all but the newest N have landed).  No scalar loads may be issued inside the loop (they
+// means all but the newest N have landed).  No scalar loads may be issued inside the loops (they
 // share the counter and return out of order), which the launch parameters being read up front ensures.
-//
-// Registers: 8 accumulators of the planes (4 token blocks x h, l), 4 of y, 6 operands: 216 of a wave's 256.
 struct GemmDmaParams {
   const uint8_t *wt;       // tile-planar weights (headers: d, dmin, mins)
   const uint8_t *planes;   // ogm_gemm_build_planes_kernel's output
@@ -683,44 +713,14 @@ struct GemmDmaParams {
 #define GD_NW 4u                       // waves of a workgroup
 #define GD_ROWS (32u * GD_NW)
 #define GD_TOK 128u
-// timing experiments only (results are wrong with any of these set)
-#ifndef GD_ABL_SAMEROW
-#define GD_ABL_SAMEROW 0   // every workgroup reads row block 0's planes
-#endif
-#ifndef GD_ABL_NOSWZ
-#define GD_ABL_NOSWZ 0     // workgroups keep the grid's order
-#endif
-#ifndef GD_ABL_NOPASS1
-#define GD_ABL_NOPASS1 0
-#endif
-#ifndef GD_ABL_NOEPI
-#define GD_ABL_NOEPI 0
-#endif
-#ifndef GD_ABL_NOMFMA
-#define GD_ABL_NOMFMA 0
-#endif
-#ifndef GD_ABL_NODMA
-#define GD_ABL_NODMA 0
-#endif
-#ifndef GD_ABL_NOBAR
-#define GD_ABL_NOBAR 0
-#endif
-#ifndef GD_ABL_NOLDS
-#define GD_ABL_NOLDS 0
-#endif
-#ifndef GD_RING
-#define GD_RING 6u
-#endif
+#define GD_RING 5u
 #define GD_AHEAD (GD_RING - 1u)        // steps fetched ahead of the one multiplied
 #define GD_XOFF (GD_NW * 2048u)        // activations of a step, after the weights' 2 KiB per wave
-#define GD_SLOT (GD_XOFF + 4096u)      // bytes of a step in LDS (one-plane types leave half the weights' part unused)
-#define GD_TAB (GD_RING * GD_SLOT)     // two slots of per-super-block tables: 128 ad, then the rows' header words
-#define GD_TAB_SLOT (512u + 4u * GD_ROWS)
+#define GD_SLOT (GD_XOFF + 4096u)      // bytes of a step in LDS
+#define GD_TAB (GD_RING * GD_SLOT)     // two slots of per-super-block tables:
+// 128 ad, the rows' 16-byte headers, the tokens' sums per 32 as f16 pairs (32 bytes a token)
+#define GD_TAB_SLOT (512u + 16u * GD_ROWS + 32u * GD_TOK)
 #define GD_LDS_BYTES (GD_TAB + 2u * GD_TAB_SLOT)
-// one-pass variant: 128 ad, the rows' 16-byte headers, the tokens' sums per 32 as f16 pairs (32 bytes a token)
-#define GD_RING_ONEPASS 5u
-#define GD_TAB_SLOT_ONEPASS (512u + 16u * GD_ROWS + 32u * GD_TOK)
-#define GD_LDS_BYTES_ONEPASS (GD_RING_ONEPASS * GD_SLOT + 2u * GD_TAB_SLOT_ONEPASS)
 
 __device__ __forceinline__ void gd_dma16(const uint8_t *src, uint8_t *lds_chunk) {
   // 16 bytes per lane from src (per lane) to lds_chunk + 16 * lane (lds_chunk is wave-uniform)
@@ -739,11 +739,7 @@ __device__ __forceinline__ void gd_dma4(const uint8_t *src, uint8_t *lds_chunk) 
 #define GD_WAIT2(N, A, B) asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(A), "+v"(B) : "n"(N))
 // all loads of this wave but the newest N have landed; then the workgroup's barrier (no fence: the
 // data other waves wait for came by load-to-LDS, which the wait covers)
-#if GD_ABL_NOBAR
-#define GD_SYNC(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
-#else
 #define GD_SYNC(N) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory")
-#endif
 
 // The activations in the matrix instruction's operand order: chunk (token block of 32, step of 32 k)
 // is 1 KiB, lane (l32, lh)'s 16 bytes -- the activations 32 step + 16 lh .. of token 32 block + l32 --
@@ -766,29 +762,17 @@ __global__ __launch_bounds__(256) void ogm_gemm_xtile_kernel(const int8_t *__res
   *(uint4 *)(xt + ((size_t)tb * (in_dim / 32u) + k0 / 32u + step) * 1024u + slot * 16u) = v;
 }
 
-#if GD_ABL_NOMFMA
-#define GD_MFMA(A, B, C, X, Y, Z) ((C) + (A).x + (B).x)
-#else
 #define GD_MFMA(A, B, C, X, Y, Z) __builtin_amdgcn_mfma_i32_32x32x32_i8(A, B, C, X, Y, Z)
-#endif
-#if GD_ABL_NOLDS
-#define GD_RD if (0)
-#else
-#define GD_RD
-#endif
-// ONEPASS (Q4_K, Q5_K): no first pass; a super-block's step is acc += ad * (d * isum - dmin * imin), the
-// single-token expression (vecdot.rs:3152-3178), with imin from the same K = 16 f16 instruction.  The integer
-// sums are the same; the f32 result differs from the two-pass order by rounding only.  The rows' whole headers
-// and the tokens' sums per 32 then travel with the tables, and the ring is one step shorter to make room.
-template <int KIND, bool ONEPASS = false>
-__global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_dma_kernel(GemmDmaParams p) {
-  constexpr bool Q3 = KIND == GP_Q3K, Q45 = KIND == GP_Q4K || KIND == GP_Q5K, Q5 = KIND == GP_Q5K, Q6 = KIND == GP_Q6K;
-  constexpr bool XS = KIND == GP_IQ4XS;   // (no first pass, as Q6_K; its d is the first half of the header word, as Q4_K's)
-  static_assert(!ONEPASS || Q45, "only the types with mins have a first pass to fold");
-  constexpr uint32_t RING = ONEPASS ? GD_RING_ONEPASS : GD_RING, AHEAD = RING - 1u;
-  constexpr uint32_t TAB = RING * GD_SLOT, TAB_SLOT = ONEPASS ? GD_TAB_SLOT_ONEPASS : GD_TAB_SLOT;
-  constexpr uint32_t TILE_BYTES = Q3 ? 7168u : (KIND == GP_Q4K || XS) ? 9216u : Q5 ? 11264u : 13440u;
-  constexpr uint32_t NPL = Q3 ? 1u : 2u;
+// Q4_K and Q5_K without a first pass ("gemm_one_pass"): a super-block's step is acc += ad * (d * isum - dmin * imin), the
+// single-token expression (vecdot.rs:3152-3178), with imin from a K = 16 f16 instruction.  The integer sums are those of
+// the kernels below; the f32 result differs from the two-pass order by rounding only.  The rows' whole headers and the
+// tokens' sums per 32 travel with the tables.
+template <int KIND>
+__global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_onepass_kernel(GemmDmaParams p) {
+  static_assert(KIND == GP_Q4K || KIND == GP_Q5K, "only the types with mins have a first pass to fold");
+  constexpr uint32_t RING = GD_RING, AHEAD = GD_AHEAD, TAB = GD_TAB, TAB_SLOT = GD_TAB_SLOT;
+  constexpr uint32_t TILE_BYTES = KIND == GP_Q4K ? 9216u : 11264u;
+  constexpr uint32_t NPL = 2u;
   constexpr int PER = (int)NPL + 1;   // loads a wave issues per step
   extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -799,7 +783,7 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_dma_kernel(GemmDmaPara
   uint32_t tok_tile = blockIdx.x, row_tile = blockIdx.y;
   {
     const uint32_t nt = gridDim.x, lin = blockIdx.y * nt + blockIdx.x;
-    if (!GD_ABL_NOSWZ && lin < (gridDim.y & ~7u) * nt) {
+    if (lin < (gridDim.y & ~7u) * nt) {
       const uint32_t j = lin >> 3;
       tok_tile = j % nt;
       row_tile = (j / nt) * 8u + (lin & 7u);
@@ -829,68 +813,11 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_dma_kernel(GemmDmaPara
 #pragma unroll
     for (int r = 0; r < 16; r++) y[tb][r] = 0.0f;
 
-  if constexpr (Q45 && !ONEPASS && !GD_ABL_NOPASS1) {
-    // ---------------- pass 1 of gemm_k_q4_k: acc -= (ad * dmin) * sum_j m_j * bsum_j over all
-    // super-blocks first (vecdot.rs:2226-2240), as gemm_q6k_i8_body does it: 64 m_j against bsum_j / 64
-    // and m_j against bsum_j % 64 in one K = 16 f16 instruction per 32 x 32 outputs.  The tokens' ad of
-    // every super-block sit in LDS (where the ring will be) for this pass.
-    // this lane's weight row (clamped: rows past the matrix are computed and never stored)
-    const uint32_t row = min(r0 + 32u * wave + l32, p.out_dim - 1u);
-    const uint32_t uo = (row >> p.r_shift) * p.nct * TILE_BYTES + (row & ((1u << p.r_shift) - 1u)) * 16u;
-    float *ad_all = (float *)lds;   // [nsb][128]
-    for (uint32_t i = tid; i < GD_TOK * p.nsb; i += 64u * GD_NW) {
-      const uint32_t k = i / p.nsb, su = i - k * p.nsb;
-      ad_all[su * GD_TOK + k] = p.ad[min(t0 + k, p.n_tokens - 1u) * p.nsb + su];
-    }
-    __syncthreads();
-    float16v zero;
-#pragma unroll
-    for (int r = 0; r < 16; r++) zero[r] = 0.0f;
-    uint32_t tk[4];
-#pragma unroll
-    for (int tb = 0; tb < 4; tb++) tk[tb] = min(t0 + 32u * tb + l32, p.n_tokens - 1u) * p.nsb;
-    const float side_scale = lh ? 1.0f : 64.0f;
-    // the header and the four tokens' sums of the next super-block are loaded while this one is added up
-    uint4 hd_n = *(const uint4 *)(p.wt + uo);
-    half8 b2_n[4];
-#pragma unroll
-    for (int tb = 0; tb < 4; tb++) b2_n[tb] = *(const half8 *)(p.bs16 + (tk[tb] * 16u + 8u * lh));
-    for (uint32_t su = 0; su < p.nsb; su++) {
-      const uint4 hd0 = hd_n;
-      half8 b2[4];
-#pragma unroll
-      for (int tb = 0; tb < 4; tb++) b2[tb] = b2_n[tb];
-      {
-        const uint32_t sn = min(su + 1u, p.nsb - 1u);   // past the end: loaded again, never used
-        hd_n = *(const uint4 *)(p.wt + (uo + sb_off(sn)));
-#pragma unroll
-        for (int tb = 0; tb < 4; tb++) b2_n[tb] = *(const half8 *)(p.bs16 + ((tk[tb] + sn) * 16u + 8u * lh));
-      }
-      uint32_t mna, mnb;
-      q4k_mins(hd0, mna, mnb);
-      const half8 a1 = side_operand(mna, mnb, side_scale);
-      const float dm = gm_f16_bits_to_f32(hd0.x >> 16);
-#pragma unroll
-      for (int tb = 0; tb < 4; tb++) {
-        const float16v im = __builtin_amdgcn_mfma_f32_32x32x16_f16(b2[tb], a1, zero, 0, 0, 0);
-        const float *adp = &ad_all[su * GD_TOK + 32u * tb + 4u * lh];
-#pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-          const float4 a4 = *(const float4 *)(adp + 8 * q4);
-          const float a4v[4] = {a4.x, a4.y, a4.z, a4.w};
-#pragma unroll
-          for (int e = 0; e < 4; e++) y[tb][4 * q4 + e] -= a4v[e] * dm * im[4 * q4 + e];
-        }
-      }
-    }
-    __syncthreads();   // the table's LDS becomes the ring
-  }
-
   // ---------------- the products
   // What this wave fetches per step: the plane chunks of its 32 rows (lane (l32, lh): the 16 weights
   // 16 lh .. of row l32, the matrix instruction's operand), and token block `wave` of the activations
   // (one chunk of ogm_gemm_xtile_kernel's layout).
-  const uint32_t prb = GD_ABL_SAMEROW ? 0u : min((r0 + 32u * wave) >> 6, (p.out_dim - 1u) >> 6);
+  const uint32_t prb = min((r0 + 32u * wave) >> 6, (p.out_dim - 1u) >> 6);
   uint32_t w_src = (prb * p.nsb * 16u + lh) * (NPL * 1024u) + (32u * (wave & 1u) + l32) * 16u;   // + step * NPL * 2048
   // (token blocks past the last one read it again; their outputs are never stored)
   uint32_t x_src = min((t0 >> 5) + wave, (p.n_tokens - 1u) >> 5) * (p.in_dim / 32u) * 1024u + lane * 16u;   // + step * 1024
@@ -902,38 +829,26 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_dma_kernel(GemmDmaPara
   } else {
     const uint32_t tab_row = min(r0 + 64u * ((wave - 2u) & 3u) + lane, p.out_dim - 1u);
     const uint32_t tab_rb = tab_row >> p.r_shift, tab_r = tab_row & ((1u << p.r_shift) - 1u);
-    if constexpr (Q6)        // d is the block's two-byte tail behind the 13 pieces: the aligned word that holds it
-      tab_src = tab_rb * p.nct * TILE_BYTES + 13u * 1024u + ((tab_r * 2u) & ~3u);
-    else if constexpr (Q3)   // scales[12] | d | padding
-      tab_src = tab_rb * p.nct * TILE_BYTES + tab_r * 16u + 6u * 1024u + 12u;
-    else                     // d | dmin
-      tab_src = tab_rb * p.nct * TILE_BYTES + tab_r * 16u;
+    tab_src = tab_rb * p.nct * TILE_BYTES + tab_r * 16u;
   }
-  // one-pass: token block `wave`'s sums per 32 (lane (l32, lh): the eight f16 of half lh of token l32)
+  // token block `wave`'s sums per 32 (lane (l32, lh): the eight f16 of half lh of token l32)
   const uint32_t bs_src = (min(t0 + 32u * wave + l32, p.n_tokens - 1u) * p.nsb * 16u + 8u * lh) * 2u;   // + 32 s
   auto fetch_tables = [&](uint32_t s) {   // for super-block s, into table slot s & 1
     uint8_t *slot = lds + TAB + (s & 1u) * TAB_SLOT;
     if (wave < 2u) {
       gd_dma4((const uint8_t *)p.ad + (tab_src + 4u * s), slot + 256u * wave);
     } else {
-      const uint32_t so = Q6 ? (s >> p.c_shift) * TILE_BYTES + ((s & ((1u << p.c_shift) - 1u)) << p.r_shift) * 2u : sb_off(s);
-      if constexpr (ONEPASS) gd_dma16(p.wt + (tab_src + so), slot + 512u + 1024u * (wave - 2u));
-      else gd_dma4(p.wt + (tab_src + so), slot + 512u + 256u * (wave - 2u));
+      gd_dma16(p.wt + (tab_src + sb_off(s)), slot + 512u + 1024u * (wave - 2u));
     }
-    if constexpr (ONEPASS)
-      gd_dma16((const uint8_t *)p.bs16 + (bs_src + 32u * s), slot + 512u + 16u * GD_ROWS + 1024u * wave);
+    gd_dma16((const uint8_t *)p.bs16 + (bs_src + 32u * s), slot + 512u + 16u * GD_ROWS + 1024u * wave);
   };
   uint32_t slot_fetch = 0;   // byte offset of the ring slot of the next step to fetch
   auto fetch_step = [&]() {   // the next step (they are fetched in ascending order) into its ring slot
     uint8_t *slot = lds + slot_fetch;
     slot_fetch = slot_fetch == (RING - 1u) * GD_SLOT ? 0u : slot_fetch + GD_SLOT;
-#if !GD_ABL_NOWDMA
     gd_dma16(p.planes + w_src, slot + w_dst);
-    if constexpr (!Q3) gd_dma16(p.planes + (w_src + 1024u), slot + w_dst + 1024u);
-#endif
-#if !GD_ABL_NOXDMA
+    gd_dma16(p.planes + (w_src + 1024u), slot + w_dst + 1024u);
     gd_dma16((const uint8_t *)p.xt + x_src, slot + x_dst);
-#endif
     w_src += NPL * 2048u;
     x_src += 1024u;
   };
@@ -946,19 +861,18 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_dma_kernel(GemmDmaPara
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
   const uint32_t w_rd = lds0 + w_dst + lane * 16u, x_rd = lds0 + GD_XOFF + lane * 16u;
   const uint32_t tab_rd = lds0 + TAB + 16u * lh;                    // + 128 tb + 32 q4: four tokens' ad
-  // the row's header word (one-pass: its 16-byte header)
-  const uint32_t hw_rd = lds0 + TAB + 512u + (ONEPASS ? 16u : 4u) * (32u * wave + l32);
-  const uint32_t bs_rd = lds0 + TAB + 512u + 16u * GD_ROWS + 16u * lane;   // one-pass: + 1024 tb
+  const uint32_t hw_rd = lds0 + TAB + 512u + 16u * (32u * wave + l32);   // the row's 16-byte header
+  const uint32_t bs_rd = lds0 + TAB + 512u + 16u * GD_ROWS + 16u * lane;   // + 1024 tb
   int16v h[4], l[4];
   const int16v zi = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   int4v wh, wl = {0, 0, 0, 0}, x0, x1, x2, x3;
-  // LDS reads outstanding at the top of a step, oldest first: wh, x0, x1, x2, x3, wl (one-plane types: no wl)
+  // LDS reads outstanding at the top of a step, oldest first: wh, x0, x1, x2, x3, wl
   GD_READ16(wh, w_rd, 0);
   GD_READ16(x0, x_rd, 0);
   GD_READ16(x1, x_rd, 1024);
   GD_READ16(x2, x_rd, 2048);
   GD_READ16(x3, x_rd, 3072);
-  if constexpr (!Q3) GD_READ16(wl, w_rd, 1024);
+  GD_READ16(wl, w_rd, 1024);
   uint32_t slot_next = GD_SLOT;   // byte offset of step k + 1's ring slot
   for (uint32_t s = 0; s < p.nsb; s++) {
 #pragma unroll
@@ -969,103 +883,55 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_dma_kernel(GemmDmaPara
       if (kk + AHEAD <= 8u || more) GD_SYNC((AHEAD - 2) * PER);
       else GD_SYNC(kk >= 6u ? 0 : (int)(6u - kk) * PER);
       if (kk == 0u && more) fetch_tables(s + 1u);
-      if ((kk + AHEAD < 8u || more) && !GD_ABL_NODMA) fetch_step();   // step k + AHEAD
+      if ((kk + AHEAD < 8u || more)) fetch_step();   // step k + AHEAD
       const uint32_t w_nx = w_rd + slot_next, x_nx = x_rd + slot_next;
       slot_next = slot_next == (RING - 1u) * GD_SLOT ? 0u : slot_next + GD_SLOT;
-      if constexpr (!Q3) {
-        constexpr int A0 = 4;   // outstanding after wh and x0: x1, x2, x3, wl
-        GD_WAIT2(A0, wh, x0);
-        h[0] = GD_MFMA(x0, wh, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : h[0], 0, 0, 0);
+      {
+        GD_WAIT2(4, wh, x0);   // outstanding after wh and x0: x1, x2, x3, wl
+        h[0] = GD_MFMA(x0, wh, kk == 0u ? zi : h[0], 0, 0, 0);
         GD_WAIT1(3, x1);
-        h[1] = GD_MFMA(x1, wh, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : h[1], 0, 0, 0);
+        h[1] = GD_MFMA(x1, wh, kk == 0u ? zi : h[1], 0, 0, 0);
         GD_WAIT1(2, x2);
-        h[2] = GD_MFMA(x2, wh, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : h[2], 0, 0, 0);
+        h[2] = GD_MFMA(x2, wh, kk == 0u ? zi : h[2], 0, 0, 0);
         GD_WAIT1(1, x3);
-        h[3] = GD_MFMA(x3, wh, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : h[3], 0, 0, 0);
-        GD_RD asm volatile("ds_read_b128 %0, %2 offset:0" : "=v"(wh) : "0"(wh), "v"(w_nx));
+        h[3] = GD_MFMA(x3, wh, kk == 0u ? zi : h[3], 0, 0, 0);
+        asm volatile("ds_read_b128 %0, %2 offset:0" : "=v"(wh) : "0"(wh), "v"(w_nx));
         GD_WAIT1(1, wl);
-        l[0] = GD_MFMA(x0, wl, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : l[0], 0, 0, 0);
-        GD_RD asm volatile("ds_read_b128 %0, %2 offset:0" : "=v"(x0) : "0"(x0), "v"(x_nx));
-        l[1] = GD_MFMA(x1, wl, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : l[1], 0, 0, 0);
-        GD_RD asm volatile("ds_read_b128 %0, %2 offset:1024" : "=v"(x1) : "0"(x1), "v"(x_nx));
-        l[2] = GD_MFMA(x2, wl, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : l[2], 0, 0, 0);
-        GD_RD asm volatile("ds_read_b128 %0, %2 offset:2048" : "=v"(x2) : "0"(x2), "v"(x_nx));
-        l[3] = GD_MFMA(x3, wl, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : l[3], 0, 0, 0);
-        GD_RD asm volatile("ds_read_b128 %0, %2 offset:3072" : "=v"(x3) : "0"(x3), "v"(x_nx));
-        GD_RD asm volatile("ds_read_b128 %0, %2 offset:1024" : "=v"(wl) : "0"(wl), "v"(w_nx));
-      } else {
-        // one plane: the next step's weights go to a second register set (this one is in use to the
-        // end); outstanding at the top, oldest first: wh, x0, x1, x2, x3
-        int4v wn;
-        GD_READ16(wn, w_nx, 0);
-        GD_WAIT2(4, wh, x0);
-        h[0] = GD_MFMA(x0, wh, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : h[0], 0, 0, 0);
-        GD_RD asm volatile("ds_read_b128 %0, %2 offset:0" : "=v"(x0) : "0"(x0), "v"(x_nx));
-        GD_WAIT1(4, x1);
-        h[1] = GD_MFMA(x1, wh, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : h[1], 0, 0, 0);
-        GD_RD asm volatile("ds_read_b128 %0, %2 offset:1024" : "=v"(x1) : "0"(x1), "v"(x_nx));
-        GD_WAIT1(4, x2);
-        h[2] = GD_MFMA(x2, wh, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : h[2], 0, 0, 0);
-        GD_RD asm volatile("ds_read_b128 %0, %2 offset:2048" : "=v"(x2) : "0"(x2), "v"(x_nx));
-        GD_WAIT1(4, x3);
-        h[3] = GD_MFMA(x3, wh, (kk == 0u && (!GD_ABL_NOEPI || s == 0u)) ? zi : h[3], 0, 0, 0);
-        GD_RD asm volatile("ds_read_b128 %0, %2 offset:3072" : "=v"(x3) : "0"(x3), "v"(x_nx));
-        // the next step wants wn first in line: it was issued before these four
-        GD_WAIT1(4, wn);
-        wh = wn;
+        l[0] = GD_MFMA(x0, wl, kk == 0u ? zi : l[0], 0, 0, 0);
+        asm volatile("ds_read_b128 %0, %2 offset:0" : "=v"(x0) : "0"(x0), "v"(x_nx));
+        l[1] = GD_MFMA(x1, wl, kk == 0u ? zi : l[1], 0, 0, 0);
+        asm volatile("ds_read_b128 %0, %2 offset:1024" : "=v"(x1) : "0"(x1), "v"(x_nx));
+        l[2] = GD_MFMA(x2, wl, kk == 0u ? zi : l[2], 0, 0, 0);
+        asm volatile("ds_read_b128 %0, %2 offset:2048" : "=v"(x2) : "0"(x2), "v"(x_nx));
+        l[3] = GD_MFMA(x3, wl, kk == 0u ? zi : l[3], 0, 0, 0);
+        asm volatile("ds_read_b128 %0, %2 offset:3072" : "=v"(x3) : "0"(x3), "v"(x_nx));
+        asm volatile("ds_read_b128 %0, %2 offset:1024" : "=v"(wl) : "0"(wl), "v"(w_nx));
       }
-      if (kk == 7u && (!GD_ABL_NOEPI || s + 1u == p.nsb)) {
-        // acc += ad * (d * isum) for the super-block (vecdot.rs:2242-2300 in the order of its sums)
+      if (kk == 7u) {   // acc += ad * (d * isum - dmin * imin)
         const uint32_t tsl = (s & 1u) * TAB_SLOT;
-        uint32_t hw;
-        half8 a1 = {0, 0, 0, 0, 0, 0, 0, 0};
-        if constexpr (ONEPASS) {
-          int4v hd;
-          GD_READ16(hd, hw_rd + tsl, 0);
-          GD_WAIT1(0, hd);
-          hw = (uint32_t)hd.x;
-          uint32_t mna, mnb;
-          q4k_mins(make_uint4((uint32_t)hd.x, (uint32_t)hd.y, (uint32_t)hd.z, (uint32_t)hd.w), mna, mnb);
-          a1 = side_operand(mna, mnb, lh ? 1.0f : 64.0f);
-        } else {
-          GD_READ4(hw, hw_rd + tsl, 0);
-          GD_WAIT1(0, hw);
-        }
-        // Q6_K's word holds the d of a pair of rows
-        const float d0 = gm_f16_bits_to_f32(Q6 && (l32 & 1u) ? (hw >> 16) : (hw & 0xFFFFu));
-        const float ndm = -gm_f16_bits_to_f32(hw >> 16);   // one-pass: -dmin
+        int4v hd;
+        GD_READ16(hd, hw_rd + tsl, 0);
+        GD_WAIT1(0, hd);
+        const uint32_t hw = (uint32_t)hd.x;
+        uint32_t mna, mnb;
+        q4k_mins(make_uint4((uint32_t)hd.x, (uint32_t)hd.y, (uint32_t)hd.z, (uint32_t)hd.w), mna, mnb);
+        const half8 a1 = side_operand(mna, mnb, lh ? 1.0f : 64.0f);
+        const float d0 = gm_f16_bits_to_f32(hw & 0xFFFFu), ndm = -gm_f16_bits_to_f32(hw >> 16);
         const uint32_t ta = tab_rd + tsl;
 #pragma unroll
         for (int tb = 0; tb < 4; tb++) {
           typedef float float4v __attribute__((ext_vector_type(4)));
           float4v a40, a41, a42, a43;
-          if constexpr (ONEPASS) {
-            // d * isum of the block's 16 outputs first (the integer sums die here), then imin into the registers
-            // they leave, then one multiply-add each for the mins and for the token's scale
-            half8 b2;
-            GD_READ16(b2, bs_rd + tsl, 1024 * tb);
-            float t[16];
+          // d * isum of the block's 16 outputs first (the integer sums die here), then imin into the registers
+          // they leave, then one multiply-add each for the mins and for the token's scale
+          half8 b2;
+          GD_READ16(b2, bs_rd + tsl, 1024 * tb);
+          float t[16];
 #pragma unroll
-            for (int r = 0; r < 16; r++) t[r] = d0 * (float)(h[tb][r] * 256 + l[tb][r]);
-            GD_WAIT1(0, b2);
-            const float16v zf = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-            const float16v im = __builtin_amdgcn_mfma_f32_32x32x16_f16(b2, a1, zf, 0, 0, 0);
-            GD_READ16(a40, ta, 128 * tb);
-            GD_READ16(a41, ta, 128 * tb + 32);
-            GD_READ16(a42, ta, 128 * tb + 64);
-            GD_READ16(a43, ta, 128 * tb + 96);
-            GD_WAIT2(0, a40, a41);
-            GD_WAIT2(0, a42, a43);
-            const float4v a4[4] = {a40, a41, a42, a43};
-#pragma unroll
-            for (int q4 = 0; q4 < 4; q4++) {
-              const float a4v[4] = {a4[q4].x, a4[q4].y, a4[q4].z, a4[q4].w};
-#pragma unroll
-              for (int e = 0; e < 4; e++)
-                y[tb][4 * q4 + e] = __builtin_fmaf(a4v[e], __builtin_fmaf(ndm, im[4 * q4 + e], t[4 * q4 + e]), y[tb][4 * q4 + e]);
-            }
-            continue;
-          }
+          for (int r = 0; r < 16; r++) t[r] = d0 * (float)(h[tb][r] * 256 + l[tb][r]);
+          GD_WAIT1(0, b2);
+          const float16v zf = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+          const float16v im = __builtin_amdgcn_mfma_f32_32x32x16_f16(b2, a1, zf, 0, 0, 0);
           GD_READ16(a40, ta, 128 * tb);
           GD_READ16(a41, ta, 128 * tb + 32);
           GD_READ16(a42, ta, 128 * tb + 64);
@@ -1077,10 +943,8 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_dma_kernel(GemmDmaPara
           for (int q4 = 0; q4 < 4; q4++) {
             const float a4v[4] = {a4[q4].x, a4[q4].y, a4[q4].z, a4[q4].w};
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-              const int is = Q3 ? -h[tb][4 * q4 + e] : h[tb][4 * q4 + e] * 256 + l[tb][4 * q4 + e];
-              y[tb][4 * q4 + e] += a4v[e] * (d0 * (float)is);
-            }
+            for (int e = 0; e < 4; e++)
+              y[tb][4 * q4 + e] = __builtin_fmaf(a4v[e], __builtin_fmaf(ndm, im[4 * q4 + e], t[4 * q4 + e]), y[tb][4 * q4 + e]);
           }
         }
       }
@@ -1100,77 +964,83 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_dma_kernel(GemmDmaPara
 }
 
 // ------------------------------------------------------------------------------------------
-// The same multiplication on 64-row tiles, for launches too small to fill the 128-row kernel's places (its grid
-// wants 384 tiles of 128 x 128; a 4096 x 4096 matrix at 512 tokens has 128), with the f32 step of a super-block
-// issued *between* the matrix instructions of the next one.  A SIMD runs a matrix instruction for 32 clocks; the
-// wave that issued it can issue about five vector instructions behind it for nothing (measured: eight matrix
-// instructions 128 ns, with five dependent v_fma behind each 131 ns, with eight 166 ns), while vector work that
-// waits for the end of a run of matrix instructions is paid in full: a workgroup that has a compute unit to itself
-// has no second wave on its SIMDs to hide it behind.  The step acc += ad * (d * isum) is five vector instructions
-// per output: one output per matrix instruction.  For that the planes' sums live in two register sets, one filled
-// while the other is added up, which a wave tile of 32 rows x 64 tokens leaves room for (2 sets x 64 + 32 of y).
-// On grids that fill the 128-row kernel this one is slower (4096 -> 14336 at 512 / 2048 tokens: 115 / 375 us
-// against 98 / 322): a step of four matrix instructions a wave carries the same waits, barrier and loads as one
-// of eight.
+// The K-quant GEMMs over planes in the reference's float order: 128-row tiles (ogm_gemm_dma_kernel) for launches that fill
+// the device with them, 64-row tiles (ogm_gemm_dmx_kernel) for smaller ones.
 //
-//   workgroup  256 threads = 4 waves; 64 rows x 128 tokens; wave w: rows 32 (w & 1) .. + 31, tokens
-//              64 (w >> 1) .. + 63.  Two workgroups share a compute unit (67 KiB of LDS each).
-//   step       32 weights of k: the row block's two planes (4 KiB, one piece of 1 KiB per wave) and
-//              four token blocks of activations (1 KiB each, one per wave), by load-to-LDS, issued behind
-//              the step's first matrix instruction
-//   ring       eight steps in LDS = the steps of a super-block (step kk of any super-block sits in slot kk:
-//              every LDS address of the loop is a constant), six in flight; one wait + barrier per step
-//   tables     per super-block the tokens' activation scales and the rows' header words, three slots:
-//              the one being added up, the one being multiplied, the one arriving
-//   LDS reads  of a step, in issue order: [header word], four tokens' ad, h plane, two token blocks,
-//              l plane -- issued one step ahead, between the matrix instructions, waited for by count
-//   first pass (Q4_K, Q5_K) two super-blocks in turn: the matrix instructions of the next are issued before the
-//              vector work of this one
-// Same arithmetic and f32 order as ogm_gemm_dma_kernel; bit-identical results.
-#define GX_NW 4u
-#define GX_ROWS 64u
-#define GX_TOK 128u
-#define GX_RING 8u
-#define GX_AHEAD (GX_RING - 1u)
-#define GX_SLOT 8192u                 // a step's planes (4 KiB) and activations (4 KiB)
-#define GX_TAB (GX_RING * GX_SLOT)
-#define GX_TAB_SLOT 1024u             // 128 ad | 64 header words | 256 bytes that absorb wave 3's load
-#define GX_LDS_BYTES (GX_TAB + 3u * GX_TAB_SLOT)
-// timing experiments only (results are wrong with any of these set)
-#ifndef GX_ABL_NOEPI
-#define GX_ABL_NOEPI 0   // the f32 step left out of the loop
-#endif
-#ifndef GX_ABL_NOPASS1
-#define GX_ABL_NOPASS1 0
-#endif
-#ifndef GX_ABL_NOMFMA
-#define GX_ABL_NOMFMA 0
-#endif
-#ifndef GX_ABL_NODMA
-#define GX_ABL_NODMA 0
-#endif
-#if GX_ABL_NOMFMA
-#define GX_MFMA(A, B, C) (C)
-#else
-#define GX_MFMA(A, B, C) __builtin_amdgcn_mfma_i32_32x32x32_i8(A, B, C, 0, 0, 0)
-#endif
-#define GX_SYNC(N) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory")
-#define GX_PIN() __builtin_amdgcn_sched_barrier(0)
-#define GX_WAITN(N) asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory")
+// What bounds them on this card is power as much as any one unit: eight matrix instructions with five vector instructions
+// behind each take 1.02 times the cycles of the matrix instructions alone (two waves a SIMD), but at 1.71 GHz instead of
+// 1.89; a launch of 4096 -> 14336 at 2048 tokens runs at 1.9 GHz with the matrix pipe busy for half of its 521 k cycles.
+// So what counts is instructions and bytes moved, not only what overlaps:
+//   * a wave multiplies one token block of 32 with every row block of its tile.  The block's operand chunks of a
+//     super-block stay in 32 registers for all of them (loaded a super-block ahead, straight from memory) and only the
+//     weights go through LDS: 16 KiB a super-block and row block, one piece, shared by the four waves;
+//   * piece after piece, so only one row block's two plane sums are being filled (32 registers) while the row block
+//     before is added up from a second set: acc += ad * (d * isum), five vector instructions an output, one output
+//     behind every matrix instruction;
+//   * a barrier and a wait per piece (sixteen matrix instructions a wave), not per 32 k;
+//   * the first pass of Q4_K / Q5_K keeps to registers -- no LDS, no barrier, its operands laid out with the planes
+//     (gp_mins_offset) -- while the ring fills, and takes the scales' products ad * dmin from an outer product on the
+//     matrix cores (32 x 32 x 1, two row blocks an instruction; a product rounded once, as the vector multiply): two
+//     vector instructions an output instead of three.
+// Whole calls, us, against the kernels these replaced (a wave 32 rows x 128 or 64 tokens with both operands through LDS step
+// by step, a barrier per 32 k): Q4_K 4096 -> 2 x 14336 at 512 tokens 175 -> 164, 4096 -> 14336 at 2048 315 -> 294, 2048 ->
+// 2 x 8192 at 1901 174 -> 162; 64-row tiles: 4096 -> 4096 at 512 38.9 -> 32.9, 14336 -> 4096 112 -> 97, Q6_K 14336 -> 4096
+// 89 -> 83.  Where the device is full the 128-row tiles lead (4096 -> 2 x 14336 at 512: 164 against 184, they fetch 6 KiB per
+// 32 x 32 x 256 products, not 8), on one workgroup a compute unit the 64-row ones (4096 -> 4096 at 512: 33 against 46).
+// Eight waves and 256 tokens a workgroup fetch less still (4 KiB) but stand at one barrier: 164 and 308.
+//
+//   workgroup  256 threads = 4 waves of 32 tokens; RB row blocks of 32.  Two workgroups share a compute unit.
+//   ring       four pieces in LDS; at the top of piece p a wave waits until its loads of piece p + 1 have landed, meets the
+//              others at a barrier, and fetches piece p + 3 into the slot piece p - 1 left
+//   tables     per super-block the tokens' ad and the rows' d, four slots, fetched a super-block ahead
+//   LDS reads  a step's two operand chunks and two ad, issued three steps ahead, waited for by count
+// Registers: 16 RB of y, 64 of the plane sums, 64 of x, 32 of weights: 247 of a wave's 256 at RB = 4.
+#define GB_PIN() __builtin_amdgcn_sched_barrier(0)
+#define GB_SYNC(N) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory")
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef float float32v __attribute__((ext_vector_type(32)));
 
-template <int KIND>
-__global__ __launch_bounds__(64 * GX_NW, 2) void ogm_gemm_dmx_kernel(GemmDmaParams p) {
-  constexpr uint32_t NW = GX_NW, ROWS = GX_ROWS, SLOT = GX_SLOT, TAB = GX_TAB, TAB_SLOT = GX_TAB_SLOT;
-  constexpr bool Q45 = KIND == GP_Q4K || KIND == GP_Q5K, Q5 = KIND == GP_Q5K, Q6 = KIND == GP_Q6K, XS = KIND == GP_IQ4XS;
-  static_assert(Q45 || Q6 || XS, "two-plane types only");
-  constexpr uint32_t TILE_BYTES = (KIND == GP_Q4K || XS) ? 9216u : Q5 ? 11264u : 13440u;
-  constexpr uint32_t AHEAD = GX_AHEAD, PER = 2u;   // loads a wave issues per step
+// Load-to-LDS by buffer instructions: `voff` a lane, `soff` and `ioff` the wave's; lane l's bytes land at lds_chunk +
+// l * size.  (The compiler counts them like any other load; behind the flat form it would wait for all of them at every
+// use of a loaded register.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gb_buffer(const void *base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0xFFFFFFFF, 0x00027000);
+}
+template <int IOFF>
+__device__ __forceinline__ void gb_dma16(__amdgpu_buffer_rsrc_t b, uint32_t voff, uint32_t soff, uint8_t *lds_chunk) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (__attribute__((address_space(3))) void *)lds_chunk, 16, voff, soff, IOFF, 0);
+}
+__device__ __forceinline__ void gb_dma4(__amdgpu_buffer_rsrc_t b, uint32_t voff, uint32_t soff, uint8_t *lds_chunk) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (__attribute__((address_space(3))) void *)lds_chunk, 4, voff, soff, 0, 0);
+}
+
+template <int KIND, uint32_t RB>
+struct GbShape {
+  static constexpr uint32_t NW = 4;                          // waves, each a token block of 32
+  static constexpr uint32_t NPL = KIND == GP_Q3K ? 1u : 2u;
+  static constexpr uint32_t PIECE = 8192u * NPL;             // a super-block of 32 rows: eight steps of 32 k, NPL planes
+  static constexpr uint32_t SLOTS = 4;                       // pieces in the ring
+  static constexpr uint32_t TAB = SLOTS * PIECE;
+  static constexpr uint32_t TAB_SLOT = NW * 128u + RB * 128u + 256u;   // the tokens' ad | the rows' d | spare
+  static constexpr uint32_t LDS_BYTES = TAB + 4u * TAB_SLOT;
+  static_assert(SLOTS % RB == 0 && RB % 2u == 0, "a super-block's pieces sit in the same slots every turn of the ring");
+};
+
+template <int KIND, uint32_t RB>
+__device__ __forceinline__ void gemm_planes_body(GemmDmaParams &p) {
+  using Shape = GbShape<KIND, RB>;
+  constexpr uint32_t NW = Shape::NW;
+  constexpr bool Q45 = KIND == GP_Q4K || KIND == GP_Q5K;
+  constexpr uint32_t NPL = Shape::NPL, PIECE = Shape::PIECE, SLOTS = Shape::SLOTS, TAB = Shape::TAB, TAB_SLOT = Shape::TAB_SLOT;
+  constexpr uint32_t TURN = SLOTS / RB;         // super-blocks the ring holds
+  constexpr uint32_t KSTEP = NPL * 1024u;       // bytes of a step of 32 k: 32 rows, NPL planes
+  constexpr uint32_t PER = 8u * NPL / NW;       // loads a wave issues per piece
+  constexpr uint32_t ROWS = 32u * RB, TOK = 32u * NW;
   extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t l32 = lane & 31u, lh = lane >> 5;
-  const uint32_t rs = wave & 1u, th = wave >> 1;   // row slice of 32, token half
-  // token tiles of one row tile go to one XCD back to back (see ogm_gemm_dma_kernel)
+  // token tiles of one row tile go to one XCD back to back (see ogm_gemm_onepass_kernel)
   uint32_t tok_tile = blockIdx.x, row_tile = blockIdx.y;
   {
     const uint32_t nt = gridDim.x, lin = blockIdx.y * nt + blockIdx.x;
@@ -1180,12 +1050,13 @@ __global__ __launch_bounds__(64 * GX_NW, 2) void ogm_gemm_dmx_kernel(GemmDmaPara
       row_tile = (j / nt) * 8u + (lin & 7u);
     }
   }
+  tok_tile = __builtin_amdgcn_readfirstlane(tok_tile);   // (divided in vector registers)
+  row_tile = __builtin_amdgcn_readfirstlane(row_tile);
 #pragma unroll
   for (uint32_t m = 0; m < OGM_GEMM_MAX_MATS - 1; m++) {   // the matrix this row tile belongs to
     const uint32_t tiles = (p.out_dim + ROWS - 1u) / ROWS;
     if (m < p.n_extra && row_tile >= tiles) {
       row_tile -= tiles;
-      p.wt = p.extra_wt[m];
       p.planes = p.extra_planes[m];
       p.y = p.extra_y[m];
       p.out_dim = p.extra_out_dim[m];
@@ -1193,242 +1064,212 @@ __global__ __launch_bounds__(64 * GX_NW, 2) void ogm_gemm_dmx_kernel(GemmDmaPara
       break;
     }
   }
-  const uint32_t t0 = tok_tile * GX_TOK, r0 = row_tile * ROWS;
-  auto sb_off = [&](uint32_t s) -> uint32_t {
-    return (s >> p.c_shift) * TILE_BYTES + ((s & ((1u << p.c_shift) - 1u)) << p.r_shift) * 16u;
+  const uint32_t t0 = tok_tile * TOK, r0 = row_tile * ROWS;
+  const uint32_t nsb = p.nsb, nrb = (p.out_dim + 63u) / 64u;
+  const bool live = t0 + 32u * wave < p.n_tokens;   // the wave has a token to multiply (else it only fetches)
+  uint32_t rb32[RB];                                // the row blocks of 32 (past the matrix: its last one again, never stored)
+#pragma unroll
+  for (uint32_t i = 0; i < RB; i++) rb32[i] = min(row_tile * RB + i, 2u * nrb - 1u);
+
+  // ---- what goes to LDS.  A piece is a super-block of a row block of 32: step k of its eight in chunks of 1 KiB, one a
+  // plane (lane (l32, lh): the 16 weights 16 lh .. of row l32); wave w fetches steps w, w + NW
+  const uint32_t w_lane = lh * KSTEP + l32 * 16u;
+  const __amdgpu_buffer_rsrc_t planes = gb_buffer(p.planes);
+  auto fetch_piece = [&](uint32_t s, uint32_t i, uint32_t slot) {   // super-block s of row block i
+    uint32_t b = rb32[0];
+#pragma unroll
+    for (uint32_t j = 1; j < RB; j++) b = i == j ? rb32[j] : b;
+    const uint32_t src = ((b >> 1) * nsb + s) * (16u * KSTEP) + (b & 1u) * 512u;
+#pragma unroll
+    for (uint32_t j = 0; j < 8u / NW; j++) {
+      const uint32_t k = wave + NW * j;
+      uint8_t *dst = lds + slot * PIECE + k * KSTEP;
+      gb_dma16<0>(planes, w_lane, src + k * (2u * KSTEP), dst);
+      if constexpr (NPL == 2u) gb_dma16<1024>(planes, w_lane, src + k * (2u * KSTEP), dst);
+    }
   };
+  // a super-block's tables: 64 tokens' ad from each of the first NW / 2 waves, 64 rows' d from each of the next RB / 2
+  const bool tab_ad = wave < NW / 2u;
+  const bool tab_d = !tab_ad && wave - NW / 2u < RB / 2u;
+  const __amdgpu_buffer_rsrc_t tab = gb_buffer(tab_ad ? (const uint8_t *)p.ad : p.planes + gp_d_offset(nrb, nsb, NPL));
+  uint32_t tab_lane;
+  if (tab_ad) {
+    tab_lane = min(t0 + 64u * wave + lane, p.n_tokens - 1u) * nsb * 4u;
+  } else {
+    const uint32_t i = (tab_d ? 2u * (wave - NW / 2u) : 0u) + lh;
+    tab_lane = min(row_tile * RB + i, 2u * nrb - 1u) * nsb * 128u + l32 * 4u;
+  }
+  const uint32_t tab_step = tab_ad ? 4u : 128u;
+  const uint32_t tab_dst = TAB + (tab_ad ? 256u * wave : NW * 128u + (tab_d ? 256u * (wave - NW / 2u) : RB * 128u));
+  auto fetch_tables = [&](uint32_t s, uint32_t slot) { gb_dma4(tab, tab_lane, tab_step * s, lds + tab_dst + slot * TAB_SLOT); };
+  // at the top of a piece: the piece after it has landed for every wave and the one before it is no longer read; its
+  // slot takes the piece SLOTS - 1 on (past the end: the last super-block again, never read)
+  auto top = [&](auto i_c, auto n_c, uint32_t s) {
+    constexpr uint32_t i = decltype(i_c)::value;
+    GB_PIN();
+    GB_SYNC(decltype(n_c)::value);
+    if (i == 0u) fetch_tables(min(s + 1u, nsb - 1u), (s + 1u) & 3u);
+    constexpr uint32_t it = (i + SLOTS - 1u) % RB, ds = (i + SLOTS - 1u) / RB;
+    fetch_piece(min(s + ds, nsb - 1u), it, ((s + ds) % TURN) * RB + it);
+    GB_PIN();
+  };
+  // loads newer than the ones a piece's top waits for
+  constexpr uint32_t AHEAD = PER * (SLOTS - 3u);
+  fetch_tables(0u, 0u);
+#pragma unroll
+  for (uint32_t q = 0; q < SLOTS - 1u; q++) fetch_piece(min(q / RB, nsb - 1u), q % RB, q);
+  asm volatile("" ::: "memory");
 
-  float16v y[2];
-#pragma unroll
-  for (int tb = 0; tb < 2; tb++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) y[tb][r] = 0.0f;
-
-  if constexpr (Q45 && !GX_ABL_NOPASS1) {
-    // pass 1 of gemm_k_q4_k: acc -= (ad * dmin) * sum_j m_j * bsum_j over all super-blocks first
-    // (vecdot.rs:2226-2240), as in ogm_gemm_dma_kernel, for this wave's two token blocks
-    const uint32_t row = min(r0 + 32u * rs + l32, p.out_dim - 1u);
-    const uint32_t uo = (row >> p.r_shift) * p.nct * TILE_BYTES + (row & ((1u << p.r_shift) - 1u)) * 16u;
-    float *ad_all = (float *)lds;   // [nsb][128]
-    {
-      // element i of the tile's [128 tokens][nsb] block goes to [su][token]; eight loads in flight a thread, and the
-      // (token, su) of i + 256 from those of i without dividing again
-      const uint32_t total = GX_TOK * p.nsb, dq = (64u * NW) / p.nsb, dr = (64u * NW) % p.nsb;
-      uint32_t k = tid / p.nsb, su = tid - k * p.nsb;
-      for (uint32_t i0 = tid; i0 < total; i0 += 8u * 64u * NW) {
-        float v[8];
-        uint32_t dst[8];
-#pragma unroll
-        for (uint32_t j = 0; j < 8u; j++) {
-          const bool in = i0 + j * 64u * NW < total;
-          dst[j] = in ? su * GX_TOK + k : 0xFFFFFFFFu;
-          v[j] = in ? p.ad[min(t0 + k, p.n_tokens - 1u) * p.nsb + su] : 0.0f;
-          k += dq;
-          su += dr;
-          if (su >= p.nsb) {
-            su -= p.nsb;
-            k++;
-          }
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < 8u; j++)
-          if (dst[j] != 0xFFFFFFFFu) ad_all[dst[j]] = v[j];
+  if (!live) {
+    // (no loads of x among its own: the tables of the super-block that begins are older than RB pieces' fetches)
+    auto idle = [&](auto i_c, uint32_t s) { top(i_c, std::integral_constant<int, (int)(AHEAD < RB * PER ? AHEAD : RB * PER)>{}, s); };
+    for (uint32_t s = 0; s < nsb; s++) {
+      idle(std::integral_constant<uint32_t, 0u>{}, s);
+      idle(std::integral_constant<uint32_t, 1u>{}, s);
+      if constexpr (RB == 4u) {
+        idle(std::integral_constant<uint32_t, 2u>{}, s);
+        idle(std::integral_constant<uint32_t, 3u>{}, s);
       }
     }
-    __syncthreads();
-    float16v zero;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return;
+  }
+
+  // this wave's token block: its operand chunks of a super-block stay in registers for all the row blocks
+  const uint32_t tb = (t0 >> 5) + wave;
+  const uint8_t *xsrc = (const uint8_t *)p.xt + (size_t)tb * (p.in_dim / 32u) * 1024u + lane * 16u;
+  int4v xA[8], xB[8];
 #pragma unroll
-    for (int r = 0; r < 16; r++) zero[r] = 0.0f;
-    uint32_t tk[2];
+  for (int k = 0; k < 8; k++) xA[k] = *(const int4v *)(xsrc + k * 1024);
+  asm volatile("" ::: "memory");
+
+  float16v y[RB];
 #pragma unroll
-    for (int tb = 0; tb < 2; tb++) tk[tb] = min(t0 + 64u * th + 32u * tb + l32, p.n_tokens - 1u) * p.nsb;
-    const float side_scale = lh ? 1.0f : 64.0f;
-    // Two super-blocks in turn (sets X and Y): the matrix instructions of the next one are issued before the vector
-    // work of this one, and each set's header and token sums are loaded two super-blocks ahead.
-    uint4 hdX, hdY;
-    half8 b2X[2], b2Y[2];
-    float16v imX[2], imY[2];
-    float dmX = 0.0f, dmY = 0.0f;
-    auto load = [&](uint32_t su, uint4 &hd, half8(&b2)[2]) {
-      const uint32_t sn = min(su, p.nsb - 1u);   // past the end: loaded again, never used
-      hd = *(const uint4 *)(p.wt + (uo + sb_off(sn)));
+  for (uint32_t i = 0; i < RB; i++)
 #pragma unroll
-      for (int tb = 0; tb < 2; tb++) b2[tb] = *(const half8 *)(p.bs16 + ((tk[tb] + sn) * 16u + 8u * lh));
+    for (int r = 0; r < 16; r++) y[i][r] = 0.0f;
+
+  if constexpr (Q45) {
+    // ---------------- pass 1 of gemm_k_q4_k: acc -= (ad * dmin) * sum_j m_j * bsum_j over all super-blocks first
+    // (vecdot.rs:2226-2240)
+    const uint32_t tok = min(t0 + 32u * wave + l32, p.n_tokens - 1u);
+    const _Float16 *bs = p.bs16 + ((size_t)tok * nsb * 16u + 8u * lh);
+    const float *adp = p.ad + (size_t)tok * nsb;
+    const float *dmin = (const float *)(p.planes + gp_dmin_offset(nrb, nsb, NPL));
+    const uint8_t *mins = p.planes + gp_mins_offset(nrb, nsb, NPL) + lane * 16u;
+    uint32_t dm_at[RB / 2];
+#pragma unroll
+    for (uint32_t j = 0; j < RB / 2u; j++) dm_at[j] = min(row_tile * RB + 2u * j + lh, 2u * nrb - 1u) * nsb * 32u + l32;
+    struct Set {
+      half8 b2, m[RB];
+      float ad, dm[RB / 2];
     };
-    auto stage = [&](const uint4 &hd, const half8(&b2)[2], float16v(&im)[2], float &dm) {
-      uint32_t mna, mnb;
-      q4k_mins(hd, mna, mnb);
-      const half8 a1 = side_operand(mna, mnb, side_scale);
-      dm = gm_f16_bits_to_f32(hd.x >> 16);
+    auto load = [&](uint32_t s, Set &q) {
+      s = min(s, nsb - 1u);
+      q.b2 = *(const half8 *)(bs + s * 16u);
+      q.ad = adp[s];
 #pragma unroll
-      for (int tb = 0; tb < 2; tb++) im[tb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(b2[tb], a1, zero, 0, 0, 0);
+      for (uint32_t j = 0; j < RB / 2u; j++) q.dm[j] = dmin[dm_at[j] + s * 32u];
+#pragma unroll
+      for (uint32_t i = 0; i < RB; i++) q.m[i] = *(const half8 *)(mins + (size_t)(rb32[i] * nsb + s) * 1024u);
     };
-    auto consume = [&](uint32_t su, const float16v(&im)[2], float dm) {
+    auto use = [&](const Set &q) {
+      const float16v z16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+      const float32v z32 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-      for (int tb = 0; tb < 2; tb++) {
-        const float *adp = &ad_all[su * GX_TOK + 64u * th + 32u * tb + 4u * lh];
+      for (uint32_t j = 0; j < RB / 2u; j++) {
+        const float16v im0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(q.b2, q.m[2 * j], z16, 0, 0, 0);
+        const float32v pr = __builtin_amdgcn_mfma_f32_32x32x1f32(q.ad, q.dm[j], z32, 0, 0, 0);
+        const float16v im1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(q.b2, q.m[2 * j + 1], z16, 0, 0, 0);
 #pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) {
-          const float4 a4 = *(const float4 *)(adp + 8 * q4);
-          const float a4v[4] = {a4.x, a4.y, a4.z, a4.w};
+        for (int r = 0; r < 16; r++) y[2 * j][r] -= pr[r] * im0[r];
 #pragma unroll
-          for (int e = 0; e < 4; e++) y[tb][4 * q4 + e] -= a4v[e] * dm * im[tb][4 * q4 + e];
-        }
+        for (int r = 0; r < 16; r++) y[2 * j + 1][r] -= pr[16 + r] * im1[r];
       }
     };
-    load(0u, hdX, b2X);
-    load(1u, hdY, b2Y);
-    stage(hdX, b2X, imX, dmX);
-    load(2u, hdX, b2X);
-    for (uint32_t su = 0; su < p.nsb; su += 2u) {
-      const bool two = su + 1u < p.nsb;
-      if (two) {
-        stage(hdY, b2Y, imY, dmY);
-        load(su + 3u, hdY, b2Y);
-      }
-      GX_PIN();
-      consume(su, imX, dmX);
-      GX_PIN();
-      if (two) {
-        if (su + 2u < p.nsb) {
-          stage(hdX, b2X, imX, dmX);
-          load(su + 4u, hdX, b2X);
-        }
-        GX_PIN();
-        consume(su + 1u, imY, dmY);
-        GX_PIN();
-      }
+    Set a, b;
+    load(0u, a);
+    for (uint32_t s = 0; s + 1u < nsb; s += 2u) {   // one super-block's loads in flight behind the other's work
+      load(s + 1u, b);
+      GB_PIN();
+      use(a);
+      GB_PIN();
+      load(s + 2u, a);
+      GB_PIN();
+      use(b);
+      GB_PIN();
     }
-    __syncthreads();   // the table's LDS becomes the ring
+    if (nsb & 1u) use(a);
   }
 
   // ---------------- the products
-  // per step wave w fetches piece w of the row block's planes ((half of k, plane) = (w >> 1, w & 1): 64 rows x 16
-  // bytes) and token block w of the activations.  The ring has as many slots as a super-block has steps: step kk of
-  // any super-block sits in slot kk, so every LDS address of the loop is a constant.
-  static_assert(GX_RING == 8u, "the ring's slots are the steps of a super-block");
-  uint32_t w_src = row_tile * p.nsb * 8u * 4096u + wave * 1024u + lane * 16u;   // + 4096 per step
-  uint32_t x_src = min((t0 >> 5) + wave, (p.n_tokens - 1u) >> 5) * (p.in_dim / 32u) * 1024u + lane * 16u;   // + 1024 per step
-  const uint32_t w_dst = wave * 1024u, x_dst = 4096u + wave * 1024u;
-  // tables: waves 0, 1 fetch 64 tokens' ad each, wave 2 the header words of the 64 rows (wave 3 the same again,
-  // into spare bytes: every wave has the same number of loads in flight)
-  uint32_t tab_src;
-  if (wave < 2u) {
-    tab_src = min(t0 + 64u * wave + lane, p.n_tokens - 1u) * p.nsb * 4u;
-  } else {
-    const uint32_t tab_row = min(r0 + lane, p.out_dim - 1u);
-    const uint32_t tab_rb = tab_row >> p.r_shift, tab_r = tab_row & ((1u << p.r_shift) - 1u);
-    if constexpr (Q6) tab_src = tab_rb * p.nct * TILE_BYTES + 13u * 1024u + ((tab_r * 2u) & ~3u);
-    else tab_src = tab_rb * p.nct * TILE_BYTES + tab_r * 16u;
-  }
-  uint32_t tsl_prev = 0u, tsl_cur = 0u, tsl_next = TAB_SLOT;   // table slots of super-blocks s - 1, s, s + 1
-  auto fetch_tables = [&](uint32_t s, uint32_t tsl) {
-    uint8_t *slot = lds + TAB + tsl;
-    if (wave < 2u) {
-      gd_dma4((const uint8_t *)p.ad + (tab_src + 4u * s), slot + 256u * wave);
-    } else {
-      const uint32_t so = Q6 ? (s >> p.c_shift) * TILE_BYTES + ((s & ((1u << p.c_shift) - 1u)) << p.r_shift) * 2u : sb_off(s);
-      gd_dma4(p.wt + (tab_src + so), slot + 512u + 256u * (wave - 2u));
-    }
-  };
-  auto fetch_step = [&](uint32_t slot_off) {   // the next step (they are fetched in ascending order) into ring slot slot_off / SLOT
-    uint8_t *slot = lds + slot_off;
-    gd_dma16(p.planes + w_src, slot + w_dst);
-    gd_dma16((const uint8_t *)p.xt + x_src, slot + x_dst);
-    w_src += 4096u;
-    x_src += 1024u;
-  };
-
-  fetch_tables(0u, 0u);
-#pragma unroll
-  for (uint32_t k = 0; k < AHEAD; k++) fetch_step(k * SLOT);
-#define GX_SYNC_STEPS(N) GX_SYNC((N) * (int)PER)   // all but the newest N steps' loads of this wave have landed, then the barrier
-  GX_SYNC_STEPS(AHEAD - 1);   // step 0 and the first tables have landed
-
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
-  const uint32_t w_rd = lds0 + lh * 2048u + (32u * rs + l32) * 16u;      // h plane; l plane + 1024
-  const uint32_t x_rd = lds0 + 4096u + 2048u * th + lane * 16u;          // token block 0 of the wave; block 1 + 1024
-  const uint32_t ad_rd = lds0 + TAB + 4u * (64u * th + 4u * lh);      // + 128 tb + 32 q4: four tokens' ad
-  const uint32_t hw_rd = lds0 + TAB + 512u + 4u * (32u * rs + l32);   // the row's header word
-  typedef float float4v __attribute__((ext_vector_type(4)));
-  int16v hA[2], lA[2], hB[2], lB[2];
+  const uint32_t w_rd = lds0 + lane * 16u;
+  const uint32_t ad_rd = lds0 + TAB + wave * 128u + lh * 16u;      // + 32 (r / 4) + 4 (r % 4): the ad of output r
+  const uint32_t d_rd = lds0 + TAB + NW * 128u + l32 * 4u;         // + 128 i: row block i's d
+  int16v hA, lA, hB, lB;
   const int16v zi = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  int4v wh, wl, x0, x1;
-  float4v a4[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
-  uint32_t hw = 0;
-  float d0 = 0.0f;
-  GD_READ16(wh, w_rd, 0);
-  GD_READ16(x0, x_rd, 0);
-  GD_READ16(x1, x_rd, 1024);
-  GD_READ16(wl, w_rd, 1024);
+  int4v w[4][NPL];
+  float2v a2[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+  float dn = 0.0f, d0 = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+#pragma unroll
+    for (uint32_t pl = 0; pl < NPL; pl++) w[j][pl] = zi.s0123;
+  constexpr int OPS = 1 + (int)NPL;   // LDS reads issued per step
 
-  // One super-block: its 8 steps accumulate into (hc, lc) while, with EPI, the sums of the one before in
-  // (hp, lp) are added to y, one output behind every matrix instruction.
-  auto super_block = [&](auto set_c, auto epi_c, uint32_t s) {
-    constexpr bool SET = decltype(set_c)::value, EPI = decltype(epi_c)::value && !GX_ABL_NOEPI;
-    const bool more = s + 1u < p.nsb;   // in the last super-block the steps in flight run out
-    int16v(&hc)[2] = SET ? hB : hA;
-    int16v(&lc)[2] = SET ? lB : lA;
-    int16v(&hp)[2] = SET ? hA : hB;
-    int16v(&lp)[2] = SET ? lA : lB;
+  // the reads of step kk of a piece that starts at LDS address `wa`, with the activation scales at `aa` of the outputs that
+  // step adds up
+#define GB_READS(KK, B, WA, WOFF, AA)                                                                                      \
+  do {                                                                                                                     \
+    asm volatile("ds_read_b64 %0, %2 offset:%3" : "=v"(a2[B]) : "0"(a2[B]), "v"(AA), "n"(32u * ((KK) >> 1) + 8u * ((KK) & 1u))); \
+    asm volatile("ds_read_b128 %0, %2 offset:%3" : "=v"(w[B][0]) : "0"(w[B][0]), "v"(WA), "n"((WOFF) + (KK) * KSTEP));     \
+    if constexpr (NPL == 2u)                                                                                               \
+      asm volatile("ds_read_b128 %0, %2 offset:%3" : "=v"(w[B][NPL - 1u]) : "0"(w[B][NPL - 1u]), "v"(WA), "n"((WOFF) + (KK) * KSTEP + 1024u)); \
+  } while (0)
+
+  uint32_t tab_prev = 0u;   // table slot of the super-block before this one
+  const uint8_t *xn = xsrc;
+  auto piece = [&](auto i_c, auto epi_c, int4v(&x)[8], int4v(&xnext)[8], uint32_t w_cur, uint32_t w_next, uint32_t tab_cur) {
+    constexpr uint32_t i = decltype(i_c)::value, ip = (i + RB - 1u) % RB;   // row block, and the one before it
+    constexpr bool EPI = decltype(epi_c)::value, SET = (i & 1u) != 0u;
+    int16v &hc = SET ? hB : hA, &lc = SET ? lB : lA, &hp = SET ? hA : hB, &lp = SET ? lA : lB;
+    const uint32_t ad_this = ad_rd + (i == 0u ? tab_prev : tab_cur), ad_after = ad_rd + tab_cur;
+    const uint32_t d_here = d_rd + tab_cur;
     auto step = [&](auto kk_c) {
-      constexpr uint32_t kk = decltype(kk_c)::value;
-      // step k = 8 s + kk: step k + 1 has landed for every wave (all but the loads of the steps after it)
-      if (kk + AHEAD <= 8u || more) GX_SYNC_STEPS(AHEAD - 2);
-      else GX_SYNC_STEPS(kk >= 6u ? 0 : (int)(6u - kk));
-      constexpr uint32_t NX = ((kk + 1u) & 7u) * SLOT;   // step k + 1's ring slot
-      constexpr int tq = (int)(kk >> 2), q4 = (int)(kk & 3u);   // the four outputs added up in this step: y[tq][4 q4 ..]
-      constexpr int cur = (int)(kk & 1u), nxt = cur ^ 1;
-      // the next step's four ad: of the same super-block, or (from step 7) of this one, whose sums are complete then
-      const uint32_t ad_nx = ad_rd + (kk == 7u ? tsl_cur : tsl_prev) + 128u * (((kk + 1u) & 7u) >> 2) + 32u * ((kk + 1u) & 3u);
+      constexpr uint32_t kk = decltype(kk_c)::value, b = kk & 3u, kn = (kk + 3u) & 7u, bn = (kk + 3u) & 3u;
+      constexpr bool over = kk + 3u >= 8u;   // the reads issued here are the next piece's
       auto add_up = [&](auto e_c) {
-        constexpr int e = decltype(e_c)::value;
+        constexpr uint32_t r = 2u * kk + decltype(e_c)::value;
         if constexpr (EPI) {
-          const int is = hp[tq][4 * q4 + e] * 256 + lp[tq][4 * q4 + e];
-          y[tq][4 * q4 + e] += a4[cur][e] * (d0 * (float)is);
+          const int is = NPL == 2u ? hp[r] * 256 + lp[r] : hp[r];
+          y[ip][r] += a2[b][decltype(e_c)::value] * (d0 * (float)is);
         }
       };
-      GX_PIN();
-      // outstanding, oldest first: [hw at step 0], a4[cur], wh, x0, x1, wl  (without EPI and before step 7: no a4)
-      GX_WAITN(2);
-      asm volatile("" : "+v"(wh), "+v"(x0), "+v"(a4[cur]), "+v"(hw));
-      if (EPI && kk == 0u) d0 = gm_f16_bits_to_f32(Q6 && (l32 & 1u) ? (hw >> 16) : (hw & 0xFFFFu));
-      hc[0] = GX_MFMA(x0, wh, kk == 0u ? zi : hc[0]);
-      GX_PIN();
-      // the loads of step k + AHEAD (into the slot step k - 1 left) go out behind a matrix instruction
-      if (kk == 0u && more) fetch_tables(s + 1u, tsl_next);
-      if ((kk + AHEAD < 8u || more) && !GX_ABL_NODMA) fetch_step(((kk + AHEAD) & 7u) * SLOT);
-      GX_PIN();
-      add_up(std::integral_constant<int, 0>{});
-      GX_PIN();
-      GX_WAITN(1);
-      asm volatile("" : "+v"(x1));
-      hc[1] = GX_MFMA(x1, wh, kk == 0u ? zi : hc[1]);
-      GX_PIN();
-      if (kk == 7u) asm volatile("ds_read_b32 %0, %1" : "=v"(hw) : "v"(hw_rd + tsl_cur));
-      if (EPI || kk == 7u) asm volatile("ds_read_b128 %0, %1" : "=v"(a4[nxt]) : "v"(ad_nx));
-      asm volatile("ds_read_b128 %0, %2 offset:%3" : "=v"(wh) : "0"(wh), "v"(w_rd), "n"(NX));
-      GX_PIN();
-      add_up(std::integral_constant<int, 1>{});
-      GX_PIN();
-      // outstanding: wl, [hw], [a4 next], wh
-      if (kk == 7u) GX_WAITN(3);
-      else if (EPI) GX_WAITN(2);
-      else GX_WAITN(1);
-      asm volatile("" : "+v"(wl));
-      lc[0] = GX_MFMA(x0, wl, kk == 0u ? zi : lc[0]);
-      GX_PIN();
-      asm volatile("ds_read_b128 %0, %2 offset:%3" : "=v"(x0) : "0"(x0), "v"(x_rd), "n"(NX));
-      GX_PIN();
-      add_up(std::integral_constant<int, 2>{});
-      GX_PIN();
-      lc[1] = GX_MFMA(x1, wl, kk == 0u ? zi : lc[1]);
-      GX_PIN();
-      asm volatile("ds_read_b128 %0, %2 offset:%3" : "=v"(x1) : "0"(x1), "v"(x_rd), "n"(NX + 1024u));
-      asm volatile("ds_read_b128 %0, %2 offset:%3" : "=v"(wl) : "0"(wl), "v"(w_rd), "n"(NX + 1024u));
-      GX_PIN();
-      add_up(std::integral_constant<int, 3>{});
-      GX_PIN();
+      using E0 = std::integral_constant<uint32_t, 0u>;
+      using E1 = std::integral_constant<uint32_t, 1u>;
+      GB_PIN();
+      // this step's reads were issued three steps ago; outstanding after them: those of two steps (and d's)
+      if constexpr (NPL == 2u)
+        asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(w[b][0]), "+v"(w[b][NPL - 1u]), "+v"(a2[b]), "+v"(dn) : "n"(2 * OPS + (kk == 4u || kk == 5u ? 1 : 0)));
+      else
+        asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(w[b][0]), "+v"(a2[b]), "+v"(dn) : "n"(2 * OPS + (kk == 4u || kk == 5u ? 1 : 0)));
+      if (kk == 0u) d0 = dn;
+      hc = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[kk], w[b][0], kk == 0u ? zi : hc, 0, 0, 0);
+      GB_PIN();
+      if constexpr (!over) GB_READS(kn, bn, w_cur, i * PIECE, ad_this);
+      else if constexpr (i + 1u < RB) GB_READS(kn, bn, w_cur, (i + 1u) * PIECE, ad_after);
+      else GB_READS(kn, bn, w_next, 0u, ad_after);
+      if constexpr (kk == 3u) asm volatile("ds_read_b32 %0, %2 offset:%3" : "=v"(dn) : "0"(dn), "v"(d_here), "n"(128u * i));
+      GB_PIN();
+      if constexpr (kk != 0u) add_up(E0{});
+      GB_PIN();
+      if constexpr (NPL == 2u) lc = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[kk], w[b][NPL - 1u], kk == 0u ? zi : lc, 0, 0, 0);
+      GB_PIN();
+      if constexpr (i == 0u) xnext[kk] = *(const int4v *)(xn + kk * 1024u);   // the next super-block's
+      if constexpr (kk == 0u) add_up(E0{});
+      add_up(E1{});
+      GB_PIN();
     };
     step(std::integral_constant<uint32_t, 0u>{});
     step(std::integral_constant<uint32_t, 1u>{});
@@ -1438,56 +1279,77 @@ __global__ __launch_bounds__(64 * GX_NW, 2) void ogm_gemm_dmx_kernel(GemmDmaPara
     step(std::integral_constant<uint32_t, 5u>{});
     step(std::integral_constant<uint32_t, 6u>{});
     step(std::integral_constant<uint32_t, 7u>{});
-    const uint32_t t = tsl_prev;   // the slots turn: s - 1's is free for s + 2
-    tsl_prev = tsl_cur;
-    tsl_cur = tsl_next;
-    tsl_next = (s == 0u) ? 2u * TAB_SLOT : t;
   };
   using std::false_type;
   using std::true_type;
-  super_block(false_type{}, false_type{}, 0u);
-  for (uint32_t s = 1; s < p.nsb; s += 2u) {
-    super_block(true_type{}, true_type{}, s);
-    if (s + 1u < p.nsb) super_block(false_type{}, true_type{}, s + 1u);
+  // (piece 1's top knows the wave's eight loads of x, issued in piece 0, among the newer ones; the tables the first top needs
+  // are older than a whole super-block's loads)
+  constexpr int N0 = (int)AHEAD, N1 = (int)AHEAD + 8;
+  static_assert(AHEAD <= RB * PER + 8u, "");
+  auto super_block = [&](auto first_c, int4v(&x)[8], int4v(&xnext)[8], uint32_t s) {
+    constexpr bool FIRST = decltype(first_c)::value;
+    const uint32_t w_cur = w_rd + (s % TURN) * (RB * PIECE), w_next = w_rd + ((s + 1u) % TURN) * (RB * PIECE);
+    const uint32_t tab_cur = (s & 3u) * TAB_SLOT;
+    xn = xsrc + min(s + 1u, nsb - 1u) * 8192u;
+    top(std::integral_constant<uint32_t, 0u>{}, std::integral_constant<int, N0>{}, s);
+    if constexpr (FIRST) {
+      GB_READS(0u, 0, w_cur, 0u, ad_rd);
+      GB_READS(1u, 1, w_cur, 0u, ad_rd);
+      GB_READS(2u, 2, w_cur, 0u, ad_rd);
+    }
+    piece(std::integral_constant<uint32_t, 0u>{}, std::integral_constant<bool, !FIRST>{}, x, xnext, w_cur, w_next, tab_cur);
+    top(std::integral_constant<uint32_t, 1u>{}, std::integral_constant<int, N1>{}, s);
+    piece(std::integral_constant<uint32_t, 1u>{}, true_type{}, x, xnext, w_cur, w_next, tab_cur);
+    if constexpr (RB == 4u) {
+      top(std::integral_constant<uint32_t, 2u>{}, std::integral_constant<int, N0>{}, s);
+      piece(std::integral_constant<uint32_t, 2u>{}, true_type{}, x, xnext, w_cur, w_next, tab_cur);
+      top(std::integral_constant<uint32_t, 3u>{}, std::integral_constant<int, N0>{}, s);
+      piece(std::integral_constant<uint32_t, 3u>{}, true_type{}, x, xnext, w_cur, w_next, tab_cur);
+    }
+    tab_prev = tab_cur;
+  };
+  super_block(true_type{}, xA, xB, 0u);
+  for (uint32_t s = 1; s < nsb; s += 2u) {
+    super_block(false_type{}, xB, xA, s);
+    if (s + 1u == nsb) break;
+    super_block(false_type{}, xA, xB, s + 1u);
   }
-  // the last super-block's sums (its header word and first four ad were asked for in its last step)
-  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wh), "+v"(x0), "+v"(x1), "+v"(wl), "+v"(a4[0]), "+v"(hw));
+  // the last piece's sums; the reads and fetches past the end
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : "+v"(w[0][0]), "+v"(w[1][0]), "+v"(w[2][0]), "+v"(w[3][0]), "+v"(w[0][NPL - 1u]), "+v"(w[1][NPL - 1u]),
+               "+v"(w[2][NPL - 1u]), "+v"(w[3][NPL - 1u]), "+v"(a2[0]), "+v"(a2[1]), "+v"(a2[2]), "+v"(a2[3]), "+v"(dn)::"memory");
   {
-    d0 = gm_f16_bits_to_f32(Q6 && (l32 & 1u) ? (hw >> 16) : (hw & 0xFFFFu));
-    const uint32_t ta = ad_rd + tsl_prev;   // (the slots have turned once more)
-    const bool odd = (p.nsb & 1u) == 0u;    // the last super-block filled set B
+    const uint32_t ta = ad_rd + tab_prev;
+    typedef float float4v __attribute__((ext_vector_type(4)));
 #pragma unroll
-    for (int tb = 0; tb < 2; tb++) {
-      float4v b40, b41, b42, b43;
-      GD_READ16(b40, ta, 128 * tb);
-      GD_READ16(b41, ta, 128 * tb + 32);
-      GD_READ16(b42, ta, 128 * tb + 64);
-      GD_READ16(b43, ta, 128 * tb + 96);
-      GD_WAIT2(0, b40, b41);
-      GD_WAIT2(0, b42, b43);
-      const float4v b4[4] = {b40, b41, b42, b43};
+    for (int q4 = 0; q4 < 4; q4++) {
+      float4v a4;
+      GD_READ16(a4, ta, 32 * q4);
+      GD_WAIT1(0, a4);
 #pragma unroll
-      for (int q4 = 0; q4 < 4; q4++) {
-        const float b4v[4] = {b4[q4].x, b4[q4].y, b4[q4].z, b4[q4].w};
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const int is = odd ? hB[tb][4 * q4 + e] * 256 + lB[tb][4 * q4 + e] : hA[tb][4 * q4 + e] * 256 + lA[tb][4 * q4 + e];
-          y[tb][4 * q4 + e] += b4v[e] * (d0 * (float)is);
-        }
+      for (int e = 0; e < 4; e++) {
+        const int r = 4 * q4 + e;
+        const int is = NPL == 2u ? hB[r] * 256 + lB[r] : hB[r];
+        y[RB - 1u][r] += a4[e] * (dn * (float)is);
       }
     }
   }
-  const uint32_t row0 = r0 + 32u * rs + l32;
-  if (row0 < p.out_dim) {
 #pragma unroll
-    for (int tb = 0; tb < 2; tb++)
+  for (uint32_t i = 0; i < RB; i++) {
+    const uint32_t row = r0 + 32u * i + l32;
+    if (row < p.out_dim) {
 #pragma unroll
       for (int r = 0; r < 16; r++) {
-        const uint32_t t = t0 + 64u * th + 32u * tb + 8u * (r >> 2) + 4u * lh + (r & 3);
-        if (t < p.n_tokens) p.y[(size_t)t * p.out_dim + row0] = y[tb][r];
+        const uint32_t t = t0 + 32u * wave + 8u * (r >> 2) + 4u * lh + (r & 3);
+        if (t < p.n_tokens) p.y[(size_t)t * p.out_dim + row] = y[i][r];
       }
+    }
   }
 }
+
+template <int KIND>
+__global__ __launch_bounds__(256, 2) void ogm_gemm_dma_kernel(GemmDmaParams p) { gemm_planes_body<KIND, 4u>(p); }
+template <int KIND>
+__global__ __launch_bounds__(256, 2) void ogm_gemm_dmx_kernel(GemmDmaParams p) { gemm_planes_body<KIND, 2u>(p); }
 
 // ------------------------------------------------------------------------------------------
 // Small batches (up to a few dozen tokens): the tiled kernels above cost the same for 9 tokens as
@@ -2958,7 +2820,7 @@ size_t ogm_gemm_plane_bytes(uint32_t ggml_type, uint32_t in_dim, uint32_t out_di
       in_dim == 0 || in_dim % 256u != 0 || out_dim == 0)
     return 0;
   const uint32_t npl = ggml_type == OGM_Q3_K ? 1u : 2u;
-  return gp_plane_offset((out_dim + 63u) / 64u, in_dim / 256u, 0, 0, 0, npl);
+  return gp_total_bytes((out_dim + 63u) / 64u, in_dim / 256u, npl, ggml_type == OGM_Q4_K || ggml_type == OGM_Q5_K);
 }
 
 hipError_t ogm_gemm_build_planes(uint32_t ggml_type, const uint8_t *wt, uint32_t in_dim, uint32_t out_dim,
@@ -2975,13 +2837,20 @@ hipError_t ogm_gemm_build_planes(uint32_t ggml_type, const uint8_t *wt, uint32_t
   p.nct = tl.nct;
   const dim3 grid(4u * p.nsb, (out_dim + 63u) / 64u);
   if (grid.y > 65535u) return hipErrorInvalidValue;
+  const dim3 side(2u * grid.y, p.nsb);
+  if (side.y > 65535u) return hipErrorInvalidValue;
+#define GP_BUILD(K)                                                                              \
+  hipLaunchKernelGGL(ogm_gemm_build_planes_kernel<K>, grid, dim3(256), 0, stream, p);            \
+  hipLaunchKernelGGL(ogm_gemm_build_side_kernel<K>, side, dim3(64), 0, stream, p);               \
+  break
   switch (ggml_type) {
-    case OGM_Q6_K: hipLaunchKernelGGL(ogm_gemm_build_planes_kernel<GP_Q6K>, grid, dim3(256), 0, stream, p); break;
-    case OGM_Q3_K: hipLaunchKernelGGL(ogm_gemm_build_planes_kernel<GP_Q3K>, grid, dim3(256), 0, stream, p); break;
-    case OGM_Q4_K: hipLaunchKernelGGL(ogm_gemm_build_planes_kernel<GP_Q4K>, grid, dim3(256), 0, stream, p); break;
-    case OGM_IQ4_XS: hipLaunchKernelGGL(ogm_gemm_build_planes_kernel<GP_IQ4XS>, grid, dim3(256), 0, stream, p); break;
-    default: hipLaunchKernelGGL(ogm_gemm_build_planes_kernel<GP_Q5K>, grid, dim3(256), 0, stream, p); break;
+    case OGM_Q6_K: GP_BUILD(GP_Q6K);
+    case OGM_Q3_K: GP_BUILD(GP_Q3K);
+    case OGM_Q4_K: GP_BUILD(GP_Q4K);
+    case OGM_IQ4_XS: GP_BUILD(GP_IQ4XS);
+    default: GP_BUILD(GP_Q5K);
   }
+#undef GP_BUILD
   return hipGetLastError();
 }
 
@@ -3008,7 +2877,7 @@ hipError_t ogm_gemm_build_planes(uint32_t ggml_type, const uint8_t *wt, uint32_t
 static bool gemm_interleaved(const OgmGemmArgs &a, bool for_small_batch = false) {
   const uint32_t nsb = a.in_dim / 256;
   const bool q45 = a.ggml_type == OGM_Q4_K || a.ggml_type == OGM_Q5_K, xs = a.ggml_type == OGM_IQ4_XS;
-  if (a.interleave == 1u || a.ggml_type == OGM_Q3_K || (q45 && a.one_pass != 0u) || nsb * 512u > GX_TAB ||
+  if (a.interleave == 1u || a.ggml_type == OGM_Q3_K || (q45 && a.one_pass != 0u) ||
       a.n_tokens < (xs ? 17u : 32u))
     return false;
   if (a.interleave == 2u) return true;
@@ -3034,10 +2903,8 @@ static bool gemm_interleaved(const OgmGemmArgs &a, bool for_small_batch = false)
 // activations in operand chunks, and everything within 32-bit byte offsets.  (plane_kernel 2: whatever the
 // grid.)
 static bool gemm_dma_eligible(const OgmGemmArgs &a) {
-  const uint32_t nsb = a.in_dim / 256;
-  const bool q45 = a.ggml_type == OGM_Q4_K || a.ggml_type == OGM_Q5_K;
   const uint32_t t_pad = (a.n_tokens + 31u) & ~31u;
-  if ((q45 && nsb * 512u > GD_TAB) || a.n_tokens < (a.ggml_type == OGM_IQ4_XS ? 17u : 32u) || !a.xh ||
+  if (a.n_tokens < (a.ggml_type == OGM_IQ4_XS ? 17u : 32u) || !a.xh ||
       (uint64_t)t_pad * a.in_dim >= (1ull << 32))
     return false;
   uint32_t tiles = 0;
@@ -3354,16 +3221,17 @@ hipError_t ogm_launch_gemm(const OgmGemmArgs &a, hipStream_t stream, const char 
       if (m < a.n_extra) tiles += (a.extra_out_dim[m] + GD_ROWS - 1u) / GD_ROWS;
     }
     if (interleaved) {
-      uint32_t tiles_x = (a.out_dim + GX_ROWS - 1u) / GX_ROWS;
-      for (uint32_t m = 0; m < a.n_extra; m++) tiles_x += (a.extra_out_dim[m] + GX_ROWS - 1u) / GX_ROWS;
+      uint32_t tiles_x = (a.out_dim + 63u) / 64u;
+      for (uint32_t m = 0; m < a.n_extra; m++) tiles_x += (a.extra_out_dim[m] + 63u) / 64u;
+      const uint32_t lds_x = GbShape<GP_Q4K, 2u>::LDS_BYTES;
       const void *fx = a.ggml_type == OGM_Q6_K     ? (const void *)ogm_gemm_dmx_kernel<GP_Q6K>
                        : a.ggml_type == OGM_IQ4_XS ? (const void *)ogm_gemm_dmx_kernel<GP_IQ4XS>
                        : a.ggml_type == OGM_Q4_K   ? (const void *)ogm_gemm_dmx_kernel<GP_Q4K>
                                                    : (const void *)ogm_gemm_dmx_kernel<GP_Q5K>;
-      hipError_t ex = hipFuncSetAttribute(fx, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GX_LDS_BYTES);
+      hipError_t ex = hipFuncSetAttribute(fx, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_x);
       if (ex != hipSuccess) return ex;
       void *xargs[] = {(void *)&d};
-      ex = hipLaunchKernel(fx, dim3((a.n_tokens + GX_TOK - 1u) / GX_TOK, tiles_x), dim3(64u * GX_NW), xargs, GX_LDS_BYTES, stream);
+      ex = hipLaunchKernel(fx, dim3((a.n_tokens + GD_TOK - 1u) / GD_TOK, tiles_x), dim3(256), xargs, lds_x, stream);
       if (ex != hipSuccess) return ex;
       if (kernel_name)
         *kernel_name = a.ggml_type == OGM_Q6_K     ? "ogm_gemm_q6k_dmx_kernel"
@@ -3376,11 +3244,11 @@ hipError_t ogm_launch_gemm(const OgmGemmArgs &a, hipStream_t stream, const char 
     const void *fn = a.ggml_type == OGM_Q6_K   ? (const void *)ogm_gemm_dma_kernel<GP_Q6K>
                      : a.ggml_type == OGM_IQ4_XS ? (const void *)ogm_gemm_dma_kernel<GP_IQ4XS>
                      : a.ggml_type == OGM_Q3_K ? (const void *)ogm_gemm_dma_kernel<GP_Q3K>
-                     : a.ggml_type == OGM_Q4_K ? (one_pass ? (const void *)ogm_gemm_dma_kernel<GP_Q4K, true>
+                     : a.ggml_type == OGM_Q4_K ? (one_pass ? (const void *)ogm_gemm_onepass_kernel<GP_Q4K>
                                                            : (const void *)ogm_gemm_dma_kernel<GP_Q4K>)
-                                               : (one_pass ? (const void *)ogm_gemm_dma_kernel<GP_Q5K, true>
+                                               : (one_pass ? (const void *)ogm_gemm_onepass_kernel<GP_Q5K>
                                                            : (const void *)ogm_gemm_dma_kernel<GP_Q5K>);
-    const uint32_t dma_lds = one_pass ? GD_LDS_BYTES_ONEPASS : GD_LDS_BYTES;
+    const uint32_t dma_lds = one_pass ? GD_LDS_BYTES : a.ggml_type == OGM_Q3_K ? GbShape<GP_Q3K, 4u>::LDS_BYTES : GbShape<GP_Q4K, 4u>::LDS_BYTES;
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dma_lds);
     if (e != hipSuccess) return e;
     void *kargs[] = {(void *)&d};
