@@ -2854,67 +2854,63 @@ hipError_t ogm_gemm_build_planes(uint32_t ggml_type, const uint8_t *wt, uint32_t
   return hipGetLastError();
 }
 
-// Whether a launch over planes takes the kernel with 64-row tiles that adds a super-block up between the next one's
-// matrix instructions (ogm_gemm_dmx_kernel) instead of the one with 128-row tiles (ogm_gemm_dma_kernel).
-// interleave: 0 by the size of the launch, 1 never, 2 whenever the type allows.  Measured on MI355X, whole calls at
-// 512 tokens, us, 64-row interleaved / 128-row / feeding waves: Q6_K 14336 -> 4096 103 / 153 / 126, Q4_K 4096 ->
-// 4096 42 / 64 / 49, 4096 -> 6144 54 / 67 / 64, 14336 -> 4096 130 / 204 / 150; but 4096 -> 14336 115 / 98 / -.
-// Its workgroups (64 rows x 128 tokens) must fit the device in one round, two to a compute unit: beyond 512 of
-// them the 128-row kernel is ahead (Q4_K 4096 -> 14336 at 384 tokens, 672 workgroups: 91 against 87; 5120 -> 13824
-// at 288: 104 against 99; 8192 -> 10240 at 512: 174 against 165).
-//   Q6_K has no first pass to pay for and no medium-batch kernel beside it, so it takes this kernel from 128
-// workgroups on, and from 96 with at least 192 tokens, before the small-batch kernel is asked (against the small-batch
-// and feeding-wave kernels: 14336 -> 4096 at 256 tokens 87 against 101, 4096 -> 4096 at 256 28 against 38, 8192 ->
-// 2048 at 384 50 against 61, 13824 -> 5120 at 160 79 against 93, 28672 -> 8192 at 128 171 against 199; level with
-// them at 160 tokens of the 4096-row matrices; behind with fewer workgroups: 8192 -> 2048 at 256 tokens, 64 of them,
-// 47 against 38).  A lone token tile wants to be nearly full.
-//   Q4_K / Q5_K want three token tiles and 160 workgroups (at 256 tokens it only draws with the medium-batch kernel,
-// which needs no planes: 4096 -> 6144 37 against 37), and with longer rows than 5120 inputs no more workgroups than
-// compute units (8192 -> 8192 at 384 / 512 tokens, 384 / 512 workgroups, 114 / 127 against 101 / 113 for the
-// feeding-wave kernel, 8192 -> 10240 at 384 120 against 108; but 14336 -> 4096 at 384 / 512 tokens, 192 / 256
-// workgroups, 121 / 127 against 135 / 143).
+// Workgroups of a launch over planes, in row tiles of `rows`.
+static uint32_t gemm_plane_wgs(const OgmGemmArgs &a, uint32_t rows) {
+  uint32_t tiles = 0;
+  for (uint32_t m = 0; m <= a.n_extra; m++) tiles += ((m ? a.extra_out_dim[m - 1] : a.out_dim) + rows - 1u) / rows;
+  return (a.n_tokens + GD_TOK - 1u) / GD_TOK * tiles;
+}
+
+// Whether a launch over planes takes 64-row tiles (ogm_gemm_dmx_kernel) instead of 128-row ones (ogm_gemm_dma_kernel).
+// interleave: 0 by the size of the launch, 1 never, 2 whenever the type allows.  Measured on MI355X, whole calls, us, 64-row /
+// 128-row / the best kernel without planes.
+//   Where the 64-row workgroups come at most one to a compute unit (256 of them) they lead: Q4_K 4096 -> 4096 at 512
+// tokens (256) 32 / 45, 14336 -> 4096 at 512 102 / 138, Q6_K 14336 -> 4096 at 512 90 / 115.  Beyond, two to a compute unit up
+// to 512, the 128-row tiles -- one to a compute unit then -- fetch less: Q4_K 4096 -> 6144 at 512 (384) 48.8 / 47.2 / 60,
+// 8192 -> 8192 at 300 (384) 87 / 85 / 105, 8192 -> 8192 at 512 107 / 103 / 118, 14336 -> 4096 at 768 163 / 152 / 185, 14336 ->
+// 8192 at 300 162 / 146 / 178, 8192 -> 2048 at 1901 (480) 110 / 103 / 120.  Level below 4096 inputs (2048 -> 8192 at 300 / 512
+// 26.9 / 27.6, 31.5 / 31.1) and without a first pass (Q6_K 4096 -> 4096 at 768 43.0 / 43.2, 14336 -> 4096 at 768 138 / 135).
+//   At the lower end: Q6_K from 128 workgroups with two token tiles (4096 -> 4096 at 160 tokens 22.9 against 24.7, 14336 ->
+// 4096 61.6 / 66.2 for the small-batch kernel; below 4096 inputs, as Q6_K did before, from 160, or 128 with a nearly full last
+// tile or three tiles) and with a lone token tile when it is nearly full.  Q4_K / Q5_K with three token tiles from 160
+// workgroups (2048 -> 2048 at 512, 128 of them, 19.0 against 17.3), with two from 160 (4096 -> 6144 at 160 / 256 tokens
+// 28 / 29 against 38 / 37 for the medium-batch kernel, 2048 -> 8192 19 / 21 against 23 / 24, 5120 -> 5120 32 / 33 against 43 /
+// 44, 8192 -> 8192 51 / 60 against 71 / 74) or, beyond 160 tokens of rows of 4096 inputs and more, from 128 (4096 -> 4096 at
+// 160 / 256 27.7 / 28.4 against 27.5 / 31.1, 11008 -> 4096 60 / 64 against 66 / 73, 14336 -> 4096 78 / 82 against 80 / 91 for the
+// small-batch kernel); rows of fewer than 2048 inputs leave two token tiles to the kernels without planes.
 // for_small_batch: asked by gemm_small_batch, whether the launch is one this kernel takes ahead of the small batches.
 static bool gemm_interleaved(const OgmGemmArgs &a, bool for_small_batch = false) {
   const uint32_t nsb = a.in_dim / 256;
   const bool q45 = a.ggml_type == OGM_Q4_K || a.ggml_type == OGM_Q5_K, xs = a.ggml_type == OGM_IQ4_XS;
-  if (a.interleave == 1u || a.ggml_type == OGM_Q3_K || (q45 && a.one_pass != 0u) ||
-      a.n_tokens < (xs ? 17u : 32u))
-    return false;
+  if (a.interleave == 1u || a.ggml_type == OGM_Q3_K || (q45 && a.one_pass != 0u) || a.n_tokens < (xs ? 17u : 32u)) return false;
   if (a.interleave == 2u) return true;
-  uint32_t tiles64 = 0;
-  for (uint32_t m = 0; m <= a.n_extra; m++) tiles64 += ((m ? a.extra_out_dim[m - 1] : a.out_dim) + 63u) / 64u;
-  const uint32_t tok_tiles = (a.n_tokens + 127u) / 128u;
-  const uint32_t n_wg = tok_tiles * tiles64;
-  if (n_wg > 512u) return false;
-  // (beyond its small batches IQ4_XS has the two plane kernels only: 4096 -> 4096 at 32 tokens 28 us against 46 on the
-  // 128-row tiles, 14336 -> 4096 77 against 141, 4096 -> 14336 33 against 50)
+  const uint32_t tok_tiles = (a.n_tokens + GD_TOK - 1u) / GD_TOK, n_wg = gemm_plane_wgs(a, 64u);
+  if (n_wg > (q45 && nsb >= 16u ? 256u : 512u)) return false;
+  // (beyond its small batches IQ4_XS has the two plane kernels only)
   if (xs && !for_small_batch) return true;
   if (!q45) {
-    const uint32_t last = a.n_tokens - (tok_tiles - 1u) * 128u;   // tokens of the last token tile
-    return (n_wg >= 160u && (tok_tiles >= 2u || a.n_tokens > 96u)) || (n_wg >= 128u && last > 96u) ||
-           (n_wg >= 128u && tok_tiles >= 3u);
+    const uint32_t last = a.n_tokens - (tok_tiles - 1u) * GD_TOK;   // tokens of the last token tile
+    return (n_wg >= 160u && (tok_tiles >= 2u || a.n_tokens > 96u)) ||
+           (n_wg >= 128u && (last > 96u || tok_tiles >= 3u || (tok_tiles == 2u && nsb >= 16u)));
   }
-  return (tok_tiles >= 3u || (tok_tiles == 2u && nsb > 32u)) && n_wg >= 160u && (nsb <= 20u || n_wg <= 256u);
+  if (tok_tiles == 2u) return nsb >= 8u && (n_wg >= 160u || (n_wg >= 128u && nsb >= 16u && a.n_tokens > 160u));
+  return tok_tiles >= 3u && n_wg >= 160u;
 }
 
-// Whether a tiled launch goes to a kernel whose waves all multiply, given planes.  The one with 128 x 128
-// workgroups wants more of them than there are compute units (two share one, and one alone is slower than the
-// feeding-wave kernels: Q4_K 4096 -> 14336 at 256 tokens 69 us against 57, at 384 tokens 87 against 104), the
-// activations in operand chunks, and everything within 32-bit byte offsets.  (plane_kernel 2: whatever the
-// grid.)
+// Whether a tiled launch goes to a kernel whose waves all multiply, given planes: more 128-row workgroups than compute units
+// (or, rows of 4096 inputs and more of Q4_K / Q5_K, more 64-row ones: see gemm_interleaved) or a launch for the 64-row tiles,
+// the activations in operand chunks, and everything within 32-bit byte offsets.  (plane_kernel 2: whatever the grid.)
 static bool gemm_dma_eligible(const OgmGemmArgs &a) {
+  const bool q45 = a.ggml_type == OGM_Q4_K || a.ggml_type == OGM_Q5_K;
   const uint32_t t_pad = (a.n_tokens + 31u) & ~31u;
-  if (a.n_tokens < (a.ggml_type == OGM_IQ4_XS ? 17u : 32u) || !a.xh ||
-      (uint64_t)t_pad * a.in_dim >= (1ull << 32))
-    return false;
-  uint32_t tiles = 0;
+  if (a.n_tokens < (a.ggml_type == OGM_IQ4_XS ? 17u : 32u) || !a.xh || (uint64_t)t_pad * a.in_dim >= (1ull << 32)) return false;
   for (uint32_t m = 0; m <= a.n_extra; m++) {
     const uint32_t od = m ? a.extra_out_dim[m - 1] : a.out_dim;
     if ((uint64_t)((od + 63u) / 64u) * 64u * a.in_dim * 2u >= (1ull << 32)) return false;
-    tiles += (od + GD_ROWS - 1u) / GD_ROWS;
   }
   // (IQ4_XS has no other GEMM kernel)
-  if (a.plane_kernel == 2u || a.ggml_type == OGM_IQ4_XS || ((a.n_tokens + GD_TOK - 1u) / GD_TOK) * tiles > 256u) return true;
+  if (a.plane_kernel == 2u || a.ggml_type == OGM_IQ4_XS || gemm_plane_wgs(a, GD_ROWS) > 256u) return true;
+  if (q45 && a.in_dim >= 4096u && a.n_tokens > GD_TOK && gemm_plane_wgs(a, 64u) > 256u) return true;
   return gemm_interleaved(a);
 }
 
@@ -2924,9 +2920,9 @@ static bool gemm_dma_eligible(const OgmGemmArgs &a) {
 static bool gemm_small_batch(const OgmGemmArgs &a, bool planes_possible) {
   const uint32_t nsb = a.in_dim / 256;
   const bool q45 = a.ggml_type == OGM_Q4_K || a.ggml_type == OGM_Q5_K;
-  // Q6_K and IQ4_XS launches the interleaved plane kernel wants by their size go there (see gemm_interleaved)
-  if ((a.ggml_type == OGM_Q6_K || a.ggml_type == OGM_IQ4_XS) && a.small_max_tokens == 0u && a.interleave == 0u &&
-      planes_possible && gemm_dma_eligible(a) && gemm_interleaved(a, true))
+  // launches the 64-row plane kernel wants by their size go there (see gemm_interleaved)
+  if (a.ggml_type != OGM_Q3_K && a.small_max_tokens == 0u && a.interleave == 0u && planes_possible && gemm_dma_eligible(a) &&
+      gemm_interleaved(a, true))
     return false;
   uint32_t tiles64_all = (a.out_dim + 63u) / 64u;
   for (uint32_t m = 0; m < a.n_extra; m++) tiles64_all += (a.extra_out_dim[m] + 63u) / 64u;
