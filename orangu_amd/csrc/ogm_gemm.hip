@@ -2432,10 +2432,11 @@ struct GemmFlatParams {
 #define GF_STAGE (128u * GF_A_ROW)         // f16 of one operand's stage
 #define GF_LDS (4u * GF_STAGE * 2u + 2u * 2u * 128u * 4u)   // bytes: two stages of both operands and of the weight scales
 
-// KIND 0: Q4_0, 1: Q5_0, 2: IQ4_NL, 3: Q8_0
+// KIND 0: Q4_0, 1: Q5_0, 2: IQ4_NL.  Launches of the nibble types that fill the device: unpacked once a workgroup by its
+// feeding waves (ogm_gemm_flat_kernel below unpacks in every multiplying wave).
 template <int KIND>
-__global__ __launch_bounds__(768) void ogm_gemm_flat_kernel(GemmFlatParams p) {
-  constexpr uint32_t PIECES = KIND == 3 ? 2u : 1u;
+__global__ __launch_bounds__(768) void ogm_gemm_flat_f16_kernel(GemmFlatParams p) {
+  constexpr uint32_t PIECES = 1u;
   constexpr uint32_t TAIL = KIND == 1 ? 6u : 2u;
   constexpr uint32_t TILE = 64u * (16u * PIECES + TAIL);
   extern __shared__ __align__(16) uint8_t gf_lds[];
@@ -2470,7 +2471,7 @@ __global__ __launch_bounds__(768) void ogm_gemm_flat_kernel(GemmFlatParams p) {
     const uint32_t bso = btok0 * GF_A_ROW + 16u * bch;   // f16
     const uint32_t aso = arow * GF_A_ROW + 32u * abl;   // f16 offset of the block's first chunk
 
-    uint4 qa_0, qa_1, qa_2, qb_0, qb_1, qb_2;          // weight pieces (qb only for Q8_0)
+    uint4 qa_0, qa_1, qa_2;                            // weight pieces
     uint32_t tl_0, tl_1, tl_2, th_0, th_1, th_2;       // tail: d16 (and qh for Q5_0)
     uint4 bx_0, bx_1, bx_2, by_0, by_1, by_2;          // activation chunks
 
@@ -2480,7 +2481,6 @@ __global__ __launch_bounds__(768) void ogm_gemm_flat_kernel(GemmFlatParams p) {
     uint32_t tail_;                                                                                \
     const uint32_t uo_ = unit_off(2u * st_ + abl, &tail_);                                         \
     qa_##K = *(const uint4 *)(p.wt + uo_);                                                         \
-    if (KIND == 3) qb_##K = *(const uint4 *)(p.wt + uo_ + 1024u);                                  \
     const uint16_t *tp_ = (const uint16_t *)(p.wt + tail_);                                        \
     tl_##K = tp_[0];                                                                               \
     th_##K = KIND == 1 ? ((uint32_t)tp_[1] | ((uint32_t)tp_[2] << 16)) : 0u;                       \
@@ -2491,16 +2491,11 @@ __global__ __launch_bounds__(768) void ogm_gemm_flat_kernel(GemmFlatParams p) {
 #define GF_STORE(BUF, K)                                                                           \
   do {                                                                                             \
     uint32_t w_[8]; /* the block's 32 int8 weights, k order */                                     \
-    if (KIND == 3) {                                                                               \
-      w_[0] = qa_##K.x; w_[1] = qa_##K.y; w_[2] = qa_##K.z; w_[3] = qa_##K.w;                      \
-      w_[4] = qb_##K.x; w_[5] = qb_##K.y; w_[6] = qb_##K.z; w_[7] = qb_##K.w;                      \
-    } else {                                                                                       \
-      const uint32_t q_[4] = {qa_##K.x, qa_##K.y, qa_##K.z, qa_##K.w};                             \
-      _Pragma("unroll") for (int k_ = 0; k_ < 4; k_++) {                                           \
-        w_[k_] = ogm_nib32_weights<KIND>(q_[k_] & 0x0F0F0F0Fu, (th_##K >> (4 * k_)) & 0xFu);       \
-        w_[4 + k_] = ogm_nib32_weights<KIND>((q_[k_] >> 4) & 0x0F0F0F0Fu,                          \
-                                             (th_##K >> (16 + 4 * k_)) & 0xFu);                    \
-      }                                                                                            \
+    const uint32_t q_[4] = {qa_##K.x, qa_##K.y, qa_##K.z, qa_##K.w};                               \
+    _Pragma("unroll") for (int k_ = 0; k_ < 4; k_++) {                                             \
+      w_[k_] = ogm_nib32_weights<KIND>(q_[k_] & 0x0F0F0F0Fu, (th_##K >> (4 * k_)) & 0xFu);         \
+      w_[4 + k_] = ogm_nib32_weights<KIND>((q_[k_] >> 4) & 0x0F0F0F0Fu,                            \
+                                           (th_##K >> (16 + 4 * k_)) & 0xFu);                      \
     }                                                                                              \
     _Float16 *ab_ = A_l + (BUF) * GF_STAGE + aso;                                                  \
     _Pragma("unroll") for (int c_ = 0; c_ < 4; c_++)                                               \
@@ -2604,6 +2599,281 @@ __global__ __launch_bounds__(768) void ogm_gemm_flat_kernel(GemmFlatParams p) {
           for (int e = 0; e < 4; e++)
             if (row + e < p.out_dim) dst[e] = yy[4 * q4 + e];
         }
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------
+// The per-32 types' tiled GEMM on int8 operands as they lie (dot_flat_pair, vecdot.rs:2598-2629), rows of any number of blocks.
+// A block is one 32 x 32 x 32 matrix instruction per 32 x 32 outputs; the scales' products come from an outer product
+// (32 x 32 x 1, two row blocks an instruction); three vector instructions an output and block remain -- convert, multiply,
+// add, in the reference's order -- and bound it: two waves a SIMD issue a vector instruction every 2.2 clocks, which is
+// 107 clocks a block beside 64 of the matrix pipe.  The f16 kernel above needs two, its products being floats already, but
+// converts both operands from int8 once a workgroup and moves twice the bytes: Q8_0, whole calls, us, 4096 -> 14336 at
+// 512 / 2048 tokens 130 / 461 there, 105 / 366 here, 4096 -> 4096 at 512 66 / 48, 14336 -> 4096 at 512 210 / 140.
+//   As in gemm_planes_body a wave multiplies one token block of 32 with every row block of the tile, the activations come
+// straight from their rows into registers (a piece of four blocks ahead), the weights through a ring of four pieces in LDS,
+// a barrier a piece.  A step is a block of a row block: its product, its operand's read two steps ahead, and behind it the 48
+// vector instructions of the step before; every second step the outer product of two row blocks' scales.
+//   The nibble types' operands are unpacked by the wave that multiplies (Q4_0 16 instructions a step, IQ4_NL 36), which
+// costs less than the f16 kernel's feeding waves only on launches of one workgroup a compute unit: Q4_0 4096 -> 4096 at 384
+// tokens 65 / 53, 14336 -> 4096 at 512 206 / 168; 4096 -> 14336 at 512 127 / 129, IQ4_NL the same 134 / 156.
+// KIND 0: Q4_0, 1: Q5_0, 2: IQ4_NL, 3: Q8_0; RB: row blocks of 32 a workgroup.
+template <int KIND, uint32_t RB>
+struct FlatShape {
+  static constexpr bool Q8 = KIND == 3;
+  static constexpr uint32_t PIECES = Q8 ? 2u : 1u, TAIL = KIND == 1 ? 6u : 2u, TILE = 64u * (16u * PIECES + TAIL);
+  static constexpr uint32_t W_BYTES = RB * 4u * 512u * PIECES;   // four blocks of 32 RB rows
+  static constexpr uint32_t T_BYTES = RB * 128u * TAIL;          // their tails, tile after tile
+  static constexpr uint32_t T_OFF = W_BYTES, A_OFF = T_OFF + T_BYTES, SLOT = A_OFF + 4u * 512u;   // a wave's 32 tokens' scales
+  static constexpr uint32_t SLOTS = 4;
+  static constexpr uint32_t LDS_BYTES = SLOTS * SLOT;
+  static constexpr uint32_t W_OPS = W_BYTES / 4096u, T_OPS = (T_BYTES / 256u + 3u) / 4u;   // loads a wave issues per piece
+};
+
+template <int KIND, uint32_t RB>
+__global__ __launch_bounds__(256, 2) void ogm_gemm_flat_kernel(GemmFlatParams p) {
+  using Shape = FlatShape<KIND, RB>;
+  constexpr bool Q8 = Shape::Q8;
+  constexpr uint32_t TAIL = Shape::TAIL, TILE = Shape::TILE, SLOT = Shape::SLOT, SLOTS = Shape::SLOTS;
+  constexpr uint32_t ROWS = 32u * RB, TOK = 128u;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t l32 = lane & 31u, lh = lane >> 5;
+  uint32_t tok_tile = blockIdx.x, row_tile = blockIdx.y;   // token tiles of one row tile go to one XCD back to back
+  {
+    const uint32_t nt = gridDim.x, lin = blockIdx.y * nt + blockIdx.x;
+    if (lin < (gridDim.y & ~7u) * nt) {
+      const uint32_t j = lin >> 3;
+      tok_tile = j % nt;
+      row_tile = (j / nt) * 8u + (lin & 7u);
+    }
+  }
+  tok_tile = __builtin_amdgcn_readfirstlane(tok_tile);
+  row_tile = __builtin_amdgcn_readfirstlane(row_tile);
+  const uint32_t t0 = tok_tile * TOK, r0 = row_tile * ROWS;
+  const uint32_t nblk = p.nblk, np = (nblk + 3u) >> 2;
+  const uint32_t cs = p.c_shift, rs = p.r_shift, cm = (1u << cs) - 1u, rm = (1u << rs) - 1u;
+  const bool live = t0 + 32u * wave < p.n_tokens;
+
+  // ---- what goes to LDS
+  const __amdgpu_buffer_rsrc_t wt = gb_buffer(p.wt);
+  const __amdgpu_buffer_rsrc_t adb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.ad), 0, (int)(p.n_tokens * nblk * 4u), 0x00027000);
+  // weights: Q8_0 a chunk is a block of a row block of 32 (lane (l32, lh): half lh of row l32's block), the nibble types' one
+  // of two row blocks (lane: a row's sixteen bytes); per wave one row block or pair, W_OPS blocks
+  const uint32_t w_rb = Q8 ? wave % RB : (RB == 4u ? (wave & 1u) : 0u);
+  const uint32_t w_b0 = Q8 ? (wave / RB) * Shape::W_OPS : (RB == 4u ? (wave >> 1) * 2u : wave);
+  uint32_t w_lane;
+  {
+    const uint32_t row = min(r0 + (Q8 ? 32u * w_rb + l32 : 64u * w_rb + lane), p.out_dim - 1u);
+    w_lane = (row >> rs) * p.nct * TILE + (row & rm) * 16u + (Q8 ? lh * 1024u : 0u);
+  }
+  constexpr uint32_t W_BLOCK = Shape::W_BYTES / 4u;   // LDS bytes of a block
+  auto w_soff = [&](uint32_t b) -> uint32_t { return (b >> cs) * TILE + ((b & cm) << rs) * 16u; };
+  // tails: the piece's 2 RB tiles one after the other, 16 TAIL words each
+  uint32_t t_lane[Shape::T_OPS], t_ct[Shape::T_OPS];
+#pragma unroll
+  for (uint32_t q = 0; q < Shape::T_OPS; q++) {
+    const uint32_t word = ((wave * Shape::T_OPS + q) * 64u + lane) % (Shape::T_BYTES / 4u);
+    const uint32_t i = word / (16u * TAIL), ctn_shift = 2u - cs;   // the tile, and how many a row block has in a piece
+    const uint32_t nrb = (p.out_dim + rm) >> rs;
+    const uint32_t rb = min((r0 >> rs) + (i >> ctn_shift), nrb - 1u);
+    t_ct[q] = i & ((1u << ctn_shift) - 1u);
+    t_lane[q] = rb * p.nct * TILE + Shape::PIECES * 1024u + (word - i * (16u * TAIL)) * 4u;
+  }
+  // scales: this wave's 32 tokens, four blocks each
+  uint32_t a_lane[2];
+#pragma unroll
+  for (uint32_t q = 0; q < 2u; q++) {
+    const uint32_t w = q * 64u + lane;
+    a_lane[q] = (min(t0 + 32u * wave + (w >> 2), p.n_tokens - 1u) * nblk + (w & 3u)) * 4u;
+  }
+  auto fetch = [&](uint32_t pc, uint32_t slot) {   // piece pc (past the end: the last one again, never read)
+    const uint32_t pp = min(pc, np - 1u);
+    uint8_t *dst = lds + slot * SLOT;
+#pragma unroll
+    for (uint32_t j = 0; j < Shape::W_OPS; j++)
+      gb_dma16<0>(wt, w_lane, w_soff(min(4u * pp + w_b0 + j, nblk - 1u)), dst + (w_b0 + j) * W_BLOCK + w_rb * 1024u);
+#pragma unroll
+    for (uint32_t q = 0; q < Shape::T_OPS; q++)
+      gb_dma4(wt, t_lane[q] + min((pp << (2u - cs)) + t_ct[q], p.nct - 1u) * TILE, 0u,
+              dst + Shape::T_OFF + ((wave * Shape::T_OPS + q) % (Shape::T_BYTES / 256u)) * 256u);
+#pragma unroll
+    for (uint32_t q = 0; q < 2u; q++) gb_dma4(adb, a_lane[q], pp * 16u, dst + Shape::A_OFF + wave * 512u + q * 256u);
+  };
+  constexpr int FETCH = (int)(Shape::W_OPS + Shape::T_OPS + 2u);
+  auto top = [&](auto n_c, uint32_t pc) {   // piece pc + 1 has landed, piece pc - 1 is no longer read
+    GB_PIN();
+    GB_SYNC(decltype(n_c)::value);
+    fetch(pc + SLOTS - 1u, (pc + SLOTS - 1u) % SLOTS);
+    GB_PIN();
+  };
+#pragma unroll
+  for (uint32_t q = 0; q < SLOTS - 1u; q++) fetch(q, q);
+  asm volatile("" ::: "memory");
+  if (!live) {
+    for (uint32_t pc = 0; pc < np; pc++) top(std::integral_constant<int, FETCH>{}, pc);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return;
+  }
+
+  // ---- this wave's tokens
+  const int8_t *xsrc = p.xq + ((size_t)min(t0 + 32u * wave + l32, p.n_tokens - 1u) * p.in_dim + 16u * lh);
+  int4v x[4];
+#pragma unroll
+  for (uint32_t b = 0; b < 4u; b++) x[b] = *(const int4v *)(xsrc + 32u * min(b, nblk - 1u));
+  asm volatile("" ::: "memory");
+  float16v y[RB];
+#pragma unroll
+  for (uint32_t i = 0; i < RB; i++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) y[i][r] = 0.0f;
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds;
+  const uint32_t w_rd = lds0 + (Q8 ? lane * 16u : l32 * 16u);
+  const uint32_t a_rd = lds0 + Shape::A_OFF + wave * 512u + l32 * 16u;
+  // the tail of (row, block bb of the piece): tile (row >> rs) * tiles a row block + (bb >> cs), lane ((bb & cm) << rs) + (row & rm)
+  auto tail_row = [&](uint32_t row) -> uint32_t { return lds0 + Shape::T_OFF + (((row >> rs) << (2u - cs)) * 64u + (row & rm)) * TAIL; };
+  auto tail_blk = [&](uint32_t bb) -> uint32_t { return ((bb >> cs) * 64u + ((bb & cm) << rs)) * TAIL; };
+  uint32_t d_rd[RB / 2], h_rd[RB];
+#pragma unroll
+  for (uint32_t j = 0; j < RB / 2u; j++) d_rd[j] = tail_row(64u * j + 32u * lh + l32);
+#pragma unroll
+  for (uint32_t i = 0; i < RB; i++) h_rd[i] = tail_row(32u * i + l32) + 2u;
+
+  // a step is a block of a row block: its operand (read two steps ahead), every second step a pair of row blocks' scales
+  int4v w[4];
+  uint32_t dh[2];                    // the f16 of row 32 (2 j + lh) + l32
+  float as[2];                       // the token's scale
+  uint32_t qh[4][2];                 // Q5_0: the fifth bits, as two halves
+  const int4v zi4 = {0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    w[q] = zi4;
+    qh[q][0] = qh[q][1] = 0u;
+    dh[q & 1] = 0u;
+    as[q & 1] = 0.0f;
+  }
+#define GF_I(N) std::integral_constant<int, (N)>{}
+#define GF_U(N) std::integral_constant<uint32_t, (N)>{}
+  constexpr int OPS_W = 1 + (KIND == 1 ? 2 : 0);   // LDS reads of a step; two more in an even one
+  auto reads = [&](auto n_c, uint32_t slot_at) {   // of step n of the piece in the slot
+    constexpr uint32_t n = decltype(n_c)::value, bb = n / RB, i = n % RB, B = n & 3u, S = (n >> 1) & 1u;
+    constexpr uint32_t o = bb * W_BLOCK + (Q8 ? i * 1024u : i * 512u);
+    asm volatile("ds_read_b128 %0, %2 offset:%3" : "=v"(w[B]) : "0"(w[B]), "v"(w_rd + slot_at), "n"(o));
+    auto &bits = qh;
+    auto &bits_rd = h_rd;
+    auto &d16 = dh;
+    auto &sc = as;
+    auto &at = d_rd;
+    const uint32_t tb = slot_at + tail_blk(bb), aa = a_rd + slot_at;
+    if constexpr (KIND == 1) {
+      asm volatile("ds_read_u16 %0, %2" : "=v"(bits[B][0]) : "0"(bits[B][0]), "v"(bits_rd[i] + tb));
+      asm volatile("ds_read_u16 %0, %2 offset:2" : "=v"(bits[B][1]) : "0"(bits[B][1]), "v"(bits_rd[i] + tb));
+    }
+    if constexpr ((i & 1u) == 0u) {
+      asm volatile("ds_read_u16 %0, %2" : "=v"(d16[S]) : "0"(d16[S]), "v"(at[i / 2u] + tb));
+      asm volatile("ds_read_b32 %0, %2 offset:%3" : "=v"(sc[S]) : "0"(sc[S]), "v"(aa), "n"(4u * bb));
+    }
+  };
+  auto operand = [&](auto b_c) -> int4v {   // the wave's int8 operand out of buffer B: as it lies, or this lane's half of the nibbles
+    constexpr uint32_t B = decltype(b_c)::value;
+    if constexpr (Q8) {
+      return w[B];
+    } else {
+      const uint32_t h = KIND == 1 ? (lh ? qh[B][1] : qh[B][0]) : 0u;
+      int4v o;
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        o[k] = (int)ogm_nib32_weights<KIND>(((uint32_t)w[B][k] >> (4u * lh)) & 0x0F0F0F0Fu, (h >> (4 * k)) & 0xFu);
+      return o;
+    }
+  };
+  float32v pr[2];   // the scales' products (ad * dw, rounded once: an outer product) of a pair of row blocks
+  int16v c[2];      // dot32
+  const int16v zi = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  const float32v zf = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  auto add_up = [&](auto n_c, auto lo_c, auto cnt_c) {   // outputs lo .. of step n: acc += (ad * dw) * dot32 (vecdot.rs:2622)
+    constexpr uint32_t n = decltype(n_c)::value, i = n % RB, S = (n >> 1) & 1u, C = n & 1u;
+#pragma unroll
+    for (int r = decltype(lo_c)::value; r < decltype(lo_c)::value + decltype(cnt_c)::value; r++)
+      y[i][r] += pr[S][16 * (i & 1u) + r] * (float)c[C][r];
+  };
+  auto piece = [&](auto first_c, uint32_t pc, uint32_t slot_at, uint32_t slot_next) {
+    constexpr uint32_t N = 4u * RB;
+    const uint32_t left = nblk - 4u * pc;   // blocks from this piece on
+    auto step = [&](auto n_c) {
+      constexpr uint32_t n = decltype(n_c)::value, bb = n / RB, i = n % RB, B = n & 3u, S = (n >> 1) & 1u;
+      constexpr bool EPI = !(decltype(first_c)::value && n == 0u);
+      constexpr uint32_t before = (n + N - 1u) % N;   // the step before
+      GB_PIN();
+      // this step's reads were issued two steps ago; outstanding after them: the next step's
+      auto &bits = qh;
+      auto &d16 = dh;
+      auto &sc = as;
+      constexpr int OUT = OPS_W + ((i & 1u) == 1u ? 2 : 0);
+      if constexpr (KIND == 1)
+        asm volatile("s_waitcnt lgkmcnt(%5)" : "+v"(w[B]), "+v"(d16[S]), "+v"(sc[S]), "+v"(bits[B][0]), "+v"(bits[B][1]) : "n"(OUT));
+      else
+        asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(w[B]), "+v"(d16[S]), "+v"(sc[S]) : "n"(OUT));
+      c[n & 1u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(x[bb], operand(GF_U(B)), zi, 0, 0, 0);
+      GB_PIN();
+      if constexpr (n + 2u < N) reads(GF_U(n + 2u), slot_at);
+      else reads(GF_U(n + 2u - N), slot_next);
+      if constexpr (i + 1u == RB) x[bb] = *(const int4v *)(xsrc + 32u * min(4u * pc + 4u + bb, nblk - 1u));   // the next piece's
+      GB_PIN();
+      if constexpr (EPI) add_up(GF_U(before), GF_I(0), GF_I(8));
+      GB_PIN();
+      if constexpr ((i & 1u) == 0u) {
+        float ad = sc[S], dw = gm_f16_bits_to_f32(d16[S] & 0xFFFFu);
+        if (bb != 0u) {   // (blocks past the row's last: nothing, whatever their scales)
+          ad = bb < left ? ad : 0.0f;
+          dw = bb < left ? dw : 0.0f;
+        }
+        pr[S] = __builtin_amdgcn_mfma_f32_32x32x1f32(ad, dw, zf, 0, 0, 0);
+        GB_PIN();
+      }
+      if constexpr (EPI) add_up(GF_U(before), GF_I(8), GF_I(8));
+      GB_PIN();
+    };
+    auto block = [&](auto bb_c) {
+      constexpr uint32_t b0 = decltype(bb_c)::value * RB;
+      step(GF_U(b0));
+      step(GF_U(b0 + 1u));
+      if constexpr (RB == 4u) {
+        step(GF_U(b0 + 2u));
+        step(GF_U(b0 + 3u));
+      }
+    };
+    block(GF_U(0u));
+    block(GF_U(1u));
+    block(GF_U(2u));
+    block(GF_U(3u));
+  };
+  top(GF_I(FETCH + 4), 0u);
+  reads(GF_U(0u), 0u);
+  reads(GF_U(1u), 0u);
+  piece(std::true_type{}, 0u, 0u, SLOT);
+  for (uint32_t pc = 1; pc < np; pc++) {
+    top(GF_I(FETCH + 4), pc);
+    piece(std::false_type{}, pc, (pc % SLOTS) * SLOT, ((pc + 1u) % SLOTS) * SLOT);
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(dh[0]), "+v"(dh[1]), "+v"(as[0]), "+v"(as[1])::"memory");
+  if constexpr (KIND == 1) {
+    auto &bits = qh;
+    asm volatile("" : "+v"(bits[0][0]), "+v"(bits[0][1]), "+v"(bits[1][0]), "+v"(bits[1][1]), "+v"(bits[2][0]), "+v"(bits[2][1]), "+v"(bits[3][0]), "+v"(bits[3][1]));
+  }
+  add_up(GF_U(4u * RB - 1u), GF_I(0), GF_I(16));   // the last step's sums
+#pragma unroll
+  for (uint32_t i = 0; i < RB; i++) {
+    const uint32_t row = r0 + 32u * i + l32;
+    if (row < p.out_dim) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const uint32_t t = t0 + 32u * wave + 8u * (r >> 2) + 4u * lh + (r & 3);
+        if (t < p.n_tokens) p.y[(size_t)t * p.out_dim + row] = y[i][r];
       }
     }
   }
@@ -2761,19 +3031,35 @@ size_t ogm_gemm_xh_bytes(uint32_t in_dim, uint32_t n_tokens) {
 static uint32_t gemm_flat_small_lds(uint32_t nw) { return nw * SBF_NB * 4096u + 2u * nw * SBF_NB * 36u * 4u; }
 
 // Whether a launch of the per-32 types takes their small-batch kernel: while its workgroups of 32 rows x 32 tokens
-// are few enough, about seven rounds of the device's compute units (two workgroups share one).  Measured on MI355X,
-// Q8_0, whole calls, us, small-batch against tiled: 4096 -> 4096 at 32 / 128 / 384 / 512 tokens 14.5 / 24.5 / 62 / 91
-// against 72 / 76 / 82 / 84; 4096 -> 14336 at 32 / 128 / 192: 26 / 73 / 125 against 77 / 82 / 89; 14336 -> 4096 at 32 /
-// 128 / 256: 42 / 73 / 134 against 239 / 243 / 252; 8192 -> 2048 at 128 / 384: 28 / 67.  (Q4_0, Q5_0, IQ4_NL within a
-// few per cent.)
-static bool gemm_flat_small(uint32_t n_tokens, uint32_t out_dim) {
+// are few, as long as the tiled kernel's one round of them takes.  Measured on MI355X, Q8_0, whole calls, us, small-batch
+// against tiled, with the workgroups: 4096 -> 4096 at 128 / 256 / 384 tokens (512 / 1024 / 1536) 24 / 42 / 60 against 43 / 44 /
+// 46; 4096 -> 14336 at 64 / 128 (896 / 1792): 40 / 70 against 43 / 45; 14336 -> 4096 at 256 / 384: 133 / 193 against 138 / 141;
+// 8192 -> 8192 at 128 / 200 (1024 / 1792): 78 / 133 against 80 / 83; Q4_0 4096 -> 4096 at 256 / 384 40 / 58 against 52 / 53, 4096 ->
+// 14336 at 64 / 128 38 / 66 against 50 / 52; IQ4_NL 4096 -> 4096 at 330 (1408) 58 against 59, 4096 -> 14336 at 120 68 / 58.
+static bool gemm_flat_small(uint32_t ggml_type, uint32_t n_tokens, uint32_t out_dim) {
   const uint32_t wgs = ((n_tokens + 31u) / 32u) * ((out_dim + 31u) / 32u);
-  return wgs <= 1792u;
+  return wgs <= (ggml_type == OGM_Q8_0 ? 1024u : ggml_type == OGM_Q4_0 ? 1280u : 1408u);
+}
+
+// Row blocks of a workgroup of ogm_gemm_flat_kernel (4 or 2), or 0 where the nibble types' f16 kernel is ahead: on rows of an
+// even number of blocks and more than a workgroup of two a compute unit.  Two or four by the rounds a launch takes, two
+// workgroups to a compute unit, a last round of at most one each the shorter: measured, Q8_0 of 4096 inputs, us, 97 a full
+// round and 72 a half one with four row blocks, 53 and 40 with two.
+static uint32_t gemm_flat_row_blocks(uint32_t ggml_type, uint32_t nblk, uint32_t out_dim, uint32_t n_tokens) {
+  const uint32_t tok_tiles = (n_tokens + 127u) / 128u, n4 = tok_tiles * ((out_dim + 127u) / 128u), n2 = tok_tiles * ((out_dim + 63u) / 64u);
+  if (ggml_type != OGM_Q8_0 && nblk % 2u == 0u && n2 > 256u) return 0;
+  auto rounds = [](uint32_t n, uint32_t full, uint32_t half) { return n / 512u * full + (n % 512u == 0u ? 0u : n % 512u <= 256u ? half : full); };
+  return (out_dim + 63u) / 64u > 65535u || rounds(n4, 97u, 72u) <= rounds(n2, 53u, 40u) ? 4u : 2u;
+}
+
+// Rows a GEMM of the per-32 types takes: any number of blocks; Q5_1's odd counts, whose only GEMM kernel does nothing for rows of a
+// few blocks (96 inputs: the GEMV kernel's three passes at 20 tokens are as short), from eight.
+static bool flat_rows(uint32_t ggml_type, uint32_t in_dim) {
+  return in_dim != 0 && in_dim % 32u == 0 && (ggml_type != OGM_Q5_1 || in_dim % 64u == 0 || in_dim >= 256u);
 }
 
 bool ogm_gemm_flat_small_batch(uint32_t ggml_type, uint32_t in_dim, uint32_t out_dim, uint32_t n_tokens) {
-  if (in_dim % 64u != 0) return false;
-  return ggml_type == OGM_Q5_1 || gemm_flat_small(n_tokens, out_dim);   // (Q5_1 has no other GEMM kernel)
+  return flat_rows(ggml_type, in_dim) && (ggml_type == OGM_Q5_1 || gemm_flat_small(ggml_type, n_tokens, out_dim));   // (Q5_1 has no other GEMM kernel)
 }
 
 // The per-32 types with a GEMM kernel: the four symmetric ones (small-batch and tiled), and Q5_1 (small-batch only).
@@ -2785,8 +3071,7 @@ bool ogm_gemm_supported(uint32_t ggml_type, uint32_t in_dim, uint32_t out_dim, u
   // the kernels address weights and activations with 32-bit byte offsets
   const uint64_t lim = 0xFFFFFFFFull;
   if (is_flat32(ggml_type)) {
-    // two blocks per stage
-    if (in_dim == 0 || in_dim % 64u != 0) return false;
+    if (!flat_rows(ggml_type, in_dim) || (out_dim + 127u) / 128u > 65535u) return false;
     OgmLayout l;
     ogm_layout_for(ggml_type, &l);
     return (uint64_t)ogm_tiling_for(in_dim / 32u, out_dim).nrb * 64u * (in_dim / 32u) * l.block_bytes <= lim &&
@@ -3005,14 +3290,14 @@ hipError_t ogm_launch_gemm(const OgmGemmArgs &a, hipStream_t stream, const char 
     p.n_tokens = a.n_tokens;
     p.nblk = a.in_dim / 32;
     const OgmTiling tl = ogm_tiling_for(p.nblk, a.out_dim);
-    p.c_shift = tl.C == 4 ? 2 : 1;   // in_dim % 64 == 0: at least two blocks per tile row
+    p.c_shift = tl.C == 4 ? 2 : (tl.C == 2 ? 1 : 0);
     p.r_shift = 6 - p.c_shift;
     p.nct = tl.nct;
     // small batches: the kernel whose waves take different blocks (small_max_tokens as for the K-quants: 0 by the
     // size of the launch, 1 never, otherwise up to that many tokens)
     const uint32_t sbf_lds = gemm_flat_small_lds(8u);
     const bool q51 = a.ggml_type == OGM_Q5_1;   // (this kernel only, whatever the batch)
-    const bool sbf = q51 || (a.small_max_tokens ? a.n_tokens <= a.small_max_tokens : gemm_flat_small(a.n_tokens, a.out_dim));
+    const bool sbf = q51 || (a.small_max_tokens ? a.n_tokens <= a.small_max_tokens : gemm_flat_small(a.ggml_type, a.n_tokens, a.out_dim));
     if ((q51 || a.small_max_tokens != 1u) && sbf && sbf_lds <= GM_LDS_MAX) {
       GemmSbParams q{};
       q.wt = a.wt;
@@ -3045,15 +3330,34 @@ hipError_t ogm_launch_gemm(const OgmGemmArgs &a, hipStream_t stream, const char 
       return hipGetLastError();
     }
     if (q51) return hipErrorInvalidValue;
-    const dim3 grid((a.n_tokens + 127u) / 128u, (a.out_dim + 127u) / 128u);
-    void (*const flat)(GemmFlatParams) = a.ggml_type == OGM_Q4_0     ? ogm_gemm_flat_kernel<0>
-                                         : a.ggml_type == OGM_Q5_0   ? ogm_gemm_flat_kernel<1>
-                                         : a.ggml_type == OGM_IQ4_NL ? ogm_gemm_flat_kernel<2>
-                                                                     : ogm_gemm_flat_kernel<3>;
-    const hipError_t e = hipFuncSetAttribute((const void *)flat, hipFuncAttributeMaxDynamicSharedMemorySize, (int)GF_LDS);
+    const uint32_t rb = gemm_flat_row_blocks(a.ggml_type, p.nblk, a.out_dim, a.n_tokens);
+    const void *fn = nullptr;
+    uint32_t lds_here = GF_LDS;
+    const char *name = "ogm_gemm_flat_kernel";
+    if (rb == 0u) {
+      fn = a.ggml_type == OGM_Q4_0   ? (const void *)ogm_gemm_flat_f16_kernel<0>
+           : a.ggml_type == OGM_Q5_0 ? (const void *)ogm_gemm_flat_f16_kernel<1>
+                                     : (const void *)ogm_gemm_flat_f16_kernel<2>;
+      name = "ogm_gemm_flat_f16_kernel";
+    } else {
+#define GF_PICK(K) fn = rb == 4u ? (const void *)ogm_gemm_flat_kernel<K, 4u> : (const void *)ogm_gemm_flat_kernel<K, 2u>; \
+  lds_here = rb == 4u ? FlatShape<K, 4u>::LDS_BYTES : FlatShape<K, 2u>::LDS_BYTES; \
+  break
+      switch (a.ggml_type) {
+        case OGM_Q4_0: GF_PICK(0);
+        case OGM_Q5_0: GF_PICK(1);
+        case OGM_IQ4_NL: GF_PICK(2);
+        default: GF_PICK(3);
+      }
+#undef GF_PICK
+    }
+    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_here);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(flat, grid, dim3(768), GF_LDS, stream, p);
-    if (kernel_name) *kernel_name = "ogm_gemm_flat_kernel";
+    const uint32_t rows = rb ? 32u * rb : 128u;
+    void *kargs[] = {(void *)&p};
+    e = hipLaunchKernel(fn, dim3((a.n_tokens + 127u) / 128u, (a.out_dim + rows - 1u) / rows), dim3(rb ? 256 : 768), kargs, lds_here, stream);
+    if (e != hipSuccess) return e;
+    if (kernel_name) *kernel_name = name;
     return hipGetLastError();
   }
   const uint32_t nsb = a.in_dim / 256;
