@@ -222,7 +222,7 @@ __device__ __forceinline__ AttnPart attn_merge_chunks(const float *part_o, const
 // row is in the cache already (ogm_qkv_pre_kernel), workgroups past a token's last chunk leave at
 // once, and nothing is quantized: the next matmul is a GEMM that quantizes its own input.
 template <int HD, int G, int GROUP, bool PREFILL = false, int CHUNK = (int)OGM_ATTN_CHUNK, bool MULTI = false>
-__global__ __launch_bounds__(4 * CHUNK, (MULTI && G <= 4) ? 4 : 1) void ogm_attn_kernel(const float *__restrict__ q, const float *__restrict__ k_new,
+__global__ __launch_bounds__(CHUNK < 128 ? 4 * CHUNK : 512, (MULTI && G <= 4) ? 4 : 1) void ogm_attn_kernel(const float *__restrict__ q, const float *__restrict__ k_new,
                                                        const float *__restrict__ v_new,
                                                        const float2 *__restrict__ cs, uint32_t rope_half,
                                                        OgmAttnPre pre, uint32_t gq,
@@ -232,7 +232,8 @@ __global__ __launch_bounds__(4 * CHUNK, (MULTI && G <= 4) ? 4 : 1) void ogm_attn
                                                        uint32_t *counters, float *__restrict__ attn_out,
                                                        OgmActDev act, uint32_t n_sub) {
   static_assert(!MULTI || CHUNK == 128, "several chunks a workgroup: chunks of 128");
-  constexpr int NT = 4 * CHUNK, NW = NT / 64;   // four threads per cache position
+  constexpr int NT = CHUNK < 128 ? 4 * CHUNK : 512, NW = NT / 64;
+  constexpr int RPT = 4 * CHUNK / NT;     // cache positions that four threads share
   constexpr int KU = HD / 32;             // 16-byte pieces of a K row per thread
   constexpr int TPR = HD / 8;             // threads per V row
   constexpr int ROWS = NT / TPR;          // V rows in flight per step
@@ -285,10 +286,14 @@ __global__ __launch_bounds__(4 * CHUNK, (MULTI && G <= 4) ? 4 : 1) void ogm_attn
   const uint32_t c = tid & 3u;
   const uint32_t r = MULTI ? (uint32_t)ROWS * ((lane >> 2) / R2) + R2 * wave + ((lane >> 2) % R2) : tid >> 2;
   // rows past the chunk's end read the last row; their scores are discarded (weight 0)
-  const __half *krow = kc + (size_t)(p0 + min(r, n_here - 1u)) * kv_dim + kvh * HD;
-  uint4 kr[KU];
+  uint4 krs[RPT][KU];
 #pragma unroll
-  for (int j = 0; j < KU; j++) kr[j] = *(const uint4 *)(krow + 8 * (c + 4 * j));
+  for (int k = 0; k < RPT; k++) {
+    const __half *krow = kc + (size_t)(p0 + min(r + (uint32_t)(k * NT / 4), n_here - 1u)) * kv_dim + kvh * HD;
+#pragma unroll
+    for (int j = 0; j < KU; j++) krs[k][j] = *(const uint4 *)(krow + 8 * (c + 4 * j));
+  }
+  uint4(&kr)[KU] = krs[0];
   const __half *vbase = vc + (size_t)p0 * kv_dim + kvh * HD + 8u * dc;
   uint4 vr[STEPS];
 #pragma unroll
@@ -370,7 +375,9 @@ __global__ __launch_bounds__(4 * CHUNK, (MULTI && G <= 4) ? 4 : 1) void ogm_attn
   // The cache loads requested above must stay up there: without this the row substitutions
   // below let the compiler move each load down to its use, one trip to memory after the other.
 #pragma unroll
-  for (int j = 0; j < KU; j++) asm volatile("" : "+v"(kr[j].x), "+v"(kr[j].y), "+v"(kr[j].z), "+v"(kr[j].w));
+  for (int k = 0; k < RPT; k++)
+#pragma unroll
+    for (int j = 0; j < KU; j++) asm volatile("" : "+v"(krs[k][j].x), "+v"(krs[k][j].y), "+v"(krs[k][j].z), "+v"(krs[k][j].w));
 #pragma unroll
   for (int st = 0; st < STEPS; st++) asm volatile("" : "+v"(vr[st].x), "+v"(vr[st].y), "+v"(vr[st].z), "+v"(vr[st].w));
   __syncthreads();
@@ -573,64 +580,73 @@ __global__ __launch_bounds__(4 * CHUNK, (MULTI && G <= 4) ? 4 : 1) void ogm_attn
     }
   } else {
   // ---- phase 1: scores
-  if (is_last && r == cur) {
-#pragma unroll
-    for (int j = 0; j < KU; j++) kr[j] = *(const uint4 *)&kcur[8 * (c + 4 * j)];
-  }
-  float acc[G];
-#pragma unroll
-  for (int g = 0; g < G; g++) acc[g] = 0.0f;
-#pragma unroll
-  for (int j = 0; j < KU; j++) {
-    const __half2 *h2 = (const __half2 *)&kr[j];
-    float kf[8];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const float2 f = __half22float2(h2[e]);
-      kf[2 * e] = f.x;
-      kf[2 * e + 1] = f.y;
-    }
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      const float4 qa = *(const float4 *)&qs[g][8 * (c + 4 * j)];
-      const float4 qb = *(const float4 *)&qs[g][8 * (c + 4 * j) + 4];
-      acc[g] = fmaf(qa.x, kf[0], acc[g]); acc[g] = fmaf(qa.y, kf[1], acc[g]);
-      acc[g] = fmaf(qa.z, kf[2], acc[g]); acc[g] = fmaf(qa.w, kf[3], acc[g]);
-      acc[g] = fmaf(qb.x, kf[4], acc[g]); acc[g] = fmaf(qb.y, kf[5], acc[g]);
-      acc[g] = fmaf(qb.z, kf[6], acc[g]); acc[g] = fmaf(qb.w, kf[7], acc[g]);
-    }
-  }
-  // sum over the row's four lanes: while a lane holds two or more heads it keeps one half and
-  // hands the other to its partner; afterwards plain butterflies
   uint32_t g0 = 0;        // first head this lane holds
   bool owner = true;      // of several lanes holding the same head, the one that stores
-  {
-    int n = G;
+  float sv[RPT][NF], mv[NF];
 #pragma unroll
-    for (int b = 1; b < 4; b <<= 1) {
-      const bool up = (lane & b) != 0;
-      if (n >= 2) {
-        n >>= 1;
+  for (int k = 0; k < RPT; k++) {
+    const uint32_t rk = r + (uint32_t)(k * NT / 4);
+    if (is_last && rk == cur) {
 #pragma unroll
-        for (int i = 0; i < n; i++) {
-          float lo = acc[i], hi = acc[n + i];
-          asm volatile("" : "+v"(lo), "+v"(hi));   // keeps the selects on values, not on array slots
-          acc[i] = (up ? hi : lo) + (b == 1 ? ogm_quad_xor<1>(up ? lo : hi) : ogm_quad_xor<2>(up ? lo : hi));
-        }
-        g0 += up ? n : 0;
-      } else {
-        acc[0] += b == 1 ? ogm_quad_xor<1>(acc[0]) : ogm_quad_xor<2>(acc[0]);
-        owner = owner && !up;
+      for (int j = 0; j < KU; j++) krs[k][j] = *(const uint4 *)&kcur[8 * (c + 4 * j)];
+    }
+    float acc[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) acc[g] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < KU; j++) {
+      const __half2 *h2 = (const __half2 *)&krs[k][j];
+      float kf[8];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float2 f = __half22float2(h2[e]);
+        kf[2 * e] = f.x;
+        kf[2 * e + 1] = f.y;
+      }
+#pragma unroll
+      for (int g = 0; g < G; g++) {
+        const float4 qa = *(const float4 *)&qs[g][8 * (c + 4 * j)];
+        const float4 qb = *(const float4 *)&qs[g][8 * (c + 4 * j) + 4];
+        acc[g] = fmaf(qa.x, kf[0], acc[g]); acc[g] = fmaf(qa.y, kf[1], acc[g]);
+        acc[g] = fmaf(qa.z, kf[2], acc[g]); acc[g] = fmaf(qa.w, kf[3], acc[g]);
+        acc[g] = fmaf(qb.x, kf[4], acc[g]); acc[g] = fmaf(qb.y, kf[5], acc[g]);
+        acc[g] = fmaf(qb.z, kf[6], acc[g]); acc[g] = fmaf(qb.w, kf[7], acc[g]);
       }
     }
+    // sum over the row's four lanes: while a lane holds two or more heads it keeps one half and
+    // hands the other to its partner; afterwards plain butterflies
+    g0 = 0;
+    owner = true;
+    {
+      int n = G;
+#pragma unroll
+      for (int b = 1; b < 4; b <<= 1) {
+        const bool up = (lane & b) != 0;
+        if (n >= 2) {
+          n >>= 1;
+#pragma unroll
+          for (int i = 0; i < n; i++) {
+            float lo = acc[i], hi = acc[n + i];
+            asm volatile("" : "+v"(lo), "+v"(hi));   // keeps the selects on values, not on array slots
+            acc[i] = (up ? hi : lo) + (b == 1 ? ogm_quad_xor<1>(up ? lo : hi) : ogm_quad_xor<2>(up ? lo : hi));
+          }
+          g0 += up ? n : 0;
+        } else {
+          acc[0] += b == 1 ? ogm_quad_xor<1>(acc[0]) : ogm_quad_xor<2>(acc[0]);
+          owner = owner && !up;
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NF; i++) sv[k][i] = rk < n_here ? acc[i] * scale : -INFINITY;
   }
-  const bool valid = r < n_here;
-  float sv[NF], mv[NF];
 #pragma unroll
   for (int i = 0; i < NF; i++) {
-    sv[i] = valid ? acc[i] * scale : -INFINITY;
+    float m = sv[0][i];
+#pragma unroll
+    for (int k = 1; k < RPT; k++) m = fmaxf(m, sv[k][i]);
     // over the wave's sixteen rows of four lanes, lane by lane of the row
-    float m = ogm_row_quads_allreduce(sv[i], OgmOpMax());
+    m = ogm_row_quads_allreduce(m, OgmOpMax());
     m = ogm_butterfly_step<16>(m, OgmOpMax());
     m = ogm_butterfly_step<32>(m, OgmOpMax());
     if (lane < 4u && owner) red[0][g0 + i][wave] = m;
@@ -642,15 +658,23 @@ __global__ __launch_bounds__(4 * CHUNK, (MULTI && G <= 4) ? 4 : 1) void ogm_attn
 #pragma unroll
     for (int w = 1; w < NW; w++) m = fmaxf(m, red[0][g0 + i][w]);
     mv[i] = m;
-    const float e = valid ? expf(sv[i] - m) : 0.0f;
-    if (owner) sc[g0 + i][r] = e;
-    float l = ogm_row_quads_allreduce(e, OgmOpAdd());
+    float l = 0.0f;
+#pragma unroll
+    for (int k = 0; k < RPT; k++) {
+      const uint32_t rk = r + (uint32_t)(k * NT / 4);
+      const float e = rk < n_here ? expf(sv[k][i] - m) : 0.0f;
+      if (owner) sc[g0 + i][rk] = e;
+      l = k == 0 ? e : l + e;
+    }
+    l = ogm_row_quads_allreduce(l, OgmOpAdd());
     l = ogm_butterfly_step<16>(l, OgmOpAdd());
     l = ogm_butterfly_step<32>(l, OgmOpAdd());
     if (lane < 4u && owner) red[1][g0 + i][wave] = l;
   }
   __syncthreads();
-  if (tid < gq) {
+  // a head whose cache one workgroup holds: nothing is handed over
+  const bool alone = GROUP != 0 && n_splits == 1u;
+  if (tid < gq && !alone) {
     float m = red[0][tid][0], l = red[1][tid][0];
 #pragma unroll
     for (int w = 1; w < NW; w++) {
@@ -717,7 +741,29 @@ __global__ __launch_bounds__(4 * CHUNK, (MULTI && G <= 4) ? 4 : 1) void ogm_attn
       float t = 0.0f;
 #pragma unroll
       for (int w = 0; w < NW; w++) t += osum[w][g][d];
-      if (g < gq) st_one<GROUP != 0>(&part_o[((size_t)(hg * gq + g) * max_splits + split) * HD + d], t);
+      if (alone) osum[0][g][d] = t;   // (this thread's own column)
+      else if (g < gq) st_one<GROUP != 0>(&part_o[((size_t)(hg * gq + g) * max_splits + split) * HD + d], t);
+    }
+  }
+  if constexpr (GROUP != 0) {
+    if (alone) {   // the merge of one partial result, and the quantizer
+      __syncthreads();
+      constexpr int NG = G * HD / 4;
+      for (int run = wave; run < (NG + 63) / 64; run += NW) {
+        const uint32_t eg = run * 64u + lane, g = 4u * eg / HD, e0 = hg * (uint32_t)(G * HD) + 4u * eg;
+        const bool active = eg < (uint32_t)NG;
+        float4 ov = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (active) {
+          float l = red[1][g][0];
+#pragma unroll
+          for (int w = 1; w < NW; w++) l += red[1][g][w];
+          ov = *(const float4 *)&osum[0][g][4u * eg % HD];
+          ov.x /= l; ov.y /= l; ov.z /= l; ov.w /= l;
+          if (attn_out) *(float4 *)(attn_out + e0) = ov;
+        }
+        ogm_quantize_store<GROUP>(ov, e0, active, lane, act.q, act.d, act.sums, act.bsum, act.bs16);
+      }
+      return;
     }
   }
   }   // one chunk
@@ -818,21 +864,32 @@ hipError_t ogm_launch_attn_decode(const float *q, const float *k_new, const floa
                                   hipStream_t stream, uint32_t chunk, uint32_t chunks_per_wg) {
   if (n_head_kv == 0 || n_head % n_head_kv != 0) return hipErrorInvalidValue;
   if (rope_dim > head_dim || rope_dim % 2u != 0) return hipErrorInvalidValue;
-  // Cache positions per workgroup: 128; 64 only for short contexts.  The kernel is a chain of
-  // latencies (cache loads 2.1 us, scores 1.5, V sum 1.5, hand-over of the partial results 0.9,
-  // merge 2.8, quantizer 1.0 at 2048 positions) of which only the two middle ones shrink with the
-  // chunk, while the merge grows with the number of chunks: measured on MI355X with eight K/V heads,
-  // 64 against 128 positions per workgroup take 8.4 against 8.9 us at 512 cached positions but 13.6
-  // against 10.7 at 2048 and 20.5 against 14.1 at 4096.
-  if (chunk == 0) chunk = (chunks_per_wg <= 1u && (pos / 64u + 1u) * n_head_kv <= 96u) ? 64u : 128u;
-  if (chunk != 64u && chunk != 128u) return hipErrorInvalidValue;
-  const uint32_t n_chunks = pos / chunk + 1u;
   const uint32_t n = n_head * head_dim;
   if (n % 32u != 0) return hipErrorInvalidValue;
   // more than eight query heads per K/V head: in equal parts of at most eight, a workgroup each
   const uint32_t parts = ogm_attn_head_parts(n_head / n_head_kv);
   if (parts == 0u) return hipErrorInvalidValue;
   const uint32_t gq = n_head / n_head_kv / parts;
+  const uint32_t G = gq <= 2u ? gq : (gq <= 4u ? 4u : 8u);   // head slots of the kernel
+  const uint32_t group = mode == 0 ? 32u : 256u;
+  // the merge rides in the attention kernel when every head slot is a head and a K/V head's
+  // outputs are whole quantizer groups
+  const uint32_t fused = (G == gq && (G * head_dim) % group == 0) ? group : 0u;
+  // Cache positions per workgroup: 128; 64 only for short contexts.  The kernel is a chain of
+  // latencies (cache loads 2.1 us, scores 1.5, V sum 1.5, hand-over of the partial results 0.9,
+  // merge 2.8, quantizer 1.0 at 2048 positions) of which only the two middle ones shrink with the
+  // chunk, while the merge grows with the number of chunks: measured on MI355X with eight K/V heads,
+  // 64 against 128 positions per workgroup take 8.4 against 8.9 us at 512 cached positions but 13.6
+  // against 10.7 at 2048 and 20.5 against 14.1 at 4096.
+  //   A context that one workgroup holds is not handed over, drawn a ticket for or merged, which at 64 to 127 positions
+  // saves more than the second workgroup of 64 (us a token, 64 / 128 positions a workgroup: 8 layers of the 8B shapes at 100
+  // cached positions 445 / 432, 16 of the 1B ones 493 / 462), and with heads of 64 at 128 to 255 in chunks of 256, two
+  // positions to four threads (498 / 481 at 200; with heads of 128 447 / 448).
+  if (chunk == 0 && chunks_per_wg <= 1u && fused != 0u && pos >= 64u && pos < (head_dim == 64u ? 256u : 128u))
+    chunk = pos < 128u ? 128u : 256u;
+  else if (chunk == 0) chunk = (chunks_per_wg <= 1u && (pos / 64u + 1u) * n_head_kv <= 96u) ? 64u : 128u;
+  else if (chunk != 64u && chunk != 128u) return hipErrorInvalidValue;
+  const uint32_t n_chunks = pos / chunk + 1u;
   // Chunks a workgroup takes in a row (chunks of 128 only): one while the launch has fewer workgroups than the
   // device has compute units, then as many as keep it near OGM_ATTN_SUB_TARGET workgroups, at most
   // OGM_ATTN_SUB_MAX.  A workgroup pays for the rotation of q, the hand-over of its partial results and its
@@ -853,19 +910,15 @@ hipError_t ogm_launch_attn_decode(const float *q, const float *k_new, const floa
   const uint32_t n_splits = (n_chunks + n_sub - 1u) / n_sub;
   if (n_splits > max_splits) return hipErrorInvalidValue;
   const dim3 grid(n_head_kv * parts, n_splits);
-  const uint32_t G = gq <= 2u ? gq : (gq <= 4u ? 4u : 8u);   // head slots of the kernel
-  const uint32_t group = mode == 0 ? 32u : 256u;
-  // the merge rides in the attention kernel when every head slot is a head and a K/V head's
-  // outputs are whole quantizer groups
-  const uint32_t fused = (G == gq && (G * head_dim) % group == 0) ? group : 0u;
 #define OGM_ATTN_LAUNCH_C(HD_, G_, GR_, CH_, MULTI_)                                                    \
-  hipLaunchKernelGGL((ogm_attn_kernel<HD_, G_, GR_, false, CH_, MULTI_>), grid, dim3(4 * CH_), 0, stream, q, k_new, \
+  hipLaunchKernelGGL((ogm_attn_kernel<HD_, G_, GR_, false, CH_, MULTI_>), grid, dim3(CH_ < 128 ? 4 * CH_ : 512), 0, stream, q, k_new, \
                      v_new, (const float2 *)cs, rope_dim / 2u, pre, gq, (__half *)k_cache_layer,        \
                      (__half *)v_cache_layer, pos, max_splits, n_head_kv, scale, part_o, part_ml, \
                      counters, attn_out, act, n_sub)
 #define OGM_ATTN_LAUNCH(HD_, G_, GR_)                    \
   do {                                                   \
     if (chunk == 64u) OGM_ATTN_LAUNCH_C(HD_, G_, GR_, 64, false); \
+    else if (chunk == 256u) OGM_ATTN_LAUNCH_C(HD_, G_, GR_, (HD_ == 64 && GR_ != 0 ? 256 : 128), false); \
     else if (n_sub == 1u) OGM_ATTN_LAUNCH_C(HD_, G_, GR_, 128, false); \
     else OGM_ATTN_LAUNCH_C(HD_, G_, GR_, 128, true);     \
   } while (0)
