@@ -494,7 +494,10 @@ int ogm_llama_load_gguf(ogm_ctx *ctx, ogm_gguf *g, uint32_t max_ctx, ogm_llama *
  *                              waiting on the stream; after 5 ms without the word, and on every 256th call,
  *                              the stream is synchronized after all; 0 = always hipStreamSynchronize; 2 = for
  *                              tests of the bounded wait: the word never matches and every call runs into the
- *                              5 ms */
+ *                              5 ms.  The model calls' results in pageable host memory of 16 KiB and more
+ *                              (ogm_llama_decode, ogm_llama_prefill*, ogm_llama_forward_all_logits,
+ *                              ogm_llama_hidden_states) come through 4 MiB of such memory under the same two
+ *                              switches: a kernel stores them there in chunks, each with a word of its own */
 int ogm_set_tuning(ogm_ctx *ctx, const char *key, int value);
 /* For benchmarks driven from an interpreter: runs host-pointer calls from compiled code and writes each
  * repetition's wall time in microseconds to us_out[reps].  `ops` holds n_variants sets of n_ops ops;

@@ -138,9 +138,14 @@ hipError_t ogm_launch_f16_to_f32(const uint16_t *bits, size_t n, float *out, hip
 #define OGM_PROBE_MAX_BUFS 4u
 hipError_t ogm_launch_read_probe(const uint8_t *const *bufs, const size_t *bytes, uint32_t n, uint32_t *sink,
                                  hipStream_t stream);
-// Stores `value` to the pinned host word `flag` once everything before it on the stream has finished.
 hipError_t ogm_launch_empty(uint32_t workgroups, uint32_t *sink, hipStream_t stream);
+// Stores `value` to the pinned host word `flag` once everything before it on the stream has finished.
 hipError_t ogm_launch_host_flag(uint32_t *flag, uint32_t value, hipStream_t stream);
+// Copies n_words to coherent pinned host memory (both 16-byte aligned) and stores `value` to flags[c] once chunk c
+// of OGM_HOST_CHUNK_WORDS words is there; the n_tail words of `tail` are there with chunk 0.
+#define OGM_HOST_CHUNK_WORDS 4096u
+hipError_t ogm_launch_host_copy(const void *src, void *dst, size_t n_words, const void *tail, void *tail_dst,
+                                size_t n_tail, uint32_t *flags, uint32_t value, hipStream_t stream);
 
 // The library's static scratch (ogm_static.hip): a file-scope device array every GPU holds its own
 // copy of, for the entry point that must not allocate.  It takes the quantized activations of up to
