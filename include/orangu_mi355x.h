@@ -450,16 +450,14 @@ int ogm_llama_load_gguf(ogm_ctx *ctx, ogm_gguf *g, uint32_t max_ctx, ogm_llama *
  *                              ogm_weight_download is unaffected
  *   "gemm_plane_kernel"        when the kernel that multiplies the planes (all waves multiply, operands loaded
  *                              straight into LDS) runs: 0 = default, when the launch has more than 256 tiles of
- *                              128 rows x 128 tokens (the feeding-wave kernels unpack otherwise); 2 = whatever
- *                              the grid, from 32 tokens
- *   "gemm_interleave"          the plane kernel with 64-row tiles that adds a super-block up between the next
- *                              one's matrix instructions (Q4_K, Q5_K, Q6_K): 0 = default, on launches of at most
- *                              512 tiles of 64 rows x 128 tokens: Q6_K from 128 such tiles with the last token
- *                              tile more than three quarters full or with three token tiles, or from 160 with
- *                              more than 96 tokens; Q4_K / Q5_K from three token tiles (two over rows of more
- *                              than 8192 inputs) and 160 tiles, with rows longer than 5120 inputs at most 256 (the
- *                              8B shapes' q/k/v, wo and down projections at 257 to 1024 tokens; their planes are
- *                              built then); 1 = never; 2 = wherever the plane kernel runs.  Same bits
+ *                              128 rows x 128 tokens, or more than 256 of 64 rows (Q4_K / Q5_K rows of 4096 inputs
+ *                              and more beyond 128 tokens), or "gemm_interleave" takes it (the feeding-wave kernels
+ *                              unpack otherwise); 2 = whatever the grid, from 32 tokens.  A prefill's gate and up on
+ *                              128-row tiles leave silu(gate) * up in one launch
+ *   "gemm_interleave"          the plane kernel with 64-row tiles (Q4_K, Q5_K, Q6_K, IQ4_XS): 0 = default, on launches
+ *                              of at most 512 tiles of 64 rows x 128 tokens (256 for Q4_K / Q5_K rows of 4096 inputs and
+ *                              more) and, by type and token tiles, at least 128 to 160 (their planes are built then);
+ *                              1 = never; 2 = wherever the plane kernel runs.  Same bits
  *   "gemm_one_pass"            0 = default.  1: Q4_K and Q5_K on that kernel skip the reference GEMM's separate
  *                              first pass over the mins (vecdot.rs:2229-2240) and add
  *                              ad * (d * isum - dmin * imin) per super-block, the single-token expression of

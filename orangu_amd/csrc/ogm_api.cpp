@@ -536,7 +536,7 @@ struct Target {
 
 static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_tokens, int decode,
                         hipStream_t stream, int32_t *dump_isum, int32_t *dump_imin,
-                        const OgmActDev *act_base = nullptr);
+                        const OgmActDev *act_base = nullptr, bool *did_swiglu = nullptr);
 
 // Whether a one-token launch over these matrices (one type and in_dim) prepares its own activations: where the work
 // that every workgroup repeats -- row blocks times runs of 1024 inputs -- costs less than the launch it saves.  Measured,
@@ -701,7 +701,8 @@ static bool all_gemm_supported(const Target *tg, size_t n_tg, uint32_t n_tokens)
 // act_base: the quantized activations to read instead of the context's scratch; such a call stays
 // on the GEMV kernels whatever the token count (the tiled GEMMs stage through context buffers).
 static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_tokens, int decode,
-                        hipStream_t stream, int32_t *dump_isum, int32_t *dump_imin, const OgmActDev *act_base) {
+                        hipStream_t stream, int32_t *dump_isum, int32_t *dump_imin, const OgmActDev *act_base,
+                        bool *did_swiglu) {
   const ogm_weight *w0 = tg[0].w;
   const int mode = act_mode_for(w0->ggml_type, n_tokens, decode);
   // backend/cpu.rs:55-167: matmul at n_tokens > 1 takes the GEMM kernels (their float order);
@@ -854,9 +855,11 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
         if (all) {
           g.planes = tg[i].w->planes;
           for (size_t j = 1; j < ng; j++) g.extra_planes[j - 1] = tg[i + j].w->planes;
+          g.swiglu = did_swiglu && n_tg == 2 && ogm_gemm_does_swiglu(g);
         }
       }
       HIPCHK(ctx, ogm_launch_gemm(g, stream, &ctx->last_kernel));
+      if (did_swiglu) *did_swiglu = g.swiglu;
     }
     if (planes_or_nothing) return OGM_OK;
   }
@@ -2139,7 +2142,8 @@ static int llama_matmul_rows(ogm_ctx *ctx, const ogm_weight *const *ws, float *c
 // scratch (mode `mode`, `in_dim` wide, T rows): the weights are grouped by type as in
 // llama_matmul_rows; all of them must take that mode.
 static int llama_matmul_quantized_rows(ogm_ctx *ctx, const ogm_weight *const *ws, float *const *ys, size_t n,
-                                       int mode, uint32_t in_dim, uint32_t T, hipStream_t s, bool xt_written = false) {
+                                       int mode, uint32_t in_dim, uint32_t T, hipStream_t s, bool xt_written = false,
+                                       bool *did_swiglu = nullptr) {
   ctx->act_mode = mode;
   ctx->act_in_dim = in_dim;
   ctx->act_tokens = T;
@@ -2152,7 +2156,7 @@ static int llama_matmul_quantized_rows(ogm_ctx *ctx, const ogm_weight *const *ws
       tg[e - i] = Target{ws[e], ys[e]};
       e++;
     }
-    int rc = enqueue_gemv(ctx, tg, e - i, T, 0, s, nullptr, nullptr);
+    int rc = enqueue_gemv(ctx, tg, e - i, T, 0, s, nullptr, nullptr, nullptr, e - i == n ? did_swiglu : nullptr);
     if (rc != OGM_OK) return rc;
     i = e;
   }
@@ -2174,7 +2178,8 @@ static int llama_producer_xt(ogm_ctx *ctx, const ogm_weight *w, int mode, uint32
 // x += delta, RMSNorm, and the matmuls over the normed rows: the norm kernel quantizes its own
 // output (the decode step's kernel, one workgroup per row) and the f32 rows are never stored.
 static int llama_norm_matmul_rows(ogm_ctx *ctx, ogm_llama *m, const ogm_weight *const *ws, float *const *ys, size_t n,
-                                  const float *delta, const float *norm_w, uint32_t T, hipStream_t s) {
+                                  const float *delta, const float *norm_w, uint32_t T, hipStream_t s,
+                                  bool *did_swiglu = nullptr) {
   const ogm_llama_config &c = m->cfg;
   int rc = ensure_act(ctx, c.n_embd, T);
   if (rc != OGM_OK) return rc;
@@ -2195,7 +2200,8 @@ static int llama_norm_matmul_rows(ogm_ctx *ctx, ogm_llama *m, const ogm_weight *
     if ((rc = llama_producer_xt(ctx, wm[0], mode, c.n_embd, T, &act.xt)) != OGM_OK) return rc;
     HIPCHK(ctx, ogm_launch_norm_quant(mode, m->pf.x, first ? delta : nullptr, norm_w, c.n_embd, c.rms_eps, nullptr, act, s, T));
     first = false;
-    if ((rc = llama_matmul_quantized_rows(ctx, wm, ym, k, mode, c.n_embd, T, s, act.xt != nullptr)) != OGM_OK) return rc;
+    if ((rc = llama_matmul_quantized_rows(ctx, wm, ym, k, mode, c.n_embd, T, s, act.xt != nullptr,
+                                          k == n ? did_swiglu : nullptr)) != OGM_OK) return rc;
   }
   return OGM_OK;
 }
@@ -2256,16 +2262,21 @@ static int llama_prefill_chunk(ogm_ctx *ctx, ogm_llama *m, uint32_t pos0, uint32
     }
     const ogm_weight *w2[2] = {L.w_gate, L.w_up};
     float *y2[2] = {P.gate, P.up};
-    if ((rc = llama_norm_matmul_rows(ctx, m, w2, y2, 2, P.proj, ffn_norm, T, s)) != OGM_OK) return rc;
-    // SwiGLU quantizes its own output for the down projection: h is never stored as f32
+    bool h_ready = false;   // P.gate holds silu(gate) * up
+    if ((rc = llama_norm_matmul_rows(ctx, m, w2, y2, 2, P.proj, ffn_norm, T, s, &h_ready)) != OGM_OK) return rc;
     const ogm_weight *wd[1] = {L.w_down};
+    delta = P.proj;
+    if (h_ready) {
+      if ((rc = llama_matmul_rows(ctx, wd, y1, 1, P.gate, T, s)) != OGM_OK) return rc;
+      continue;
+    }
+    // SwiGLU quantizes its own output for the down projection: h is never stored as f32
     const int mode_d = act_mode_for(L.w_down->ggml_type, T, 0);
     if ((rc = ensure_act(ctx, c.n_ff, T)) != OGM_OK) return rc;
     OgmActDev act_d = act_view(ctx, c.n_ff, mode_d, 0);
     if ((rc = llama_producer_xt(ctx, L.w_down, mode_d, c.n_ff, T, &act_d.xt)) != OGM_OK) return rc;
     HIPCHK(ctx, ogm_launch_swiglu_quant(mode_d, P.gate, P.up, c.n_ff, nullptr, act_d, s, T));
     if ((rc = llama_matmul_quantized_rows(ctx, wd, y1, 1, mode_d, c.n_ff, T, s, act_d.xt != nullptr)) != OGM_OK) return rc;
-    delta = P.proj;
   }
   ctx->act_mode = -1;   // the activation scratch was the matmuls'
   if (all_logits) {

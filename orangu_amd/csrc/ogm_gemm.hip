@@ -1026,8 +1026,10 @@ struct GbShape {
   static_assert(SLOTS % RB == 0 && RB % 2u == 0, "a super-block's pieces sit in the same slots every turn of the ring");
 };
 
-template <int KIND, uint32_t RB>
+template <int KIND, uint32_t RB, bool SWIGLU = false>
 __device__ __forceinline__ void gemm_planes_body(GemmDmaParams &p) {
+  static_assert(!SWIGLU || RB == 4u, "the first RB / 2 row blocks are gate's, the others up's");
+  constexpr uint32_t RBM = SWIGLU ? RB / 2u : RB;   // row blocks of one matrix
   using Shape = GbShape<KIND, RB>;
   constexpr uint32_t NW = Shape::NW;
   constexpr bool Q45 = KIND == GP_Q4K || KIND == GP_Q5K;
@@ -1035,7 +1037,7 @@ __device__ __forceinline__ void gemm_planes_body(GemmDmaParams &p) {
   constexpr uint32_t TURN = SLOTS / RB;         // super-blocks the ring holds
   constexpr uint32_t KSTEP = NPL * 1024u;       // bytes of a step of 32 k: 32 rows, NPL planes
   constexpr uint32_t PER = 8u * NPL / NW;       // loads a wave issues per piece
-  constexpr uint32_t ROWS = 32u * RB, TOK = 32u * NW;
+  constexpr uint32_t ROWS = 32u * RBM, TOK = 32u * NW;
   extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1055,7 +1057,7 @@ __device__ __forceinline__ void gemm_planes_body(GemmDmaParams &p) {
 #pragma unroll
   for (uint32_t m = 0; m < OGM_GEMM_MAX_MATS - 1; m++) {   // the matrix this row tile belongs to
     const uint32_t tiles = (p.out_dim + ROWS - 1u) / ROWS;
-    if (m < p.n_extra && row_tile >= tiles) {
+    if (!SWIGLU && m < p.n_extra && row_tile >= tiles) {
       row_tile -= tiles;
       p.planes = p.extra_planes[m];
       p.y = p.extra_y[m];
@@ -1069,13 +1071,15 @@ __device__ __forceinline__ void gemm_planes_body(GemmDmaParams &p) {
   const bool live = t0 + 32u * wave < p.n_tokens;   // the wave has a token to multiply (else it only fetches)
   uint32_t rb32[RB];                                // the row blocks of 32 (past the matrix: its last one again, never stored)
 #pragma unroll
-  for (uint32_t i = 0; i < RB; i++) rb32[i] = min(row_tile * RB + i, 2u * nrb - 1u);
+  for (uint32_t i = 0; i < RB; i++) rb32[i] = min(row_tile * RBM + i % RBM, 2u * nrb - 1u);
 
   // ---- what goes to LDS.  A piece is a super-block of a row block of 32: step k of its eight in chunks of 1 KiB, one a
   // plane (lane (l32, lh): the 16 weights 16 lh .. of row l32); wave w fetches steps w, w + NW
   const uint32_t w_lane = lh * KSTEP + l32 * 16u;
-  const __amdgpu_buffer_rsrc_t planes = gb_buffer(p.planes);
+  const uint8_t *const planes2 = SWIGLU ? p.extra_planes[0] : p.planes;   // of the row blocks from RBM on
+  const __amdgpu_buffer_rsrc_t planes_a = gb_buffer(p.planes), planes_b = gb_buffer(planes2);
   auto fetch_piece = [&](uint32_t s, uint32_t i, uint32_t slot) {   // super-block s of row block i
+    const __amdgpu_buffer_rsrc_t planes = i < RBM ? planes_a : planes_b;
     uint32_t b = rb32[0];
 #pragma unroll
     for (uint32_t j = 1; j < RB; j++) b = i == j ? rb32[j] : b;
@@ -1091,13 +1095,14 @@ __device__ __forceinline__ void gemm_planes_body(GemmDmaParams &p) {
   // a super-block's tables: 64 tokens' ad from each of the first NW / 2 waves, 64 rows' d from each of the next RB / 2
   const bool tab_ad = wave < NW / 2u;
   const bool tab_d = !tab_ad && wave - NW / 2u < RB / 2u;
-  const __amdgpu_buffer_rsrc_t tab = gb_buffer(tab_ad ? (const uint8_t *)p.ad : p.planes + gp_d_offset(nrb, nsb, NPL));
+  const __amdgpu_buffer_rsrc_t tab = gb_buffer(
+      tab_ad ? (const uint8_t *)p.ad : (SWIGLU && wave == NW / 2u + 1u ? planes2 : p.planes) + gp_d_offset(nrb, nsb, NPL));
   uint32_t tab_lane;
   if (tab_ad) {
     tab_lane = min(t0 + 64u * wave + lane, p.n_tokens - 1u) * nsb * 4u;
   } else {
     const uint32_t i = (tab_d ? 2u * (wave - NW / 2u) : 0u) + lh;
-    tab_lane = min(row_tile * RB + i, 2u * nrb - 1u) * nsb * 128u + l32 * 4u;
+    tab_lane = min(row_tile * RBM + i % RBM, 2u * nrb - 1u) * nsb * 128u + l32 * 4u;
   }
   const uint32_t tab_step = tab_ad ? 4u : 128u;
   const uint32_t tab_dst = TAB + (tab_ad ? 256u * wave : NW * 128u + (tab_d ? 256u * (wave - NW / 2u) : RB * 128u));
@@ -1155,11 +1160,11 @@ __device__ __forceinline__ void gemm_planes_body(GemmDmaParams &p) {
     const uint32_t tok = min(t0 + 32u * wave + l32, p.n_tokens - 1u);
     const _Float16 *bs = p.bs16 + ((size_t)tok * nsb * 16u + 8u * lh);
     const float *adp = p.ad + (size_t)tok * nsb;
-    const float *dmin = (const float *)(p.planes + gp_dmin_offset(nrb, nsb, NPL));
-    const uint8_t *mins = p.planes + gp_mins_offset(nrb, nsb, NPL) + lane * 16u;
+    auto dmin = [&](uint32_t i) { return (const float *)((i < RBM ? p.planes : planes2) + gp_dmin_offset(nrb, nsb, NPL)); };
+    auto mins = [&](uint32_t i) { return (i < RBM ? p.planes : planes2) + gp_mins_offset(nrb, nsb, NPL) + lane * 16u; };
     uint32_t dm_at[RB / 2];
 #pragma unroll
-    for (uint32_t j = 0; j < RB / 2u; j++) dm_at[j] = min(row_tile * RB + 2u * j + lh, 2u * nrb - 1u) * nsb * 32u + l32;
+    for (uint32_t j = 0; j < RB / 2u; j++) dm_at[j] = min(row_tile * RBM + (2u * j) % RBM + lh, 2u * nrb - 1u) * nsb * 32u + l32;
     struct Set {
       half8 b2, m[RB];
       float ad, dm[RB / 2];
@@ -1169,9 +1174,9 @@ __device__ __forceinline__ void gemm_planes_body(GemmDmaParams &p) {
       q.b2 = *(const half8 *)(bs + s * 16u);
       q.ad = adp[s];
 #pragma unroll
-      for (uint32_t j = 0; j < RB / 2u; j++) q.dm[j] = dmin[dm_at[j] + s * 32u];
+      for (uint32_t j = 0; j < RB / 2u; j++) q.dm[j] = dmin(2u * j)[dm_at[j] + s * 32u];
 #pragma unroll
-      for (uint32_t i = 0; i < RB; i++) q.m[i] = *(const half8 *)(mins + (size_t)(rb32[i] * nsb + s) * 1024u);
+      for (uint32_t i = 0; i < RB; i++) q.m[i] = *(const half8 *)(mins(i) + (size_t)(rb32[i] * nsb + s) * 1024u);
     };
     auto use = [&](const Set &q) {
       const float16v z16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -1334,13 +1339,15 @@ __device__ __forceinline__ void gemm_planes_body(GemmDmaParams &p) {
     }
   }
 #pragma unroll
-  for (uint32_t i = 0; i < RB; i++) {
+  for (uint32_t i = 0; i < RBM; i++) {
     const uint32_t row = r0 + 32u * i + l32;
     if (row < p.out_dim) {
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         const uint32_t t = t0 + 32u * wave + 8u * (r >> 2) + 4u * lh + (r & 3);
-        if (t < p.n_tokens) p.y[(size_t)t * p.out_dim + row] = y[i][r];
+        float v = y[i][r];
+        if constexpr (SWIGLU) v = v / (1.0f + expf(-v)) * y[i + RBM][r];   // (ogm_swiglu_quant_run's order)
+        if (t < p.n_tokens) p.y[(size_t)t * p.out_dim + row] = v;
       }
     }
   }
@@ -1350,6 +1357,12 @@ template <int KIND>
 __global__ __launch_bounds__(256, 2) void ogm_gemm_dma_kernel(GemmDmaParams p) { gemm_planes_body<KIND, 4u>(p); }
 template <int KIND>
 __global__ __launch_bounds__(256, 2) void ogm_gemm_dmx_kernel(GemmDmaParams p) { gemm_planes_body<KIND, 2u>(p); }
+// Gate and up of a feed-forward block in one launch of 128-row tiles, 64 rows of each: a wave holds both sums of its outputs
+// and stores silu(gate) * up alone, so that half as many outputs go to memory and come back for the quantizer.  2048 -> 2 x
+// 8192 at 1901 tokens 156.9 us and 26.6 for the quantizing SwiGLU launch, 154.9 and 19.2 for the quantizer here (a forward
+// pass 7345 -> 7227, the 8B shapes at 1500 tokens 7635 -> 7475, at 512 3116 -> 3101).
+template <int KIND>
+__global__ __launch_bounds__(256, 2) void ogm_gemm_swiglu_kernel(GemmDmaParams p) { gemm_planes_body<KIND, 4u, true>(p); }
 
 // ------------------------------------------------------------------------------------------
 // Small batches (up to a few dozen tokens): the tiled kernels above cost the same for 9 tokens as
@@ -3275,9 +3288,17 @@ bool ogm_gemm_uses_planes(const OgmGemmArgs &a) {
   return !gemm_small_batch(a, true) && gemm_dma_eligible(a);
 }
 
+// Gate and up may leave silu(gate) * up where their launch takes 128-row tiles over planes; 64-row tiles, the small and
+// medium batches and the one-pass kernel store both.
+bool ogm_gemm_does_swiglu(const OgmGemmArgs &a) {
+  return a.n_extra == 1u && a.extra_out_dim[0] == a.out_dim && ogm_gemm_uses_planes(a) && !gemm_interleaved(a) &&
+         !(a.medium == 2u && gemm_medium_batch(a)) && a.one_pass == 0u;
+}
+
 hipError_t ogm_launch_gemm(const OgmGemmArgs &a, hipStream_t stream, const char **kernel_name) {
   if (a.n_tokens == 0 || a.out_dim == 0) return hipSuccess;
   if (!ogm_gemm_supported(a.ggml_type, a.in_dim, a.out_dim, a.n_tokens)) return hipErrorInvalidValue;
+  if (a.swiglu && !(a.planes && a.extra_planes[0] && ogm_gemm_does_swiglu(a))) return hipErrorInvalidValue;
   if (a.n_extra > OGM_GEMM_MAX_MATS - 1 || (is_flat32(a.ggml_type) && a.n_extra != 0)) return hipErrorInvalidValue;
   if (is_flat32(a.ggml_type)) {
     GemmFlatParams p;
@@ -3538,6 +3559,21 @@ hipError_t ogm_launch_gemm(const OgmGemmArgs &a, hipStream_t stream, const char 
                        : a.ggml_type == OGM_IQ4_XS ? "ogm_gemm_iq4xs_dmx_kernel"
                        : a.ggml_type == OGM_Q4_K   ? "ogm_gemm_q4k_dmx_kernel"
                                                    : "ogm_gemm_q5k_dmx_kernel";
+      return hipGetLastError();
+    }
+    if (a.swiglu) {
+      const void *fs = a.ggml_type == OGM_Q6_K     ? (const void *)ogm_gemm_swiglu_kernel<GP_Q6K>
+                       : a.ggml_type == OGM_IQ4_XS ? (const void *)ogm_gemm_swiglu_kernel<GP_IQ4XS>
+                       : a.ggml_type == OGM_Q3_K   ? (const void *)ogm_gemm_swiglu_kernel<GP_Q3K>
+                       : a.ggml_type == OGM_Q4_K   ? (const void *)ogm_gemm_swiglu_kernel<GP_Q4K>
+                                                   : (const void *)ogm_gemm_swiglu_kernel<GP_Q5K>;
+      const uint32_t lds_s = a.ggml_type == OGM_Q3_K ? GbShape<GP_Q3K, 4u>::LDS_BYTES : GbShape<GP_Q4K, 4u>::LDS_BYTES;
+      hipError_t es = hipFuncSetAttribute(fs, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_s);
+      if (es != hipSuccess) return es;
+      void *sargs[] = {(void *)&d};
+      es = hipLaunchKernel(fs, dim3((a.n_tokens + GD_TOK - 1u) / GD_TOK, (a.out_dim + 63u) / 64u), dim3(256), sargs, lds_s, stream);
+      if (es != hipSuccess) return es;
+      if (kernel_name) *kernel_name = "ogm_gemm_swiglu_kernel";
       return hipGetLastError();
     }
     const bool one_pass = q45 && a.one_pass != 0u;

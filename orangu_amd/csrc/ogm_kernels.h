@@ -101,10 +101,13 @@ struct OgmGemmArgs {
   // the grid
   uint32_t plane_kernel = 0;
   uint32_t interleave = 0;   // the plane kernel with 64-row tiles that adds a super-block up between the next one's matrix instructions: 0 by the size of the launch, 1 never, 2 whenever it can
+  bool swiglu = false;     // the two matrices are gate and up: y gets silu(gate) * up, extra_y is not written (ogm_gemm_does_swiglu)
   uint32_t one_pass = 0;   // Q4_K / Q5_K on the all-waves-multiply kernel: fold the min pass into the super-block step (f32 to rounding, not to the bit)
 };
 // Whether this launch would run a tiled int8 plane kernel, i.e. whether planes would be read.
 bool ogm_gemm_uses_planes(const OgmGemmArgs &a);
+// Whether this launch, given its matrices' planes, could store silu(first) * second alone.
+bool ogm_gemm_does_swiglu(const OgmGemmArgs &a);
 // Whether this K-quant or IQ4_XS launch would run the small-batch kernel of its type (which needs no planes).
 bool ogm_gemm_takes_small_batch(const OgmGemmArgs &a);
 // Bytes of a K-quant matrix's planes (0: the type has none), and the kernel that builds them from
