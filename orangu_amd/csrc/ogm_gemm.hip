@@ -1959,7 +1959,13 @@ __global__ __launch_bounds__(512) void ogm_gemm_sb_q2k_kernel(GemmSbParams p) {
 // instruction each), then the sweep of the products as above.  A lane's 16 weights of sub-block j
 // are the low (j even) or high nibbles of one 16-byte piece of qs, Q5_K's fifth bit is bit j of
 // its piece of qh.
-template <bool Q5, uint32_t NW>
+// AHEAD: a round's loads -- header and sums in the first sweep, the eight operand chunks of the activations in the second --
+// are under way a round before (the weights always are), so that a round starts on registers and not on a trip to memory; past
+// the last super-block every lane asks for one line.  Whole calls, us, before / now: Q4_K 14336 -> 4096 at 64 tokens 30.5 /
+// 26.1, 8192 -> 8192 at 100 52.8 / 47.7, 8192 -> 2048 at 300 50.5 / 40.9, 3072 -> 3072 at 64 14.3 / 11.9, 4096 -> 14336 at 40
+// 29.4 / 26.8, Q5_K 11008 -> 4096 at 77 36.6 / 35.6, -> 8192 60.3 / 55.5, 14336 -> 4096 at 9 24.9 / 23.1.  (Q6_K, which has one
+// sweep and two plain chains of matrix instructions to wait behind, lost 3 to 12 % of its short rows and won 4 % of the longest.)
+template <bool Q5, uint32_t NW, bool AHEAD>
 __device__ __forceinline__ void gemm_sb_q45k_body(GemmSbParams p) {
   constexpr uint32_t NT = 64u * NW, NACC = 1024u / NT;
   constexpr uint32_t TILE_BYTES = Q5 ? 11264u : 9216u;
@@ -1968,7 +1974,7 @@ __device__ __forceinline__ void gemm_sb_q45k_body(GemmSbParams p) {
   float *terms = (float *)sb_lds;             // [NW super-blocks][32 tokens][32 rows]
   float *ad_l = terms + NW * 32u * 32u;       // [nsb][32 tokens]
 
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t l32 = lane & 31u, lh = lane >> 5;
   uint32_t row_tile = blockIdx.y;
 #pragma unroll
@@ -2003,8 +2009,8 @@ __device__ __forceinline__ void gemm_sb_q45k_body(GemmSbParams p) {
   uint4 hdr, w0, w1, w2, w3, qh5 = make_uint4(0, 0, 0, 0);
 #define SB_LOADW(S)                                                                               \
   do {                                                                                            \
-    const uint32_t s_ = min((uint32_t)(S), p.nsb - 1u); /* past the end: loaded, never used */    \
-    const uint32_t so_ = uo + sb_off(s_);                                                         \
+    const uint32_t s_ = S; /* past the end: one line for all lanes, never used */                 \
+    const uint32_t so_ = s_ < p.nsb ? uo + sb_off(s_) : 0u;                                       \
     hdr = *(const uint4 *)(p.wt + so_);                                                           \
     w0 = *(const uint4 *)(p.wt + (so_ + (QS_PIECE0 + 0u + lh) * 1024u));                          \
     w1 = *(const uint4 *)(p.wt + (so_ + (QS_PIECE0 + 2u + lh) * 1024u));                          \
@@ -2012,6 +2018,13 @@ __device__ __forceinline__ void gemm_sb_q45k_body(GemmSbParams p) {
     w3 = *(const uint4 *)(p.wt + (so_ + (QS_PIECE0 + 6u + lh) * 1024u));                          \
     if constexpr (Q5) qh5 = *(const uint4 *)(p.wt + (so_ + (1u + lh) * 1024u));                   \
   } while (0)
+#define SB_LOADX(S)                                                                               \
+  do {                                                                                            \
+    const uint32_t s_ = S, xs_ = s_ < p.nsb ? xro + 256u * s_ * xmul : 0u;                        \
+    _Pragma("unroll") for (int j_ = 0; j_ < 8; j_++)                                              \
+      xa[j_] = *(const int4v *)(p.xq + (xs_ + 32u * j_ * xmul));                                  \
+  } while (0)
+  int4v xa[8];
   SB_LOADW(wave);   // the second sweep's first weights: under way during the first sweep
   for (uint32_t i = tid; i < 32u * p.nsb; i += NT) {
     const uint32_t k = i / p.nsb, s = i - k * p.nsb;
@@ -2028,12 +2041,24 @@ __device__ __forceinline__ void gemm_sb_q45k_body(GemmSbParams p) {
 #pragma unroll
     for (int r = 0; r < 16; r++) zero[r] = 0.0f;
     const float side_scale = lh ? 1.0f : 64.0f;
+    uint4 hd_n = hdr;
+    half8 b2_n = *(const half8 *)(p.bs16 + (wave < p.nsb ? (tk + wave) * 16u + 8u * lh : 0u));
     for (uint32_t s0 = 0; s0 < p.nsb; s0 += NW) {
       {
         const uint32_t sl = wave, s = s0 + sl;
+        if (!AHEAD && s0 != 0u && s < p.nsb) {
+          hd_n = *(const uint4 *)(p.wt + (uo + sb_off(s)));
+          b2_n = *(const half8 *)(p.bs16 + ((tk + s) * 16u + 8u * lh));
+        }
+        const uint4 hd = hd_n;
+        const half8 b2 = b2_n;
+        if constexpr (AHEAD) {   // the next round's (past the end: one line for all lanes, never used)
+          const uint32_t sn = s + NW;
+          hd_n = *(const uint4 *)(p.wt + (sn < p.nsb ? uo + sb_off(sn) : 0u));
+          b2_n = *(const half8 *)(p.bs16 + (sn < p.nsb ? (tk + sn) * 16u + 8u * lh : 0u));
+          __builtin_amdgcn_sched_barrier(0);
+        }
         if (s < p.nsb) {   // wave-uniform
-          const uint4 hd = *(const uint4 *)(p.wt + (uo + sb_off(s)));
-          const half8 b2 = *(const half8 *)(p.bs16 + ((tk + s) * 16u + 8u * lh));
           uint32_t mna, mnb;
           q4k_mins(hd, mna, mnb);
           const half8 a1 = side_operand(mna, mnb, side_scale);
@@ -2072,8 +2097,8 @@ __device__ __forceinline__ void gemm_sb_q45k_body(GemmSbParams p) {
       if constexpr (Q5) v_[w_] |= ((q5w_[w_] >> (J)) & 0x01010101u) << 4;                         \
     }                                                                                             \
     const int4v b_ = {(int)v_[0], (int)v_[1], (int)v_[2], (int)v_[3]};                            \
-    const int4v xa_ = *(const int4v *)(p.xq + (xs_ + 32u * (J) * xmul));                          \
-    D = __builtin_amdgcn_mfma_i32_32x32x32_i8(xa_, b_, zi, 0, 0, 0);                              \
+    if constexpr (!AHEAD) xa[J] = *(const int4v *)(p.xq + (xs_ + 32u * (J) * xmul));              \
+    D = __builtin_amdgcn_mfma_i32_32x32x32_i8(xa[J], b_, zi, 0, 0, 0);                            \
   } while (0)
 #define SB_ACC(D, J, FIRST)                                                                       \
   do {                                                                                            \
@@ -2082,6 +2107,7 @@ __device__ __forceinline__ void gemm_sb_q45k_body(GemmSbParams p) {
       I[r_] = (FIRST) ? __mul24(sc_, D[r_]) : __mul24(sc_, D[r_]) + I[r_];                        \
   } while (0)
   const int16v zi = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  if constexpr (AHEAD) SB_LOADX(wave);
   for (uint32_t s0 = 0; s0 < p.nsb; s0 += NW) {
     const uint32_t s = s0 + wave;
     if (s < p.nsb) {   // wave-uniform
@@ -2119,7 +2145,12 @@ __device__ __forceinline__ void gemm_sb_q45k_body(GemmSbParams p) {
         }
       }
     }
-    SB_LOADW(s + NW);   // the next round's weights, in flight over the barrier and the additions
+    // the next round's weights and activations, in flight over the barrier and the additions
+    SB_LOADW(s + NW);
+    if constexpr (AHEAD) {
+      SB_LOADX(s + NW);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     __syncthreads();
     {
       const uint32_t n_here = min(NW, p.nsb - s0);
@@ -2131,6 +2162,7 @@ __device__ __forceinline__ void gemm_sb_q45k_body(GemmSbParams p) {
     __syncthreads();
   }
 #undef SB_LOADW
+#undef SB_LOADX
 #undef SB_MMA
 #undef SB_ACC
   {
@@ -2143,10 +2175,10 @@ __device__ __forceinline__ void gemm_sb_q45k_body(GemmSbParams p) {
   }
 }
 
-template <bool Q5>
-__global__ __launch_bounds__(512) void ogm_gemm_sb_q45k_kernel(GemmSbParams p) { gemm_sb_q45k_body<Q5, 8u>(p); }
-template <bool Q5>
-__global__ __launch_bounds__(1024) void ogm_gemm_sb_q45k_w16_kernel(GemmSbParams p) { gemm_sb_q45k_body<Q5, 16u>(p); }
+template <bool Q5, bool AHEAD>
+__global__ __launch_bounds__(512) void ogm_gemm_sb_q45k_kernel(GemmSbParams p) { gemm_sb_q45k_body<Q5, 8u, AHEAD>(p); }
+template <bool Q5, bool AHEAD>
+__global__ __launch_bounds__(1024) void ogm_gemm_sb_q45k_w16_kernel(GemmSbParams p) { gemm_sb_q45k_body<Q5, 16u, AHEAD>(p); }
 
 // ------------------------------------------------------------------------------------------
 // Medium batches of Q4_K / Q5_K (some 65 to 256 tokens over a matrix whose 128 x 128 tiles would leave compute
@@ -3455,11 +3487,19 @@ hipError_t ogm_launch_gemm(const OgmGemmArgs &a, hipStream_t stream, const char 
     const bool w16 = (a.sb_waves ? a.sb_waves == 16u : (n_wg <= 256u && nsb >= 16u)) &&
                      16u * 4096u + 128u * nsb <= GM_LDS_MAX;
     const uint32_t lds_bytes = (w16 ? 16u : 8u) * 4096u + 128u * nsb;
+    // a round's loads a round ahead where there is a round to spare: from two rounds, Q5_K from three (Q4_K 4096 -> 4096 at 20
+    // tokens in one round 10.1 against 10.7, 2048 -> 2048 at 12 7.7 / 7.9; Q5_K 4096 -> 4096 at 96 in two 17.8 / 18.3)
+    const uint32_t nw = w16 ? 16u : 8u;
+    const bool ahead = nsb > (a.ggml_type == OGM_Q5_K ? 2u * nw : nw);
+    auto q45_fn = [&](auto q5_c) {
+      constexpr bool Q5 = decltype(q5_c)::value;
+      return w16 ? (ahead ? (const void *)ogm_gemm_sb_q45k_w16_kernel<Q5, true> : (const void *)ogm_gemm_sb_q45k_w16_kernel<Q5, false>)
+                 : (ahead ? (const void *)ogm_gemm_sb_q45k_kernel<Q5, true> : (const void *)ogm_gemm_sb_q45k_kernel<Q5, false>);
+    };
     const void *fn = a.ggml_type == OGM_Q6_K   ? (w16 ? (const void *)ogm_gemm_sb_q6k_w16_kernel : (const void *)ogm_gemm_sb_q6k_kernel)
                      : a.ggml_type == OGM_Q3_K ? (w16 ? (const void *)ogm_gemm_sb_q3k_w16_kernel : (const void *)ogm_gemm_sb_q3k_kernel)
                      : a.ggml_type == OGM_IQ4_XS ? (w16 ? (const void *)ogm_gemm_sb_iq4xs_w16_kernel : (const void *)ogm_gemm_sb_iq4xs_kernel)
-                     : a.ggml_type == OGM_Q4_K ? (w16 ? (const void *)ogm_gemm_sb_q45k_w16_kernel<false> : (const void *)ogm_gemm_sb_q45k_kernel<false>)
-                                               : (w16 ? (const void *)ogm_gemm_sb_q45k_w16_kernel<true> : (const void *)ogm_gemm_sb_q45k_kernel<true>);
+                     : a.ggml_type == OGM_Q4_K ? q45_fn(std::false_type{}) : q45_fn(std::true_type{});
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
     if (e != hipSuccess) return e;
     void *kargs[] = {(void *)&p};
