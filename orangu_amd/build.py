@@ -43,7 +43,7 @@ EXTRA_FLAGS = {"ogm_gemm_ft.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 def build(verbose: bool = False, defines=(), out: str | None = None) -> str:
     """Compiles every source to an object of its own (in parallel) and links the shared library.
     `defines` (NAME=VALUE strings, passed as -D) and `out` build a variant beside the library instead of it: the
-    kernels' timing switches (GD_ABL_*, SBW_ABL, FK_ABL: wrong results, for `bench.py --lib`)."""
+    kernels' timing switches (SBW_ABL, FK_ABL: wrong results, for `bench.py --lib`)."""
     from concurrent.futures import ThreadPoolExecutor
     names = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
     if defines and not out:
