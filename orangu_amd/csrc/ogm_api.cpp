@@ -380,7 +380,7 @@ extern "C" size_t ogm_scratch_bytes(ogm_ctx *ctx) {
   if (!ctx) return 0;
   std::lock_guard<std::mutex> lock(ctx->mu);
   const DevBuf *all[] = {&ctx->x,    &ctx->y,    &ctx->q,  &ctx->d,          &ctx->sums, &ctx->bsum, &ctx->bs16,
-                         &ctx->isum, &ctx->imin, &ctx->xh, &ctx->probe_sink, &ctx->hx,   &ctx->hy,   &ctx->hflag};
+                         &ctx->isum, &ctx->imin, &ctx->xh, &ctx->probe_sink, &ctx->hx,   &ctx->hy,   &ctx->hflag, &ctx->hstage};
   size_t n = 0;
   for (const DevBuf *b : all) n += b->cap;
   return n;
