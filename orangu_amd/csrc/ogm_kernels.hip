@@ -1204,7 +1204,12 @@ __device__ __forceinline__ T *of_matrix(T *const (&v)[OGM_GEMV_MAX_MATS], uint32
 
 // NQ: runs of 1024 elements a wave prepares.  bid: the workgroup's number among those of its type; leads: it stores the
 // quantized row and the residual stream.
-template <class F, int UPR, int PRE, int NQ, bool SWIGLU>
+// NB 2 (SWIGLU): a second row block of both matrices, gridDim.x after the first.  Where one block a workgroup is more waves than
+// the device holds at once (twenty a compute unit at these registers) a second round of workgroups pays the whole chain again --
+// its start, the trip for the row, the preparation; here its weights are under way over the first block's sum instead.  8B shapes
+// (4096 -> 2 x 14336: 896 workgroups of eight waves, now 448), a step of 8 layers at 300 / 2048 / 16000 positions 447.7 / 460.1 /
+// 567.5 -> 436.0 / 448.6 / 556.0 us.  Not for launches without SwiGLU: 4096 -> 28672, two teams of different row blocks, 10.7 -> 11.9.
+template <class F, int UPR, int PRE, int NQ, int NB, bool SWIGLU>
 __device__ __forceinline__ void gemv_fused_body(const GemvFusedParams &fp, const uint32_t bid, const bool leads) {
   extern __shared__ __align__(16) uint8_t lds[];
   const GemvParams &p = fp.g;
@@ -1224,8 +1229,8 @@ __device__ __forceinline__ void gemv_fused_body(const GemvFusedParams &fp, const
   uint4 *l_aux = l_xq + xch;
   float *l_d = (float *)(l_aux + upr * F::AUX16);
   const uint32_t head = (xch * 16 + upr * F::AUX16 * 16 + n_scale * 4 + 15) & ~15u;
-  float *l_term = (float *)(lds + head);               // [teams][upr][R]
-  float *l_red = l_term + (size_t)teams * term_stride; // PRE 2: a run of 256's sum of squares each
+  float *l_term = (float *)(lds + head);               // [NB][teams][upr][R]
+  float *l_red = l_term + (size_t)NB * teams * term_stride; // PRE 2: a run of 256's sum of squares each
 
   // ---- this wave's team and its row block (a team past the last one multiplies the last again and stores nothing)
   const uint32_t team = teams == 1u ? 0u : wave / tw, wv = wave - team * tw;
@@ -1372,24 +1377,46 @@ __device__ __forceinline__ void gemv_fused_body(const GemvFusedParams &fp, const
   a.d = l_d;
   a.upr = upr;
   float *my_term = l_term + (size_t)team * term_stride;
-  for (; it < nct; it += tw) {
-    const uint32_t col_own = it * C + c_local;
-    const bool live = col_own < upr;
-    const uint32_t col = live ? col_own : upr - 1u;
-    int isum, imin;
-    F::template sums<UPR>(cur, a, col, isum, imin);
-    if (live) my_term[col * R + r_local] = F::term_gemv(cur, a.d[col], isum, imin);
-    if (it + tw < nct) F::load(cur, wt, tile0 + it + tw, lane);
+  auto tiles = [&](size_t tile, float *term) {
+    for (; it < nct; it += tw) {
+      const uint32_t col_own = it * C + c_local;
+      const bool live = col_own < upr;
+      const uint32_t col = live ? col_own : upr - 1u;
+      int isum, imin;
+      F::template sums<UPR>(cur, a, col, isum, imin);
+      if (live) term[col * R + r_local] = F::term_gemv(cur, a.d[col], isum, imin);
+      if (it + tw < nct) F::load(cur, wt, tile + it + tw, lane);
+    }
+  };
+  tiles(tile0, my_term);
+  // SWIGLU, R <= 32: the first wave adds gate and up of a row up, one in each half
+  auto product = [&](uint32_t rb, const float *term) {
+    const uint32_t t = lane / R, r = lane - t * R, orow = rb * R + r;
+    const bool have = t < 2u && orow < out_dim;
+    const float acc = have ? ordered_sum<false>(0.0f, term + (size_t)t * term_stride + r, upr, R) : 0.0f;
+    const float up = __shfl(acc, (int)((lane + R) & 63u));
+    if (have && t == 0u) y[orow] = acc / (1.0f + expf(-acc)) * up;
+  };
+  if constexpr (NB == 2) {
+    static_assert(SWIGLU, "a second row block of gate and up");
+    const uint32_t rb1 = rb0 + gridDim.x;
+    const bool more = rb1 < p.wg_end[0];
+    const size_t tile1 = (size_t)min(rb1, p.wg_end[0] - 1u) * nct;
+    it = wv;
+    F::load(cur, wt, tile1 + it, lane);   // its first tile, under way over the first block's sum
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    if (wave == 0u) product(rb0, l_term);
+    if (!more) return;
+    tiles(tile1, my_term + 2u * term_stride);
+    __syncthreads();
+    if (wave == 0u) product(rb1, l_term + 2u * term_stride);
+    return;
   }
   __syncthreads();
 
-  if constexpr (SWIGLU) {   // R <= 32: the first wave adds gate and up of a row up, one in each half
-    if (wave != 0u) return;
-    const uint32_t t = lane / R, r = lane - t * R, orow = rb0 * R + r;
-    const bool have = t < 2u && orow < out_dim;
-    const float acc = have ? ordered_sum<false>(0.0f, l_term + (size_t)t * term_stride + r, upr, R) : 0.0f;
-    const float up = __shfl(acc, (int)((lane + R) & 63u));
-    if (have && t == 0u) y[orow] = acc / (1.0f + expf(-acc)) * up;
+  if constexpr (SWIGLU) {
+    if (wave == 0u) product(rb0, l_term);
   } else {   // a team's first wave adds its row block up
     if (wv != 0u || !mine) return;
     const uint32_t orow = rb0 * R + lane;
@@ -1397,17 +1424,17 @@ __device__ __forceinline__ void gemv_fused_body(const GemvFusedParams &fp, const
   }
 }
 
-template <class F, int UPR, int PRE, int NQ, bool SWIGLU>
+template <class F, int UPR, int PRE, int NQ, int NB, bool SWIGLU>
 __global__ __launch_bounds__(F::ELEMS == 32 ? 1024 : 512) void ogm_gemv_fused_kernel(GemvFusedParams fp) {
-  gemv_fused_body<F, UPR, PRE, NQ, SWIGLU>(fp, blockIdx.x, blockIdx.x == 0);
+  gemv_fused_body<F, UPR, PRE, NQ, NB, SWIGLU>(fp, blockIdx.x, blockIdx.x == 0);
 }
 
 // Matrices of two K-quants over one normed row (q and k in Q4_K beside v in Q6_K, as mixed files have them in half of
 // their layers): the workgroups of both in one launch.
 template <class F1, class F2, int UPR>
 __global__ __launch_bounds__(512) void ogm_gemv_fused_pair_kernel(GemvFusedParams fp1, GemvFusedParams fp2, uint32_t wgs1) {
-  if (blockIdx.x < wgs1) gemv_fused_body<F1, UPR, 2, 1, false>(fp1, blockIdx.x, blockIdx.x == 0);
-  else gemv_fused_body<F2, UPR, 2, 1, false>(fp2, blockIdx.x - wgs1, false);
+  if (blockIdx.x < wgs1) gemv_fused_body<F1, UPR, 2, 1, 1, false>(fp1, blockIdx.x, blockIdx.x == 0);
+  else gemv_fused_body<F2, UPR, 2, 1, 1, false>(fp2, blockIdx.x - wgs1, false);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1695,9 +1722,14 @@ static hipError_t launch_fused_t(const OgmGemvArgs &a, const OgmGemvSrc &src, hi
   const dim3 g(src.swiglu ? p.wg_end[0] : (n_rb + f.teams - 1u) / f.teams), b(f.team_waves * f.teams * 64u);
   constexpr bool K = F::ELEMS == 256;
   constexpr int HOT = K ? 16 : 128;   // rows of 4096
-#define OGM_FUSED(UPR, PRE, NQ, SW) hipLaunchKernelGGL((ogm_gemv_fused_kernel<F, UPR, PRE, NQ, SW>), g, b, f.lds, stream, fp)
+#define OGM_FUSED(UPR, PRE, NQ, SW) hipLaunchKernelGGL((ogm_gemv_fused_kernel<F, UPR, PRE, NQ, 1, SW>), g, b, f.lds, stream, fp)
   if (norm && src.swiglu) {
-    if (p.upr == HOT) OGM_FUSED(HOT, 2, 1, true);
+    // two row blocks a workgroup beyond the waves the device holds at once, for the K-quants' rows of 4096 (see the kernel)
+    const dim3 g2((g.x + 1u) / 2u);
+    const size_t lds2 = f.lds + (size_t)f.teams * p.upr * (64u / p.C) * 4u;
+    if (K && p.upr == HOT && g.x * f.team_waves * f.teams > 20u * 256u && lds2 <= OGM_LDS_UNASKED)
+      hipLaunchKernelGGL((ogm_gemv_fused_kernel<F, HOT, 2, 1, K ? 2 : 1, true>), g2, b, lds2, stream, fp);
+    else if (p.upr == HOT) OGM_FUSED(HOT, 2, 1, true);
     else OGM_FUSED(0, 2, 1, true);
   } else if (norm) {
     if (p.upr == HOT) OGM_FUSED(HOT, 2, 1, false);
