@@ -549,16 +549,28 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
 // Q6_K 19.0 / 18.2, IQ4_XS -> 28672 16.1 / 15.3.  The per-32 types, whose quantizer launch has more to do, lead to 8192 at any
 // length: Q8_0 4096 -> 4096 (1024) 7.5 / 4.8, -> 28672 (7168) 21.9 / 20.6, 8192 -> 14336 24.7 / 23.7, 14336 -> 8192 27.0 / 25.6, 14336 ->
 // 14336 (12544) level; Q4_0 4096 -> 28672 17.1 / 16.2, Q5_1 19.8 / 18.7.
+//   A norm in front of per-32 matrices is as short as one in front of K-quants, and the launch behind it has more rows' scales
+// to make again in every workgroup: beyond 512 such launches that end in their products lose.  Two layers of a decode step at
+// 300 positions, us, separate / prepared: Q8_0 4096 / 14336 150 / 171, 2048 / 16384 126 / 139, 2048 / 5632 88.6 / 90.1, Q4_0 4096 /
+// 14336 131 / 154, 4096 / 4096 87.7 / 93.1, 2048 / 8192 90.0 / 93.5, Q5_1 4096 / 14336 138 / 162; ahead in a few (Q8_0 3072 / 4096
+// 94.7 / 92.9).  Those that end in silu(gate) * up (rows of at most 1024 inputs) gain: Q8_0 1024 / 32768 159 / 156, 1024 / 49152
+// 213 / 207.
 //   A band above 2048 (512 for the per-32 types) keeps the quantizer launch that calls of these widths have had since prepared
 // launches began, and that the tests expect of them there, though prepared ones lead in it as well (Q4_K 4096 -> 9216, 2304,
 // 7.2 / 5.5, Q6_K 2816 -> 10928, 2049, 7.9 / 7.6, Q8_0 2048 -> 4112, 514, 7.4 / 4.7); it is as narrow as they allow.
-struct PrepareLine {
-  uint32_t to, from, last;   // prepared at up to `to` and between `from` and `last`
-};
-static PrepareLine prepare_line(uint32_t ggml_type, uint32_t in_dim) {
-  if (block_elems_of(ggml_type) == 32) return {512, 640, 8192};
-  return {2048, 2560, in_dim == 4096 ? 8192u : 4096u};
+// rb: row blocks of all the matrices.  norm: the launch prepares the row through the residual add and RMSNorm; swiglu: it ends in
+// silu(gate) * up.
+static bool preparing_pays(uint32_t ggml_type, uint32_t in_dim, uint32_t rb, bool norm, bool swiglu) {
+  const uint32_t runs = (in_dim + 1023u) / 1024u;
+  const uint64_t work = (uint64_t)rb * runs;
+  if (block_elems_of(ggml_type) == 32) {
+    if (work <= 512u) return true;
+    if (norm && !swiglu) return false;
+    return work >= 640u && work <= 8192u;
+  }
+  return work <= 2048u || (work >= 2560u && work <= (in_dim == 4096u ? 8192u : 4096u));
 }
+
 static bool gemv_prepares(const ogm_ctx *ctx, const Target *tg, size_t n_tg, bool norm, bool swiglu) {
   if (ctx->tune_gemv_prologue == 1 || n_tg == 0 || n_tg > OGM_GEMV_MAX_MATS) return false;
   const uint32_t type = tg[0].w->ggml_type, in_dim = tg[0].w->in_dim;
@@ -566,9 +578,7 @@ static bool gemv_prepares(const ogm_ctx *ctx, const Target *tg, size_t n_tg, boo
   for (size_t i = 0; i < n_tg; i++) rb += ogm_gemv_row_blocks(type, in_dim, tg[i].w->out_dim);
   if (rb == 0 || !ogm_gemv_fused_can(type, in_dim, rb, norm, swiglu, (uint32_t)ctx->tune_wg_waves)) return false;
   if (ctx->tune_gemv_prologue == 2) return true;
-  const uint64_t work = (uint64_t)rb * ((in_dim + 1023u) / 1024u);
-  const PrepareLine line = prepare_line(type, in_dim);
-  return work <= line.to || (work >= line.from && work <= line.last);
+  return preparing_pays(type, in_dim, rb, norm, swiglu);
 }
 
 static OgmGemvArgs prepared_args(ogm_ctx *ctx, const Target *tg, size_t n_tg) {

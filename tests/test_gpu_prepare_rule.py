@@ -1,0 +1,70 @@
+"""Which one-token launches prepare their own rows: the families of shapes that the limit on row blocks times runs of 1024
+inputs alone gets wrong, each on both sides of its own line -- read from a capture of the call, over weights of zero bytes
+(both routes give the same bits; test_gpu_gemv_prologue.py and test_gpu_llama.py compare them)."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import BLOCK, IQ4_NL, IQ4_XS, Q2_K, Q3_K, Q4_0, Q4_K, Q5_0, Q5_1, Q5_K, Q6_K, Q8_0, captured_launches
+
+pytestmark = pytest.mark.gpu
+PREPARED, SEPARATE = ["ogm_gemv_fused_kernel"], ["ogm_quantize_kernel", "ogm_gemv_kernel"]
+
+
+@pytest.fixture(scope="module")
+def be():
+    from orangu_amd import Mi355xBackend
+    b = Mi355xBackend()
+    yield b
+    b.close()
+
+
+@pytest.fixture(scope="module")
+def stream():
+    from orangu_amd import hiprt
+    s = hiprt.Stream()
+    yield s
+    s.destroy()
+
+
+def zeros(be, t, in_dim, out_dim):
+    bytes_, elems = BLOCK[t]
+    return be.upload_raw(np.zeros(out_dim * (in_dim // elems) * bytes_, np.uint8), t, in_dim, out_dim)
+
+
+LETTER = {"ogm_norm_quant_kernel": "n", "ogm_gemv_kernel": "m", "ogm_attn_kernel": "a", "ogm_swiglu_quant_kernel": "s",
+          "ogm_quantize_kernel": "q", "ogm_gemv_fused_pair_kernel": "P"}
+
+
+def decode_launches(be, stream, t, n_embd, n_head, n_kv, hd, n_ff):
+    """The launches of a decode step's one layer, every matrix of one type, as letters: norm, matmul, attention, SwiGLU and
+    quantizer launches small, matmuls that prepare their row F, gate and up that leave silu(gate) * up G."""
+    from orangu_amd import LlamaDecoder
+    shapes = {"wq": (n_embd, n_head * hd), "wk": (n_embd, n_kv * hd), "wv": (n_embd, n_kv * hd), "wo": (n_head * hd, n_embd),
+              "w_gate": (n_embd, n_ff), "w_up": (n_embd, n_ff), "w_down": (n_ff, n_embd)}
+    layer = {k: zeros(be, t, *s) for k, s in shapes.items()}
+    ws = [*layer.values(), zeros(be, t, n_embd, 32)]
+    layer["attn_norm"] = layer["ffn_norm"] = np.ones(n_embd, np.float32)
+    dev = LlamaDecoder(be, n_embd=n_embd, n_head=n_head, n_head_kv=n_kv, head_dim=hd, n_ff=n_ff, n_vocab=32, layers=[layer],
+                       output_norm=np.ones(n_embd, np.float32), output=ws[-1], max_ctx=8, rms_eps=1e-5,
+                       rope_freq_base=10000.0, upload=lambda handle: handle)
+    x, lg, tok = torch.ones(n_embd, device="cuda"), torch.empty(32, device="cuda"), torch.empty(1, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    ran = captured_launches(stream.ptr, lambda: dev.decode_dev(x.data_ptr(), 2, lg.data_ptr(), tok.data_ptr(), stream.ptr))
+    dev.close()
+    for w in ws:
+        be.free_weight(w)
+    assert [k[0] for k in ran[-2:]] == ["ogm_argmax_kernel"] * 2   # behind the last norm and the output matrix
+    return "".join("G" if k[0] == "ogm_gemv_fused_kernel" and "Lb1EEv" in k[1] else LETTER.get(k[0], "F") for k in ran[:-4])
+
+
+# (row blocks of sixteen rows times runs of 1024: up to 512 the launch prepares the normed row, beyond it the norm has a launch
+# of its own; silu(gate) * up, of rows of at most 1024 inputs, beyond it too)
+@pytest.mark.parametrize("t", [Q8_0, Q4_0, Q5_0, Q5_1, IQ4_NL])
+@pytest.mark.parametrize("n_embd,n_head,n_kv,hd,n_ff,want", [
+    (2048, 32, 16, 64, 2048, "FamFsm"), (2048, 32, 32, 64, 2080, "nmamnmsm"), (4096, 32, 8, 128, 4096, "nmamnmsm"),
+    (1024, 16, 8, 64, 8192, "FamGF")])
+def test_norms_before_per_32_matrices(be, stream, t, n_embd, n_head, n_kv, hd, n_ff, want):
+    got = decode_launches(be, stream, t, n_embd, n_head, n_kv, hd, n_ff)
+    print(t, n_embd, n_ff, got, flush=True)
+    assert got == want
