@@ -558,14 +558,22 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
 //   A band above 2048 (512 for the per-32 types) keeps the quantizer launch that calls of these widths have had since prepared
 // launches began, and that the tests expect of them there, though prepared ones lead in it as well (Q4_K 4096 -> 9216, 2304,
 // 7.2 / 5.5, Q6_K 2816 -> 10928, 2049, 7.9 / 7.6, Q8_0 2048 -> 4112, 514, 7.4 / 4.7); it is as narrow as they allow.
+//   Per-32 rows of at most 1024 inputs are one run, which one wave prepares while the others wait: such matmuls lose beyond 48 Mi
+// weights, where the row's last tile is padded beyond 2048 row blocks.  us, separate / prepared: Q8_0 1024 -> 49152 11.5 / 11.4,
+// -> 57344 12.8 / 13.9, -> 126400 24.4 / 28.4, Q4_0 1024 -> 65536 12.9 / 13.6, Q5_1 512 -> 81920 9.7 / 9.5, -> 128000 12.7 / 13.8,
+// IQ4_NL 768 -> 65536 12.5 / 11.9; padded, Q8_0 864 -> 33280 (2080 row blocks) 9.0 / 8.4, -> 44800 10.5 / 10.8, -> 131072 22.3 / 26.3,
+// IQ4_NL 864 -> 33280 9.7 / 9.9.
 // rb: row blocks of all the matrices.  norm: the launch prepares the row through the residual add and RMSNorm; swiglu: it ends in
 // silu(gate) * up.
 static bool preparing_pays(uint32_t ggml_type, uint32_t in_dim, uint32_t rb, bool norm, bool swiglu) {
-  const uint32_t runs = (in_dim + 1023u) / 1024u;
+  const uint32_t runs = (in_dim + 1023u) / 1024u, be = block_elems_of(ggml_type);
   const uint64_t work = (uint64_t)rb * runs;
-  if (block_elems_of(ggml_type) == 32) {
+  const uint32_t R = ogm_tiling_for(in_dim / be, 1).R;
+  const bool whole_tiles = in_dim / be % 4u == 0u;   // no blocks of zeros in a row's last tile
+  if (be == 32) {
     if (work <= 512u) return true;
     if (norm && !swiglu) return false;
+    if (runs == 1u && !swiglu && (whole_tiles ? (uint64_t)rb * R * in_dim > 48u << 20 : rb > 2048u)) return false;
     return work >= 640u && work <= 8192u;
   }
   return work <= 2048u || (work >= 2560u && work <= (in_dim == 4096u ? 8192u : 4096u));

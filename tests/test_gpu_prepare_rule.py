@@ -32,6 +32,27 @@ def zeros(be, t, in_dim, out_dim):
     return be.upload_raw(np.zeros(out_dim * (in_dim // elems) * bytes_, np.uint8), t, in_dim, out_dim)
 
 
+def check(be, stream, t, in_dim, out_dim, prepared):
+    w = zeros(be, t, in_dim, out_dim)
+    x, y = torch.ones(in_dim, device="cuda"), torch.empty(out_dim, device="cuda")
+    torch.cuda.synchronize()
+    be.matmul_dev(w, x.data_ptr(), 1, y.data_ptr(), True, stream.ptr)   # (its scratch is there before the capture)
+    stream.synchronize()
+    ran = captured_launches(stream.ptr, lambda: be.matmul_dev(w, x.data_ptr(), 1, y.data_ptr(), True, stream.ptr))
+    be.free_weight(w)
+    print(t, in_dim, out_dim, [k[0] for k in ran], flush=True)
+    assert [k[0] for k in ran] == (PREPARED if prepared else SEPARATE)
+
+
+# (48 Mi weights of rows without padded tiles, 2048 row blocks of sixteen rows with)
+@pytest.mark.parametrize("t,in_dim,out_dim,prepared", [
+    (Q8_0, 1024, 49152, True), (Q8_0, 1024, 49153, False), (Q4_0, 512, 98304, True), (Q4_0, 512, 98305, False),
+    (IQ4_NL, 768, 65536, True), (IQ4_NL, 768, 65537, False), (Q5_1, 864, 32768, True), (Q5_1, 864, 32769, False),
+    (Q8_0, 1056, 32768, True), (Q5_0, 256, 131072, True)])
+def test_one_run_of_per_32_blocks(be, stream, t, in_dim, out_dim, prepared):
+    check(be, stream, t, in_dim, out_dim, prepared)
+
+
 LETTER = {"ogm_norm_quant_kernel": "n", "ogm_gemv_kernel": "m", "ogm_attn_kernel": "a", "ogm_swiglu_quant_kernel": "s",
           "ogm_quantize_kernel": "q", "ogm_gemv_fused_pair_kernel": "P"}
 
