@@ -563,6 +563,10 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
 // -> 57344 12.8 / 13.9, -> 126400 24.4 / 28.4, Q4_0 1024 -> 65536 12.9 / 13.6, Q5_1 512 -> 81920 9.7 / 9.5, -> 128000 12.7 / 13.8,
 // IQ4_NL 768 -> 65536 12.5 / 11.9; padded, Q8_0 864 -> 33280 (2080 row blocks) 9.0 / 8.4, -> 44800 10.5 / 10.8, -> 131072 22.3 / 26.3,
 // IQ4_NL 864 -> 33280 9.7 / 9.9.
+//   K-quant rows of more than 8192 inputs are two runs a wave: such matmuls lead while a compute unit has one workgroup.  us, separate /
+// prepared at 256 row blocks or just below and above: Q4_K 12288 8.5 / 7.7, 10.1 / 10.8, 14336 8.7 / 7.7, 10.8 / 10.3, 10240 (260)
+// 9.0 / 9.2, Q6_K 11264 10.6 / 9.3, 12.9 / 12.9, 13312 11.2 / 10.3, 14.7 / 15.3, IQ4_XS 11264 11.3 / 10.5, 14.4 / 15.3, Q3_K 9728 (260)
+// 11.1 / 11.8, Q5_K 12288 9.0 / 8.5, 12.1 / 12.9; 9216 inputs level above (Q4_K 8.8 / 8.8, Q3_K 10.8 / 10.5).
 // rb: row blocks of all the matrices.  norm: the launch prepares the row through the residual add and RMSNorm; swiglu: it ends in
 // silu(gate) * up.
 static bool preparing_pays(uint32_t ggml_type, uint32_t in_dim, uint32_t rb, bool norm, bool swiglu) {
@@ -576,7 +580,9 @@ static bool preparing_pays(uint32_t ggml_type, uint32_t in_dim, uint32_t rb, boo
     if (runs == 1u && !swiglu && (whole_tiles ? (uint64_t)rb * R * in_dim > 48u << 20 : rb > 2048u)) return false;
     return work >= 640u && work <= 8192u;
   }
-  return work <= 2048u || (work >= 2560u && work <= (in_dim == 4096u ? 8192u : 4096u));
+  if (work <= 2048u) return true;
+  if (runs > 8u && rb > 256u) return false;
+  return work >= 2560u && work <= (in_dim == 4096u ? 8192u : 4096u);
 }
 
 static bool gemv_prepares(const ogm_ctx *ctx, const Target *tg, size_t n_tg, bool norm, bool swiglu) {

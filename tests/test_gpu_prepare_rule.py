@@ -53,6 +53,14 @@ def test_one_run_of_per_32_blocks(be, stream, t, in_dim, out_dim, prepared):
     check(be, stream, t, in_dim, out_dim, prepared)
 
 
+# (two runs a wave: 256 row blocks of sixteen rows)
+@pytest.mark.parametrize("t", [Q4_K, Q6_K, IQ4_XS])
+@pytest.mark.parametrize("in_dim,prepared_to", [(10240, 4096), (11008, 4096), (14336, 4096)])
+def test_two_runs_a_wave(be, stream, t, in_dim, prepared_to):
+    check(be, stream, t, in_dim, prepared_to, True)
+    check(be, stream, t, in_dim, prepared_to + 1, False)
+
+
 LETTER = {"ogm_norm_quant_kernel": "n", "ogm_gemv_kernel": "m", "ogm_attn_kernel": "a", "ogm_swiglu_quant_kernel": "s",
           "ogm_quantize_kernel": "q", "ogm_gemv_fused_pair_kernel": "P"}
 
