@@ -567,21 +567,33 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
 // prepared at 256 row blocks or just below and above: Q4_K 12288 8.5 / 7.7, 10.1 / 10.8, 14336 8.7 / 7.7, 10.8 / 10.3, 10240 (260)
 // 9.0 / 9.2, Q6_K 11264 10.6 / 9.3, 12.9 / 12.9, 13312 11.2 / 10.3, 14.7 / 15.3, IQ4_XS 11264 11.3 / 10.5, 14.4 / 15.3, Q3_K 9728 (260)
 // 11.1 / 11.8, Q5_K 12288 9.0 / 8.5, 12.1 / 12.9; 9216 inputs level above (Q4_K 8.8 / 8.8, Q3_K 10.8 / 10.5).
+//   Rows of three tiles make workgroups of six waves, two row blocks each, of which 512 run at once.  Beyond, us, separate / prepared:
+// 3072 inputs, IQ4_XS -> 16448 10.4 / 11.7, -> 21328 11.7 / 12.8, Q3_K -> 18656 9.1 / 9.8, Q6_K -> 17408 10.3 / 10.4, -> 21328 11.4 / 10.8,
+// Q4_K 8.8 / 8.0, Q5_K 10.1 / 9.5, Q2_K 8.7 / 7.3 (IQ4_XS -> 16000 still 10.3 / 9.2); 1536, IQ4_XS -> 34816 10.7 / 12.1, Q3_K 9.3 / 9.8,
+// Q6_K -> 52800 12.7 / 15.1, Q4_K 9.5 / 9.3, Q5_K -> 65536 12.9 / 12.3; 768 (rows of 64 a block), Q4_K -> 131840 10.7 / 10.8, Q5_K 12.8 /
+// 13.2, Q6_K 14.8 / 17.1.  Two layers of a decode step whose gate and up are such a launch: 3072 / 8704 IQ4_XS 103.2 / 104.5, / 10752
+// 107.5 / 110.9, Q5_K / 8704 94.7 / 91.3, Q6_K 99.5 / 97.0, / 10752 level; 1536 / 20480 IQ4_XS 109.6 / 113.6, Q2_K 85.3 / 87.1, the others
+// level.
 // rb: row blocks of all the matrices.  norm: the launch prepares the row through the residual add and RMSNorm; swiglu: it ends in
 // silu(gate) * up.
 static bool preparing_pays(uint32_t ggml_type, uint32_t in_dim, uint32_t rb, bool norm, bool swiglu) {
   const uint32_t runs = (in_dim + 1023u) / 1024u, be = block_elems_of(ggml_type);
   const uint64_t work = (uint64_t)rb * runs;
-  const uint32_t R = ogm_tiling_for(in_dim / be, 1).R;
+  const OgmTiling tl = ogm_tiling_for(in_dim / be, 1);
   const bool whole_tiles = in_dim / be % 4u == 0u;   // no blocks of zeros in a row's last tile
   if (be == 32) {
     if (work <= 512u) return true;
     if (norm && !swiglu) return false;
-    if (runs == 1u && !swiglu && (whole_tiles ? (uint64_t)rb * R * in_dim > 48u << 20 : rb > 2048u)) return false;
+    if (runs == 1u && !swiglu && (whole_tiles ? (uint64_t)rb * tl.R * in_dim > 48u << 20 : rb > 2048u)) return false;
     return work >= 640u && work <= 8192u;
   }
   if (work <= 2048u) return true;
   if (runs > 8u && rb > 256u) return false;
+  if (tl.nct == 3u && rb > 1024u) {
+    if (norm) return swiglu && tl.C == 4u && ggml_type != OGM_IQ4_XS && work <= 4096u;
+    const bool light = ggml_type == OGM_Q4_K || ggml_type == OGM_Q5_K || ggml_type == OGM_Q2_K || (ggml_type == OGM_Q6_K && tl.C == 4u);
+    if (!light || tl.C == 1u) return false;
+  }
   return work >= 2560u && work <= (in_dim == 4096u ? 8192u : 4096u);
 }
 

@@ -61,13 +61,23 @@ def test_two_runs_a_wave(be, stream, t, in_dim, prepared_to):
     check(be, stream, t, in_dim, prepared_to + 1, False)
 
 
+# (rows of three tiles, up to two row blocks in each of 512 workgroups; by type beyond)
+@pytest.mark.parametrize("t,in_dim,out_dim,prepared", [
+    (IQ4_XS, 3072, 16384, True), (IQ4_XS, 3072, 16385, False), (Q3_K, 2816, 16384, True), (Q3_K, 2816, 16385, False),
+    (Q6_K, 3072, 16385, True), (Q4_K, 3072, 21840, True), (Q2_K, 3072, 16385, True), (IQ4_XS, 1536, 32768, True),
+    (IQ4_XS, 1536, 40992, False), (Q6_K, 1536, 40992, False), (Q5_K, 1536, 40992, True), (Q4_K, 768, 131072, True),
+    (Q4_K, 768, 163904, False)])
+def test_three_tiles(be, stream, t, in_dim, out_dim, prepared):
+    check(be, stream, t, in_dim, out_dim, prepared)
+
+
 LETTER = {"ogm_norm_quant_kernel": "n", "ogm_gemv_kernel": "m", "ogm_attn_kernel": "a", "ogm_swiglu_quant_kernel": "s",
-          "ogm_quantize_kernel": "q", "ogm_gemv_fused_pair_kernel": "P"}
+          "ogm_attn_combine_quant_kernel": "c", "ogm_quantize_kernel": "q", "ogm_gemv_fused_kernel": "F"}
 
 
 def decode_launches(be, stream, t, n_embd, n_head, n_kv, hd, n_ff):
-    """The launches of a decode step's one layer, every matrix of one type, as letters: norm, matmul, attention, SwiGLU and
-    quantizer launches small, matmuls that prepare their row F, gate and up that leave silu(gate) * up G."""
+    """The launches of a decode step's one layer, every matrix of one type, as letters: norm, matmul, attention (and its merge),
+    SwiGLU and quantizer launches small, matmuls that prepare their row F, gate and up that leave silu(gate) * up G."""
     from orangu_amd import LlamaDecoder
     shapes = {"wq": (n_embd, n_head * hd), "wk": (n_embd, n_kv * hd), "wv": (n_embd, n_kv * hd), "wo": (n_head * hd, n_embd),
               "w_gate": (n_embd, n_ff), "w_up": (n_embd, n_ff), "w_down": (n_ff, n_embd)}
@@ -84,7 +94,7 @@ def decode_launches(be, stream, t, n_embd, n_head, n_kv, hd, n_ff):
     for w in ws:
         be.free_weight(w)
     assert [k[0] for k in ran[-2:]] == ["ogm_argmax_kernel"] * 2   # behind the last norm and the output matrix
-    return "".join("G" if k[0] == "ogm_gemv_fused_kernel" and "Lb1EEv" in k[1] else LETTER.get(k[0], "F") for k in ran[:-4])
+    return "".join("G" if k[0] == "ogm_gemv_fused_kernel" and "Lb1EEv" in k[1] else LETTER[k[0]] for k in ran[:-4])
 
 
 # (row blocks of sixteen rows times runs of 1024: up to 512 the launch prepares the normed row, beyond it the norm has a launch
@@ -94,6 +104,15 @@ def decode_launches(be, stream, t, n_embd, n_head, n_kv, hd, n_ff):
     (2048, 32, 16, 64, 2048, "FamFsm"), (2048, 32, 32, 64, 2080, "nmamnmsm"), (4096, 32, 8, 128, 4096, "nmamnmsm"),
     (1024, 16, 8, 64, 8192, "FamGF")])
 def test_norms_before_per_32_matrices(be, stream, t, n_embd, n_head, n_kv, hd, n_ff, want):
+    got = decode_launches(be, stream, t, n_embd, n_head, n_kv, hd, n_ff)
+    print(t, n_embd, n_ff, got, flush=True)
+    assert got == want
+
+
+@pytest.mark.parametrize("t,n_embd,n_head,n_kv,hd,n_ff,want", [
+    (IQ4_XS, 3072, 24, 8, 128, 8192, "FacmGF"), (IQ4_XS, 3072, 24, 8, 128, 8704, "Facmnmsm"), (Q5_K, 3072, 24, 8, 128, 8704, "FacmGF"),
+    (Q2_K, 1536, 24, 8, 64, 20480, "Facmnmsm"), (Q4_K, 1536, 24, 8, 64, 16384, "FacmGF")])
+def test_three_tiles_gate_and_up(be, stream, t, n_embd, n_head, n_kv, hd, n_ff, want):
     got = decode_launches(be, stream, t, n_embd, n_head, n_kv, hd, n_ff)
     print(t, n_embd, n_ff, got, flush=True)
     assert got == want
