@@ -574,6 +574,10 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
 // 13.2, Q6_K 14.8 / 17.1.  Two layers of a decode step whose gate and up are such a launch: 3072 / 8704 IQ4_XS 103.2 / 104.5, / 10752
 // 107.5 / 110.9, Q5_K / 8704 94.7 / 91.3, Q6_K 99.5 / 97.0, / 10752 level; 1536 / 20480 IQ4_XS 109.6 / 113.6, Q2_K 85.3 / 87.1, the others
 // level.
+//   Gate and up of 4096 inputs: 512 workgroups of eight waves run at once, and a second round less than a quarter full costs the heavier
+// types more than the launches that it saves.  Two layers of a decode step, us, separate / prepared, at 8448, 9216 and 10240 rows each:
+// Q5_K 97.2 / 99.7, 97.8 / 99.6, 100.5 / 100.4, Q6_K 104.7 / 106.9, 105.8 / 107.2, 108.8 / 108.1, IQ4_XS 105.6 / 107.1, 106.7 / 108.1, 111.8 /
+// 109.3; Q3_K level, Q4_K and Q2_K ahead throughout.
 // rb: row blocks of all the matrices.  norm: the launch prepares the row through the residual add and RMSNorm; swiglu: it ends in
 // silu(gate) * up.
 static bool preparing_pays(uint32_t ggml_type, uint32_t in_dim, uint32_t rb, bool norm, bool swiglu) {
@@ -593,6 +597,10 @@ static bool preparing_pays(uint32_t ggml_type, uint32_t in_dim, uint32_t rb, boo
     if (norm) return swiglu && tl.C == 4u && ggml_type != OGM_IQ4_XS && work <= 4096u;
     const bool light = ggml_type == OGM_Q4_K || ggml_type == OGM_Q5_K || ggml_type == OGM_Q2_K || (ggml_type == OGM_Q6_K && tl.C == 4u);
     if (!light || tl.C == 1u) return false;
+  }
+  if (in_dim == 4096u && norm && work > 4096u) {
+    const bool light = ggml_type == OGM_Q4_K || ggml_type == OGM_Q3_K || ggml_type == OGM_Q2_K;
+    return swiglu && (light || work >= 5120u) && work <= 8192u;
   }
   return work >= 2560u && work <= (in_dim == 4096u ? 8192u : 4096u);
 }

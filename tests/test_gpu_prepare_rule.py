@@ -116,3 +116,13 @@ def test_three_tiles_gate_and_up(be, stream, t, n_embd, n_head, n_kv, hd, n_ff, 
     got = decode_launches(be, stream, t, n_embd, n_head, n_kv, hd, n_ff)
     print(t, n_embd, n_ff, got, flush=True)
     assert got == want
+
+
+# (512 workgroups run at once; the heavier types' second round from a quarter of it on)
+@pytest.mark.parametrize("t", [Q4_K, Q2_K, Q3_K, Q5_K, Q6_K, IQ4_XS])
+def test_gate_and_up_of_4096_inputs(be, stream, t):
+    light = t in (Q4_K, Q2_K, Q3_K)
+    for n_ff, prepared in ((8192, True), (8448, light), (9984, light), (10240, True), (14336, True), (16384, True), (16640, False)):
+        got = decode_launches(be, stream, t, 4096, 32, 8, 128, n_ff)
+        print(t, n_ff, got, flush=True)
+        assert got.startswith("FamG") if prepared else got == "Famnmsm", n_ff
