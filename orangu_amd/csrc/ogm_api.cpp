@@ -540,14 +540,14 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
 
 // Whether a one-token launch over these matrices (one type and in_dim) prepares its own activations: where the work
 // that every workgroup repeats -- row blocks times runs of 1024 inputs -- costs less than the launch it saves.  Measured,
-// whole calls, us, separate / prepared, with that work: Q4_K 4096 -> 8192 (2048) 6.1 / 4.4, 2048 -> 16384 6.8 / 5.4, 5120 ->
-// 8192 (2560) 7.0 / 6.5, 4096 -> 14336 (3584) 7.3 / 5.7, 14336 -> 4096 (3584) 8.1 / 7.7, 8192 -> 8192 (4096) 8.5 / 7.9, 5120 -> 14336
+// whole calls, us, separate / prepared, with that work: Q4_K 4096 -> 8192 (2048) 6.1 / 4.4, 2048 -> 16384 6.8 / 5.4, 4096 ->
+// 9216 (2304) 7.2 / 5.5, 5120 -> 8192 (2560) 7.0 / 6.5, 4096 -> 14336 (3584) 7.3 / 5.7, 14336 -> 4096 (3584) 8.1 / 7.7, 8192 -> 8192 (4096) 8.5 / 7.9, 5120 -> 14336
 // (4480) 9.7 / 9.5, 2816 -> 28672 (5376) 9.5 / 9.9, 8192 -> 14336 (7168) level, 11008 -> 8192 (5632) 10.3 / 11.4; Q6_K 14336 ->
 // 4096 10.3 / 9.6, 2816 -> 28672 13.7 / 16.9; Q5_K 8192 -> 8192 10.1 / 9.6; Q3_K 14336 -> 4096 9.6 / 8.7; IQ4_XS the same 11.4 /
 // 10.7: the line of the K-quants is 4096, eight a compute unit twice over.  Rows of 4096 inputs, whose length the kernel has as a
 // constant and whose waves have one tile each, lead to 8192: Q4_K -> 28672 (7168) 11.6 / 10.8, -> 32768 12.8 / 11.6, Q5_K 16.3 / 15.2,
 // Q6_K 19.0 / 18.2, IQ4_XS -> 28672 16.1 / 15.3.  The per-32 types, whose quantizer launch has more to do, lead to 8192 at any
-// length: Q8_0 4096 -> 4096 (1024) 7.5 / 4.8, -> 28672 (7168) 21.9 / 20.6, 8192 -> 14336 24.7 / 23.7, 14336 -> 8192 27.0 / 25.6, 14336 ->
+// length: Q8_0 2048 -> 4112 (514) 7.4 / 4.7, 4096 -> 4096 (1024) 7.5 / 4.8, -> 28672 (7168) 21.9 / 20.6, 8192 -> 14336 24.7 / 23.7, 14336 -> 8192 27.0 / 25.6, 14336 ->
 // 14336 (12544) level; Q4_0 4096 -> 28672 17.1 / 16.2, Q5_1 19.8 / 18.7.
 //   A norm in front of per-32 matrices is as short as one in front of K-quants, and the launch behind it has more rows' scales
 // to make again in every workgroup: beyond 512 such launches that end in their products lose.  Two layers of a decode step at
@@ -555,9 +555,6 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
 // 14336 131 / 154, 4096 / 4096 87.7 / 93.1, 2048 / 8192 90.0 / 93.5, Q5_1 4096 / 14336 138 / 162; ahead in a few (Q8_0 3072 / 4096
 // 94.7 / 92.9).  Those that end in silu(gate) * up (rows of at most 1024 inputs) gain: Q8_0 1024 / 32768 159 / 156, 1024 / 49152
 // 213 / 207.
-//   A band above 2048 (512 for the per-32 types) keeps the quantizer launch that calls of these widths have had since prepared
-// launches began, and that the tests expect of them there, though prepared ones lead in it as well (Q4_K 4096 -> 9216, 2304,
-// 7.2 / 5.5, Q6_K 2816 -> 10928, 2049, 7.9 / 7.6, Q8_0 2048 -> 4112, 514, 7.4 / 4.7); it is as narrow as they allow.
 //   Per-32 rows of at most 1024 inputs are one run, which one wave prepares while the others wait: such matmuls lose beyond 48 Mi
 // weights, where the row's last tile is padded beyond 2048 row blocks.  us, separate / prepared: Q8_0 1024 -> 49152 11.5 / 11.4,
 // -> 57344 12.8 / 13.9, -> 126400 24.4 / 28.4, Q4_0 1024 -> 65536 12.9 / 13.6, Q5_1 512 -> 81920 9.7 / 9.5, -> 128000 12.7 / 13.8,
@@ -589,7 +586,7 @@ static bool preparing_pays(uint32_t ggml_type, uint32_t in_dim, uint32_t rb, boo
     if (work <= 512u) return true;
     if (norm && !swiglu) return false;
     if (runs == 1u && !swiglu && (whole_tiles ? (uint64_t)rb * tl.R * in_dim > 48u << 20 : rb > 2048u)) return false;
-    return work >= 640u && work <= 8192u;
+    return work <= 8192u;
   }
   if (work <= 2048u) return true;
   if (runs > 8u && rb > 256u) return false;
@@ -602,7 +599,7 @@ static bool preparing_pays(uint32_t ggml_type, uint32_t in_dim, uint32_t rb, boo
     const bool light = ggml_type == OGM_Q4_K || ggml_type == OGM_Q3_K || ggml_type == OGM_Q2_K;
     return swiglu && (light || work >= 5120u) && work <= 8192u;
   }
-  return work >= 2560u && work <= (in_dim == 4096u ? 8192u : 4096u);
+  return work <= (in_dim == 4096u ? 8192u : 4096u);
 }
 
 static bool gemv_prepares(const ogm_ctx *ctx, const Target *tg, size_t n_tg, bool norm, bool swiglu) {
@@ -1847,6 +1844,8 @@ static int llama_norm_matmul(ogm_ctx *ctx, ogm_llama *m, DecodeRow &row, const f
   // layer, one launch / prepared q and k, then a launch for v / norm and two launches: 4096 wide, q/k 2048 + v 1024
   // 33.5 / 34.9 / 40.3; 3072 wide, 1536 + 768 31.7 / 33.7 / 39.9; 5120 wide, 1920 + 320 43.9 / 47.9 / 50.5; gate 2048 + up
   // 2048 at 4096 wide 39.9 / 39.9 / 41.7, at 2048 wide 40.7 / 40.2 / 42.1.
+  // Two layers, one of them so, one launch / norm and two launches, at larger shares: 4096 wide, 13312 + 1024 85.7 / 90.4; 6144 wide,
+  // 7168 + 1024 93.5 / 99.1; 5120 wide, 10240 + 5120 level.
   Target tg2[OGM_GEMV_MAX_MATS];
   bool both = e < n && n - e <= OGM_GEMV_MAX_MATS && ogm_gemv_fused_pair_can(ws[0]->ggml_type, ws[e]->ggml_type, ws[0]->in_dim, (uint32_t)ctx->tune_wg_waves);
   for (size_t i = e; both && i < n; i++) {

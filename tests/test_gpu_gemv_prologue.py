@@ -150,8 +150,8 @@ def test_decode_steps_give_the_same_bits(be, types, n_embd, n_ff, layer):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
-# (each type's share of q/k + v within the line of 2048 row blocks x runs, together 3072; q/k above it)
-@pytest.mark.parametrize("n_head,n_kv,layer,wgs", [(32, 32, "PAGSF", 512 + 256), (64, 8, "NGGAGSF", 512 + 64)])
+# (each type's share of q/k + v within the line of 4096 row blocks x runs; q/k above it)
+@pytest.mark.parametrize("n_head,n_kv,layer,wgs", [(32, 32, "PAGSF", 512 + 256), (64, 8, "PAGSF", 576 + 64), (128, 8, "NGGAGSF", 1024 + 64)])
 def test_two_types_at_the_line(be, n_head, n_kv, layer, wgs):
     from orangu_amd import hiprt
     _, dev, rng = build(be, n_embd=4096, n_head=n_head, n_kv=n_kv, hd=128, n_ff=256, n_vocab=300, n_layer=1,

@@ -101,10 +101,13 @@ def test_prepared_rows_use_no_private_memory(be, stream, t):
         be.set_tuning("gemv_prologue", 0)
 
 
-# (row blocks x runs of 1024 up to 2048, 512 for the per-32 types; row blocks of 16 rows, of 64 at 7 blocks a row)
+# (row blocks x runs of 1024 up to 4096, 8192 at 4096 inputs and for the per-32 types; row blocks of 16 rows, of 64 at 7 blocks a
+# row; the shapes that end earlier are in test_gpu_prepare_rule.py)
 @pytest.mark.parametrize("t,in_dim,out_dim,prepared", [
-    (Q4_K, 4096, 512 * 16, True), (Q4_K, 4096, 512 * 16 + 1, False), (Q6_K, 2816, 682 * 16, True), (Q6_K, 2816, 682 * 16 + 1, False),
-    (Q4_K, 1792, 1024 * 64, True), (Q8_0, 2048, 256 * 16, True), (Q8_0, 2048, 256 * 16 + 1, False)])
+    (Q4_K, 4096, 512 * 16, True), (Q4_K, 4096, 512 * 16 + 1, True), (Q4_K, 4096, 2048 * 16, True), (Q4_K, 4096, 2048 * 16 + 1, False),
+    (Q6_K, 2816, 682 * 16, True), (Q6_K, 2816, 682 * 16 + 1, True), (Q6_K, 2816, 1365 * 16, True), (Q6_K, 2816, 1365 * 16 + 1, False),
+    (Q4_K, 1792, 1024 * 64, True), (Q4_K, 1792, 2048 * 64, True), (Q4_K, 1792, 2048 * 64 + 1, False),
+    (Q8_0, 2048, 256 * 16, True), (Q8_0, 2048, 256 * 16 + 1, True), (Q8_0, 2048, 4096 * 16, True), (Q8_0, 2048, 4096 * 16 + 1, False)])
 def test_the_line(be, stream, t, in_dim, out_dim, prepared):
     bytes_, elems = BLOCK[t]
     raw = np.zeros(out_dim * (in_dim // elems) * bytes_, np.uint8)
