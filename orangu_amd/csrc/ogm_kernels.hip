@@ -1204,9 +1204,9 @@ __device__ __forceinline__ T *of_matrix(T *const (&v)[OGM_GEMV_MAX_MATS], uint32
 
 // NQ: runs of 1024 elements a wave prepares.  bid: the workgroup's number among those of its type; leads: it stores the
 // quantized row and the residual stream.
-// NB 2 (SWIGLU): a second row block of both matrices, gridDim.x after the first.  Where one block a workgroup is more waves than
-// the device holds at once (twenty a compute unit at these registers) a second round of workgroups pays the whole chain again --
-// its start, the trip for the row, the preparation; here its weights are under way over the first block's sum instead.  8B shapes
+// NB 2 (SWIGLU): a second row block of both matrices, gridDim.x after the first.  Where one block a workgroup is more
+// workgroups than run at once, a second round of them pays the whole chain again -- its start, the trip for the row, the
+// preparation; here its weights are under way over the first block's sum instead.  (Which launches: launch_fused_t.)  8B shapes
 // (4096 -> 2 x 14336: 896 workgroups of eight waves, now 448), a step of 8 layers at 300 / 2048 / 16000 positions 447.7 / 460.1 /
 // 567.5 -> 436.0 / 448.6 / 556.0 us.  Not for launches without SwiGLU: 4096 -> 28672, two teams of different row blocks, 10.7 -> 11.9.
 template <class F, int UPR, int PRE, int NQ, int NB, bool SWIGLU>
@@ -1724,10 +1724,24 @@ static hipError_t launch_fused_t(const OgmGemvArgs &a, const OgmGemvSrc &src, hi
   constexpr int HOT = K ? 16 : 128;   // rows of 4096
 #define OGM_FUSED(UPR, PRE, NQ, SW) hipLaunchKernelGGL((ogm_gemv_fused_kernel<F, UPR, PRE, NQ, 1, SW>), g, b, f.lds, stream, fp)
   if (norm && src.swiglu) {
-    // two row blocks a workgroup beyond the waves the device holds at once, for the K-quants' rows of 4096 (see the kernel)
+    // Two row blocks a workgroup where a compute unit gets no more of them that way than with one each, and one each are more
+    // workgroups than run at once (eight waves of 82 to 118 registers: two a compute unit, 512): from 769 to 1024 row blocks.  Two
+    // layers of a decode step, 4096 / n_ff, us, one block / two:
+    //            10752 (672)     12288 (768)     12800 (800)     14336 (896)     16384 (1024)
+    //   Q4_K     92.8 /  93.5    92.6 /  91.2    95.3 /  92.1    95.1 /  92.3    99.6 /  97.0
+    //   Q5_K     97.8 / 100.1   100.8 / 101.2   105.6 / 102.1   105.5 / 102.3   111.3 / 107.8
+    //   Q6_K    105.5 / 110.0   109.1 / 111.6   115.6 / 112.7   115.1 / 112.9   121.8 / 120.0
+    //   Q3_K     90.5 /  94.0    92.0 /  95.0    96.7 /  95.5    95.5 /  94.4    99.4 /  98.4
+    //   Q2_K     79.4 /  82.6    81.4 /  81.8    86.8 /  82.1    85.7 /  80.7    88.5 /  86.7
+    //   IQ4_XS  106.4 / 108.4   108.6 / 109.2   113.9 / 110.0   113.7 / 109.8   117.9 / 116.7
+    // (513 to 640: 3 to 7 % of the step slower with two.)  Q4_K already where one each nearly fill the third place of every compute
+    // unit: 11776 (736) 94.6 / 95.6, 12032 (752) 97.1 / 96.0.  Only for rows of 4096 inputs: launches of other lengths end, at 4096 row
+    // blocks x runs, with what runs at once or, three tiles a row, a third more.
     const dim3 g2((g.x + 1u) / 2u);
     const size_t lds2 = f.lds + (size_t)f.teams * p.upr * (64u / p.C) * 4u;
-    if (K && p.upr == HOT && g.x * f.team_waves * f.teams > 20u * 256u && lds2 <= OGM_LDS_UNASKED)
+    const uint32_t waves = f.team_waves * f.teams, at_once = 256u * (waves < 16u ? 16u / waves : 1u);
+    const bool no_more = 2u * ((g2.x + 255u) / 256u) <= (g.x + 255u) / 256u || (a.ggml_type == OGM_Q4_K && g.x > 744u && g.x <= 768u);
+    if (K && p.upr == HOT && g.x > at_once && no_more && lds2 <= OGM_LDS_UNASKED)
       hipLaunchKernelGGL((ogm_gemv_fused_kernel<F, HOT, 2, 1, K ? 2 : 1, true>), g2, b, lds2, stream, fp);
     else if (p.upr == HOT) OGM_FUSED(HOT, 2, 1, true);
     else OGM_FUSED(0, 2, 1, true);

@@ -1,11 +1,11 @@
-"""Gate and up of a decode step in one launch, two row blocks a workgroup: from the first size that takes it (641 and more row
-blocks of sixteen rows at 4096 inputs) against the last that doesn't, with a down projection per 32 (10272 rows) and per 256, for
+"""Gate and up of a decode step in one launch, two row blocks a workgroup: from the first size that takes it (769 and more row
+blocks of sixteen rows at 4096 inputs, Q4_K 745) against the last that doesn't, with a down projection per 32 (12320 rows) and per 256, for
 each K-quant -- the bits of the step whose norm, products and SwiGLU are launches of their own, and the workgroups launched."""
 import numpy as np
 import pytest
 import torch
 
-from helpers import IQ4_XS, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, captured_launches
+from helpers import IQ4_XS, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, captured_launches
 from test_gpu_llama import build, f32
 
 pytestmark = pytest.mark.gpu
@@ -19,9 +19,10 @@ def be():
     b.close()
 
 
-@pytest.mark.parametrize("gate,down,n_ff,workgroups", [(Q4_K, Q6_K, 10240, 640), (Q4_K, Q8_0, 10272, 321), (Q4_K, Q4_K, 14336, 448),
-                                                       (Q5_K, Q8_0, 10272, 321), (Q6_K, Q6_K, 10496, 328), (Q3_K, Q8_0, 10304, 322),
-                                                       (IQ4_XS, Q6_K, 10496, 328)])
+@pytest.mark.parametrize("gate,down,n_ff,workgroups", [(Q4_K, Q6_K, 10240, 640), (Q4_K, Q8_0, 10272, 642), (Q6_K, Q6_K, 10496, 656),
+                                                       (Q4_K, Q6_K, 11776, 736), (Q4_K, Q6_K, 12288, 384), (Q6_K, Q6_K, 12288, 768), (Q4_K, Q4_K, 14336, 448),
+                                                       (Q5_K, Q8_0, 12320, 385), (Q6_K, Q6_K, 12544, 392), (Q3_K, Q8_0, 12352, 386),
+                                                       (IQ4_XS, Q6_K, 12544, 392), (Q2_K, Q6_K, 16384, 512)])
 def test_two_row_blocks(be, gate, down, n_ff, workgroups):
     from orangu_amd import hiprt
     _, dev, rng = build(be, n_embd=4096, n_head=4, n_kv=2, hd=64, n_ff=n_ff, n_vocab=320, n_layer=2, types=(gate, gate, down, Q8_0),
