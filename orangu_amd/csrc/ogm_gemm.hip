@@ -3191,6 +3191,28 @@ static uint32_t gemm_plane_wgs(const OgmGemmArgs &a, uint32_t rows) {
   return (a.n_tokens + GD_TOK - 1u) / GD_TOK * tiles;
 }
 
+// Whether a Q4_K / Q5_K launch of two token tiles (129 to 256 tokens) over rows of 4096 inputs and more is the small-batch kernel's
+// although 64-row tiles over planes could take it: that kernel's time goes by rounds of its workgroups of 32 rows x 32 tokens over
+// the compute units, the plane kernel's hardly at all.  Whole calls, us, small-batch / 64-row tiles:
+//   three rounds   4096 -> 4096 at 192 tokens 24.4 / 27.8 (Q5_K 26.0 / 27.8), 11008 -> 4096 50.4 / 61.2 (54.6 / 61.1), 14336 -> 4096
+//                  60.4 / 77.3 (66.1 / 77.9), 5120 -> 4608 at 160 29.2 / 31.9 (31.5 / 32.0)
+//   four           14336 -> 4096 at 208 / 256 75.1 / 77.6, 73.0 / 80.1 (Q5_K 81.7 / 78.1, 80.3 / 80.2), 14336 -> 5120 at 160 71.7 / 77.1
+//                  (79.4 / 77.9), 11008 -> 4096 at 208 / 256 61.6 / 61.6, 59.7 / 62.8 (67.0 / 61.5), 8192 -> 5000 at 192 45.7 / 47.8 (50.3 /
+//                  47.7), 6144 -> 6144 at 160 37.1 / 37.6 (40.5 / 37.5), 5120 -> 4608 at 192 32.8 / 32.2, 4096 -> 4096 at 256 28.1 / 28.4
+//                  (30.1 / 28.3), 2048 -> 5120 at 192 18.5 / 18.0
+//   five           14336 -> 5120 at 256 88.2 / 80.4, 8192 -> 5000 55.5 / 48.8, 8192 -> 8192 at 160 56.6 / 48.3
+// so three for both types and four for Q4_K from 6144 inputs on.  (The medium-batch kernel is behind both: 8192 -> 5000 at 160 62.5.)
+static bool gemm_small_leads(const OgmGemmArgs &a) {
+  const uint32_t nsb = a.in_dim / 256;
+  if ((a.ggml_type != OGM_Q4_K && a.ggml_type != OGM_Q5_K) || a.n_tokens <= GD_TOK || a.n_tokens > 2u * GD_TOK || nsb < 16u ||
+      a.small_max_tokens != 0u || a.interleave != 0u || a.medium == 2u || a.one_pass != 0u)
+    return false;
+  uint64_t blocks = (a.out_dim + 31u) / 32u;
+  for (uint32_t m = 0; m < a.n_extra; m++) blocks += (a.extra_out_dim[m] + 31u) / 32u;
+  const uint64_t rounds = (blocks * ((a.n_tokens + 31u) / 32u) + 255u) / 256u;
+  return rounds <= (a.ggml_type == OGM_Q4_K && nsb >= 24u ? 4u : 3u);
+}
+
 // Whether a launch over planes takes 64-row tiles (ogm_gemm_dmx_kernel) instead of 128-row ones (ogm_gemm_dma_kernel).
 // interleave: 0 by the size of the launch, 1 never, 2 whenever the type allows.  Measured on MI355X, whole calls, us, 64-row /
 // 128-row / the best kernel without planes.
@@ -3203,11 +3225,9 @@ static uint32_t gemm_plane_wgs(const OgmGemmArgs &a, uint32_t rows) {
 //   At the lower end: Q6_K from 128 workgroups with two token tiles (4096 -> 4096 at 160 tokens 22.9 against 24.7, 14336 ->
 // 4096 61.6 / 66.2 for the small-batch kernel; below 4096 inputs, as Q6_K did before, from 160, or 128 with a nearly full last
 // tile or three tiles) and with a lone token tile when it is nearly full.  Q4_K / Q5_K with three token tiles from 160
-// workgroups (2048 -> 2048 at 512, 128 of them, 19.0 against 17.3), with two from 160 (4096 -> 6144 at 160 / 256 tokens
-// 28 / 29 against 38 / 37 for the medium-batch kernel, 2048 -> 8192 19 / 21 against 23 / 24, 5120 -> 5120 32 / 33 against 43 /
-// 44, 8192 -> 8192 51 / 60 against 71 / 74) or, beyond 160 tokens of rows of 4096 inputs and more, from 128 (4096 -> 4096 at
-// 160 / 256 27.7 / 28.4 against 27.5 / 31.1, 11008 -> 4096 60 / 64 against 66 / 73, 14336 -> 4096 78 / 82 against 80 / 91 for the
-// small-batch kernel); rows of fewer than 2048 inputs leave two token tiles to the kernels without planes.
+// workgroups (2048 -> 2048 at 512, 128 of them, 19.0 against 17.3), with two from 160, or from 128 over rows of 4096 inputs and
+// more, unless the small batches' kernel is through in few rounds (gemm_small_leads); rows of fewer than 2048 inputs leave two
+// token tiles to the kernels without planes.
 // for_small_batch: asked by gemm_small_batch, whether the launch is one this kernel takes ahead of the small batches.
 static bool gemm_interleaved(const OgmGemmArgs &a, bool for_small_batch = false) {
   const uint32_t nsb = a.in_dim / 256;
@@ -3223,7 +3243,7 @@ static bool gemm_interleaved(const OgmGemmArgs &a, bool for_small_batch = false)
     return (n_wg >= 160u && (tok_tiles >= 2u || a.n_tokens > 96u)) ||
            (n_wg >= 128u && (last > 96u || tok_tiles >= 3u || (tok_tiles == 2u && nsb >= 16u)));
   }
-  if (tok_tiles == 2u) return nsb >= 8u && (n_wg >= 160u || (n_wg >= 128u && nsb >= 16u && a.n_tokens > 160u));
+  if (tok_tiles == 2u) return nsb >= 8u && n_wg >= (nsb >= 16u ? 128u : 160u) && !gemm_small_leads(a);
   return tok_tiles >= 3u && n_wg >= 160u;
 }
 
@@ -3256,24 +3276,22 @@ static bool gemm_small_batch(const OgmGemmArgs &a, bool planes_possible) {
     return false;
   uint32_t tiles64_all = (a.out_dim + 63u) / 64u;
   for (uint32_t m = 0; m < a.n_extra; m++) tiles64_all += (a.extra_out_dim[m] + 63u) / 64u;
-  // Measured on MI355X with the activations in operand chunks, whole calls, us, small-batch against the best other
-  // kernel.  Q4_K: 4096 -> 4096 (64 tiles of 64 rows) at 128 / 192 / 256 / 384 tokens 20 / 30 / 32 / 41 against 33 / 33 /
-  // 34 / 40; 4096 -> 6144 (96 tiles) at 128 / 192 / 256: 29 / 38 / 43 against 33 / 37 / 38; 8192 -> 8192 (128 tiles) at
-  // 128 / 192: 54 / 76 against 57 / 70; 4096 -> 14336 (224 tiles) at 64 / 96 / 128: 31 / 42 / 48 against 37 / 38 / 39;
-  // 2048 -> 2048 (32 tiles) at 256 / 512: 14 / 23 against 20 / 22.  Rows of more than 8192 inputs, where the plane
-  // kernels' first pass weighs most and no medium-batch kernel runs: 14336 -> 4096 (64 tiles) at 192 / 256 / 384: 81 /
-  // 90 / 117 against 95 / 95 / 121; 14336 -> 5120 (80 tiles) at 192 / 256 / 384: 87 / 118 / 149 against 116 / 122 / 123;
-  // 14336 -> 8192 (128 tiles) at 128 / 192 / 256: 89 / 127 / 168 against 94 / 126 / 131.  Q6_K: 8192 -> 2048 (32 tiles)
-  // at 256 / 384 / 512: 32 / 48 / 50 against 47 / 50 / 51; 4096 -> 2048 at 384 / 512: 25 / 31 against 29 / 29; the
-  // launches of more tiles leave earlier for the 64-row plane kernel (gemm_interleaved).
-  const bool long_rows = q45 && nsb > 32u;   // no medium-batch kernel there, and a first pass in the plane kernels
+  // By tiles of 64 rows.  Whole calls, us, small-batch against the best other kernel without planes, Q4_K (Q5_K, Q6_K): 4096 ->
+  // 2048 (32 tiles) at 256 / 512 tokens 17.7 / 26.7 against 32.1 / 41.6 (18.9 / 27.4 against 36.9 / 43.6), Q6_K at 256 / 384 19.5 /
+  // 23.3 against 32.1 / 33.7, at 448 27.6 against the plane kernel's 24.7; 4096 -> 4096 (64) at 128 16.8 against 31.7 (18.6 / 36.6, 19.2 /
+  // 31.7); 4096 -> 6144 (96) at 128 23.7 against 31.9 (25.2 / 37.0, 23.9 / 32.0); 8192 -> 8192 (128) at 96 / 128 38.6 / 45.3 against
+  // 54.7 / 56.2 (41.6 / 49.8 against 64.6 / 66.0, Q6_K at 128 49.0 against the plane kernel's 38.4); 4096 -> 14336 (224) at 64 / 96 / 128
+  // 26.8 / 35.9 / 42.1 against 39.0 / 34.8 / 36.2 (28.9 / 40.3 / 46.7 against 40.5 / 38.9 / 40.2, 28.7 / 40.1 / 45.9 against 31.9 / 32.2 /
+  // 26.8).  Beyond 128 tokens 64-row tiles over planes come first where they can (gemm_interleaved, gemm_small_leads); without planes
+  // rows of more than 8192 inputs, which no medium-batch kernel takes, stay here: 14336 -> 5120 (80) at 160 / 256 72 / 88.
+  const bool long_rows = q45 && nsb > 32u;
   const uint32_t small_max = a.small_max_tokens ? a.small_max_tokens
                              : (tiles64_all <= 32u   ? (q45 ? 512u : 384u)
                                 : tiles64_all <= 64u ? 256u
                                 : tiles64_all <= 96u ? (long_rows ? 256u : 128u)
                                 : tiles64_all <= 128u ? 128u
                                                       : 64u);
-  return a.small_max_tokens != 1u && a.n_tokens <= small_max &&
+  return a.small_max_tokens != 1u && (a.n_tokens <= small_max || gemm_small_leads(a)) &&
          8u * 4096u + 128u * nsb <= GM_LDS_MAX;
 }
 
