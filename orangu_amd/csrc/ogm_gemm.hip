@@ -562,7 +562,7 @@ __global__ __launch_bounds__(256) void ogm_gemm_build_planes_kernel(GemmPlaneBui
   const uint32_t so = (s >> p.c_shift) * TILE_BYTES + ((s & ((1u << p.c_shift) - 1u)) << p.r_shift) * 16u;
   const uint8_t *u0 = p.wt + uo + so;
   const uint32_t h_ = g >> 1;
-  uint4 ql, qh = make_uint4(0, 0, 0, 0);
+  uint4 ql, qh = make_uint4(0, 0, 0, 0), hd = make_uint4(0, 0, 0, 0);
   int sc;
   short addc;   // the constant added to sc * q
   uint32_t shift_q = 0, mask_q, hi_shift = 0, hi_mask = 0, hi_lsh = 0;   // q = (ql >> shift_q) & mask_q | ((qh >> hi_shift) & hi_mask) << hi_lsh
@@ -571,6 +571,7 @@ __global__ __launch_bounds__(256) void ogm_gemm_build_planes_kernel(GemmPlaneBui
     ql = *(const uint4 *)(u0 + (2u + 2u * h_ + (t16 & 1u)) * 1024u);
     qh = *(const uint4 *)(u0 + (t16 & 1u) * 1024u);
     const uint4 scx = *(const uint4 *)(u0 + 6u * 1024u);
+    hd.x = scx.w;
     const uint32_t lw = (g & 1u) ? scx.y : scx.x;
     const uint32_t low = ((lw >> (8u * t16)) >> (g >= 2u ? 4u : 0u)) & 0xFu;
     const uint32_t high = ((scx.z >> (8u * t16)) >> (2u * g)) & 3u;
@@ -589,7 +590,7 @@ __global__ __launch_bounds__(256) void ogm_gemm_build_planes_kernel(GemmPlaneBui
     // the byte level + 128: u = ls (level + 128) + (128 - 128 ls)
     const uint32_t ib = 2u * g + (t16 >> 1);
     const uint4 pa = *(const uint4 *)(u0 + ib * 1024u), pb = *(const uint4 *)(u0 + (ib + 1u) * 1024u);
-    const uint4 hd = *(const uint4 *)u0;
+    hd = *(const uint4 *)u0;
     const uint32_t sh = hd.x >> 16, sl = hd.y, nsh = 4u * (t16 & 1u);
     ql = make_uint4(ogm_nib32_weights<2>((pa.z >> nsh) & 0x0F0F0F0Fu, 0u) ^ 0x80808080u,
                     ogm_nib32_weights<2>((pa.w >> nsh) & 0x0F0F0F0Fu, 0u) ^ 0x80808080u,
@@ -601,7 +602,7 @@ __global__ __launch_bounds__(256) void ogm_gemm_build_planes_kernel(GemmPlaneBui
   } else if constexpr (Q45) {
     ql = *(const uint4 *)(u0 + (QS_PIECE0 + 2u * g + (t16 & 1u)) * 1024u);
     if constexpr (Q5) qh = *(const uint4 *)(u0 + (1u + (t16 & 1u)) * 1024u);
-    const uint4 hd = *(const uint4 *)u0;
+    hd = *(const uint4 *)u0;
     uint32_t sc4a, sc4b;
     q4k_scales(hd, sc4a, sc4b);
     const uint32_t hi = t16 >> 1, j = 2u * g + hi;
@@ -616,6 +617,10 @@ __global__ __launch_bounds__(256) void ogm_gemm_build_planes_kernel(GemmPlaneBui
     ql = *(const uint4 *)(u0 + (4u * h_ + t16) * 1024u);
     qh = *(const uint4 *)(u0 + (8u + 2u * h_ + (t16 & 1u)) * 1024u);
     const uint4 scx = *(const uint4 *)(u0 + 12u * 1024u);
+    if (g == 0u && t16 == 0u) {   // d, two bytes a block behind the pieces
+      const uint32_t unit = ((s & ((1u << p.c_shift) - 1u)) << p.r_shift) + (row & ((1u << p.r_shift) - 1u));
+      hd.x = *(const uint16_t *)(u0 - unit * 16u + 13u * 1024u + unit * 2u);
+    }
     const uint32_t scw[4] = {scx.x, scx.y, scx.z, scx.w};
     sc = (int)(int8_t)((scw[g] >> (8u * t16)) & 0xFFu);
     addc = (short)(128 - 32 * sc);
@@ -646,30 +651,22 @@ __global__ __launch_bounds__(256) void ogm_gemm_build_planes_kernel(GemmPlaneBui
   uint8_t *dst = p.planes + gp_plane_offset(rb, p.nsb, s, g, t16, NPL) + r * 16u;
   *(uint4 *)dst = make_uint4(ph[0], ph[1], ph[2], ph[3]);
   if constexpr (!Q3) *(uint4 *)(dst + 1024u) = make_uint4(pl[0], pl[1], pl[2], pl[3]);
-}
-
-// What the plane kernels read of a block's header, in their order (gp_d_offset ..): a wave per 32 rows of a super-block.
-template <int KIND>
-__global__ __launch_bounds__(64) void ogm_gemm_build_side_kernel(GemmPlaneBuildParams p) {
-  constexpr bool Q3 = KIND == GP_Q3K, Q45 = KIND == GP_Q4K || KIND == GP_Q5K, Q6 = KIND == GP_Q6K, XS = KIND == GP_IQ4XS;
-  constexpr uint32_t TILE_BYTES = Q3 ? 7168u : (KIND == GP_Q4K || XS) ? 9216u : Q6 ? 13440u : 11264u;
-  constexpr uint32_t NPL = Q3 ? 1u : 2u;
-  const uint32_t lane = threadIdx.x, l32 = lane & 31u, lh = lane >> 5, b = blockIdx.x, s = blockIdx.y;
-  const uint32_t row = min(32u * b + l32, p.out_dim - 1u);   // rows past the matrix repeat its last one
-  const uint32_t r = row & ((1u << p.r_shift) - 1u), c = s & ((1u << p.c_shift) - 1u);
-  const uint8_t *tile = p.wt + ((size_t)(row >> p.r_shift) * p.nct + (s >> p.c_shift)) * TILE_BYTES;
-  const uint32_t unit = (c << p.r_shift) + r;   // this row's lane of the tile
-  const uint4 hd = *(const uint4 *)(tile + unit * 16u + (Q3 ? 6u * 1024u : 0u));
-  const uint32_t db = Q3 ? hd.w : Q6 ? *(const uint16_t *)(tile + 13u * 1024u + unit * 2u) : hd.x;
-  const float d = gm_f16_bits_to_f32(db & 0xFFFFu);
-  const uint32_t nrb = (p.out_dim + 63u) / 64u;
-  const size_t at = ((size_t)b * p.nsb + s) * 32u;
-  if (lh == 0u) ((float *)(p.planes + gp_d_offset(nrb, p.nsb, NPL)))[at + l32] = Q3 ? -d : d;
+  // What the kernels over planes read of a block's header, in their order (gp_d_offset ..), from the waves of the super-block's
+  // first two workgroups that hold it anyway.  (As a launch of its own 3 to 6 us a
+  // matrix: Q4_K 4096 -> 14336 31.2 + 6.2 us, here 30.6; Q6_K 33.4 + 4.7 / 34.6.)
+  const size_t at = ((size_t)(2u * rb + (r >> 5)) * p.nsb + s) * 32u;
+  if (g == 0u && t16 == 0u) {
+    const float d = gm_f16_bits_to_f32(hd.x & 0xFFFFu);
+    ((float *)(p.planes + gp_d_offset(gridDim.y, p.nsb, NPL)))[at + (r & 31u)] = Q3 ? -d : d;
+    if constexpr (Q45) ((float *)(p.planes + gp_dmin_offset(gridDim.y, p.nsb, NPL)))[at + (r & 31u)] = gm_f16_bits_to_f32(hd.x >> 16);
+  }
   if constexpr (Q45) {
-    if (lh == 0u) ((float *)(p.planes + gp_dmin_offset(nrb, p.nsb, NPL)))[at + l32] = gm_f16_bits_to_f32(hd.x >> 16);
-    uint32_t mna, mnb;
-    q4k_mins(hd, mna, mnb);
-    *(half8 *)(p.planes + gp_mins_offset(nrb, p.nsb, NPL) + at * 32u + lane * 16u) = side_operand(mna, mnb, lh ? 1.0f : 64.0f);
+    if (g == 1u && t16 < 2u) {   // half t16 of the operand
+      uint32_t mna, mnb;
+      q4k_mins(hd, mna, mnb);
+      *(half8 *)(p.planes + gp_mins_offset(gridDim.y, p.nsb, NPL) + at * 32u + (32u * t16 + (r & 31u)) * 16u) =
+          side_operand(mna, mnb, t16 ? 1.0f : 64.0f);
+    }
   }
 }
 
@@ -3167,11 +3164,8 @@ hipError_t ogm_gemm_build_planes(uint32_t ggml_type, const uint8_t *wt, uint32_t
   p.nct = tl.nct;
   const dim3 grid(4u * p.nsb, (out_dim + 63u) / 64u);
   if (grid.y > 65535u) return hipErrorInvalidValue;
-  const dim3 side(2u * grid.y, p.nsb);
-  if (side.y > 65535u) return hipErrorInvalidValue;
 #define GP_BUILD(K)                                                                              \
   hipLaunchKernelGGL(ogm_gemm_build_planes_kernel<K>, grid, dim3(256), 0, stream, p);            \
-  hipLaunchKernelGGL(ogm_gemm_build_side_kernel<K>, side, dim3(64), 0, stream, p);               \
   break
   switch (ggml_type) {
     case OGM_Q6_K: GP_BUILD(GP_Q6K);

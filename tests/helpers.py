@@ -182,10 +182,10 @@ def synth_x(n_tokens: int, in_dim: int, seed: int) -> np.ndarray:
     return rng.standard_normal((n_tokens, in_dim)).astype(np.float32)
 
 
-def captured_launches(stream, enqueue):
+def captured_launches(stream, enqueue, relaxed=False):
     """The kernels that `enqueue` puts on `stream` (a hipStream_t), in order, as (name, template arguments as mangled,
     workgroups, threads, bytes of private memory a lane): taken from a stream capture whose graph is never launched.  What `enqueue` allocates on first
-    use must be there already."""
+    use must be there already, unless the capture is relaxed (what it fills then never is)."""
     import ctypes as C
     import re
     from orangu_amd import hiprt
@@ -204,7 +204,7 @@ def captured_launches(stream, enqueue):
     L = hiprt.hip()
     L.hipKernelNameRefByPtr.restype = C.c_char_p
     s, graph, n = C.c_void_p(stream), C.c_void_p(), C.c_size_t()
-    hiprt.check(L.hipStreamBeginCapture(s, C.c_int(0)), "hipStreamBeginCapture")
+    hiprt.check(L.hipStreamBeginCapture(s, C.c_int(2 if relaxed else 0)), "hipStreamBeginCapture")
     try:
         enqueue()
     finally:

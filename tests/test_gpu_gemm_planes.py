@@ -5,9 +5,10 @@ only fetch), several matrices a launch, and scales whose product with dmin, form
 infinite or not a number.  Every bit of the CPU restatement."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
-from helpers import BLOCK, F16_FIELDS, IQ4_XS, Q3_K, Q4_K, Q5_K, Q6_K, TYPE_NAME, synth_weights, synth_x
+from helpers import BLOCK, F16_FIELDS, IQ4_XS, Q3_K, Q4_K, Q5_K, Q6_K, TYPE_NAME, captured_launches, synth_weights, synth_x
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +68,24 @@ def test_min_products(be, t, rows64):
     x[5, 7] = np.inf
     x[6, 9] = np.nan
     check(be, t, raw, 256 * nsb, out_dim, x, tokens, rows64)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K, IQ4_XS, Q3_K])
+def test_planes_are_one_launch(be, t):
+    """A matrix's first tiled call: the quantizer, one launch that builds all that the GEMM reads of the matrix, the GEMM."""
+    from orangu_amd import hiprt
+    in_dim, out_dim, tokens = 512, 200, 130
+    raw = synth_weights(t, in_dim, out_dim, seed=t)
+    first, second = (be.upload_raw(raw, t, in_dim, out_dim) for _ in range(2))
+    x, y = torch.ones(tokens, in_dim, device="cuda"), torch.empty(tokens, out_dim, device="cuda")
+    torch.cuda.synchronize()
+    stream = hiprt.Stream()
+    be.set_tuning("gemm_interleave", 1)
+    be.matmul_dev(first, x.data_ptr(), tokens, y.data_ptr(), False, stream.ptr)   # (allocates the scratch)
+    stream.synchronize()
+    ran = captured_launches(stream.ptr, lambda: be.matmul_dev(second, x.data_ptr(), tokens, y.data_ptr(), False, stream.ptr), relaxed=True)
+    be.free_weight(first)
+    be.free_weight(second)   # (its planes were never filled)
+    stream.destroy()
+    print(t, [k[0] for k in ran], flush=True)
+    assert [k[0] for k in ran[1:]] == ["ogm_gemm_build_planes_kernel", "ogm_gemm_dma_kernel"]
