@@ -524,6 +524,11 @@ int ogm_enqueue_repeated(ogm_ctx *ctx, int kind, const ogm_weight *const *ws, si
 size_t ogm_scratch_bytes(ogm_ctx *ctx);
 /* Name of the kernel the last matmul on this context launched (for profiles). */
 const char *ogm_last_kernel(ogm_ctx *ctx);
+/* The names (static strings) of the matmul kernels, plane builds and result copies that calls on this context have
+ * launched since the last ogm_kernels_run, oldest first: the newest `max` of the last OGM_KERNELS_RUN_MAX.  Returns
+ * how many were written (for tests: which route a whole call took). */
+#define OGM_KERNELS_RUN_MAX 256
+size_t ogm_kernels_run(ogm_ctx *ctx, const char **names, size_t max);
 
 #ifdef __cplusplus
 }

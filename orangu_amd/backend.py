@@ -370,6 +370,11 @@ class Mi355xBackend:
     def last_kernel(self) -> str:
         return self._lib.ogm_last_kernel(self._ctx).decode()
 
+    def kernels_run(self) -> list[str]:
+        """The matmul kernels, plane builds and result copies launched since the last call, oldest first (up to 256)."""
+        names = (C.c_char_p * 256)()
+        return [names[i].decode() for i in range(self._lib.ogm_kernels_run(self._ctx, names, 256))]
+
     def argmax(self, logits: np.ndarray) -> int:
         """sampling::argmax (engine/sampling.rs:336-343) on the device: the decode step's greedy pick."""
         logits = np.ascontiguousarray(logits, dtype=np.float32).reshape(-1)

@@ -82,6 +82,8 @@ struct ogm_ctx {
   int tune_plane_cache_mb = 32768;   // MiB the K-quant matrices' prefill planes may take in all
   size_t plane_bytes_used = 0;
   const char *last_kernel = "";
+  const char *ran[OGM_KERNELS_RUN_MAX];   // ogm_kernels_run
+  uint64_t n_ran = 0;
   uint8_t *static_scratch = nullptr;   // this device's copy of the library's static scratch array (ogm_static.hip)
   // what the activation buffer currently holds (ogm_act_quantize_dev)
   int act_mode = -1;
@@ -386,6 +388,19 @@ extern "C" size_t ogm_scratch_bytes(ogm_ctx *ctx) {
   return n;
 }
 
+static void note_run(ogm_ctx *ctx, const char *name) { ctx->ran[ctx->n_ran++ % OGM_KERNELS_RUN_MAX] = name; }
+
+extern "C" size_t ogm_kernels_run(ogm_ctx *ctx, const char **names, size_t max) {
+  if (!ctx) return 0;
+  std::lock_guard<std::mutex> lock(ctx->mu);
+  size_t n = ctx->n_ran < OGM_KERNELS_RUN_MAX ? (size_t)ctx->n_ran : (size_t)OGM_KERNELS_RUN_MAX;
+  if (!names) max = 0;
+  if (n > max) n = max;
+  for (size_t i = 0; i < n; i++) names[i] = ctx->ran[(ctx->n_ran - n + i) % OGM_KERNELS_RUN_MAX];
+  ctx->n_ran = 0;
+  return n;
+}
+
 extern "C" const char *ogm_last_kernel(ogm_ctx *ctx) {
   if (!ctx) return "";
   std::lock_guard<std::mutex> lock(ctx->mu);   // launches write it under the same lock
@@ -637,6 +652,7 @@ static OgmGemvArgs prepared_args(ogm_ctx *ctx, const Target *tg, size_t n_tg) {
 // Enqueues that launch; the quantized row also ends in the context's scratch.  The scratch is large enough.
 static int enqueue_prepared(ogm_ctx *ctx, const Target *tg, size_t n_tg, const OgmGemvSrc &src, hipStream_t stream) {
   HIPCHK(ctx, ogm_launch_gemv_fused(prepared_args(ctx, tg, n_tg), src, stream, &ctx->last_kernel));
+  note_run(ctx, ctx->last_kernel);
   return OGM_OK;
 }
 
@@ -726,6 +742,7 @@ static bool ensure_planes(ogm_ctx *ctx, const ogm_weight *cw, hipStream_t stream
     w->planes_refused = true;
     return false;
   }
+  note_run(ctx, "ogm_gemm_build_planes_kernel");
   w->planes = p;
   w->plane_bytes = bytes;
   ctx->plane_bytes_used += bytes;
@@ -777,6 +794,7 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
         g.y = tg[i].y;
         g.xh = nullptr;
         HIPCHK(ctx, ogm_launch_gemm_ft(g, gemm_order, stream, &ctx->last_kernel));
+        note_run(ctx, ctx->last_kernel);
       }
       return OGM_OK;
     }
@@ -829,6 +847,7 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
         a.extra_y[i - 1] = tg[g0 + i].y;
       }
       HIPCHK(ctx, ogm_launch_gemv_mma(a, stream, &ctx->last_kernel));
+      note_run(ctx, ctx->last_kernel);
     }
     return OGM_OK;
   }
@@ -900,6 +919,7 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
         }
       }
       HIPCHK(ctx, ogm_launch_gemm(g, stream, &ctx->last_kernel));
+      note_run(ctx, ctx->last_kernel);
       if (did_swiglu) *did_swiglu = g.swiglu;
     }
     if (planes_or_nothing) return OGM_OK;
@@ -930,6 +950,7 @@ static int enqueue_gemv(ogm_ctx *ctx, const Target *tg, size_t n_tg, uint32_t n_
         a.extra_y[i - 1] = tg[g0 + i].y + (size_t)t0 * tg[g0 + i].w->out_dim;
       }
       HIPCHK(ctx, ogm_launch_gemv(a, stream, &ctx->last_kernel));
+      note_run(ctx, ctx->last_kernel);
     }
   }
   return OGM_OK;
@@ -1045,6 +1066,7 @@ static int results_to_host(ogm_ctx *ctx, void *dst, const void *src, size_t byte
   auto launch = [&]() -> hipError_t {
     const size_t i = launched++, off = i * OGM_STAGE_HALF, nb = bytes - off < OGM_STAGE_HALF ? bytes - off : OGM_STAGE_HALF;
     const uint32_t epoch = epoch0 + 1 + (uint32_t)i;
+    note_run(ctx, "ogm_host_copy_kernel");
     return ogm_launch_host_copy((const uint8_t *)src + off, stage + (i & 1) * (size_t)OGM_STAGE_HALF, nb / 4, tail, stage_tail,
                                 i == 0 && tail_dst ? tail_bytes / 4 : 0, flags + (i & 1) * half_flags,
                                 ctx->tune_host_flag_wait == 2 ? epoch ^ 0x80000000u : epoch, s);
@@ -1869,6 +1891,7 @@ static int llama_norm_matmul(ogm_ctx *ctx, ogm_llama *m, DecodeRow &row, const f
     }
     if (both) {
       HIPCHK(ctx, ogm_launch_gemv_fused_pair(prepared_args(ctx, tg, e), prepared_args(ctx, tg2, n - e), src, s, &ctx->last_kernel));
+      note_run(ctx, ctx->last_kernel);
     } else {
       if ((rc = enqueue_prepared(ctx, tg, e, src, s)) != OGM_OK) return rc;
       if (e < n && (rc = llama_matmul(ctx, ws + e, ys + e, n - e, s)) != OGM_OK) return rc;

@@ -48,11 +48,17 @@ def test_results_arrive_whole(be, n_vocab, n_tokens):
     x = rng.standard_normal((n_tokens, 256)).astype(f32)
     try:
         be.set_tuning("host_flag_wait", 0)
+        be.kernels_run()
         want = results(be, dev, x, n_vocab)
+        assert "ogm_host_copy_kernel" not in be.kernels_run()
         for wait in (1, 1, 2):
             be.set_tuning("host_flag_wait", wait)
+            be.kernels_run()
             got = results(be, dev, x, n_vocab)
             assert [g == w for g, w in zip(got, want)] == [True] * len(want), wait
+            # the copies by kernel: of 2 MiB at most, from 16 KiB of pageable memory on (two steps, a batch, a prompt, the states)
+            sizes = [n_vocab, n_vocab, n_vocab * n_tokens, n_vocab, 256 * n_tokens]
+            assert be.kernels_run().count("ogm_host_copy_kernel") == sum(-(-n // 524288) for n in sizes if n >= 4096), wait
     finally:
         be.set_tuning("host_flag_wait", 1)
         dev.close()
@@ -69,7 +75,9 @@ def test_wide_hidden_states_take_their_pieces_in_turn(be):
         be.set_tuning("host_flag_wait", 1)
         for rep in range(70):      # past the call that synchronizes after 256 polled ones
             for a, w in zip(x, want):
+                be.kernels_run()
                 assert dev.hidden_states(a).tobytes() == w, (rep, len(a))
+                assert be.kernels_run().count("ogm_host_copy_kernel") == -(-a.size // 524288)
     finally:
         be.set_tuning("host_flag_wait", 1)
         dev.close()

@@ -20,11 +20,17 @@ def be():
     b.close()
 
 
-def hidden(be, dev, x, **tuning):
+def hidden(be, dev, x, one_launch, **tuning):
+    """The hidden states, and that both layers' gate and up ran as one launch (or neither's)."""
     try:
         for k, v in tuning.items():
             be.set_tuning(k, v)
-        return dev.hidden_states(x)
+        be.kernels_run()
+        states = dev.hidden_states(x)
+        ran = be.kernels_run()
+        print(ran, flush=True)
+        assert ran.count("ogm_gemm_swiglu_kernel") == (2 if one_launch else 0)
+        return states
     finally:
         for k in KEYS:
             be.set_tuning(k, 0)
@@ -39,8 +45,8 @@ def test_one_launch_leaves_the_product(be, gate, down, n_embd, n_ff, n_tokens):
                           types=(gate, Q8_0, down, Q8_0), max_ctx=n_tokens + 4, seed=n_ff + n_tokens)
     x = rng.standard_normal((n_tokens, n_embd)).astype(f32)
     try:
-        got = hidden(be, dev, x, gemm_plane_kernel=2, gemm_small_max_tokens=1, gemm_interleave=1)
-        want = hidden(be, dev, x, gemm_plane_kernel=0 if gate == Q3_K else 2, gemm_small_max_tokens=1, gemm_interleave=2)
+        got = hidden(be, dev, x, True, gemm_plane_kernel=2, gemm_small_max_tokens=1, gemm_interleave=1)
+        want = hidden(be, dev, x, False, gemm_plane_kernel=0 if gate == Q3_K else 2, gemm_small_max_tokens=1, gemm_interleave=2)
         assert np.isfinite(want).all() and np.array_equal(got.view(np.uint32), want.view(np.uint32))
     finally:
         dev.close()
@@ -52,7 +58,7 @@ def test_by_size(be):
                           types=(Q4_K, Q6_K, Q6_K, Q6_K), max_ctx=1104, seed=3)
     x = rng.standard_normal((1100, 512)).astype(f32)
     try:
-        got, want = hidden(be, dev, x), hidden(be, dev, x, gemm_interleave=2)
+        got, want = hidden(be, dev, x, True), hidden(be, dev, x, False, gemm_interleave=2)
         assert np.isfinite(want).all() and np.array_equal(got.view(np.uint32), want.view(np.uint32))
     finally:
         dev.close()
