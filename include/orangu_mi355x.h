@@ -422,11 +422,13 @@ int ogm_llama_load_gguf(ogm_ctx *ctx, ogm_gguf *g, uint32_t max_ctx, ogm_llama *
  *                              GEMM's float order
  *   "gemm_small_max_tokens"    GEMMs of at most this many tokens take the small-batch kernel of their type, whose
  *                              waves work on different super-blocks (blocks, for the per-32 types: by default
- *                              while the launch has at most 1792 workgroups of 32 rows x 32 tokens) of the same rows; 0 = default (K-quants: 64, more
+ *                              while the launch has at most 1024 workgroups of 32 rows x 32 tokens for Q8_0, 1280 for
+ *                              Q4_0, 1408 for Q5_0 and IQ4_NL) of the same rows; 0 = default (K-quants: 64, more
  *                              for matrices of few rows: 128 up to 8192 rows, 256 up to 4096 -- and up to 6144
  *                              for Q4_K / Q5_K rows of more than 8192 inputs --, 384 up to 2048, 512 there for
- *                              Q4_K / Q5_K; Q6_K launches that "gemm_interleave" sends to its kernel by their size
- *                              go there first), 1 = never
+ *                              Q4_K / Q5_K; launches that "gemm_interleave" sends to its kernel by their size go
+ *                              there first, but for Q4_K / Q5_K at 129 to 256 tokens of rows of 4096 inputs and more
+ *                              with at most 768 workgroups, Q4_K from 6144 inputs on 1024), 1 = never
  *   "gemm_act_chunks"          whether a K-quant batch's int8 activations are also written in the operand order
  *                              of the matrix-core kernels (1 KiB chunks of 32 tokens x 32 inputs; the small-batch
  *                              kernels then load a chunk in one piece instead of gathering 32 rows, the plane
@@ -444,7 +446,8 @@ int ogm_llama_load_gguf(ogm_ctx *ctx, ogm_gguf *g, uint32_t max_ctx, ogm_llama *
  *                              -1 = never
  *   "gemm_plane_cache_mb"      device memory, in MiB, that the K-quant and IQ4_XS matrices' prefill planes may take
  *                              in all (default 32768): on a matrix's first GEMM that would read them its scale-folded
- *                              int8 planes (2 bytes per weight, 1 for Q3_K) are built once and kept; a matrix
+ *                              int8 planes, with its rows' scales (2.02 bytes per weight, Q4_K and Q5_K 2.16, Q3_K
+ *                              1.02), are built once and kept; a matrix
  *                              that does not fit, and every matrix at 0, is unpacked on every call (IQ4_XS, whose
  *                              GEMM kernels beyond its small batches read planes, then stays on the GEMV kernel);
  *                              ogm_weight_download is unaffected
@@ -456,13 +459,15 @@ int ogm_llama_load_gguf(ogm_ctx *ctx, ogm_gguf *g, uint32_t max_ctx, ogm_llama *
  *                              128-row tiles leave silu(gate) * up in one launch
  *   "gemm_interleave"          the plane kernel with 64-row tiles (Q4_K, Q5_K, Q6_K, IQ4_XS): 0 = default, on launches
  *                              of at most 512 tiles of 64 rows x 128 tokens (256 for Q4_K / Q5_K rows of 4096 inputs and
- *                              more) and, by type and token tiles, at least 128 to 160 (their planes are built then);
+ *                              more) and, by type and token tiles, at least 128 to 160 (their planes are built then;
+ *                              two token tiles of Q4_K / Q5_K: see "gemm_small_max_tokens");
  *                              1 = never; 2 = wherever the plane kernel runs.  Same bits
  *   "gemm_one_pass"            0 = default.  1: Q4_K and Q5_K on that kernel skip the reference GEMM's separate
  *                              first pass over the mins (vecdot.rs:2229-2240) and add
  *                              ad * (d * isum - dmin * imin) per super-block, the single-token expression of
  *                              vecdot.rs:3152-3178.  The integer sums are the same; the f32 result is within
- *                              rounding of the reference GEMM's, not its bits: an output whose terms cancel to
+ *                              rounding of the reference GEMM's, not its bits (2 to 4 % faster at 4096 inputs, 10 %
+ *                              slower at 14336): an output whose terms cancel to
  *                              near zero can differ from the reference's by more than 1e-3 of itself
  *   "gemv_mma"                 2 to 16 tokens over Q4_K / Q5_K / Q6_K rows on the kernel
  *                              that gives a workgroup one row block and multiplies on the matrix cores: 1 =

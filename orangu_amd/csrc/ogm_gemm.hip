@@ -11,8 +11,9 @@
 // Kernels, by the size of the launch (ogm_launch_gemm at the end of the file):
 //   * gemm_sb_*: small batches, 32 rows x 32 tokens per workgroup, its waves on different super-blocks;
 //   * gemm_q6k_i8_body: 128 (64) rows x 128 tokens, feeding waves unpack per call, as many multiply;
-//   * ogm_gemm_dma_kernel: the same tile over planes built once per matrix, all waves multiply;
-//   * ogm_gemm_flat_kernel: the per-32 types (f16 operands, one block per accumulator).
+//   * gemm_planes_body: 128 (64) rows x 128 tokens over planes built once per matrix, all waves multiply;
+//   * ogm_gemm_flat_kernel: the per-32 types on int8 operands, one block per accumulator (ogm_gemm_flat_f16_kernel: the
+//     nibble types' largest launches, on f16 operands).
 #include <hip/hip_runtime.h>
 #include <type_traits>
 
@@ -87,8 +88,8 @@ struct GemmI8pParams {
   uint32_t extra_out_dim[OGM_GEMM_MAX_MATS - 1];
 };
 
-// The planes of a matrix, built once and kept beside its tile-planar bytes (2 bytes per weight; 1
-// for Q3_K): what the feeding waves of the kernels below otherwise recompute on every call.  Row
+// The planes of a matrix, built once and kept beside its tile-planar bytes (2 bytes per weight, 1
+// for Q3_K; with what lies behind them 2.02, 1.02 and for Q4_K and Q5_K 2.16): what the feeding waves of the kernels below otherwise recompute on every call.  Row
 // blocks of 64 rows; for row block rb, super-block s, stage g (64 weights), group t (16 weights):
 // 64 rows x 16 bytes of plane h, then (two-plane types) 64 rows x 16 bytes of plane l -- one
 // feeding wave's share of a stage is one contiguous run of 1 or 2 KiB.
@@ -731,7 +732,6 @@ __device__ __forceinline__ void gd_dma4(const uint8_t *src, uint8_t *lds_chunk) 
 // LDS reads the compiler does not see, and the waits that go with them.  A wait names the
 // registers it makes valid, so that their uses stay behind it.
 #define GD_READ16(DST, ADDR, OFF) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(DST) : "v"(ADDR), "n"(OFF))
-#define GD_READ4(DST, ADDR, OFF) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(DST) : "v"(ADDR), "n"(OFF))
 #define GD_WAIT1(N, A) asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(A) : "n"(N))
 #define GD_WAIT2(N, A, B) asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(A), "+v"(B) : "n"(N))
 // all loads of this wave but the newest N have landed; then the workgroup's barrier (no fence: the
@@ -964,10 +964,11 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_onepass_kernel(GemmDma
 // The K-quant GEMMs over planes in the reference's float order: 128-row tiles (ogm_gemm_dma_kernel) for launches that fill
 // the device with them, 64-row tiles (ogm_gemm_dmx_kernel) for smaller ones.
 //
-// What bounds them on this card is power as much as any one unit: eight matrix instructions with five vector instructions
-// behind each take 1.02 times the cycles of the matrix instructions alone (two waves a SIMD), but at 1.71 GHz instead of
-// 1.89; a launch of 4096 -> 14336 at 2048 tokens runs at 1.9 GHz with the matrix pipe busy for half of its 521 k cycles.
-// So what counts is instructions and bytes moved, not only what overlaps:
+// A launch of 4096 -> 14336 at 2048 tokens keeps the matrix pipe busy for half of its 521 k cycles at 1.9 GHz.  What the other half
+// waits for has not been measured part by part.  It isn't the vector work behind the matrix instructions: eight of these with five
+// dependent vector instructions behind each take 1.02 times the cycles of the matrix instructions alone (two waves a SIMD), at 1.71
+// GHz instead of 1.89.  What the rewrite from one wave tile a step to this form changed, and what it gained, was instructions and
+// bytes moved:
 //   * a wave multiplies one token block of 32 with every row block of its tile.  The block's operand chunks of a
 //     super-block stay in 32 registers for all of them (loaded a super-block ahead, straight from memory) and only the
 //     weights go through LDS: 16 KiB a super-block and row block, one piece, shared by the four waves;
@@ -982,7 +983,9 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_onepass_kernel(GemmDma
 // Whole calls, us, against the kernels these replaced (a wave 32 rows x 128 or 64 tokens with both operands through LDS step
 // by step, a barrier per 32 k): Q4_K 4096 -> 2 x 14336 at 512 tokens 175 -> 164, 4096 -> 14336 at 2048 315 -> 294, 2048 ->
 // 2 x 8192 at 1901 174 -> 162; 64-row tiles: 4096 -> 4096 at 512 38.9 -> 32.9, 14336 -> 4096 112 -> 97, Q6_K 14336 -> 4096
-// 89 -> 83.  Where the device is full the 128-row tiles lead (4096 -> 2 x 14336 at 512: 164 against 184, they fetch 6 KiB per
+// 89 -> 83; all five types at 512 / 2048 tokens of 4096 -> 14336, and 14336 -> 4096 at 512: Q4_K 84.7 -> 78.2, 306 -> 291, 110.5 ->
+// 93.5, Q5_K 85.6 -> 78.7, 306 -> 291, 110.6 -> 94.4, Q6_K 74.4 -> 71.8, 264 -> 257, 88.2 -> 82.0, IQ4_XS 74.6 -> 72.2, 266 -> 257,
+// 88.8 -> 82.1, Q3_K 56.4 -> 51.4, 183 -> 164.  Where the device is full the 128-row tiles lead (4096 -> 2 x 14336 at 512: 164 against 184, they fetch 6 KiB per
 // 32 x 32 x 256 products, not 8), on one workgroup a compute unit the 64-row ones (4096 -> 4096 at 512: 33 against 46).
 // Eight waves and 256 tokens a workgroup fetch less still (4 KiB) but stand at one barrier: 164 and 308.
 //
@@ -991,7 +994,8 @@ __global__ __launch_bounds__(64 * GD_NW, 2) void ogm_gemm_onepass_kernel(GemmDma
 //              others at a barrier, and fetches piece p + 3 into the slot piece p - 1 left
 //   tables     per super-block the tokens' ad and the rows' d, four slots, fetched a super-block ahead
 //   LDS reads  a step's two operand chunks and two ad, issued three steps ahead, waited for by count
-// Registers: 16 RB of y, 64 of the plane sums, 64 of x, 32 of weights: 247 of a wave's 256 at RB = 4.
+// Registers: 16 RB of y, 64 of the plane sums, 64 of x, 32 of weights: 246 of a wave's 256 at RB = 4 (Q3_K 198; Q4_K and Q5_K
+// with their first pass all of them, and one spilled outside the loops), 216 at RB = 2.
 #define GB_PIN() __builtin_amdgcn_sched_barrier(0)
 #define GB_SYNC(N) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory")
 typedef float float2v __attribute__((ext_vector_type(2)));
@@ -1952,8 +1956,8 @@ __global__ __launch_bounds__(512) void ogm_gemm_sb_q2k_kernel(GemmSbParams p) {
 
 // The same for Q4_K and Q5_K (gemm_k_q4_k, vecdot.rs:2213-2303): first a sweep over the super-blocks
 // for the terms (ad * dmin) * imin, which the reference subtracts before anything else (rounds of
-// sixteen super-blocks, two per wave: header and the quantizer's sums per 32 only, one f16 matrix
-// instruction each), then the sweep of the products as above.  A lane's 16 weights of sub-block j
+// NW super-blocks, one per wave: header and the quantizer's sums per 32 only, one f16 matrix
+// instruction), then the sweep of the products as above.  A lane's 16 weights of sub-block j
 // are the low (j even) or high nibbles of one 16-byte piece of qs, Q5_K's fifth bit is bit j of
 // its piece of qh.
 // AHEAD: a round's loads -- header and sums in the first sweep, the eight operand chunks of the activations in the second --
@@ -2443,7 +2447,7 @@ __device__ __forceinline__ half8 gw_i8_to_f16(uint32_t w0, uint32_t w1) {
 }
 
 // ------------------------------------------------------------------------------------------
-// The symmetric per-32 types (Q8_0, Q5_0, Q4_0, IQ4_NL): the flat-activation GEMM
+// The symmetric nibble types (Q5_0, Q4_0, IQ4_NL), launches that fill the device: the flat-activation GEMM
 // (dot_flat_pair, engine/vecdot.rs:2598-2629): acc += (ad * dw) * dot32 per 32-block.
 //
 // A block's integer dot is exact on the matrix cores: weights and activations are int8 values as
@@ -2453,7 +2457,7 @@ __device__ __forceinline__ half8 gw_i8_to_f16(uint32_t w0, uint32_t w1) {
 // 174 k cycles of vector instructions and 86 k of matrix instructions in the 266 k a SIMD has work for -- so the sum
 // is what counted.  Hence the scales' products ad * dw come from an outer product (one v_mfma_f32_32x32x1_2b for 64
 // rows x 32 tokens, 32 cycles a 32 x 32 block where sixteen multiplies take 64) and the activations become f16 once,
-// in the feeding waves, instead of in each of the multiplying ones: 149 -> 130 us (Q4_0) and 157 -> 133 (Q8_0).
+// in the feeding waves, instead of in each of the multiplying ones: 149 -> 130 us (Q4_0).
 // Interleaving the f32 step with the next block's matrix instructions, operands fetched a block ahead, 64 x 64 outputs
 // a wave: no faster (132 to 155), for a reason that is not known.
 //
@@ -2466,7 +2470,7 @@ struct GemmFlatParams {
   const int8_t *xq;       // [T][in_dim] int8 activations
   const float *ad;        // [T][in_dim / 32] activation scales
   float *y;               // [T][out_dim]
-  uint32_t in_dim, out_dim, n_tokens, nblk;   // nblk = in_dim / 32 (even)
+  uint32_t in_dim, out_dim, n_tokens, nblk;   // nblk = in_dim / 32 (even for ogm_gemm_flat_f16_kernel)
   uint32_t c_shift, r_shift, nct;             // tiles of R = 1 << r_shift rows x C = 1 << c_shift blocks
 };
 
@@ -3568,7 +3572,6 @@ hipError_t ogm_launch_gemm(const OgmGemmArgs &a, hipStream_t stream, const char 
     if (!a.xt_ready)
       hipLaunchKernelGGL(ogm_gemm_xtile_kernel, dim3(a.in_dim / 128u, t_pad / 32u), dim3(256), 0, stream, a.act.q,
                          (int8_t *)a.xh, a.in_dim, a.n_tokens);
-    // the kernel that adds a super-block up between the next one's matrix instructions (64-row tiles)
     const bool interleaved = gemm_interleaved(a);
     GemmDmaParams d;
     d.wt = a.wt;

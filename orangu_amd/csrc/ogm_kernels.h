@@ -100,7 +100,7 @@ struct OgmGemmArgs {
   // when that kernel runs: 0 when the grid fills the device twice (else the feeding waves unpack), 2 whatever
   // the grid
   uint32_t plane_kernel = 0;
-  uint32_t interleave = 0;   // the plane kernel with 64-row tiles that adds a super-block up between the next one's matrix instructions: 0 by the size of the launch, 1 never, 2 whenever it can
+  uint32_t interleave = 0;   // 64-row tiles over planes: 0 by the size of the launch, 1 never, 2 whenever it can
   bool swiglu = false;     // the two matrices are gate and up: y gets silu(gate) * up, extra_y is not written (ogm_gemm_does_swiglu)
   uint32_t one_pass = 0;   // Q4_K / Q5_K on the all-waves-multiply kernel: fold the min pass into the super-block step (f32 to rounding, not to the bit)
 };
@@ -111,7 +111,7 @@ bool ogm_gemm_does_swiglu(const OgmGemmArgs &a);
 // Whether this K-quant or IQ4_XS launch would run the small-batch kernel of its type (which needs no planes).
 bool ogm_gemm_takes_small_batch(const OgmGemmArgs &a);
 // Bytes of a K-quant matrix's planes (0: the type has none), and the kernel that builds them from
-// the tile-planar bytes (2 bytes per weight, 1 for Q3_K; rows padded to a multiple of 64).
+// the tile-planar bytes (2.02 bytes per weight, Q4_K and Q5_K 2.16, Q3_K 1.02; rows padded to a multiple of 64).
 size_t ogm_gemm_plane_bytes(uint32_t ggml_type, uint32_t in_dim, uint32_t out_dim);
 hipError_t ogm_gemm_build_planes(uint32_t ggml_type, const uint8_t *wt, uint32_t in_dim, uint32_t out_dim,
                                  uint8_t *planes, hipStream_t stream);
