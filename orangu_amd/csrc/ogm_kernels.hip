@@ -1377,26 +1377,27 @@ __device__ __forceinline__ void gemv_fused_body(const GemvFusedParams &fp, const
   a.d = l_d;
   a.upr = upr;
   float *my_term = l_term + (size_t)team * term_stride;
-  auto tiles = [&](size_t tile, float *term) {
-    for (; it < nct; it += tw) {
-      const uint32_t col_own = it * C + c_local;
-      const bool live = col_own < upr;
-      const uint32_t col = live ? col_own : upr - 1u;
-      int isum, imin;
-      F::template sums<UPR>(cur, a, col, isum, imin);
-      if (live) term[col * R + r_local] = F::term_gemv(cur, a.d[col], isum, imin);
-      if (it + tw < nct) F::load(cur, wt, tile + it + tw, lane);
-    }
-  };
-  tiles(tile0, my_term);
-  // SWIGLU, R <= 32: the first wave adds gate and up of a row up, one in each half
-  auto product = [&](uint32_t rb, const float *term) {
-    const uint32_t t = lane / R, r = lane - t * R, orow = rb * R + r;
-    const bool have = t < 2u && orow < out_dim;
-    const float acc = have ? ordered_sum<false>(0.0f, term + (size_t)t * term_stride + r, upr, R) : 0.0f;
-    const float up = __shfl(acc, (int)((lane + R) & 63u));
-    if (have && t == 0u) y[orow] = acc / (1.0f + expf(-acc)) * up;
-  };
+  // Text and not lambdas: through a lambda's references the kernels with one row block compile to
+  // other code than with the loop written here, and that is slower where it counts (one token, Q4_K,
+  // 4096 to 1024 / 4096 / 7600 rows: 3.09 / 3.23 / 3.97 us, so 2.98 / 3.08 / 3.85; IQ4_XS 4.02 / 4.12
+  // / 6.17, so 3.89 / 4.00 / 6.04; Q5_K, Q2_K and the 32-value blocks 0 to 2 % the other way).
+#define OGM_FUSED_TILES(TILE, TERM)   /* this wave's tiles of the row block whose first is TILE */ \
+  for (; it < nct; it += tw) {                                                                    \
+    const uint32_t col_own = it * C + c_local;                                                    \
+    const bool live = col_own < upr;                                                              \
+    const uint32_t col = live ? col_own : upr - 1u;                                               \
+    int isum, imin;                                                                               \
+    F::template sums<UPR>(cur, a, col, isum, imin);                                               \
+    if (live) (TERM)[col * R + r_local] = F::term_gemv(cur, a.d[col], isum, imin);                \
+    if (it + tw < nct) F::load(cur, wt, (TILE) + it + tw, lane);                                  \
+  }
+#define OGM_FUSED_PRODUCT(RB, TERM)   /* R <= 32: a wave adds gate and up of a row up, one in each half */                     \
+  const uint32_t t = lane / R, r = lane - t * R, orow = (RB) * R + r;                                                          \
+  const bool have = t < 2u && orow < out_dim;                                                                                  \
+  const float acc = have ? ordered_sum<false>(0.0f, (TERM) + (size_t)t * term_stride + r, upr, R) : 0.0f;                      \
+  const float up = __shfl(acc, (int)((lane + R) & 63u));                                                                       \
+  if (have && t == 0u) y[orow] = acc / (1.0f + expf(-acc)) * up;
+  OGM_FUSED_TILES(tile0, my_term)
   if constexpr (NB == 2) {
     static_assert(SWIGLU, "a second row block of gate and up");
     const uint32_t rb1 = rb0 + gridDim.x;
@@ -1406,22 +1407,28 @@ __device__ __forceinline__ void gemv_fused_body(const GemvFusedParams &fp, const
     F::load(cur, wt, tile1 + it, lane);   // its first tile, under way over the first block's sum
     __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
-    if (wave == 0u) product(rb0, l_term);
+    if (wave == 0u) {
+      OGM_FUSED_PRODUCT(rb0, l_term)
+    }
     if (!more) return;
-    tiles(tile1, my_term + 2u * term_stride);
+    OGM_FUSED_TILES(tile1, my_term + 2u * term_stride)
     __syncthreads();
-    if (wave == 0u) product(rb1, l_term + 2u * term_stride);
+    if (wave != 0u) return;
+    OGM_FUSED_PRODUCT(rb1, l_term + 2u * term_stride)
     return;
   }
   __syncthreads();
 
   if constexpr (SWIGLU) {
-    if (wave == 0u) product(rb0, l_term);
+    if (wave != 0u) return;
+    OGM_FUSED_PRODUCT(rb0, l_term)
   } else {   // a team's first wave adds its row block up
     if (wv != 0u || !mine) return;
     const uint32_t orow = rb0 * R + lane;
     if (lane < R && orow < out_dim) y[orow] = ordered_sum<false>(0.0f, my_term + lane, upr, R);
   }
+#undef OGM_FUSED_TILES
+#undef OGM_FUSED_PRODUCT
 }
 
 template <class F, int UPR, int PRE, int NQ, int NB, bool SWIGLU>
