@@ -1735,14 +1735,14 @@ static hipError_t launch_fused_t(const OgmGemvArgs &a, const OgmGemvSrc &src, hi
     // workgroups than run at once (eight waves of 82 to 118 registers: two a compute unit, 512): from 769 to 1024 row blocks.  Two
     // layers of a decode step, 4096 / n_ff, us, one block / two:
     //            10752 (672)     12288 (768)     12800 (800)     14336 (896)     16384 (1024)
-    //   Q4_K     92.8 /  93.5    92.6 /  91.2    95.3 /  92.1    95.1 /  92.3    99.6 /  97.0
-    //   Q5_K     97.8 / 100.1   100.8 / 101.2   105.6 / 102.1   105.5 / 102.3   111.3 / 107.8
-    //   Q6_K    105.5 / 110.0   109.1 / 111.6   115.6 / 112.7   115.1 / 112.9   121.8 / 120.0
-    //   Q3_K     90.5 /  94.0    92.0 /  95.0    96.7 /  95.5    95.5 /  94.4    99.4 /  98.4
-    //   Q2_K     79.4 /  82.6    81.4 /  81.8    86.8 /  82.1    85.7 /  80.7    88.5 /  86.7
-    //   IQ4_XS  106.4 / 108.4   108.6 / 109.2   113.9 / 110.0   113.7 / 109.8   117.9 / 116.7
-    // (513 to 640: 3 to 7 % of the step slower with two.)  Q4_K already where one each nearly fill the third place of every compute
-    // unit: 11776 (736) 94.6 / 95.6, 12032 (752) 97.1 / 96.0.  Only for rows of 4096 inputs: launches of other lengths end, at 4096 row
+    //   Q4_K    88.0 /  89.4    92.8 /  90.3    94.5 /  90.2    94.0 /  89.4    98.8 /  94.9
+    //   Q5_K    97.2 /  99.2   100.1 / 100.3   105.3 / 101.1   105.0 / 101.1   110.8 / 107.2
+    //   Q6_K   104.8 / 109.2   108.2 / 110.9   115.3 / 112.1   114.6 / 112.3   121.0 / 119.3
+    //   Q3_K    89.4 /  94.3    91.3 /  94.9    96.1 /  95.2    95.1 /  94.0    99.1 /  97.9
+    //   Q2_K    79.0 /  80.9    80.8 /  81.8    84.9 /  82.8    84.0 /  81.2    87.2 /  86.6
+    //   IQ4_XS 105.8 / 108.2   108.2 / 108.8   113.6 / 109.7   113.6 / 109.7   117.5 / 116.5
+    // (640: 2 to 6 % of the step slower with two.)  Q4_K already where one each nearly fill the third place of every compute
+    // unit: 11776 (736) 90.4 / 90.4, 12032 (752) 92.2 / 90.3.  Only for rows of 4096 inputs: launches of other lengths end, at 4096 row
     // blocks x runs, with what runs at once or, three tiles a row, a third more.
     const dim3 g2((g.x + 1u) / 2u);
     const size_t lds2 = f.lds + (size_t)f.teams * p.upr * (64u / p.C) * 4u;
